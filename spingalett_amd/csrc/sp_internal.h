@@ -49,6 +49,10 @@ void  sp_log(LogLevel level, const char *fmt, ...) __attribute__((format(printf,
 void *sp_aligned_calloc(size_t count, size_t elem_size);
 void  sp_aligned_free(void *p);
 ComputeMode sp_resolve_compute_mode(void);
+#define SP_MAX_THREADS 8u
+/* fn over [0, count) in parts that begin at multiples of 64, on up to SP_MAX_THREADS threads (the caller's among
+ * them); `part` numbers them from 0.  Short ranges stay on the calling thread. */
+void  sp_parallel(size_t count, void (*fn)(void *ctx, unsigned part, size_t begin, size_t end), void *ctx);
 extern const char *const sp_act_names[];
 extern const char *const sp_loss_names[];
 extern const char *const sp_init_names[];
@@ -64,7 +68,6 @@ size_t sp_array_bytes(uint64_t n, PrecisionMode p);
 /* decodes one serialized array to FP32; returns false if `avail` is too small */
 bool   sp_decode_array(const uint8_t *src, size_t avail, uint32_t n, PrecisionMode p,
                        SpingalettDequantMode mode, float *dst);
-size_t sp_encode_array(const float *src, uint32_t n, PrecisionMode p, uint8_t *dst);
 void   sp_drop_packed(sp_net *sn);
 
 /* Spingalett.HIP.c */

@@ -6,6 +6,8 @@
 #define _GNU_SOURCE
 #include "sp_internal.h"
 
+#include <pthread.h>
+#include <sched.h>
 #include <stdarg.h>
 #include <stdatomic.h>
 #include <stdio.h>
@@ -57,7 +59,7 @@ void spingalett_set_compute_mode(ComputeMode mode)
 }
 
 unsigned spingalett_get_num_threads(void) { return atomic_load(&g_threads); }
-void spingalett_set_num_threads(unsigned n) { atomic_store(&g_threads, n); }   /* no host threads here */
+void spingalett_set_num_threads(unsigned n) { atomic_store(&g_threads, n); }   /* bounds sp_parallel(); 0: its own choice */
 void spingalett_set_log_callback(LogCallback cb) { atomic_store(&g_log_cb, cb); }
 void spingalett_set_log_level(LogLevel level) { atomic_store(&g_log_level, (int)level); }
 void spingalett_set_verbose(bool enabled) { atomic_store(&g_verbose, enabled); }
@@ -97,6 +99,55 @@ ComputeMode sp_resolve_compute_mode(void)
     return COMPUTE_HIP;
 }
 
+/* ---- elementwise host work on a few threads ----
+ * A thread costs about as much to start and join as THREAD_GRAIN elements take on one core, hence the grain. */
+#define THREAD_GRAIN ((size_t)1 << 19)
+
+typedef struct {
+    void (*fn)(void *, unsigned, size_t, size_t);
+    void *ctx;
+    unsigned part;
+    size_t begin, end;
+} parallel_part;
+
+static void *parallel_main(void *arg)
+{
+    const parallel_part *p = (const parallel_part *)arg;
+    p->fn(p->ctx, p->part, p->begin, p->end);
+    return NULL;
+}
+
+void sp_parallel(size_t count, void (*fn)(void *ctx, unsigned part, size_t begin, size_t end), void *ctx)
+{
+    size_t parts = count / THREAD_GRAIN;
+    if (parts > SP_MAX_THREADS) parts = SP_MAX_THREADS;
+    if (parts > 1u) {
+        const unsigned asked = spingalett_get_num_threads();
+        cpu_set_t set;
+        const int cpus = sched_getaffinity(0, sizeof set, &set) == 0 ? CPU_COUNT(&set) : 1;
+        if (parts > (size_t)cpus) parts = (size_t)cpus;
+        if (asked && parts > asked) parts = asked;
+    }
+    if (parts <= 1u) {
+        fn(ctx, 0, 0, count);
+        return;
+    }
+    const size_t per = (count / parts + 63u) / 64u * 64u;
+    parallel_part p[SP_MAX_THREADS];
+    pthread_t id[SP_MAX_THREADS];
+    bool started[SP_MAX_THREADS] = {false};
+    for (unsigned t = 1; t < parts; ++t) {
+        const size_t begin = (size_t)t * per, end = t + 1u == parts ? count : begin + per;
+        p[t] = (parallel_part){fn, ctx, t, begin < count ? begin : count, end < count ? end : count};
+        started[t] = pthread_create(&id[t], NULL, parallel_main, &p[t]) == 0;
+    }
+    fn(ctx, 0, 0, per < count ? per : count);
+    for (unsigned t = 1; t < parts; ++t) {
+        if (started[t]) pthread_join(id[t], NULL);
+        else parallel_main(&p[t]);
+    }
+}
+
 /* Settings.c:59-80 */
 void sp_log(LogLevel level, const char *fmt, ...)
 {
@@ -120,6 +171,8 @@ void sp_log(LogLevel level, const char *fmt, ...)
  * Large blocks come from anonymous mappings, whose pages are zero and are not
  * committed until touched: the gradient and optimizer arrays that layer()
  * allocates for API compatibility cost nothing for an inference-only net.
+ * Blocks of SP_HUGE_THRESHOLD and more start on a 2 MiB boundary and ask for pages of that size: an array that is
+ * filled takes one page fault per 2 MiB instead of 512.
  * A 64-byte header in front of every block records how to release it. */
 typedef struct {
     uint64_t magic;
@@ -130,6 +183,8 @@ typedef struct {
 #define SP_BLOCK_MAGIC 0x5350424C4F434B21ull
 #define SP_MAP_THRESHOLD ((size_t)1 << 20)
 #define SP_MAP_LEAD 4096u
+#define SP_HUGE ((size_t)2 << 20)
+#define SP_HUGE_THRESHOLD (SP_HUGE + ((size_t)1 << 20))
 
 void *sp_aligned_calloc(size_t count, size_t elem_size)
 {
@@ -140,12 +195,18 @@ void *sp_aligned_calloc(size_t count, size_t elem_size)
     uint8_t *user;
     sp_block_header h = {SP_BLOCK_MAGIC, 0, NULL};
     if (bytes >= SP_MAP_THRESHOLD) {
-        size_t total = bytes + SP_MAP_LEAD;
+        const bool huge = bytes >= SP_HUGE_THRESHOLD;
+        size_t total = (huge ? (bytes + SP_HUGE - 1u) / SP_HUGE * SP_HUGE + SP_HUGE : bytes) + SP_MAP_LEAD;
+        if (total < bytes) return NULL;
         void *m = mmap(NULL, total, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
         if (m == MAP_FAILED) return NULL;
         h.map_bytes = total;
         h.base = m;
         user = (uint8_t *)m + SP_MAP_LEAD;
+        if (huge) {
+            user = (uint8_t *)(((uintptr_t)user + SP_HUGE - 1u) & ~(uintptr_t)(SP_HUGE - 1u));
+            (void)madvise(user, (bytes + SP_HUGE - 1u) / SP_HUGE * SP_HUGE, MADV_HUGEPAGE);                  /* a hint: refused, the pages are small ones */
+        }
     } else {
         void *m = aligned_alloc(SP_ALIGNMENT, bytes + SP_ALIGNMENT);
         if (!m) return NULL;

@@ -399,3 +399,46 @@ def test_bf16_activation_setting_round_trips(S):
     finally:
         L.spingalett_set_bf16_activations(0)
     assert L.spingalett_get_bf16_activations() == 0
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 5, 63, 65, 1023, 1026, 1 << 19, (1 << 20) + 67, (1 << 21) + 1])
+def test_codecs_at_block_thread_and_piece_edges(S, O, tmp_path, count):
+    """Arrays around the codecs' edges (bytes of two and four codes, blocks of 1024, half a million elements per thread,
+    pieces of a million): the file is the oracle's byte for byte and the loaded arrays are its values bit for bit,
+    infinities, NaNs, subnormals and halfway cases among them (finite ones only where a scale is taken).  The second
+    save overwrites a longer file."""
+    rng = np.random.default_rng(count)
+    src = O.Net.new([count, 1], [O.ACT["none"]])
+    w = src.W(0).ravel()
+    w[:] = rng.standard_normal(count).astype(np.float32)
+    k = min(count, 40)
+    w[:k] = (np.arange(k, dtype=np.float32) - 20) * np.float32(0.125)                # halfway between codes
+    w[-1] = -3.0
+    special = np.float32([np.inf, -np.inf, np.nan, 1e-42, -6e-8, 2.0 ** -24, 2.0 ** -25, 65520.0, 65504.0, -0.0])
+    path = str(tmp_path / "x.nn")
+    with open(path, "wb") as f:
+        f.write(b"\xff" * (4 * count + 4096))
+    for fmt in FORMATS:
+        if fmt in ("f32", "f16", "bf16") and count >= 63:
+            w[7:7 + special.size] = special
+        blob = src.serialize(O.PREC[fmt])
+        w[7:7 + special.size] = 0.25
+        net = S.new_spingalett()
+        S.layer(net, count)
+        S.layer(net, 1, S.ACT_NONE, S.WEIGHT_INITIALIZATION_NONE)
+        ref = O.Net.parse(src.serialize(O.PREC["f32"]))
+        if fmt in ("f32", "f16", "bf16") and count >= 63:
+            ref.W(0).ravel()[7:7 + special.size] = special
+        S.weights_view(net, 0)[:] = ref.W(0)
+        S.clear_error()
+        S.save_spingalett(net, path, PREC[fmt], do_not_save_optimizer=True)
+        assert S.last_error()[0] == S.SPINGALETT_OK, S.last_error()
+        S.free_network(net)
+        assert open(path, "rb").read() == blob, fmt
+        for mode in (S.DEQUANT_STRICT, S.DEQUANT_RELEASE):
+            S.lib().spingalett_set_dequant_mode(mode)
+            again = S.load_spingalett(path)
+            want = O.Net.parse(blob, mode)
+            assert np.array_equal(bits(S.weights_view(again, 0)), bits(want.W(0))), (fmt, mode)
+            S.free_network(again)
+        S.lib().spingalett_set_dequant_mode(S.DEQUANT_STRICT)
