@@ -10,6 +10,7 @@
  */
 #define _GNU_SOURCE
 #include "sp_internal.h"
+#include "sp_train_tiny.h"
 
 #include <math.h>
 #include <stdio.h>
@@ -247,8 +248,7 @@ void *spingalett_hip_handle(NeuralNetwork *net)
 }
 
 /* ------------------------------------------------------------------------- *
- *  train(), Training.c:584-949, for the two batched strategies: the epoch
- *  loop, reporting, NaN check, autosave and callback run here; each step
+ *  train(), Training.c:584-949: the epoch loop, reporting, NaN check, autosave and callback run here; each step
  *  (forward, deltas, gradients, update) runs on the device.
  * ------------------------------------------------------------------------- */
 static const char *const optimizer_names[] = {"SGD", "MOMENTUM", "RMSPROP", "ADAM", "ADAMW"};
@@ -257,6 +257,24 @@ static const char *const strategy_names[] = {"SGD", "FULL_BATCH", "SMALL_BATCH"}
 static inline bool should_report(size_t epoch, size_t epochs, size_t interval)      /* Training.c:580-582 */
 {
     return interval > 0 && ((epoch % interval == 0) || (epoch == epochs));
+}
+
+static inline bool nan_check_due(const TrainArgs *a, size_t epoch)
+{
+    return a->nan_check_interval > 0 && epoch % a->nan_check_interval == 0;
+}
+
+static inline bool autosave_due(const TrainArgs *a, size_t epoch)
+{
+    return a->autosave_mode != AUTOSAVE_OFF && a->autosave_interval > 0 && a->autosave_path &&
+           should_report(epoch, a->epochs, a->autosave_interval);
+}
+
+/* whether the host reports, checks, saves or hands out anything at the end of this epoch */
+static inline bool epoch_is_looked_at(const TrainArgs *a, size_t epoch)
+{
+    return should_report(epoch, a->epochs, a->report_interval) || nan_check_due(a, epoch) || autosave_due(a, epoch) ||
+           (a->callback && should_report(epoch, a->epochs, a->callback_interval));
 }
 
 /* weights, biases, moments and the last gradients back into the host arrays (what the reference's
@@ -373,7 +391,10 @@ void train_struct_arguments(TrainArgs args)
     /* The host arrays may have been written since the last upload: an existing FP32 device net gets them again
      * (its buffers, and the training buffers an earlier call left, are kept: allocating and freeing them costs more
      * than the uploads). */
-    if (sn->dev && !upload_arrays(sn, sn->dev)) {
+    const uint32_t eff_batch = small ? args.batch_size : per_sample ? 1u : sample_count;
+    /* a net that fits one compute unit trains inside one launch, which takes and returns the arrays itself */
+    const bool tiny = sp_train_tiny_fits && sp_train_tiny_fits(net->layers, net->topology, sample_count, eff_batch, small);
+    if (sn->dev && !tiny && !upload_arrays(sn, sn->dev)) {
         sp_hip_release(sn);
         return;
     }
@@ -382,7 +403,7 @@ void train_struct_arguments(TrainArgs args)
         report(SPINGALETT_ERR_ALLOC, "HIP back-end: train");
         return;
     }
-    for (uint32_t l = 0; l + 1 < net->layers; ++l) {
+    for (uint32_t l = 0; l + 1 < net->layers && !tiny; ++l) {
         const uint64_t wo = net->weight_offsets[l], bo = net->bias_offsets[l];
         if (sphip_train_set(sn->dev, SPHIP_TRAIN_MW, l, net->opt_m_weights + wo) || sphip_train_set(sn->dev, SPHIP_TRAIN_VW, l, net->opt_v_weights + wo) ||
             sphip_train_set(sn->dev, SPHIP_TRAIN_MB, l, net->opt_m_biases + bo) || sphip_train_set(sn->dev, SPHIP_TRAIN_VB, l, net->opt_v_biases + bo)) {
@@ -392,7 +413,7 @@ void train_struct_arguments(TrainArgs args)
         }
     }
 
-    if (per_sample)
+    if (per_sample && !tiny)
         sp_log(LOG_WARNING, "HIP back-end: the per-sample strategy runs one small device step per sample; the batched strategies are the fast ones");
     if (small)
         sp_log(LOG_INFO, "Starting training: loss=%s, strategy=%s, mode=ARRAY, optimizer=%s, compute=HIP, batch_size=%u",
@@ -402,17 +423,26 @@ void train_struct_arguments(TrainArgs args)
                sp_loss_names[net->loss_func], strategy_names[args.training_strategy], optimizer_names[args.optimizer_type]);
 
     const uint32_t in_sz = net->topology[0], out_sz = net->topology[net->layers - 1];
-    const uint32_t eff_batch = small ? args.batch_size : per_sample ? 1u : sample_count;
-    uint32_t *order = NULL;
+    uint32_t *order = NULL, *orders = NULL;
     float *bx = NULL, *bt = NULL;
+    /* One launch covers the epochs up to the next one that something on the host looks at: at most about 50 ms of them
+     * (5000 cycles and a quarter of a cycle per weight and sample for a step), and 64 K shuffled sample numbers. */
+    const uint64_t steps_per_epoch = ((uint64_t)sample_count + eff_batch - 1u) / eff_batch;
+    uint64_t tiny_epochs = 120000000u / (5000u + net->total_weights * eff_batch / 4u) / steps_per_epoch;
+    if (small && tiny_epochs > 65536u / sample_count) tiny_epochs = 65536u / sample_count;
+    if (tiny_epochs < 1u) tiny_epochs = 1u;
     if (small) {
         order = (uint32_t *)malloc((size_t)sample_count * sizeof(uint32_t));
-        bx = (float *)sp_aligned_calloc((size_t)eff_batch * in_sz, sizeof(float));
-        bt = (float *)sp_aligned_calloc((size_t)eff_batch * out_sz, sizeof(float));
-        if (!order || !bx || !bt) {
+        if (tiny) {
+            orders = (uint32_t *)malloc((size_t)tiny_epochs * sample_count * sizeof(uint32_t));
+        } else {
+            bx = (float *)sp_aligned_calloc((size_t)eff_batch * in_sz, sizeof(float));
+            bt = (float *)sp_aligned_calloc((size_t)eff_batch * out_sz, sizeof(float));
+        }
+        if (!order || (tiny ? !orders : !bx || !bt)) {
             sp_set_error(SPINGALETT_ERR_ALLOC, "Mini-batch allocation failed");
             sp_log(LOG_ERROR, "Mini-batch allocation failed");
-            free(order); sp_aligned_free(bx); sp_aligned_free(bt);
+            free(order); free(orders); sp_aligned_free(bx); sp_aligned_free(bt);
             sphip_train_end(sn->dev);
             return;
         }
@@ -433,10 +463,32 @@ void train_struct_arguments(TrainArgs args)
     }
     bool failed = false;
     for (size_t epoch = 1; epoch <= epochs && !failed; ++epoch) {
+        const size_t begin = epoch;
+        if (tiny) while (epoch < epochs && epoch - begin + 1u < tiny_epochs && !epoch_is_looked_at(&args, epoch)) ++epoch;
         const bool need_loss = should_report(epoch, epochs, args.report_interval) ||
                                (args.callback && should_report(epoch, epochs, args.callback_interval));
         float total_error = 0.0f;
-        if (per_sample) {
+        if (tiny) {
+            const uint32_t count = (uint32_t)(epoch - begin + 1u);
+            for (uint32_t e = 0; small && e < count; ++e) {
+                sp_shuffle_indices(order, sample_count);
+                memcpy(orders + (size_t)e * sample_count, order, (size_t)sample_count * sizeof(uint32_t));
+            }
+            const sp_tiny_run run = {
+                .weights = net->weights, .biases = net->biases, .m_weights = net->opt_m_weights, .m_biases = net->opt_m_biases,
+                .v_weights = net->opt_v_weights, .v_biases = net->opt_v_biases, .g_weights = net->grad_weights,
+                .g_biases = net->grad_biases, .x = args.inputs, .t = args.targets, .samples = sample_count, .batch = eff_batch,
+                .epochs = count, .order = orders, .order_room = (uint32_t)tiny_epochs * sample_count, .first = begin == 1u,
+                .args = &ta, .total_loss = need_loss ? &total_error : NULL,
+            };
+            failed = sp_train_tiny_run(sn->dev, &run) != 0;
+            sn->opt_loaded = true;
+            for (uint64_t s = 0; s < steps_per_epoch * count; ++s) {
+                net->time_step++;
+                ta.beta1_pow_t *= args.beta1;
+                ta.beta2_pow_t *= args.beta2;
+            }
+        } else if (per_sample) {
             for (uint32_t s = 0; s < sample_count && !failed; ++s) {
                 float loss = 0.0f;
                 net->time_step++;
@@ -481,11 +533,9 @@ void train_struct_arguments(TrainArgs args)
             sp_log(LOG_INFO, "Epoch: %zu/%zu, Error: %f", epoch, epochs, (double)current_error);
 
         /* whoever looks at the host arrays below needs them current */
-        const bool nan_now = args.nan_check_interval > 0 && epoch % args.nan_check_interval == 0;
-        const bool save_now = args.autosave_mode != AUTOSAVE_OFF && args.autosave_interval > 0 && args.autosave_path &&
-                              should_report(epoch, epochs, args.autosave_interval);
+        const bool nan_now = nan_check_due(&args, epoch), save_now = autosave_due(&args, epoch);
         const bool call_now = args.callback && should_report(epoch, epochs, args.callback_interval);
-        if ((nan_now || save_now || call_now) && !train_download(sn)) break;
+        if ((nan_now || save_now || call_now) && !tiny && !train_download(sn)) break;
         if (nan_now && has_nan_inf(net)) {
             sp_log(LOG_ERROR, "NaN/Inf detected in weights at epoch %zu, stopping training", epoch);
             break;
@@ -496,10 +546,11 @@ void train_struct_arguments(TrainArgs args)
             break;
         }
     }
-    (void)train_download(sn);
+    if (!tiny) (void)train_download(sn);
     /* no sphip_train_end: the training buffers stay with the device net for the next call and go with it
      * (free_network, layer(), spingalett_hip_invalidate) */
     free(order);
+    free(orders);
     sp_aligned_free(bx);
     sp_aligned_free(bt);
     sp_log(LOG_INFO, "Training completed.");

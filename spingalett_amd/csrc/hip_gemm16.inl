@@ -1,6 +1,6 @@
 // hip_gemm16.inl — the LDS-tiled 16-bit MFMA GEMM for larger batches (sp_gemm16, sp_gemm16_big,
-// sp_gemm16_reduce).  Part of hip_forward.hip's translation unit (included there, inside its unnamed
-// namespace); not compiled on its own.
+// sp_gemm16_reduce).  Part of hip_kernels.h (included there,
+// inside its namespace); not compiled on its own.
 
 // ---------------------------------------------------------------------------
 // 16-bit MFMA GEMM (n > 64): C[M][N] = act(bias + scale * A[M][K] . Wq[N][K]^T)

@@ -1,0 +1,199 @@
+// hip_kernels.h — element formats, device helpers and the template kernels that several translation units share: the
+// one that launches them (hip_forward.hip) and those that compile them (hip_part.hip).
+#ifndef SPINGALETT_HIP_KERNELS_H
+#define SPINGALETT_HIP_KERNELS_H
+
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstdint>
+#include <type_traits>
+
+namespace sphip_kernels {
+
+// ---------------------------------------------------------------------------
+// formats and small helpers
+// ---------------------------------------------------------------------------
+enum : int { F32 = 0, F16 = 1, BF16 = 2, I8 = 3, I4 = 4, I2 = 5, NFMT = 6 };
+enum : int { A_SIGMOID = 0, A_RELU, A_TANH, A_LEAKY, A_FOO52, A_SOFTMAX, A_NONE, A_COUNT };
+
+constexpr int kWave = 64;
+
+__host__ __device__ constexpr int fmt_bits(int f)
+{
+    return f == F32 ? 32 : (f == F16 || f == BF16) ? 16 : f == I8 ? 8 : f == I4 ? 4 : 2;
+}
+
+// ---------------------------------------------------------------------------
+// device-side element access
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ float bits_to_float(uint32_t u) { return __uint_as_float(u); }
+
+// binary16 -> binary32, integer arithmetic only; any NaN becomes the quiet NaN
+// of the same sign (Serialize.c:45-72).
+__device__ __forceinline__ float half_bits_to_float_exact(uint32_t h)
+{
+    uint32_t s = (h & 0x8000u) << 16;
+    uint32_t e = (h >> 10) & 31u;
+    uint32_t m = h & 1023u;
+    uint32_t f;
+    if (e == 31u) {
+        f = s | (m ? 0x7FC00000u : 0x7F800000u);
+    } else if (e != 0u) {
+        f = s | ((e + 112u) << 23) | (m << 13);
+    } else if (m == 0u) {
+        f = s;
+    } else {
+        int lz = __clz((int)m) - 21;               // shifts until bit 10 is set
+        m = (m << lz) & 1023u;
+        f = s | ((uint32_t)(113 - lz) << 23) | (m << 13);
+    }
+    return bits_to_float(f);
+}
+
+// integer code of element i of a packed INT array
+template <int FMT>
+__device__ __forceinline__ int int_code(const uint8_t *codes, uint64_t i)
+{
+    if constexpr (FMT == I8) {
+        return (int)(int8_t)codes[i];
+    } else if constexpr (FMT == I4) {
+        uint32_t byte = codes[i >> 1];
+        uint32_t nib = (i & 1u) ? (byte >> 4) : (byte & 15u);
+        return (int)nib - (int)((nib & 8u) << 1);
+    } else {
+        uint32_t c = (codes[i >> 2] >> ((i & 3u) * 2u)) & 3u;
+        return (int)c - (int)((c & 2u) << 1);
+    }
+}
+
+// unscaled value of element i: the float itself for FP formats, (float)q for INT
+template <int FMT>
+__device__ __forceinline__ float elem_value(const uint8_t *codes, uint64_t i)
+{
+    if constexpr (FMT == F32) {
+        return reinterpret_cast<const float *>(codes)[i];
+    } else if constexpr (FMT == F16) {
+        return half_bits_to_float_exact(reinterpret_cast<const uint16_t *>(codes)[i]);
+    } else if constexpr (FMT == BF16) {
+        return bits_to_float((uint32_t)reinterpret_cast<const uint16_t *>(codes)[i] << 16);
+    } else {
+        return (float)int_code<FMT>(codes, i);
+    }
+}
+
+__device__ __forceinline__ float elem_value_rt(int fmt, const uint8_t *codes, uint64_t i)
+{
+    switch (fmt) {
+    case F32:  return elem_value<F32>(codes, i);
+    case F16:  return elem_value<F16>(codes, i);
+    case BF16: return elem_value<BF16>(codes, i);
+    case I8:   return elem_value<I8>(codes, i);
+    case I4:   return elem_value<I4>(codes, i);
+    default:   return elem_value<I2>(codes, i);
+    }
+}
+
+// Activation.c:23-38 (leak factor fixed at 0.01f).  Softmax is a row operation
+// and handled by sp_softmax_rows.
+__device__ __forceinline__ float apply_act(float x, int act)
+{
+    switch (act) {
+    case A_SIGMOID: return 1.0f / (1.0f + expf(-x));
+    case A_RELU:    return x > 0.0f ? x : 0.0f;
+    case A_TANH:    return tanhf(x);
+    case A_LEAKY:   return x > 0.0f ? x : 0.01f * x;
+    case A_FOO52:   return x > 1.0f ? 1.0f + 0.01f * (x - 1.0f) : (x < 0.0f ? 0.01f * x : x);
+    default:        return x;
+    }
+}
+
+// the same for the activations that need no transcendental function (a caller has dealt with the other two)
+__device__ __forceinline__ float apply_act_cheap(float x, int act)
+{
+    switch (act) {
+    case A_RELU:    return x > 0.0f ? x : 0.0f;
+    case A_LEAKY:   return x > 0.0f ? x : 0.01f * x;
+    case A_FOO52:   return x > 1.0f ? 1.0f + 0.01f * (x - 1.0f) : (x < 0.0f ? 0.01f * x : x);
+    default:        return x;
+    }
+}
+
+// FP32 -> BF16, round to nearest even, NaNs stay NaNs: the part's own conversion instruction
+__device__ __forceinline__ uint16_t f32_to_bf16_rne(float x)
+{
+    const __bf16 h = (__bf16)x;
+    uint16_t r;
+    __builtin_memcpy(&r, &h, 2);
+    return r;
+}
+
+// FP32 -> FP16: finite values beyond the FP16 range become +-65504 (an activation that large stays finite in the
+// reference's FP32 arithmetic; an infinity here would turn into NaNs in the next layer), infinities and NaNs stay
+// what they are.
+__device__ __forceinline__ uint16_t f32_to_f16_sat(float x)
+{
+    if (x != x) return (uint16_t)0x7E00u;
+    const float c = fminf(fmaxf(x, -65504.0f), 65504.0f);
+    _Float16 h = (_Float16)(fabsf(x) == __builtin_inff() ? x : c);
+    uint16_t r;
+    __builtin_memcpy(&r, &h, 2);
+    return r;
+}
+
+template <bool F16T>
+__device__ __forceinline__ uint16_t f32_to_t16(float x)
+{
+    if constexpr (F16T) return f32_to_f16_sat(x);
+    else return f32_to_bf16_rne(x);
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<N, I + 1>(f);
+    }
+}
+
+__device__ __forceinline__ float wave_sum(float v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    return v;
+}
+
+__device__ __forceinline__ int wave_sum_i(int v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    return v;
+}
+
+__device__ __forceinline__ uint32_t wave_max_u(uint32_t v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, kWave));
+    return v;
+}
+
+__device__ __forceinline__ float wave_max(float v)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
+    return v;
+}
+
+#include "hip_gemv.inl"
+
+#include "hip_gemm16.inl"
+
+#include "hip_skinny.inl"
+
+}  // namespace sphip_kernels
+
+#endif

@@ -278,44 +278,49 @@ struct OptArgs {
     float lr, decay, momentum, b1, b2, omb1, omb2, mf, vf, eps;
 };
 
-// One optimizer step over one array: the scalar forms of SIMD.c:279-494 as called from
-// apply_gradients_batch_prescaled (Training.c:439-507).  The gradient array keeps what the reference
-// leaves in it (clipped, and with decay * W added for Adam with weight decay).
-__global__ __launch_bounds__(256) void sp_train_opt(const OptArgs a)
+// One optimizer step of one element: the scalar forms of SIMD.c:279-494 as called from apply_gradients_batch_prescaled
+// (Training.c:439-507).  g is left as the reference leaves its gradient (with decay * W added for Adam with weight decay).
+__device__ __forceinline__ void opt_update(const OptArgs &a, float &w, float &g, float &m, float &v)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-    if (i >= a.cnt) return;
-    float w = a.W[i], g = a.g[i];
-    if (a.clip) { g *= *a.clip; a.g[i] = g; }
     switch (a.opt) {
     case 0:     // SGD
         w -= a.lr * (a.decay > 0.0f ? g + a.decay * w : g);
         break;
-    case 1: {   // momentum
-        const float m = a.momentum * a.m[i] + a.decay * w + g;
-        a.m[i] = m;
+    case 1:     // momentum
+        m = a.momentum * m + a.decay * w + g;
         w -= a.lr * m;
         break;
-    }
     case 2: {   // RMSprop
-        if (a.decay_in_grad && a.decay > 0.0f) g += a.decay * w;
-        const float v = a.b2 * a.v[i] + a.omb2 * (g * g);
-        a.v[i] = v;
-        w -= a.decay_in_grad ? a.lr * g / sqrtf(v + a.eps) : a.lr * (a.decay * w + g / sqrtf(v + a.eps));
+        const float gd = a.decay_in_grad && a.decay > 0.0f ? g + a.decay * w : g;
+        v = a.b2 * v + a.omb2 * (gd * gd);
+        w -= a.decay_in_grad ? a.lr * gd / sqrtf(v + a.eps) : a.lr * (a.decay * w + gd / sqrtf(v + a.eps));
         break;
     }
     default: {  // Adam (3): decay joins the gradient; AdamW (4): decay shrinks the weight
         const bool adamw = a.opt == 4;
-        if (!adamw && a.decay > 0.0f) { g += a.decay * w; a.g[i] = g; }
-        const float m = a.b1 * a.m[i] + a.omb1 * g;
-        const float v = a.b2 * a.v[i] + a.omb2 * (g * g);
-        a.m[i] = m;
-        a.v[i] = v;
+        if (!adamw && a.decay > 0.0f) g += a.decay * w;
+        m = a.b1 * m + a.omb1 * g;
+        v = a.b2 * v + a.omb2 * (g * g);
         const float step = a.lr * ((m * a.mf) / sqrtf(v * a.vf + a.eps));
         w = (adamw && a.decay > 0.0f) ? w * (1.0f - a.lr * a.decay) - step : w - step;
         break;
     }
     }
+}
+
+// One optimizer step over one array; the gradient array keeps what the reference leaves in it (clipped, and see above)
+__global__ __launch_bounds__(256) void sp_train_opt(const OptArgs a)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (i >= a.cnt) return;
+    const bool has_m = a.opt != 0 && a.opt != 2, has_v = a.opt >= 2;
+    const float g0 = a.g[i];
+    float w = a.W[i], g = a.clip ? g0 * *a.clip : g0, m = has_m ? a.m[i] : 0.0f, v = has_v ? a.v[i] : 0.0f;
+    const bool keep_g = a.clip || (a.opt == 3 && a.decay > 0.0f);
+    opt_update(a, w, g, m, v);
+    if (keep_g) a.g[i] = g;
+    if (has_m) a.m[i] = m;
+    if (has_v) a.v[i] = v;
     a.W[i] = w;
 }
 
@@ -344,6 +349,8 @@ struct sphip_train_state {
     float *scal = nullptr;                 // clip factor, gradient norm
     float *loss_buf = nullptr;             // per-sample loss / prediction / hit, totals
     uint64_t loss_cap = 0;
+    float *tiny_pin = nullptr;             // pinned host memory of sp_train_tiny: state, results, samples
+    uint64_t tiny_cap = 0;
 };
 
 namespace {
@@ -357,6 +364,7 @@ void train_free(sphip_net *net)
     float *flat[] = {ts->gW, ts->gB, ts->mW, ts->vW, ts->mB, ts->vB, ts->targets, ts->ws, ts->scal, ts->loss_buf};
     for (float *p : flat) if (p) (void)hipFree(p);
     if (ts->sq_part) (void)hipFree(ts->sq_part);
+    if (ts->tiny_pin) (void)hipHostFree(ts->tiny_pin);
     for (float *p : ts->act) if (p) (void)hipFree(p);
     for (float *p : ts->delta) if (p) (void)hipFree(p);
     delete ts;
@@ -413,13 +421,13 @@ void launch_train_gemm(TrGemmArgs g, float *ws, uint64_t ws_floats)
         sp_train_gemm32_reduce<EPI><<<(uint32_t)(((uint64_t)g.M * g.N + 255) / 256), 256, 0, g_stream>>>(g, splits);
 }
 
-void launch_opt(const sphip_train_args &a, float *W, float *g, float *m, float *v, uint64_t cnt, float decay, const float *clip)
+// the scalars of a step's updates; decay and the arrays are the caller's to set
+OptArgs opt_args(const sphip_train_args &a)
 {
     OptArgs o{};
-    o.W = W; o.g = g; o.m = m; o.v = v; o.cnt = cnt; o.clip = clip;
     o.opt = a.optimizer;
     o.decay_in_grad = a.decay_in_grad;
-    o.lr = a.learning_rate; o.decay = decay; o.momentum = a.momentum;
+    o.lr = a.learning_rate; o.momentum = a.momentum;
     o.b1 = a.beta1; o.b2 = a.beta2;
     // formed in FP32 like the reference's locals (Training.c:447-448, 479-480)
     o.omb1 = 1.0f - a.beta1;
@@ -427,7 +435,22 @@ void launch_opt(const sphip_train_args &a, float *W, float *g, float *m, float *
     o.mf = 1.0f / (1.0f - a.beta1_pow_t);
     o.vf = 1.0f / (1.0f - a.beta2_pow_t);
     o.eps = a.epsilon;
+    return o;
+}
+
+void launch_opt(const sphip_train_args &a, float *W, float *g, float *m, float *v, uint64_t cnt, float decay, const float *clip)
+{
+    OptArgs o = opt_args(a);
+    o.W = W; o.g = g; o.m = m; o.v = v; o.cnt = cnt; o.clip = clip;
+    o.decay = decay;
     sp_train_opt<<<(uint32_t)((cnt + 255) / 256), 256, 0, g_stream>>>(o);
+}
+
+// which of sp_train_out_delta's rules a loss and an output activation take (Training.c:357-378)
+int out_delta_mode(int loss_func, int last_act)
+{
+    return (loss_func == 0 && last_act == A_SOFTMAX) ? 0
+         : (loss_func == 1 && (last_act == A_SOFTMAX || last_act == A_SIGMOID)) ? 1 : 2;
 }
 
 }  // namespace
@@ -568,8 +591,7 @@ int sphip_train_step(sphip_net *net, const float *x, const float *targets, uint3
 
     // deltas (Training.c:347-394)
     const int last_act = net->act[last - 1];
-    const int mode = (args->loss_func == 0 && last_act == A_SOFTMAX) ? 0
-                   : (args->loss_func == 1 && (last_act == A_SOFTMAX || last_act == A_SIGMOID)) ? 1 : 2;
+    const int mode = out_delta_mode(args->loss_func, last_act);
     sp_train_out_delta<<<(n + 3) / 4, 256, 0, g_stream>>>(ts->act[last], d_t, ts->delta[last], n, width, mode, last_act);
     for (uint32_t l = last - 1; l > 0; --l) {
         TrGemmArgs g{};

@@ -451,3 +451,57 @@ def test_full_size_benchmark_step_properties():
         seen.append(d.train_step(X, hot, a, want_loss=True))
     assert seen[-1] < seen[0]
     d.destroy()
+
+
+TINY_CASES = [
+    # topology, activations, loss, samples, batch (0: the full batch, 1: per sample, else mini-batch), epochs, optimizer, options
+    ([3, 2], ["sigmoid"], 0, 5, 0, 20, S.OPTIMIZER_SGD, {"weight_decay": 0.01}),                # one layer, one wave
+    ([2, 8, 1], ["tanh", "sigmoid"], 0, 4, 0, 50, S.OPTIMIZER_ADAMW, {"weight_decay": 1e-3}),
+    ([6, 16, 5], ["foo52", "softmax"], 0, 9, 0, 12, S.OPTIMIZER_MOMENTUM, {"max_grad_norm": 1e-3}),  # clipped, four waves
+    ([17, 31, 12, 7], ["leaky_relu", "tanh", "softmax"], 1, 60, 0, 6, S.OPTIMIZER_RMSPROP, {"max_grad_norm": 0.05}),
+    ([48, 48, 10], ["tanh", "softmax"], 1, 94, 0, 4, S.OPTIMIZER_ADAM, {"weight_decay": 1e-3}),   # 94 * 2784 pairs: the largest step taken
+    ([48, 48, 10], ["tanh", "softmax"], 1, 95, 0, 4, S.OPTIMIZER_ADAM, {}),                       # one sample more: launch by launch
+    ([5, 4, 6, 3, 2], ["tanh", "sigmoid", "none", "none"], 0, 13, 0, 8, S.OPTIMIZER_ADAM, {}),    # four layers ...
+    ([5, 4, 6, 3, 3, 2], ["tanh"] * 4 + ["none"], 0, 13, 0, 8, S.OPTIMIZER_ADAM, {}),             # ... and one too many
+    ([11, 20, 3], ["sigmoid", "softmax"], 1, 70, 70, 5, S.OPTIMIZER_ADAM, {}),                    # shuffled, one step an epoch
+    ([40, 9, 2], ["tanh", "softmax"], 1, 1100, 1, 1, S.OPTIMIZER_SGD, {}),                        # samples beyond LDS, read step by step
+]
+
+
+@pytest.mark.parametrize("topo,acts,loss,n,batch,epochs,opt,kw", TINY_CASES)
+def test_small_nets_match_the_oracle(topo, acts, loss, n, batch, epochs, opt, kw):
+    """Trainings that run inside one launch, at the edges of what that takes (threads per workgroup, layers, weight-sample
+    pairs, samples in LDS or not, a shuffled order), with the report of every second epoch."""
+    net, onet = public_net(topo, acts, loss, seed=3)
+    rng = np.random.default_rng(8)
+    X = rng.standard_normal((n, topo[0])).astype(np.float32)
+    T = targets_for(rng, n, topo[-1], loss == 1)
+    strategy = {0: S.STRATEGY_FULL_BATCH, 1: S.STRATEGY_SAMPLE}.get(batch, S.STRATEGY_SMALL_BATCH)
+    seen = []
+    S.clear_error()
+    S.train(net, X, T, epochs, strategy, opt, batch_size=batch, learning_rate=0.005,
+            callback=lambda p, epoch, err: seen.append((epoch, err)) or False, callback_interval=2, **kw)
+    assert S.last_error()[0] == S.SPINGALETT_OK, S.last_error()
+    st = O.TrainState(onet)
+    want = []
+    for epoch in range(1, epochs + 1):
+        total = 0.0
+        for s in range(n if batch == 1 else 1):
+            x, t = (X[s:s + 1], T[s:s + 1]) if batch == 1 else (X, T)
+            gW, gB, out = onet.batch_gradients(x, t)
+            total += O.batch_loss(out, t, loss, O.ACT[acts[-1]])
+            onet.apply_gradients(st, gW, gB, opt, lr=0.005, decay_in_grad=batch == 1, **kw)
+        if epoch % 2 == 0 or epoch == epochs:
+            want.append((epoch, total / n))
+    assert [e for e, _ in seen] == [e for e, _ in want]
+    assert [v for _, v in seen] == pytest.approx([v for _, v in want], rel=1e-4)
+    nc = net.contents
+    assert nc.time_step == epochs * (n if batch == 1 else 1)
+    arr = lambda name, cnt: np.ctypeslib.as_array(getattr(nc, name), shape=(int(cnt),))
+    for name, cnt, ref in [("weights", nc.total_weights, onet.weights), ("biases", nc.total_biases, onet.biases),
+                           ("grad_weights", nc.total_weights, gW), ("grad_biases", nc.total_biases, gB),
+                           ("opt_m_weights", nc.total_weights, st.mW), ("opt_v_weights", nc.total_weights, st.vW),
+                           ("opt_m_biases", nc.total_biases, st.mB), ("opt_v_biases", nc.total_biases, st.vB)]:
+        assert rel_max_abs(arr(name, cnt), ref) <= TOL, name
+    assert rel_max_abs(S.forward_batch(net, X[:7]), onet.forward_batch(X[:7])) <= TOL      # the device holds the results too
+    S.free_network(net)
