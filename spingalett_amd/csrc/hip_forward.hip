@@ -398,6 +398,62 @@ __global__ __launch_bounds__(256) void sp_cat3_w(const float *__restrict__ w, ui
 }
 
 // ---------------------------------------------------------------------------
+// padded layers (padded_width)
+// ---------------------------------------------------------------------------
+// [rows][cols] elements of BITS bits into [prows][pcols], zeros around; a thread makes one 32-bit word.  Packed elements
+// run on across row ends, in the source and (behind a hidden softmax, whose width stays) in the destination.  Once per
+// upload.
+template <int BITS>
+__global__ __launch_bounds__(256) void sp_pad_rows(const uint8_t *__restrict__ in, uint32_t *__restrict__ out, uint32_t rows, uint32_t cols,
+                                                   uint32_t pcols, uint64_t words)
+{
+    constexpr uint32_t EPW = 32 / BITS;
+    const uint64_t id = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (id >= words) return;
+    const uint64_t e0 = id * EPW;
+    uint32_t r = (uint32_t)(e0 / pcols), c = (uint32_t)(e0 % pcols), v = 0;
+#pragma unroll
+    for (uint32_t e = 0; e < EPW; ++e, ++c) {
+        if (c == pcols) { c = 0; ++r; }
+        if (r >= rows || c >= cols) continue;
+        const uint64_t i = (uint64_t)r * cols + c;
+        if constexpr (BITS == 16) v |= (uint32_t)reinterpret_cast<const uint16_t *>(in)[i] << (16u * e);
+        else v |= ((uint32_t)in[i * BITS / 8u] >> (i % (8u / BITS) * BITS) & ((1u << BITS) - 1u)) << (BITS * e);
+    }
+    out[id] = v;
+}
+
+// The caller's rows of K floats as rows of Kp (a multiple of 4), zeros behind; KIND 1 BF16, 2 FP16, 3 split FP16
+// (sp_cvt16_split's two matrices).  A thread makes four elements of a row.
+template <int KIND>
+__global__ __launch_bounds__(256) void sp_pad_input(const float *__restrict__ x, void *__restrict__ out, uint32_t n, uint32_t K, uint32_t Kp)
+{
+    const uint64_t id = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    const uint32_t quads = Kp / 4u, r = (uint32_t)(id / quads), k = (uint32_t)(id % quads) * 4u;
+    if (r >= n) return;
+    float v[4];
+#pragma unroll
+    for (uint32_t e = 0; e < 4u; ++e) v[e] = k + e < K ? x[(size_t)r * K + k + e] : 0.0f;
+    const size_t o = (size_t)r * Kp + k;
+    uint16_t h[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if constexpr (KIND == 3) split_f16(v[e], h[e], l[e]);
+        else h[e] = f32_to_t16<KIND == 2>(v[e]);
+    }
+    uint16_t *p = reinterpret_cast<uint16_t *>(out);
+    *reinterpret_cast<uint2 *>(p + o) = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+    if constexpr (KIND == 3)
+        *reinterpret_cast<uint2 *>(p + (size_t)n * Kp + o) = make_uint2((uint32_t)l[0] | ((uint32_t)l[1] << 16), (uint32_t)l[2] | ((uint32_t)l[3] << 16));
+}
+
+__global__ __launch_bounds__(256) void sp_fill0(float *p, uint64_t cnt)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (i < cnt) p[i] = 0.0f;
+}
+
+// ---------------------------------------------------------------------------
 // small copies (host staging of single-sample forwards)
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void sp_copy32(const float *__restrict__ src, float *__restrict__ dst, uint64_t n)
@@ -515,7 +571,7 @@ __global__ __launch_bounds__(1024) void sp_eval_total(const float *loss, const u
 // host side
 // ---------------------------------------------------------------------------
 struct DevArray {
-    uint8_t *base = nullptr;       // allocation (256-byte aligned by hipMalloc)
+    uint8_t *base = nullptr;       // inside sphip_net::arrays, at a multiple of 256 bytes
     size_t bytes = 0;
     uint64_t count = 0;
     float max_val = 0.0f;
@@ -551,7 +607,16 @@ struct sphip_net {
     std::vector<uint32_t> topo;
     std::vector<uint8_t> act;
     int prec = 0;
-    std::vector<DevArray> W, B;    // [layers-1]
+    std::vector<DevArray> W, B;    // [layers-1] as uploaded (W: zero rows behind it up to the padded outputs)
+    // Widths whose weight rows would not be whole 16-byte units run padded with zero weights (padded_width); PW / PB are
+    // the arrays of the layers this touches, base == nullptr where the uploaded ones serve.
+    uint8_t *arrays = nullptr;     // the one allocation behind every base
+    std::vector<uint32_t> ptopo;
+    std::vector<DevArray> PW, PB;
+
+    DevArray &w(uint32_t l) { return PW[l].base ? PW[l] : W[l]; }                    // what a forward multiplies with
+    const DevArray &w(uint32_t l) const { return PW[l].base ? PW[l] : W[l]; }
+    const DevArray &b(uint32_t l) const { return PB[l].base ? PB[l] : B[l]; }
     // workspace, grown on demand
     uint64_t cap_elems = 0;        // capacity of each ping-pong buffer in FP32 elements
     void *buf[2] = {nullptr, nullptr};
@@ -612,18 +677,39 @@ Regime pick_regime(const sphip_net *net, uint32_t n, uint32_t flags)
     return n <= 4 ? R_GEMV : R_GEMM16;
 }
 
-LayerArgs make_layer_args(const sphip_net *net, uint32_t l /*1-based layer*/)
+// Width a layer runs with.  Rows of weights that are not whole 16-byte units can only be read element by element or word
+// by word, and every tile of such a layer waits for those loads (1030-1531-777-33 FP16 at 1333 samples: 107 us for each
+// of three layers, 9 to 15 padded).  So an input or hidden layer of such a width gets neurons without weights up to
+// the next whole unit (wide ones up to a multiple of 64, whole cache lines): zero rows and zero biases on the producing
+// side, zero columns on the consuming side, so that whatever activation(0) is adds nothing.  Not the output layer, whose
+// rows are the caller's, and not a hidden softmax, whose sum runs over its real neurons.
+// Integer rows of eight codes' multiples (1000 INT8 codes) have kernels of their own, which are as good on small layers
+// and take the input as it is; hidden widths of that kind are padded in front of half a million weights and more, where
+// the streaming and DMA kernels, which want 16-byte rows, are the better ones.  FP32 rows stay as they are.
+uint32_t padded_width(int fmt, uint32_t w, uint32_t next, bool hidden)
+{
+    if (fmt == F32) return w;
+    const uint32_t unit = fmt_bits(fmt) == 16 ? 8u : 128u / (uint32_t)fmt_bits(fmt);
+    if (w % unit == 0) return w;
+    if (w % 8u == 0 && !(hidden && (uint64_t)w * next > (512u << 10))) return w;
+    const uint32_t to = w >= 256u ? 64u : unit;
+    return (w + to - 1u) / to * to;
+}
+
+// raw: its inputs unpadded (the first layer on the vector kernels, which take the caller's rows as they are); its outputs
+// are padded all the same
+LayerArgs make_layer_args(const sphip_net *net, uint32_t l /*1-based layer*/, bool raw = false)
 {
     LayerArgs L{};
-    const DevArray &w = net->W[l - 1], &b = net->B[l - 1];
+    const DevArray &w = raw ? net->W[l - 1] : net->w(l - 1), &b = net->b(l - 1);
     L.w = w.base;
     L.bias = b.base;
-    L.wscale = fmt_scale(net->prec, w.max_val);
-    L.bscale = fmt_scale(net->prec, b.max_val);
+    L.wscale = fmt_scale(net->prec, net->W[l - 1].max_val);
+    L.bscale = fmt_scale(net->prec, net->B[l - 1].max_val);
     L.bias_fmt = net->prec;
     L.act = net->act[l - 1] == A_SOFTMAX ? A_NONE : net->act[l - 1];
-    L.N = net->topo[l];
-    L.K = net->topo[l - 1];
+    L.N = net->ptopo[l];
+    L.K = raw ? net->topo[l - 1] : net->ptopo[l - 1];
     return L;
 }
 
@@ -889,6 +975,7 @@ struct ThinCtx {
     void *soft_out;        // softmax layer: where the normalised outputs go if the layer's kernel can do it itself ...
     int soft_kind;         // ... as 0 FP32, 1 BF16, 2 FP16
     bool *soft_done;       // ... and whether it did
+    bool padded_in;        // the first layer, with the caller's rows padded (padded_width)
 };
 
 struct ThinPlan {
@@ -1071,7 +1158,9 @@ template <int FMT, bool F16T>
 void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t M, int out_f32, const ThinCtx &ctx)
 {
     const uint32_t halves = tl_route.halves;
-    if (gemm16_small_layer(M, L.N, L.K, halves) && (reinterpret_cast<uintptr_t>(A) & 15u) == 0) {
+    // (a small layer behind a padded input stays on the single-stage kernel: its conversion is a launch of its own anyway)
+    const bool single = ctx.padded_in && gemm16_small_layer(M, L.N, L.K, halves);
+    if (!single && gemm16_small_layer(M, L.N, L.K, halves) && (reinterpret_cast<uintptr_t>(A) & 15u) == 0) {
         GemmArgs g{L, A, C, M, out_f32, nullptr, 0, 1, 1};
         tl_route.name = "sp_gemm16_small";
         if (tl_route.dry) return;
@@ -1088,7 +1177,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         return;
     }
     const ThinPlan tp = plan_thin(FMT, M, L.N, L.K);
-    if (tp.use && (!tp.mode_b || ctx.w16) &&
+    if (tp.use && !single && (!tp.mode_b || ctx.w16) &&
         ((tp.splits == 1 && halves == 1) || (uint64_t)tp.splits * halves * tp.NC * tp.R <= ctx.ws_floats)) {
         SkinnyArgs a{};
         a.halves = halves; a.half_elems = (uint64_t)M * L.K;
@@ -1153,7 +1242,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     g.ksplits = 1;
     if (halves == 2) g.ws = ctx.ws;                  // one partial sum per activation matrix, added by the reduction
     const bool words = !aligned && L.K % 8u == 0 && ((uint64_t)L.K * fmt_bits(FMT)) % 32u == 0 && (FMT == I8 || FMT == I4 || FMT == I2);
-    if (!aligned && !words) {
+    if ((!aligned && !words) || single) {
         uint32_t kper = 0;
         const uint32_t sp = gemm16_ragged_splits(M, L.N, L.K, &kper);
         if (sp > 1 && (uint64_t)sp * halves * M * L.N <= ctx.ws_floats) {
@@ -1327,7 +1416,7 @@ struct WorkspaceNeed {
 bool layer_wants_codes16(const sphip_net *net, uint32_t l /*1-based*/, uint32_t n)
 {
     if (net->prec < I8) return false;
-    const ThinPlan tp = plan_thin(net->prec, n, net->topo[l], net->topo[l - 1]);
+    const ThinPlan tp = plan_thin(net->prec, n, net->ptopo[l], net->ptopo[l - 1]);
     return tp.use && tp.mode_b;
 }
 
@@ -1348,14 +1437,14 @@ WorkspaceNeed workspace_need(const sphip_net *net, uint32_t n, uint32_t flags)
     const uint32_t halves = (flags & SPHIP_SPLIT_ACTIVATIONS) && reg == R_GEMM16 ? 2u : 1u;
     w.act_floats = (uint64_t)n * net->max_width;
     for (uint32_t l = 1; l < net->layers; ++l)
-        if (net->act[l - 1] == A_SOFTMAX && (uint64_t)n * net->topo[l] > w.soft_floats) w.soft_floats = (uint64_t)n * net->topo[l];
+        if (net->act[l - 1] == A_SOFTMAX && (uint64_t)n * net->ptopo[l] > w.soft_floats) w.soft_floats = (uint64_t)n * net->ptopo[l];
     if (n <= 64 && net->prec >= I8) {
         const uint64_t padded = (uint64_t)n * ((uint64_t)net->max_width + 4096u);
         w.plane_bytes = padded * 4u;
         w.plane_recs = padded / 64u + 64u;
     }
     for (uint32_t l = 1; l < net->layers; ++l) {
-        const uint32_t N = net->topo[l], K = net->topo[l - 1];
+        const uint32_t N = net->ptopo[l], K = net->ptopo[l - 1];
         uint32_t kper = 0;
         uint64_t ws = 0;
         if (reg == R_CAT3 && cat3_layer(n, N, K)) {
@@ -1386,6 +1475,10 @@ WorkspaceNeed workspace_need(const sphip_net *net, uint32_t n, uint32_t flags)
                     if (rs > 1) ws = (uint64_t)rs * halves * n * N;
                 }
             }
+        }
+        if (reg == R_GEMM16 && l == 1 && K != net->topo[0] && gemm16_small_layer(n, N, K, halves)) {
+            const uint32_t rs = gemm16_ragged_splits(n, N, K, &kper);
+            if ((uint64_t)rs * halves * n * N > ws) ws = (uint64_t)rs * halves * n * N;
         }
         if (ws > w.split_floats) w.split_floats = ws;
     }
@@ -1423,6 +1516,32 @@ int make_cat3(DevArray &wa, uint32_t N, uint32_t K)
     return 0;
 }
 
+// The padded arrays of one layer from the uploaded ones (sp_pad_rows).  Enqueues only.
+int pad_layer(sphip_net *net, uint32_t l, bool weights, bool biases)
+{
+    if (net->prec == F32) return 0;                        // (never padded)
+    const uint32_t N = net->topo[l + 1], K = net->topo[l], Np = net->ptopo[l + 1], Kp = net->ptopo[l];
+    DevArray &pw = net->PW[l], &pb = net->PB[l];
+    auto go = [&](const DevArray &src, DevArray &dst, uint32_t rows, uint32_t cols, uint32_t prows, uint32_t pcols) {
+        const uint64_t words = (fmt_bytes(net->prec, (uint64_t)prows * pcols) + 3u) / 4u;
+        const uint32_t grid = (uint32_t)((words + 255u) / 256u);
+        uint32_t *out = reinterpret_cast<uint32_t *>(dst.base);
+        switch (fmt_bits(net->prec)) {
+        case 16: sp_pad_rows<16><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
+        case 8:  sp_pad_rows<8><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
+        case 4:  sp_pad_rows<4><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
+        default: sp_pad_rows<2><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
+        }
+    };
+    if (weights && pw.base) {
+        go(net->W[l], pw, N, K, Np, Kp);
+        pw.codes16_valid = pw.wide16_valid = pw.cat3_valid = false;
+    }
+    if (biases && pb.base) go(net->B[l], pb, 1, N, 1, Np);
+    HCHECK(hipGetLastError());
+    return 0;
+}
+
 // grows the net's own workspace to what n samples need
 int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
 {
@@ -1435,8 +1554,8 @@ int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
     }
     if (need.cat_elems)
         for (uint32_t l = 1; l < net->layers; ++l)
-            if (cat3_layer(n, net->topo[l], net->topo[l - 1]) && !net->W[l - 1].cat3_valid && net->W[l - 1].uploaded &&
-                make_cat3(net->W[l - 1], net->topo[l], net->topo[l - 1])) return 1;
+            if (cat3_layer(n, net->ptopo[l], net->ptopo[l - 1]) && !net->w(l - 1).cat3_valid && net->W[l - 1].uploaded &&
+                make_cat3(net->w(l - 1), net->ptopo[l], net->ptopo[l - 1])) return 1;
     if (need.act_floats > net->cap_elems) {
         for (int i = 0; i < 2; ++i) {
             if (net->buf[i]) { HCHECK(hipFree(net->buf[i])); net->buf[i] = nullptr; }
@@ -1469,8 +1588,8 @@ int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
         net->split_cap = need.split_floats;
     }
     for (uint32_t l = 1; l < net->layers; ++l) {
-        DevArray &wa = net->W[l - 1];
-        if (layer_wants_codes16(net, l, n) && !wa.codes16_valid && wa.uploaded) {
+        DevArray &wa = net->w(l - 1);
+        if (layer_wants_codes16(net, l, n) && !wa.codes16_valid && net->W[l - 1].uploaded) {
             if (!wa.codes16) HCHECK(hipMalloc((void **)&wa.codes16, wa.count * sizeof(uint16_t)));
             launch_codes16(net->prec, wa.base, wa.codes16, wa.count);
             HCHECK(hipGetLastError());
@@ -1514,10 +1633,19 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
     const uint32_t last = net->layers - 1;
 
     const void *in = d_x;
-    const bool x_fused = reg == R_GEMM16 && gemm16_small_layer(n, net->topo[1], net->topo[0], tl_route.halves) &&
+    const uint32_t in_w = net->topo[0], in_pw = net->ptopo[0];
+    const bool x_fused = reg == R_GEMM16 && in_pw == in_w && gemm16_small_layer(n, net->ptopo[1], in_w, tl_route.halves) &&
                          (reinterpret_cast<uintptr_t>(d_x) & 15u) == 0;
     if (x_fused) {
         // (the first layer's kernel rounds, or splits, the FP32 input itself)
+    } else if (in_pw != in_w && reg == R_GEMM16 && !only_layer) {
+        // rows of a padded input, converted on the way
+        const uint64_t quads = (uint64_t)n * ((in_pw + 3u) / 4u);
+        const uint32_t grid = (uint32_t)((quads + 255u) / 256u);
+        if (split) sp_pad_input<3><<<grid, 256, 0, g_stream>>>(d_x, wk.buf[1], n, in_w, in_pw);
+        else if (f16t) sp_pad_input<2><<<grid, 256, 0, g_stream>>>(d_x, wk.buf[1], n, in_w, in_pw);
+        else sp_pad_input<1><<<grid, 256, 0, g_stream>>>(d_x, wk.buf[1], n, in_w, in_pw);
+        in = wk.buf[1];
     } else if (split && !only_layer) {
         const uint64_t cnt = (uint64_t)n * net->topo[0];
         sp_cvt16_split<<<(uint32_t)((cnt / 4 + 255) / 256 + 1), 256, 0, g_stream>>>(d_x, (uint16_t *)wk.buf[1], cnt);
@@ -1533,17 +1661,18 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
     }
 
     for (uint32_t l = 1; l <= last; ++l) {
-        LayerArgs L = make_layer_args(net, l);
+        const DevArray &wa = net->w(l - 1);
+        LayerArgs L = make_layer_args(net, l, l == 1 && reg == R_GEMV);
         if (wide) {
-            L.w = reinterpret_cast<const uint8_t *>(net->W[l - 1].wide16);
-            L.wscale = ldexpf(L.wscale, -net->W[l - 1].wide_shift);
+            L.w = reinterpret_cast<const uint8_t *>(wa.wide16);
+            L.wscale = ldexpf(L.wscale, -wa.wide_shift);
         }
         const bool cat3 = reg == R_CAT3 && cat3_layer(n, L.N, L.K);
         if (cat3) {
-            if (!net->W[l - 1].cat3_valid) return fail_msg("sphip: the FP16 parts of this net's FP32 weights were not made (split mode)");
-            L.w = reinterpret_cast<const uint8_t *>(net->W[l - 1].cat3);
-            L.wscale = ldexpf(L.wscale, -net->W[l - 1].cat3_shift);
-            L.K = 3u * cat3_kp(net->topo[l - 1]);
+            if (!wa.cat3_valid) return fail_msg("sphip: the FP16 parts of this net's FP32 weights were not made (split mode)");
+            L.w = reinterpret_cast<const uint8_t *>(wa.cat3);
+            L.wscale = ldexpf(L.wscale, -wa.cat3_shift);
+            L.K = 3u * cat3_kp(net->ptopo[l - 1]);
         }
         const bool softmax = net->act[l - 1] == A_SOFTMAX;
         const bool is_last = l == last;
@@ -1563,11 +1692,11 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
                                           softmax && !only_layer ? (float *)dst : nullptr);
             else if (cat3) {
                 // (timing one layer includes the conversion of its input)
-                const uint32_t K = net->topo[l - 1], Kp = cat3_kp(K);
+                const uint32_t K = net->ptopo[l - 1], Kp = cat3_kp(K);
                 const int vec = K % 4u == 0 && (reinterpret_cast<uintptr_t>(in) & 15u) == 0;
                 sp_cat3_x<<<(uint32_t)(((uint64_t)n * (Kp / 8u) + 255) / 256), 256, 0, g_stream>>>((const float *)in, wk.cat, n, K, Kp, vec);
                 ThinCtx ctx{};
-                ctx.w16 = net->W[l - 1].cat3;
+                ctx.w16 = wa.cat3;
                 ctx.ws = wk.split_ws;
                 ctx.ws_floats = wk.split_cap;
                 if (softmax && !only_layer) {
@@ -1577,7 +1706,6 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
                 }
                 launch_gemm16((int)F16, L, wk.cat, main_out, n, 1, ctx);
             } else {
-                const DevArray &wa = net->W[l - 1];
                 ThinCtx ctx{};
                 if (wide) ctx.w16 = wa.wide16;
                 else if (net->prec == F16 || net->prec == BF16) ctx.w16 = reinterpret_cast<const uint16_t *>(wa.base);
@@ -1585,6 +1713,7 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
                 ctx.ws = wk.split_ws;
                 ctx.ws_floats = wk.split_cap;
                 ctx.x_f32 = x_fused && l == 1;
+                ctx.padded_in = l == 1 && in_pw != in_w;
                 if (softmax && !only_layer) {
                     ctx.soft_out = dst;
                     ctx.soft_kind = !is_last ? (split ? 3 : f16t ? 2 : 1) : 0;
@@ -1677,25 +1806,46 @@ int sphip_create(const sphip_desc *desc, sphip_net **out)
     net->prec = desc->precision;
     net->W.resize(desc->layers - 1);
     net->B.resize(desc->layers - 1);
+    net->PW.resize(desc->layers - 1);
+    net->PB.resize(desc->layers - 1);
     net->codes16_ptrs.assign(desc->layers - 1, nullptr);
     for (uint32_t l = 0; l < desc->layers; ++l) {
-        if (net->topo[l] > net->max_width) net->max_width = net->topo[l];
+        const bool hidden_softmax = l && net->act[l - 1] == A_SOFTMAX;
+        net->ptopo.push_back(l + 1 == desc->layers || hidden_softmax ? net->topo[l] : padded_width(net->prec, net->topo[l], net->topo[l + 1], l > 0));
+        if (net->ptopo[l] > net->max_width) net->max_width = net->ptopo[l];
         net->total_neurons += net->topo[l];
         net->slot_off.push_back((uint32_t)net->slots_total);
-        net->slots_total += ((uint64_t)net->topo[l] + 3u) & ~3ull;
+        net->slots_total += ((uint64_t)net->ptopo[l] + 3u) & ~3ull;
     }
+    // All arrays in one allocation, each at a multiple of 256 bytes with 16 bytes of slack: vector loads of the last chunk
+    // never leave it.  (A hipMalloc takes 10 to 100 us.)
+    size_t at = 0;
+    auto place = [&](DevArray &a, uint64_t count, uint64_t room) {
+        a.count = count;
+        a.bytes = fmt_bytes(net->prec, count);
+        a.base = reinterpret_cast<uint8_t *>(at);
+        at += (fmt_bytes(net->prec, room) + 16u + 255u) & ~(size_t)255u;
+    };
+    std::vector<DevArray *> placed;
     for (uint32_t l = 0; l + 1 < desc->layers; ++l) {
-        DevArray &w = net->W[l], &b = net->B[l];
-        w.count = (uint64_t)net->topo[l] * net->topo[l + 1];
-        b.count = net->topo[l + 1];
-        w.bytes = fmt_bytes(net->prec, w.count);
-        b.bytes = fmt_bytes(net->prec, b.count);
-        // 16 bytes of slack: vector loads of the last chunk never leave the allocation
-        if (hipMalloc((void **)&w.base, w.bytes + 16) != hipSuccess || hipMalloc((void **)&b.base, b.bytes + 16) != hipSuccess) {
-            sphip_destroy(net);
-            return fail_msg("sphip_create: device allocation failed");
-        }
+        const uint64_t K = net->topo[l], N = net->topo[l + 1], Kp = net->ptopo[l], Np = net->ptopo[l + 1];
+        place(net->W[l], K * N, K * Np);
+        place(net->B[l], N, N);
+        placed.insert(placed.end(), {&net->W[l], &net->B[l]});
+        if (Np != N || Kp != K) { place(net->PW[l], Kp * Np, Kp * Np); placed.push_back(&net->PW[l]); }
+        if (Np != N) { place(net->PB[l], Np, Np); placed.push_back(&net->PB[l]); }
     }
+    if (hipMalloc((void **)&net->arrays, at) != hipSuccess) {
+        for (DevArray *a : placed) a->base = nullptr;
+        sphip_destroy(net);
+        return fail_msg("sphip_create: device allocation failed");
+    }
+    for (DevArray *a : placed) a->base = net->arrays + reinterpret_cast<size_t>(a->base);
+    for (uint32_t l = 0; l + 1 < desc->layers; ++l)
+        if (net->PB[l].base) {                              // zero rows behind the uploaded ones
+            const uint64_t floats = (fmt_bytes(net->prec, (uint64_t)net->topo[l] * net->ptopo[l + 1]) + 16u) / 4u;
+            sp_fill0<<<(uint32_t)((floats + 255u) / 256u), 256, 0, g_stream>>>(reinterpret_cast<float *>(net->W[l].base), floats);
+        }
     *out = net;
     return 0;
 }
@@ -1705,8 +1855,13 @@ void sphip_destroy(sphip_net *net)
     if (!net) return;
     if (g_stream) (void)hipStreamSynchronize(g_stream);
     train_free(net);
-    for (auto &a : net->W) { if (a.base) (void)hipFree(a.base); if (a.codes16) (void)hipFree(a.codes16); if (a.wide16) (void)hipFree(a.wide16); if (a.cat3) (void)hipFree(a.cat3); }
-    for (auto &a : net->B) if (a.base) (void)hipFree(a.base);
+    for (auto *arrays : {&net->W, &net->PW, &net->B, &net->PB})
+        for (auto &a : *arrays) {
+            if (a.codes16) (void)hipFree(a.codes16);
+            if (a.wide16) (void)hipFree(a.wide16);
+            if (a.cat3) (void)hipFree(a.cat3);
+        }
+    if (net->arrays) (void)hipFree(net->arrays);
     if (net->split_ws) (void)hipFree(net->split_ws);
     if (net->cat_buf) (void)hipFree(net->cat_buf);
     if (net->eval_buf) (void)hipFree(net->eval_buf);
@@ -1760,7 +1915,8 @@ int sphip_upload_array(sphip_net *net, uint32_t l, int which, const void *codes,
     a.codes16_valid = false;
     a.wide16_valid = false;
     a.cat3_valid = false;
-    if (which == 0 && net->prec == BF16 && make_wide(a)) return 1;
+    if (pad_layer(net, l, which == 0, which == 1)) return 1;
+    if (which == 0 && net->prec == BF16 && make_wide(net->w(l))) return 1;
     return 0;
 }
 
@@ -1771,9 +1927,10 @@ int sphip_clone(const sphip_net *src, sphip_net **out)
     sphip_net *net = nullptr;
     if (sphip_create(&d, &net)) return 1;
     for (uint32_t l = 0; l + 1 < src->layers; ++l) {
-        for (int which = 0; which < 2; ++which) {
-            const DevArray &s = which == 0 ? src->W[l] : src->B[l];
-            DevArray &t = which == 0 ? net->W[l] : net->B[l];
+        for (int which = 0; which < 4; ++which) {
+            const DevArray &s = which == 0 ? src->W[l] : which == 1 ? src->B[l] : which == 2 ? src->PW[l] : src->PB[l];
+            DevArray &t = which == 0 ? net->W[l] : which == 1 ? net->B[l] : which == 2 ? net->PW[l] : net->PB[l];
+            if (!s.base) continue;
             hipError_t e = hipMemcpyAsync(t.base, s.base, s.bytes, hipMemcpyDeviceToDevice, g_stream);
             if (e != hipSuccess) { sphip_destroy(net); return fail_hip("sphip_clone copy", e); }
             t.max_val = s.max_val;
@@ -1951,7 +2108,7 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
     const WorkspaceNeed need = workspace_need(net, n, flags);
     if (need.cat_elems)
         for (uint32_t l = 1; l < net->layers; ++l)
-            if (cat3_layer(n, net->topo[l], net->topo[l - 1]) && !net->W[l - 1].cat3_valid)
+            if (cat3_layer(n, net->ptopo[l], net->ptopo[l - 1]) && !net->w(l - 1).cat3_valid)
                 return fail_msg("sphip_forward_noalloc: the split mode of an FP32 net needs FP16 parts of its weights, which the first sphip_forward in that mode makes");
     size_t used = 0;
     auto take = [&](uint64_t bytes) -> unsigned char * {
@@ -1980,7 +2137,7 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
     bool fresh[kMaxLayers] = {};
     for (uint32_t l = 1; l < net->layers; ++l) {
         if (!reads_codes || !layer_wants_codes16(net, l, n)) continue;
-        const DevArray &wa = net->W[l - 1];
+        const DevArray &wa = net->w(l - 1);
         if (wa.codes16_valid) { codes[l - 1] = wa.codes16; continue; }
         codes[l - 1] = reinterpret_cast<uint16_t *>(take(wa.count * sizeof(uint16_t)));
         fresh[l - 1] = true;
@@ -1992,7 +2149,7 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
         return 1;
     }
     for (uint32_t l = 1; l < net->layers; ++l)
-        if (fresh[l - 1]) launch_codes16(net->prec, net->W[l - 1].base, codes[l - 1], net->W[l - 1].count);
+        if (fresh[l - 1]) launch_codes16(net->prec, net->w(l - 1).base, codes[l - 1], net->w(l - 1).count);
     // the integer GEMV's quantise launch is never skipped here (that shortcut belongs to the layer timer)
     net->aq_valid_layer = 0;
     return enqueue_forward(net, wk, d_x, n, d_y, fwd_flags, 0);
@@ -2217,7 +2374,7 @@ const char *sphip_layer_kernel_name(sphip_net *net, uint32_t layer, uint32_t n, 
     // pointers as aligned, which is how sphip_forward calls it
     tl_route.dry = true;
     tl_route.name = "";
-    const LayerArgs L = make_layer_args(net, layer);
+    const LayerArgs L = make_layer_args(net, layer, layer == 1 && pick_regime(net, n, flags) == R_GEMV);
     const float *aligned_ptr = reinterpret_cast<const float *>(uintptr_t{256});     // never dereferenced
     switch (pick_regime(net, n, flags)) {
     case R_GEMV:
@@ -2245,6 +2402,7 @@ const char *sphip_layer_kernel_name(sphip_net *net, uint32_t layer, uint32_t n, 
         ThinCtx ctx{};
         ctx.w16 = reinterpret_cast<const uint16_t *>(aligned_ptr);
         ctx.ws_floats = ~0ull;
+        ctx.padded_in = layer == 1 && net->ptopo[0] != net->topo[0];
         tl_route.halves = (flags & SPHIP_SPLIT_ACTIVATIONS) ? 2u : 1u;
         launch_gemm16(net->prec, L, reinterpret_cast<const uint16_t *>(aligned_ptr), nullptr, n, 1, ctx);
         break;

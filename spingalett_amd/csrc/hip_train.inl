@@ -324,12 +324,6 @@ __global__ __launch_bounds__(256) void sp_train_opt(const OptArgs a)
     a.W[i] = w;
 }
 
-__global__ __launch_bounds__(256) void sp_train_fill0(float *p, uint64_t cnt)
-{
-    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-    if (i < cnt) p[i] = 0.0f;
-}
-
 }  // namespace
 
 // Device state of a net being trained: gradients and optimizer moments laid out like the host net's
@@ -481,7 +475,7 @@ int sphip_train_begin(sphip_net *net)
         const uint64_t cnt = i < 3 ? ts->total_w : ts->total_b;
         hipError_t e = hipMalloc((void **)flat[i], cnt * sizeof(float));
         if (e != hipSuccess) { train_free(net); return fail_hip("sphip_train_begin: device allocation", e); }
-        sp_train_fill0<<<(uint32_t)((cnt + 255) / 256), 256, 0, g_stream>>>(*flat[i], cnt);
+        sp_fill0<<<(uint32_t)((cnt + 255) / 256), 256, 0, g_stream>>>(*flat[i], cnt);
     }
     hipError_t e = hipMalloc((void **)&ts->sq_part, 2u * kSqBlocks * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void **)&ts->scal, 4 * sizeof(float));

@@ -1225,3 +1225,33 @@ def test_full_batch_int2_first_layer_properties(S):
     got = np.stack([Y[first[v]] for v in range(8)])
     assert rel_max_abs(got, want) <= 2e-3
     net.destroy()
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
+@pytest.mark.parametrize("topo,acts", [
+    ([777, 1030, 515, 33], ["sigmoid", "tanh", "softmax"]),       # every layer padded (activation(0) of the padding is 0.5)
+    ([33, 7, 1, 70, 5], ["foo52", "sigmoid", "relu", "none"]),    # widths below one unit
+    ([130, 1101, 90, 9], ["softmax", "relu", "none"]),            # a hidden softmax keeps its width: the layer behind it is ragged
+    ([512, 1000, 640, 11], ["relu", "sigmoid", "softmax"]),       # whole words, padded for its half a million weights
+])
+def test_padded_widths_leave_the_outputs_alone(S, O, fmt, topo, acts):
+    """Hidden widths and inputs whose weight rows are not whole 16-byte units run padded with zero weights: outputs
+    against the float64 forward at one to four samples (vector kernels, FP32-grade) and on both sides of the small,
+    streaming and tiled kernels' ranges, plain and split; every activation of a single forward; a clone."""
+    src = make_oracle_net(O, topo, acts, seed=sum(topo), bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    X = np.random.default_rng(1).standard_normal((1500, topo[0])).astype(F32)
+    want = ref.forward_batch_f64(X)
+    for n in (1, 3, 4, 5, 33, 260, 1500):
+        assert rel_max_abs(S.forward_batch(net, X[:n]), want[:n]) <= (TOL_VEC if n <= 4 else TOL_MFMA), n
+    assert S.lib().spingalett_set_net_activations(net, S.NET_ACTIVATIONS_SPLIT) == 0
+    for n in (5, 260):
+        assert rel_max_abs(S.forward_batch(net, X[:n]), want[:n]) <= 2e-5, n
+    assert rel_max_abs(S.forward(net, X[2]), want[2]) <= TOL_VEC
+    h = S.lib().spingalett_hip_handle(net)
+    d = S.DeviceNet(topo, [O.ACT[a] for a in acts], O.PREC[fmt], handle=h)
+    d.owned = False
+    twin = d.clone()
+    assert np.array_equal(twin.forward(X[:300]), d.forward(X[:300]))
+    twin.destroy()
+    S.free_network(net)
