@@ -716,7 +716,7 @@ LayerArgs make_layer_args(const sphip_net *net, uint32_t l /*1-based layer*/, bo
 bool rows_aligned(int fmt, uint32_t K) { return ((uint64_t)K * (uint64_t)fmt_bits(fmt)) % 128u == 0; }
 
 template <int FMT>
-void launch_gemv_fmt(const LayerArgs &L, const float *x, float *y, uint32_t n)
+void launch_gemv_fmt(const LayerArgs &L, const float *x, float *y, uint32_t n, bool padded = false)
 {
     const bool aligned = rows_aligned(FMT, L.K) && (L.K % 4u == 0);
     // integer rows of whole words: a word per lane when 16-byte chunks would leave most of a wave idle (rows of at
@@ -725,9 +725,10 @@ void launch_gemv_fmt(const LayerArgs &L, const float *x, float *y, uint32_t n)
     uint32_t lpr = 64;
     if constexpr (FMT == I8 || FMT == I4 || FMT == I2) {
         const uint64_t row_bits = (uint64_t)L.K * fmt_bits(FMT);
-        // ... and for layers of at most 64 outputs, whose rows the 16-byte kernel would give to 32 waves or fewer:
+        // ... and for rows that are whole units by padding only (12000 -> 5200 -> 467 INT4 at four samples: 45 us, the chunks
+        // 52), and for layers of at most 64 outputs, whose rows the 16-byte kernel would give to 32 waves or fewer:
         // there a row of 256 words and more spans a whole workgroup (8192 -> 10 INT4 at four samples: 20 -> 11 us)
-        words = row_bits % 32u == 0 && (!aligned || row_bits <= 16u * 128u || L.N <= 64u) && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+        words = row_bits % 32u == 0 && (!aligned || padded || row_bits <= 16u * 128u || L.N <= 64u) && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
         const uint32_t wpr = (uint32_t)(row_bits / 32u);
         while (lpr > 1u && lpr / 2u >= wpr) lpr /= 2u;
         if (L.N <= 64u && wpr >= 256u) lpr = 256u;
@@ -899,15 +900,18 @@ bool launch_gemv_i8(const Workspace &wk, const LayerArgs &L, const float *x, flo
     return true;
 }
 
-void launch_gemv(int prec, const Workspace &wk, const LayerArgs &L, const float *x, float *y, uint32_t n, bool main_only)
+// padded: rows that are whole units by padding only.  They take the FP32 kernels, as they would unpadded: the integer
+// matrix cores see an activation with 22 bits of its chunk's largest, FP32 has 24 of its own.
+void launch_gemv(int prec, const Workspace &wk, const LayerArgs &L, const float *x, float *y, uint32_t n, bool main_only,
+                 bool padded = false)
 {
     switch (prec) {
     case F32:  launch_gemv_fmt<F32>(L, x, y, n); break;
     case F16:  launch_gemv_fmt<F16>(L, x, y, n); break;
     case BF16: launch_gemv_fmt<BF16>(L, x, y, n); break;
-    case I8:   if (!launch_gemv_i8<I8>(wk, L, x, y, n, main_only)) launch_gemv_fmt<I8>(L, x, y, n); break;
-    case I4:   if (!launch_gemv_i8<I4>(wk, L, x, y, n, main_only)) launch_gemv_fmt<I4>(L, x, y, n); break;
-    default:   if (!launch_gemv_i8<I2>(wk, L, x, y, n, main_only)) launch_gemv_fmt<I2>(L, x, y, n); break;
+    case I8:   if (padded || !launch_gemv_i8<I8>(wk, L, x, y, n, main_only)) launch_gemv_fmt<I8>(L, x, y, n, padded); break;
+    case I4:   if (padded || !launch_gemv_i8<I4>(wk, L, x, y, n, main_only)) launch_gemv_fmt<I4>(L, x, y, n, padded); break;
+    default:   if (padded || !launch_gemv_i8<I2>(wk, L, x, y, n, main_only)) launch_gemv_fmt<I2>(L, x, y, n, padded); break;
     }
 }
 
@@ -1683,7 +1687,8 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
         const bool run = !only_layer || only_layer == l;
         bool soft_done = false;                 // the layer's own kernel wrote the softmax
         if (run) {
-            if (reg == R_GEMV) launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n, only_layer != 0 && net->aq_valid_layer == l && net->aq_valid_n == n);
+            if (reg == R_GEMV) launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n,
+                                          only_layer != 0 && net->aq_valid_layer == l && net->aq_valid_n == n, net->ptopo[l - 1] != net->topo[l - 1]);
             if (reg == R_GEMV) { net->aq_valid_layer = l; net->aq_valid_n = n; }
             else if ((reg == R_GEMM32 || (reg == R_CAT3 && !cat3)) && f32_thin_vector(L, n))
                 launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n, false);
@@ -2378,7 +2383,7 @@ const char *sphip_layer_kernel_name(sphip_net *net, uint32_t layer, uint32_t n, 
     const float *aligned_ptr = reinterpret_cast<const float *>(uintptr_t{256});     // never dereferenced
     switch (pick_regime(net, n, flags)) {
     case R_GEMV:
-        launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false);
+        launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false, net->ptopo[layer - 1] != net->topo[layer - 1]);
         break;
     case R_GEMM32:
         if (f32_thin_vector(L, n)) launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false);
