@@ -220,36 +220,67 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32_big(const Gemm32Args g)
     }
 }
 
-// Small FP32 layers in one launch: a workgroup owns a 32 x 32 tile of the output, its eight waves split K in whole
-// steps of eight, and their sums meet in LDS.  No operand staging: lane (r, h) loads four consecutive k of row r of both
-// operands (k = 8 s + 4 h .. + 3 of step s) straight into registers and feeds them to four MFMA steps (a sum over k in
-// any order).  For outputs of up to 512 tiles and K up to 1024, where sp_gemm32_f32 needs a K split over the grid and a
-// second launch to fill the chip (256 x 512 x 784: 8 us against 12 us for the two).  A softmax layer of at most 32
-// outputs is normalised here (Activation.c:5-21), soft_out != nullptr.  Rows are 16-byte aligned (K % 4 == 0).
-__global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float *__restrict__ soft_out)
+// What a training step wants besides the outputs of its last layer: their deltas (sp_train_out_delta's modes)
+struct DeltaTail {
+    const float *targets;  // [M][N], nullptr: no deltas
+    float *delta;          // [M][N]
+    int mode, act;
+};
+
+// Small FP32 layers in one launch: a workgroup owns a T x T tile of the output, its eight waves split K in whole steps,
+// and their sums meet in LDS.  No operand staging: a lane loads four consecutive k of a row of both operands straight
+// into registers and feeds them to four MFMA steps (a sum over k in any order).  T = 32: steps of 8 k, lane (r, h)
+// takes k = 8 s + 4 h .. + 3; for outputs of up to 512 tiles and K up to 1024, where sp_gemm32_f32 needs a K split over
+// the grid and a second launch to fill the chip (256 x 512 x 784: 8 us against 12 us for the two).  T = 16: steps of 16 k;
+// where 32 x 32 tiles would leave half of the compute units and more without work: 64 x 512 x 784 is 32 of them, whose
+// waves are 49 MFMAs of 64 cycles deep, two to a SIMD (11.7 us, 128 tiles of 16 x 16: 7.7 us).
+// A softmax layer of at most T outputs is normalised here (Activation.c:5-21), soft_out != nullptr, and the deltas of a
+// training step's last layer are formed (tail.targets != nullptr).  VEC: rows are 16-byte aligned (K % 4 == 0).
+template <int T, bool VEC>
+__global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float *__restrict__ soft_out, const DeltaTail tail)
 {
-    constexpr int NW = 8, U = 4;
-    __shared__ float part[NW][32 * 33];
+    constexpr int NW = 8, U = 4, H = 64 / T, STEP = 4 * H;       // H lane groups, each with its own four k of a step
+    __shared__ float part[NW][T * (T + 1)];
     const uint32_t M = g.M, N = g.L.N, K = g.L.K;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, q = lane & 31, h = lane >> 5;
-    const uint32_t tiles_n = (N + 31u) / 32u;
-    const uint32_t m0 = (blockIdx.x / tiles_n) * 32u, n0 = (blockIdx.x % tiles_n) * 32u;
-    const uint32_t steps = (K + 7u) / 8u, per = (steps + NW - 1) / NW;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, q = lane % T, h = lane / T;
+    const uint32_t tiles_n = (N + T - 1) / T;
+    const uint32_t m0 = (blockIdx.x / tiles_n) * T, n0 = (blockIdx.x % tiles_n) * T;
+    const uint32_t steps = (K + STEP - 1) / STEP, per = (steps + NW - 1) / NW;
     const uint32_t s0 = wave * per, s1 = s0 + per < steps ? s0 + per : steps;
     const uint32_t am = m0 + q < M ? m0 + q : M - 1, wn = n0 + q < N ? n0 + q : N - 1;
-    const float *ap = g.A + (size_t)am * K + 4 * h;
-    const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)wn * K + 4 * h;
-    f32x16 acc;
+    const float *ap = g.A + (size_t)am * K;
+    const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)wn * K;
+    typedef float acc_t __attribute__((ext_vector_type(T * T / 64)));
+    acc_t acc;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    auto ld = [&](const float *p, uint32_t s) -> float4 {       // K % 4 == 0: a piece is inside the row or beyond it
-        return 8u * s + 4u * h < K ? *reinterpret_cast<const float4 *>(p + 8u * s) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int r = 0; r < T * T / 64; ++r) acc[r] = 0.0f;
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+    auto ld = [&](const float *p, uint32_t s) -> float4 {
+        const uint32_t k = (uint32_t)STEP * s + 4u * h;
+        if constexpr (VEC) {                                      // K % 4 == 0: a piece is inside the row or beyond it
+            return k < K ? *reinterpret_cast<const float4 *>(p + k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        } else if ((uint32_t)STEP * (s + 1u) <= K) {              // (uniform) rows start anywhere: 4-byte aligned loads
+            const f4u v = *reinterpret_cast<const f4u *>(p + k);
+            return make_float4(v.x, v.y, v.z, v.w);
+        } else {
+            float v[4];
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) { const float x = p[k + e < K ? k + e : K - 1]; v[e] = k + e < K ? x : 0.0f; }
+            return make_float4(v[0], v[1], v[2], v[3]);
+        }
     };
     auto fma4 = [&](const float4 &a, const float4 &b) {
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+        if constexpr (T == 32) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+        } else {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc, 0, 0, 0);
+        }
     };
     uint32_t s = s0;
     for (; s + U <= s1; s += U) {
@@ -259,32 +290,59 @@ __global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float
 #pragma unroll
         for (int u = 0; u < U; ++u) fma4(a[u], b[u]);
     }
-    for (; s < s1; ++s) fma4(ld(ap, s), ld(wp, s));
+    if (s < s1) {                                                 // fewer than U steps left: still one round of loads
+        float4 a[U - 1], b[U - 1];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) part[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 33 + q] = acc[r];
+        for (int u = 0; u < U - 1; ++u) {
+            if (s + u >= s1) break;                               // (uniform)
+            a[u] = ld(ap, s + u);
+            b[u] = ld(wp, s + u);
+        }
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+            if (s + u < s1) fma4(a[u], b[u]);                     // (uniform)
+    }
+#pragma unroll
+    for (int r = 0; r < T * T / 64; ++r) {
+        const int row = T == 32 ? 8 * (r >> 2) + 4 * h + (r & 3) : 4 * h + r;
+        part[wave][row * (T + 1) + q] = acc[r];
+    }
     __syncthreads();
-    // the waves' sums in wave order, bias, activation; 512 threads, two outputs each
+    // the waves' sums in wave order, bias, activation: T neighbouring threads hold a row of the tile
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int e = t + 512 * i, row = e >> 5, col = e & 31;
+    for (int i = 0; i < (T == 32 ? 2 : 1); ++i) {
+        const int e = t + 512 * i, row = e / T, col = e % T;
+        if (row >= T) break;                                      // (T = 16: four of the eight waves)
         float v = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) v += part[w][row * 33 + col];
+        for (int w = 0; w < NW; ++w) v += part[w][row * (T + 1) + col];
+        const bool in = m0 + row < M && n0 + col < N;
+        const size_t o = (size_t)(m0 + row) * N + n0 + col;
         const uint32_t n = n0 + col < N ? n0 + col : N - 1;
         v = apply_act(v + elem_value_rt(g.L.bias_fmt, g.L.bias, n) * g.L.bscale, g.L.act);
-        if (soft_out) part[0][row * 33 + col] = v;               // (every thread has read part[0][its own two slots] only)
-        else if (m0 + row < M && n0 + col < N) g.C[(size_t)(m0 + row) * N + n0 + col] = v;
-    }
-    if (!soft_out) return;                                        // (uniform)
-    __syncthreads();
-    if (t < 32 && m0 + t < M) {                                   // N <= 32: the tile holds whole rows of logits
-        const float *lr = &part[0][t * 33];
-        float mx = lr[0];
-        for (uint32_t c = 1; c < N; ++c) mx = fmaxf(mx, lr[c]);
-        float sum = 0.0f;
-        for (uint32_t c = 0; c < N; ++c) sum += expf(lr[c] - mx);
-        const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
-        for (uint32_t c = 0; c < N; ++c) soft_out[(size_t)(m0 + t) * N + c] = expf(lr[c] - mx) * inv;
+        if (soft_out) {                                           // (uniform; N <= T: the tile holds whole rows)
+            float mx = (uint32_t)col < N ? v : -3.402823466e+38f;
+#pragma unroll
+            for (int off = T / 2; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+            float ex = (uint32_t)col < N ? expf(v - mx) : 0.0f, sum = ex;
+#pragma unroll
+            for (int off = T / 2; off; off >>= 1) sum += __shfl_xor(sum, off);
+            v = ex * (sum > 0.0f ? 1.0f / sum : 1.0f);
+            if (in) soft_out[o] = v;
+        } else if (in) {
+            g.C[o] = v;
+        }
+        if (tail.targets) {                                       // (uniform)
+            const float d = in ? v - tail.targets[o] : 0.0f;
+            float out = tail.mode == 1 ? d : d * act_derivative(v, tail.act);
+            if (tail.mode == 0) {                                 // squared error through a softmax
+                float c = d * v;
+#pragma unroll
+                for (int off = T / 2; off; off >>= 1) c += __shfl_xor(c, off);
+                out = v * (d - c);
+            }
+            if (in) tail.delta[o] = out;
+        }
     }
 }
 

@@ -108,7 +108,21 @@ __device__ __forceinline__ float apply_act(float x, int act)
     }
 }
 
-// the same for the activations that need no transcendental function (a caller has dealt with the other two)
+// derivative of an activation as a function of its output (Activation.c:40-56, SIMD.c:90-188)
+__device__ __forceinline__ float act_derivative(float a, int act)
+{
+    switch (act) {
+    case A_RELU:    return a > 0.0f ? 1.0f : 0.0f;
+    case A_LEAKY:   return a > 0.0f ? 1.0f : 0.01f;
+    case A_SIGMOID:
+    case A_SOFTMAX: return a * (1.0f - a);
+    case A_TANH:    return 1.0f - a * a;
+    case A_FOO52:   return (a > 1.0f || a < 0.0f) ? 0.01f : 1.0f;
+    default:        return 1.0f;
+    }
+}
+
+// apply_act for the activations that need no transcendental function (a caller has dealt with the other two)
 __device__ __forceinline__ float apply_act_cheap(float x, int act)
 {
     switch (act) {

@@ -1255,3 +1255,24 @@ def test_padded_widths_leave_the_outputs_alone(S, O, fmt, topo, acts):
     assert np.array_equal(twin.forward(X[:300]), d.forward(X[:300]))
     twin.destroy()
     S.free_network(net)
+
+
+@pytest.mark.parametrize("N,K,n", [
+    (16, 16, 5), (17, 33, 16), (1, 3, 9), (512, 784, 64), (300, 2000, 33),      # 16 x 16 tiles: whole and partial steps, few rows
+    (233, 1038, 64), (65, 1, 40), (90, 1023, 100), (31, 1026, 17),               # ... rows that start anywhere
+    (1000, 512, 128), (1024, 1024, 128), (65, 1024, 1365),                       # ... at their bound, and 32 x 32 tiles beyond it
+    (500, 1000, 512), (512, 1020, 1024),
+])
+@pytest.mark.parametrize("act", ["tanh", "softmax"])
+def test_small_fp32_layers_run_in_one_launch(S, O, N, K, n, act):
+    """Small FP32 layers whose workgroups split K among their waves; a softmax of at most a tile's width in the same
+    launch, wider ones by the row kernel.  1e-4 against the float64 forward, like every FP32 path."""
+    src = make_oracle_net(O, [K, N], [act], seed=N + K, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, "f32")
+    X = np.random.default_rng(n).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    name = S.lib().sphip_layer_kernel_name(S.lib().spingalett_hip_handle(net), 1, n, 0).decode()
+    S.free_network(net)
+    assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_VEC
+    if N > 64 or n > 8:
+        assert name == "sp_gemm32_small"
