@@ -1362,25 +1362,35 @@ bool f32_thin_vector(const LayerArgs &L, uint32_t n) { return L.N <= 64u && n <=
 // layouts lose by it (235 -> 240 us, and 48 -> 53 us where K is 10 and memory decides).  `own`: the kernel's static LDS.
 size_t gemm32_lds_pad(uint64_t workgroups, size_t own) { return workgroups >= 2048u && own < (32u << 10) ? (32u << 10) - own : 0; }
 
-// Tile of sp_gemm32_small for a layer that would otherwise need a K split and a second launch (or a handful of
-// workgroups), 0 where the other kernels are the faster ones: 32 x 32 tiles up to 512 of them and K = 1024 (measured against the split path: 256 x 512 x 784 8
-// against 12 us, 1024 x 512 x 784 17 against 20 us, 1024 x 1024 x 1024 42 against 32 us); 16 x 16 tiles where the 32 x 32
+// Tile of sp_gemm32_small (32) or sp_gemm32_small16 for a layer that would otherwise need a K split and a second launch (or a handful of
+// workgroups), 0 where the other kernels are the faster ones: 32 x 32 tiles up to 512 of them and K = 1024 (measured
+// against the split path: 256 x 512 x 784 8 against 12 us, 1024 x 512 x 784 17 against 20 us, 1024 x 1024 x 1024 42 against 32 us); 16 x 16 tiles where the 32 x 32
 // ones are at most 128 (128 x 1024 x 1024 7.3 against 8.8 us in a net of three, 400 x 300 x 300 even), which pays for longer
 // and unaligned rows too (64 x 300 x 2000, 64 x 233 x 1038: 7 against 10 us), as long as their twice as many reads of K do
-// not decide (64 x 2048 x 2048: 57 against 50 us for two layers).
-uint32_t gemm32_small_tile(uint32_t M, uint32_t N, uint32_t K, bool vec, uint32_t splits)
+// not decide (64 x 2048 x 2048: 57 against 50 us for two layers).  *seg: the cut of the kernel that would take the layer
+// without the 16 x 16 tiles.
+uint32_t gemm32_small_tile(uint32_t M, uint32_t N, uint32_t K, bool vec, KSegments *seg)
 {
     const uint64_t tiles = (uint64_t)((M + 31u) / 32u) * ((N + 31u) / 32u);
+    uint32_t kper = 0;
+    const uint32_t splits = gemm32_fwd_splits(M, N, K, &kper);
+    const bool fits32 = splits > 1u && vec && tiles <= 512u && K <= 1024u;
+    if (fits32) {
+        const uint32_t steps = (K + 7u) / 8u, per = (steps + 7u) / 8u;
+        *seg = KSegments{8u * per, (steps + per - 1u) / per, 1};
+    } else {
+        *seg = KSegments{kper, splits, 0};
+    }
     if (tiles <= 128u && K <= 2048u && tiles * K <= (128u << 10)) return 16u;
-    return splits > 1u && vec && tiles <= 512u && K <= 1024u ? 32u : 0u;
+    return fits32 ? 32u : 0u;
 }
 
-void launch_gemm32_small(const Gemm32Args &g, uint32_t tile, bool vec, float *soft_out, const DeltaTail &tail)
+void launch_gemm32_small(const Gemm32Args &g, uint32_t tile, const KSegments &seg, float *soft_out, const DeltaTail &tail)
 {
     const uint32_t grid = ((g.M + tile - 1u) / tile) * ((g.L.N + tile - 1u) / tile);
-    if (tile == 32u) sp_gemm32_small<32, true><<<grid, 512, 0, g_stream>>>(g, soft_out, tail);
-    else if (vec) sp_gemm32_small<16, true><<<grid, 512, 0, g_stream>>>(g, soft_out, tail);
-    else sp_gemm32_small<16, false><<<grid, 512, 0, g_stream>>>(g, soft_out, tail);
+    if (tile == 32u) sp_gemm32_small<<<grid, 512, 0, g_stream>>>(g, soft_out);       // (no deltas: the caller's own launch)
+    else if (seg.paired) sp_gemm32_small16<true><<<grid, 512, 0, g_stream>>>(g, seg, soft_out, tail);
+    else sp_gemm32_small16<false><<<grid, 512, 0, g_stream>>>(g, seg, soft_out, tail);
 }
 
 // soft_out: the layer is a softmax layer whose normalised outputs belong there; returns true if they were written
@@ -1401,12 +1411,13 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
         return false;
     }
     uint32_t splits = gemm32_fwd_splits(M, L.N, L.K, &g.kper);
-    const uint32_t small = gemm32_small_tile(M, L.N, L.K, vec, splits);
+    KSegments seg;
+    const uint32_t small = gemm32_small_tile(M, L.N, L.K, vec, &seg);
     if (small) {
         tl_route.name = "sp_gemm32_small";
         if (tl_route.dry) return false;
         const bool soft = soft_out && L.N <= small;
-        launch_gemm32_small(g, small, vec, soft ? soft_out : nullptr, DeltaTail{});
+        launch_gemm32_small(g, small, seg, soft ? soft_out : nullptr, DeltaTail{});
         return soft;
     }
     if (splits > 1 && (uint64_t)splits * M * L.N > ws_floats) { splits = 1; g.kper = (L.K + 31u) / 32u * 32u; }

@@ -227,60 +227,103 @@ struct DeltaTail {
     int mode, act;
 };
 
-// Small FP32 layers in one launch: a workgroup owns a T x T tile of the output, its eight waves split K in whole steps,
-// and their sums meet in LDS.  No operand staging: a lane loads four consecutive k of a row of both operands straight
-// into registers and feeds them to four MFMA steps (a sum over k in any order).  T = 32: steps of 8 k, lane (r, h)
-// takes k = 8 s + 4 h .. + 3; for outputs of up to 512 tiles and K up to 1024, where sp_gemm32_f32 needs a K split over
-// the grid and a second launch to fill the chip (256 x 512 x 784: 8 us against 12 us for the two).  T = 16: steps of 16 k;
-// where 32 x 32 tiles would leave half of the compute units and more without work: 64 x 512 x 784 is 32 of them, whose
-// waves are 49 MFMAs of 64 cycles deep, two to a SIMD (11.7 us, 128 tiles of 16 x 16: 7.7 us).
-// A softmax layer of at most T outputs is normalised here (Activation.c:5-21), soft_out != nullptr, and the deltas of a
-// training step's last layer are formed (tail.targets != nullptr).  VEC: rows are 16-byte aligned (K % 4 == 0).
-template <int T, bool VEC>
-__global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float *__restrict__ soft_out, const DeltaTail tail)
+// How a sum over k is cut: `count` segments of `len` k, each one chain of fused multiply-adds, the segments' sums added in
+// order.  Inside a chain k ascends, or (paired) goes 0, 4, 1, 5, 2, 6, 3, 7 in every group of eight, as where a lane of a
+// 32 x 32 x 2 MFMA holds four consecutive k.  One layer then has the same bits whichever of these kernels computes it,
+// also where 16 x 16 x 4 MFMAs (four links of the chain each) take the place of 32 x 32 x 2 ones (two): a training run
+// whose gradients nearly cancel multiplies a last-bit difference by a thousand within ten epochs.
+struct KSegments {
+    uint32_t len, count;
+    int paired;
+};
+
+// Four consecutive k of a row per lane, lane group h = lane / 16 holding k = 4 h .. 4 h + 3 of a block of 16, as the operands
+// of four 16 x 16 x 4 MFMAs whose chain goes through the block in either order: v[i] becomes the operand of MFMA i.
+//   ascending: MFMA i takes k = 4 i + h: a 4 x 4 transpose between registers and lane groups
+//   paired:    MFMAs 0 and 1 the first eight k, lane groups 0, 4, 1, 5 and 2, 6, 3, 7; MFMAs 2 and 3 the second eight
+__device__ __forceinline__ void swap_halves(float &x, float &y)         // upper 32 lanes of x <-> lower 32 lanes of y
 {
-    constexpr int NW = 8, U = 4, H = 64 / T, STEP = 4 * H;       // H lane groups, each with its own four k of a step
-    __shared__ float part[NW][T * (T + 1)];
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(r[0]);
+    y = __uint_as_float(r[1]);
+}
+
+__device__ __forceinline__ void swap_rows(float &x, float &y)           // odd 16-lane rows of x <-> even ones of y
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(r[0]);
+    y = __uint_as_float(r[1]);
+}
+
+template <bool PAIRED>
+__device__ __forceinline__ void chain_order(float (&v)[4])
+{
+    if constexpr (PAIRED) {
+        swap_halves(v[0], v[1]);          // v[0]: first eight, even MFMA; v[1]: second eight, even MFMA
+        swap_halves(v[2], v[3]);
+        const float x = v[1];
+        v[1] = v[2];
+        v[2] = x;
+    } else {
+        swap_halves(v[0], v[2]);
+        swap_halves(v[1], v[3]);
+        swap_rows(v[0], v[1]);
+        swap_rows(v[2], v[3]);
+    }
+}
+
+// A lane's four k from kb + 4 h of a row that starts anywhere, for the block of 16 at kb; zeros from k1, the end of the
+// segment, on.  K: end of the row.  (Branches are uniform.)
+typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_piece(float (&v)[4], const float *row, uint32_t kb, uint32_t h, uint32_t k1, uint32_t K)
+{
+    const uint32_t k = kb + 4u * h;
+    if (kb + 16u <= K) {
+        const float4_any x = *reinterpret_cast<const float4_any *>(row + k);
+        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+        if (kb + 16u > k1) {
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) v[e] = k + e < k1 ? v[e] : 0.0f;
+        }
+    } else {
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; ++e) {
+            const float x = row[k + e < k1 ? k + e : k1 - 1u];
+            v[e] = k + e < k1 ? x : 0.0f;
+        }
+    }
+}
+
+// Small FP32 layers in one launch: a workgroup owns a 32 x 32 tile of the output, its eight waves split K in whole
+// steps of eight, and their sums meet in LDS.  No operand staging: lane (r, h) loads four consecutive k of row r of both
+// operands (k = 8 s + 4 h .. + 3 of step s) straight into registers and feeds them to four MFMA steps (a sum over k in
+// any order).  For outputs of up to 512 tiles and K up to 1024, where sp_gemm32_f32 needs a K split over the grid and a
+// second launch to fill the chip (256 x 512 x 784: 8 us against 12 us for the two).  A softmax layer of at most 32
+// outputs is normalised here (Activation.c:5-21), soft_out != nullptr.  Rows are 16-byte aligned (K % 4 == 0).
+__global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float *__restrict__ soft_out)
+{
+    constexpr int NW = 8, U = 4;
+    __shared__ float part[NW][32 * 33];
     const uint32_t M = g.M, N = g.L.N, K = g.L.K;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, q = lane % T, h = lane / T;
-    const uint32_t tiles_n = (N + T - 1) / T;
-    const uint32_t m0 = (blockIdx.x / tiles_n) * T, n0 = (blockIdx.x % tiles_n) * T;
-    const uint32_t steps = (K + STEP - 1) / STEP, per = (steps + NW - 1) / NW;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, q = lane & 31, h = lane >> 5;
+    const uint32_t tiles_n = (N + 31u) / 32u;
+    const uint32_t m0 = (blockIdx.x / tiles_n) * 32u, n0 = (blockIdx.x % tiles_n) * 32u;
+    const uint32_t steps = (K + 7u) / 8u, per = (steps + NW - 1) / NW;
     const uint32_t s0 = wave * per, s1 = s0 + per < steps ? s0 + per : steps;
     const uint32_t am = m0 + q < M ? m0 + q : M - 1, wn = n0 + q < N ? n0 + q : N - 1;
-    const float *ap = g.A + (size_t)am * K;
-    const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)wn * K;
-    typedef float acc_t __attribute__((ext_vector_type(T * T / 64)));
-    acc_t acc;
+    const float *ap = g.A + (size_t)am * K + 4 * h;
+    const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)wn * K + 4 * h;
+    f32x16 acc;
 #pragma unroll
-    for (int r = 0; r < T * T / 64; ++r) acc[r] = 0.0f;
-    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-    auto ld = [&](const float *p, uint32_t s) -> float4 {
-        const uint32_t k = (uint32_t)STEP * s + 4u * h;
-        if constexpr (VEC) {                                      // K % 4 == 0: a piece is inside the row or beyond it
-            return k < K ? *reinterpret_cast<const float4 *>(p + k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        } else if ((uint32_t)STEP * (s + 1u) <= K) {              // (uniform) rows start anywhere: 4-byte aligned loads
-            const f4u v = *reinterpret_cast<const f4u *>(p + k);
-            return make_float4(v.x, v.y, v.z, v.w);
-        } else {
-            float v[4];
-#pragma unroll
-            for (uint32_t e = 0; e < 4u; ++e) { const float x = p[k + e < K ? k + e : K - 1]; v[e] = k + e < K ? x : 0.0f; }
-            return make_float4(v[0], v[1], v[2], v[3]);
-        }
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    auto ld = [&](const float *p, uint32_t s) -> float4 {       // K % 4 == 0: a piece is inside the row or beyond it
+        return 8u * s + 4u * h < K ? *reinterpret_cast<const float4 *>(p + 8u * s) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     };
     auto fma4 = [&](const float4 &a, const float4 &b) {
-        if constexpr (T == 32) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
-        } else {
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc, 0, 0, 0);
-        }
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
     };
     uint32_t s = s0;
     for (; s + U <= s1; s += U) {
@@ -290,60 +333,130 @@ __global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float
 #pragma unroll
         for (int u = 0; u < U; ++u) fma4(a[u], b[u]);
     }
-    if (s < s1) {                                                 // fewer than U steps left: still one round of loads
-        float4 a[U - 1], b[U - 1];
+    for (; s < s1; ++s) fma4(ld(ap, s), ld(wp, s));
 #pragma unroll
-        for (int u = 0; u < U - 1; ++u) {
-            if (s + u >= s1) break;                               // (uniform)
-            a[u] = ld(ap, s + u);
-            b[u] = ld(wp, s + u);
-        }
-#pragma unroll
-        for (int u = 0; u < U - 1; ++u)
-            if (s + u < s1) fma4(a[u], b[u]);                     // (uniform)
-    }
-#pragma unroll
-    for (int r = 0; r < T * T / 64; ++r) {
-        const int row = T == 32 ? 8 * (r >> 2) + 4 * h + (r & 3) : 4 * h + r;
-        part[wave][row * (T + 1) + q] = acc[r];
-    }
+    for (int r = 0; r < 16; ++r) part[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 33 + q] = acc[r];
     __syncthreads();
-    // the waves' sums in wave order, bias, activation: T neighbouring threads hold a row of the tile
+    // the waves' sums in wave order, bias, activation; 512 threads, two outputs each
 #pragma unroll
-    for (int i = 0; i < (T == 32 ? 2 : 1); ++i) {
-        const int e = t + 512 * i, row = e / T, col = e % T;
-        if (row >= T) break;                                      // (T = 16: four of the eight waves)
+    for (int i = 0; i < 2; ++i) {
+        const int e = t + 512 * i, row = e >> 5, col = e & 31;
         float v = 0.0f;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) v += part[w][row * (T + 1) + col];
-        const bool in = m0 + row < M && n0 + col < N;
-        const size_t o = (size_t)(m0 + row) * N + n0 + col;
+        for (int w = 0; w < NW; ++w) v += part[w][row * 33 + col];
         const uint32_t n = n0 + col < N ? n0 + col : N - 1;
         v = apply_act(v + elem_value_rt(g.L.bias_fmt, g.L.bias, n) * g.L.bscale, g.L.act);
-        if (soft_out) {                                           // (uniform; N <= T: the tile holds whole rows)
-            float mx = (uint32_t)col < N ? v : -3.402823466e+38f;
+        if (soft_out) part[0][row * 33 + col] = v;               // (every thread has read part[0][its own two slots] only)
+        else if (m0 + row < M && n0 + col < N) g.C[(size_t)(m0 + row) * N + n0 + col] = v;
+    }
+    if (!soft_out) return;                                        // (uniform)
+    __syncthreads();
+    if (t < 32 && m0 + t < M) {                                   // N <= 32: the tile holds whole rows of logits
+        const float *lr = &part[0][t * 33];
+        float mx = lr[0];
+        for (uint32_t c = 1; c < N; ++c) mx = fmaxf(mx, lr[c]);
+        float sum = 0.0f;
+        for (uint32_t c = 0; c < N; ++c) sum += expf(lr[c] - mx);
+        const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
+        for (uint32_t c = 0; c < N; ++c) soft_out[(size_t)(m0 + t) * N + c] = expf(lr[c] - mx) * inv;
+    }
+}
+
+// The same on 16 x 16 tiles, where 32 x 32 ones would leave half of the compute units and more without work: 64 x 512 x
+// 784 is 32 of those, whose waves are 49 MFMAs of 64 cycles deep, two to a SIMD (11.6 us, 128 tiles of 16 x 16: 9.2 us).
+// A lane loads four consecutive k of a row, which may start anywhere; the operands are passed on between lane groups to
+// keep the order of the sum (chain_order).  A wave takes every eighth segment of K.  A softmax of at most 16 outputs is
+// normalised here as above, and the deltas of a training step's last layer are formed (tail.targets != nullptr).
+template <bool PAIRED>
+__global__ __launch_bounds__(512) void sp_gemm32_small16(const Gemm32Args g, const KSegments seg, float *__restrict__ soft_out,
+                                                         const DeltaTail tail)
+{
+    constexpr int T = 16, NW = 8, U = 8;                              // blocks of 16 k in flight: a segment of 128, one round of latency
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    __shared__ float part[16][T * (T + 1)];
+    const uint32_t M = g.M, N = g.L.N, K = g.L.K;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, q = lane & 15, h = lane >> 4;
+    const uint32_t tiles_n = (N + T - 1) / T;
+    const uint32_t m0 = (blockIdx.x / tiles_n) * T, n0 = (blockIdx.x % tiles_n) * T;
+    const float *ap = g.A + (size_t)(m0 + q < M ? m0 + q : M - 1) * K;
+    const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)(n0 + q < N ? n0 + q : N - 1) * K;
+    for (uint32_t sg = wave; sg < seg.count; sg += NW) {
+        const uint32_t k0 = sg * seg.len, k1 = k0 + seg.len < K ? k0 + seg.len : K;
+        f32x4 acc;
 #pragma unroll
-            for (int off = T / 2; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-            float ex = (uint32_t)col < N ? expf(v - mx) : 0.0f, sum = ex;
+        for (int r = 0; r < 4; ++r) acc[r] = 0.0f;
+        for (uint32_t k = k0; k < k1; k += 16u * U) {
+            float a[U][4], b[U][4];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t kb = k + 16u * u;
+                if (kb >= k1) break;                                  // (uniform)
+                load_piece(a[u], ap, kb, h, k1, K);
+                load_piece(b[u], wp, kb, h, k1, K);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (k + 16u * u >= k1) break;
+                chain_order<PAIRED>(a[u]);
+                chain_order<PAIRED>(b[u]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[u][i], acc, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[sg][(4 * h + r) * (T + 1) + q] = acc[r];
+    }
+    __syncthreads();
+    // the segments' sums in order, bias, activation: 16 neighbouring threads of the first four waves hold a row
+    const int row = t / T, col = t % T;
+    const bool in = t < T * T && m0 + row < M && n0 + col < N;
+    const size_t o = (size_t)(m0 + row) * N + n0 + col;
+    float v = 0.0f;
+    if (t < T * T) {
+#pragma unroll
+        for (int w0 = 0; w0 < 16; w0 += 8) {
+            if ((uint32_t)w0 >= seg.count) break;                     // (uniform)
+            float x[8];
+#pragma unroll
+            for (int w = 0; w < 8; ++w) x[w] = part[w0 + w][row * (T + 1) + col];     // (all at once; the unused ones are not added)
+#pragma unroll
+            for (int w = 0; w < 8; ++w)
+                if ((uint32_t)(w0 + w) < seg.count) v += x[w];
+        }
+        const uint32_t n = n0 + col < N ? n0 + col : N - 1;
+        v = apply_act(v + elem_value_rt(g.L.bias_fmt, g.L.bias, n) * g.L.bscale, g.L.act);
+        if (soft_out) part[0][row * (T + 1) + col] = v;               // (every thread has read its own slots only)
+    }
+    if (soft_out) {                                                   // (uniform; N <= 16: the tile holds whole rows)
+        __syncthreads();
+        if (t >= T * T) return;
+        const float *lr = &part[0][row * (T + 1)];
+        float mx = lr[0], sum = 0.0f, ex;
+        for (uint32_t c = 1; c < N; ++c) mx = fmaxf(mx, lr[c]);
+        if constexpr (PAIRED) {                                       // (the order of sp_gemm32_small)
+            for (uint32_t c = 0; c < N; ++c) sum += expf(lr[c] - mx);
+            ex = expf(v - mx);
+        } else {                                                      // (the order of sp_gemm32_reduce_softmax)
+            ex = (uint32_t)col < N ? expf(v - mx) : 0.0f;
+            sum = ex;
 #pragma unroll
             for (int off = T / 2; off; off >>= 1) sum += __shfl_xor(sum, off);
-            v = ex * (sum > 0.0f ? 1.0f / sum : 1.0f);
-            if (in) soft_out[o] = v;
-        } else if (in) {
-            g.C[o] = v;
         }
-        if (tail.targets) {                                       // (uniform)
-            const float d = in ? v - tail.targets[o] : 0.0f;
-            float out = tail.mode == 1 ? d : d * act_derivative(v, tail.act);
-            if (tail.mode == 0) {                                 // squared error through a softmax
-                float c = d * v;
-#pragma unroll
-                for (int off = T / 2; off; off >>= 1) c += __shfl_xor(c, off);
-                out = v * (d - c);
-            }
-            if (in) tail.delta[o] = out;
-        }
+        v = ex * (sum > 0.0f ? 1.0f / sum : 1.0f);
+        if (in) soft_out[o] = v;
+    } else if (in) {
+        g.C[o] = v;
     }
+    if (!tail.targets || t >= T * T) return;                          // (uniform in a wave)
+    const float d = in ? v - tail.targets[o] : 0.0f;
+    float out = tail.mode == 1 ? d : d * act_derivative(v, tail.act);
+    if (tail.mode == 0) {                                             // squared error through a softmax
+        float c = in ? d * v : 0.0f;
+#pragma unroll
+        for (int off = T / 2; off; off >>= 1) c += __shfl_xor(c, off);
+        out = v * (d - c);
+    }
+    if (in) tail.delta[o] = out;
 }
 
 // adds the K splits of sp_gemm32_f32 (in split order) and applies bias and activation

@@ -505,3 +505,42 @@ def test_small_nets_match_the_oracle(topo, acts, loss, n, batch, epochs, opt, kw
         assert rel_max_abs(arr(name, cnt), ref) <= TOL, name
     assert rel_max_abs(S.forward_batch(net, X[:7]), onet.forward_batch(X[:7])) <= TOL      # the device holds the results too
     S.free_network(net)
+
+
+@pytest.mark.parametrize("topo,acts,loss,n", [
+    ([784, 512, 1000, 10], ["relu", "relu", "softmax"], 1, 64),          # small products, deltas and grouped updates throughout
+    ([100, 333, 70, 17], ["tanh", "sigmoid", "softmax"], 0, 9),          # unaligned rows, a head wider than a 16 x 16 tile
+    ([61, 257, 31], ["sigmoid", "none"], 0, 257),                         # two chunks of bias sums, the second of one sample
+    ([48, 200, 16], ["tanh", "sigmoid"], 1, 512), ([48, 200, 16], ["tanh", "softmax"], 0, 513),   # the grouped update's bound
+    ([33, 1200, 1200, 12], ["relu", "tanh", "softmax"], 1, 300),          # wider column tiles of the small delta product
+    ([9] + [12] * 17 + [4], ["tanh"] * 17 + ["softmax"], 1, 40),          # more layers than one launch takes
+    ([20, 30, 5], ["tanh", "softmax"], 1, 4),                             # vector kernels forward
+])
+def test_steps_from_host_batches_match_oracle(topo, acts, loss, n):
+    """Twelve steps of AdamW on changing host batches (the ring of pinned slots goes round; two steps of the larger nets),
+    forward, deltas, gradients and update at the edges of the small-batch kernels.  Smooth activations where there are
+    many steps: which side of a bend a sample falls on within rounding changes a small batch's gradients by more than
+    the tolerance."""
+    onet = make_oracle_net(O, topo, acts, seed=n, bias_std=0.1, loss=loss)
+    rng = np.random.default_rng(n)
+    d = device_net(onet)
+    d.train_begin()
+    st = O.TrainState(onet)
+    a = step_args(S.OPTIMIZER_ADAMW, loss, lr=0.002, weight_decay=0.01)
+    steps = 12 if sum(a_ * b_ for a_, b_ in zip(topo, topo[1:])) * n < 3e7 else 2
+    for _ in range(steps):
+        X = rng.standard_normal((n, topo[0])).astype(np.float32)
+        T = targets_for(rng, n, topo[-1], loss == 1)
+        gW, gB, _ = onet.batch_gradients(X, T)
+        onet.apply_gradients(st, gW, gB, S.OPTIMIZER_ADAMW, lr=0.002, weight_decay=0.01)
+        a.beta1_pow_t, a.beta2_pow_t = float(st.beta1_pow), float(st.beta2_pow)
+        d.train_step(X, T, a)
+        X[:] = np.nan                                                     # the caller's memory is free again
+        T[:] = np.nan
+    for l in range(len(topo) - 1):
+        wo, wc, bo, bc = onet.woff[l], topo[l] * topo[l + 1], onet.boff[l], topo[l + 1]
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_W, l), onet.W(l).ravel()) <= TOL, l
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_B, l), onet.b(l)) <= TOL, l
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_MW, l), st.mW[wo: wo + wc]) <= 2 * TOL, l
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_VB, l), st.vB[bo: bo + bc]) <= 2 * TOL, l
+    d.destroy()
