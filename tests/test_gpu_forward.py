@@ -537,6 +537,65 @@ def test_large_fp32_layers_take_the_128_by_128_tile(S, O):
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_VEC
 
 
+@pytest.mark.parametrize("n,K,N", [
+    (4095, 520, 1000),     # 256 tiles of 128 x 128: rows of 64, a last tile of each kind in part, K 8 beyond its tiles
+    (8321, 268, 897),      # rows of 128, no split
+    (8321, 269, 897),      # ... rows that are not 16-byte aligned
+    (8200, 68, 3600),      # short sums
+    (250, 2720, 3000),     # split over K, the last share shorter
+    (250, 2721, 3000),
+    (128, 4096, 4096),
+])
+def test_large_fp32_products_on_bf16_parts(S, O, n, K, N):
+    """The kernel of products of 2 G multiply-adds and more, against float64 and the FP32 kernels' own accuracy: at most
+    6 K / 16 roundings of 2^-24 of a partial sum no larger than about its result's deviation (K = 4096 at random: 2e-6;
+    at worst one after the other 1e-4)."""
+    src = make_oracle_net(O, [K, N], ["none"], seed=n + K, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, "f32")
+    h = S.lib().spingalett_hip_handle(net)
+    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm32_f32_big"
+    X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    S.free_network(net)
+    assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 1e-5
+
+
+def test_large_fp32_products_keep_infinities_and_nans(S):
+    """Operands without BF16 parts (infinite, beyond the largest BF16, NaN), next to weights whose lower parts are zero."""
+    n, K, N = 4096, 784, 640
+    rng = np.random.default_rng(3)
+    W = (rng.standard_normal((N, K)) * 0.05).astype(F32)
+    W[:, 5], W[:, 6], W[::2, 7], W[:, 11] = 1.0, -0.5, 0.0, 0.25
+    W[9, 20] = -np.inf
+    b = rng.standard_normal(N).astype(F32)
+    X = rng.standard_normal((n, K)).astype(F32)
+    X[3, 5] = np.inf
+    X[70, 5], X[70, 6] = np.inf, np.inf
+    X[100, 7] = -np.inf
+    X[200, 100] = np.nan
+    X[300, 11] = np.finfo(F32).max
+    X[4000, 20] = 0.0
+    net = S.new_spingalett(S.LOSS_MSE)
+    S.layer(net, K)
+    S.layer(net, N, S.ACT_NONE, S.WEIGHT_INITIALIZATION_NONE)
+    S.weights_view(net, 0)[:] = W
+    S.biases_view(net, 0)[:] = b
+    got = S.forward_batch(net, X)
+    h = S.lib().spingalett_hip_handle(net)
+    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm32_f32_big"
+    S.free_network(net)
+    with np.errstate(invalid="ignore"):
+        want = X.astype(np.float64) @ W.astype(np.float64).T + b
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(got[np.isinf(got)], want[np.isinf(want)].astype(F32))
+    fine = np.isfinite(want)
+    fine[300] = False
+    assert fine.sum() > n * N - 5 * n - 5 * N
+    assert rel_max_abs(got[fine], want[fine]) <= 1e-5
+    row = np.isfinite(want[300])
+    assert rel_max_abs(got[300][row], want[300][row]) <= 1e-6
+
+
 def test_fp32_nets_leave_the_vector_kernel_beyond_four_samples(S, O):
     """From five samples on the FP32 matrix-core kernel is the faster one for FP32 weights, as the 16-bit one is for
     the other formats (configuration 1 at 64 samples: 31 us against 245 us in eight passes of the vector kernel), and
