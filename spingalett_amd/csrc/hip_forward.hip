@@ -955,6 +955,24 @@ uint32_t gemm16_splits(int fmt, uint32_t M, uint32_t N, uint32_t K, uint32_t *kp
     return (ktiles + per - 1) / per;
 }
 
+// Longest K at which the single-stage kernel is the better one for more than a round of 256 x 256 tiles.  Those have a
+// compute unit to themselves, so that the matrix cores idle during a tile's epilogue, and the last round is often mostly
+// empty; several of the single-stage kernel's smaller workgroups share a compute unit and one's epilogue runs beside
+// another's products.  A tanh or sigmoid per output (half of a short layer's time) or an uneven last round decides for it,
+// a long sum, and 16-bit weights, which reach the big kernel's LDS by DMA, against it.  Big against single-stage, input
+// conversion included: tanh behind 4567 x 4736 x 448 INT4 79 / 59, INT8 82 / 62, FP16 80 / 66 us, 4567 x 8192 x 1024 155 / 129,
+// 165 / 142, 159 / 151, at K = 2048 226 / 206, 241 / 226, 232 / 240; even rounds: 8192 x 8192 x 256 144 / 122, 151 / 126, 149 / 139,
+// x 768 196 / 188, 211 / 202, 208 / 235; a ReLU there 4567 x 8192 x 448 71 / 65, 74 / 72, 72 / 81, 8192 x 4736 x 1024 even.  One round
+// or less: 2048 x 8192 x 448 with tanh 46 / 50, 47 / 53, 47 / 57.
+uint32_t gemm16_shared_limit(int fmt, int act, uint32_t big_tiles)
+{
+    if (big_tiles <= 256u) return 0;
+    const bool slow = act == A_TANH || act == A_SIGMOID, wide = fmt_bits(fmt) == 16;
+    const bool uneven = (big_tiles + 255u) / 256u * 1024u >= 5u * big_tiles;         // a fifth of the rounds is idle
+    if (slow) return wide ? (uneven ? 1024u : 384u) : uneven ? 1536u : 768u;
+    return uneven && !wide ? 768u : 0u;
+}
+
 // K splits of the single-stage kernel for rows that are not whole 16-byte units (always 64 x 64 tiles, element-wise
 // loads): few samples give it a handful of workgroups, each walking all of K with nothing in flight (1030 x 777 at
 // 64 samples: 17 workgroups, 80 us).  Whole K tiles per split, about two workgroups per compute unit.
@@ -1214,7 +1232,8 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     const bool split_ok = splits > 1 && (uint64_t)splits * halves * M * L.N <= ctx.ws_floats;
     const bool halves_ok = halves == 1 || (uint64_t)halves * M * L.N <= ctx.ws_floats;     // (checked by the caller's reserve)
     // (too few tiles and no K split, gemm16_splits: the single-stage kernel below)
-    if (aligned && L.K >= 128u && M > 64 && L.N >= 256 && fits32 && (big_tiles >= 192u || split_ok) && halves_ok) {
+    const bool shared_cu = halves == 1 && bm == 256u && L.K <= gemm16_shared_limit(FMT, L.act, big_tiles);
+    if (aligned && !shared_cu && L.K >= 128u && M > 64 && L.N >= 256 && fits32 && (big_tiles >= 192u || split_ok) && halves_ok) {
         if (big_tiles >= 192u) g.kper = 0;
         else g.ksplits = splits;
         if (g.kper || halves == 2) g.ws = ctx.ws;
