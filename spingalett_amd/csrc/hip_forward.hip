@@ -955,22 +955,20 @@ uint32_t gemm16_splits(int fmt, uint32_t M, uint32_t N, uint32_t K, uint32_t *kp
     return (ktiles + per - 1) / per;
 }
 
-// Longest K at which the single-stage kernel is the better one for more than a round of 256 x 256 tiles.  Those have a
-// compute unit to themselves, so that the matrix cores idle during a tile's epilogue, and the last round is often mostly
-// empty; several of the single-stage kernel's smaller workgroups share a compute unit and one's epilogue runs beside
-// another's products.  A tanh or sigmoid per output (half of a short layer's time) or an uneven last round decides for it,
-// a long sum, and 16-bit weights, which reach the big kernel's LDS by DMA, against it.  Big against single-stage, input
-// conversion included: tanh behind 4567 x 4736 x 448 INT4 79 / 59, INT8 82 / 62, FP16 80 / 66 us, 4567 x 8192 x 1024 155 / 129,
-// 165 / 142, 159 / 151, at K = 2048 226 / 206, 241 / 226, 232 / 240; even rounds: 8192 x 8192 x 256 144 / 122, 151 / 126, 149 / 139,
-// x 768 196 / 188, 211 / 202, 208 / 235; a ReLU there 4567 x 8192 x 448 71 / 65, 74 / 72, 72 / 81, 8192 x 4736 x 1024 even.  One round
-// or less: 2048 x 8192 x 448 with tanh 46 / 50, 47 / 53, 47 / 57.
+// Longest K at which the single-stage kernel is the better one for more than a round of 256 x 256 tiles, of which a fifth
+// and more is idle.  A large tile has a compute unit to itself, so that the matrix cores idle during its epilogue and the
+// last round is mostly empty; several of the single-stage kernel's smaller workgroups share a compute unit and one's
+// epilogue runs beside another's products.  A tanh or sigmoid per output lengthens the epilogue; 16-bit weights, which
+// reach the big kernel's LDS by DMA, shorten the rest.  Big against single-stage, input conversion included, tanh, INT4 /
+// INT8 / FP16: 4567 x 8192 x 448 96 / 84, 99 / 88, 100 / 96 us, 8192 x 4736 x 448 99 / 90, 101 / 97, 101 / 100, 4567 x 8192 x 768
+// 119 / 105, 124 / 118, 123 / 126, x 1024 136 / 126, 143 / 139, 142 / 152, x 1536 172 / 173, 183 / 189, 177 / -; a ReLU there
+// 4567 x 8192 x 448 71 / 65, 74 / 72, 72 / 81, 4567 x 4736 x 768 66 / 63, 68 / 65, 65 / 72, 4567 x 8192 x 1024 113 / 111, 118 / 123,
+// 112 / 139.  Full rounds are the big kernel's: 8192 x 8192 x 448 with tanh 133 / 144, 140 / 152, 145 / -.
 uint32_t gemm16_shared_limit(int fmt, int act, uint32_t big_tiles)
 {
-    if (big_tiles <= 256u) return 0;
     const bool slow = act == A_TANH || act == A_SIGMOID, wide = fmt_bits(fmt) == 16;
-    const bool uneven = (big_tiles + 255u) / 256u * 1024u >= 5u * big_tiles;         // a fifth of the rounds is idle
-    if (slow) return wide ? (uneven ? 1024u : 384u) : uneven ? 1536u : 768u;
-    return uneven && !wide ? 768u : 0u;
+    if (big_tiles <= 256u || (big_tiles + 255u) / 256u * 1024u < 5u * big_tiles) return 0;
+    return slow ? (wide ? 512u : 1024u) : wide ? 0u : 768u;
 }
 
 // K splits of the single-stage kernel for rows that are not whole 16-byte units (always 64 x 64 tiles, element-wise

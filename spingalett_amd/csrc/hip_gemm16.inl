@@ -328,8 +328,7 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
         }
         return;
     }
-    // epilogue: scale, bias, activation, store.  Sigmoid and tanh have a copy of the loops to themselves: a switch
-    // over all activations behind every one of a lane's outputs is mostly their code, fetched for nothing.
+    // epilogue: scale, bias, activation, store
     const float wscale = g.L.wscale;
     // 16-bit outputs in rows of whole 16-byte units: a wave turns each 32 x 32 block around in LDS (the tiles' memory,
     // free once every wave has read its last fragments) and stores 16 bytes per lane, two store instructions per
@@ -338,8 +337,8 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
     if (rows16) __syncthreads();
     constexpr int SP = 40;                                   // row pitch of a wave's 32 x 32 staging block, elements
     uint16_t *const stage = (wave < 2 ? As : Ws) + (wave & 1) * (32 * SP);
-    auto emit = [&](auto slow_c) __attribute__((always_inline)) {
-        constexpr bool SLOW = decltype(slow_c)::value;
+    auto emit = [&](auto act_c) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_c)::value;
         if (rows16) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
@@ -350,7 +349,7 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const float pre = fmaf(acc[i][j][r], wscale, bias);
-                        const float v = SLOW ? apply_act(pre, g.L.act) : apply_act_cheap(pre, g.L.act);
+                        const float v = apply_act(pre, ACT);
                         stage[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * SP + (lane & 31)] = f32_to_t16<F16T>(v);
                     }
                     __builtin_amdgcn_wave_barrier();
@@ -378,7 +377,7 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
                     const uint32_t row = m0 + wm * TM * 32 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                     if (row >= M) continue;
                     const float pre = fmaf(acc[i][j][r], wscale, bias);
-                    const float v = SLOW ? apply_act(pre, g.L.act) : apply_act_cheap(pre, g.L.act);
+                    const float v = apply_act(pre, ACT);
                     const size_t o = (size_t)row * N + col;
                     if (g.out_f32) reinterpret_cast<float *>(g.C)[o] = v;
                     else reinterpret_cast<uint16_t *>(g.C)[o] = f32_to_t16<F16T>(v);
@@ -386,8 +385,7 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
             }
         }
     };
-    if (g.L.act == A_SIGMOID || g.L.act == A_TANH) emit(std::true_type{});
-    else emit(std::false_type{});
+    with_act(g.L.act, emit);
 }
 
 // Small layers in one launch: a workgroup owns a 32 x 32 tile of the output, its eight waves split K in whole steps of
@@ -898,18 +896,21 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
             bias[j] = (col < N && !g.ws) ? elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale : 0.0f;
         }
         char *const out = g.ws ? reinterpret_cast<char *>(g.ws + (size_t)blockIdx.y * M * N) : reinterpret_cast<char *>(g.C);
-        // Sigmoid and tanh are kept out of the common path: a run-time switch over all activations inside the
-        // unrolled loops puts a copy of their code behind each of a lane's 16 TM TN outputs, and fetching that code
-        // took longer than the stores (a tenth of an 8192-cubed launch).  The lambda is forced inline: called, it
-        // would take the accumulators through memory.
+        // Every activation has its own copy of the loops (with_act).  Sigmoid and tanh are kept out of the unrolled ones
+        // over a lane's 16 TM TN outputs, where their code takes longer to fetch than to run: the sums wait in LDS as
+        // FP32, and the loop that reads them back and stores whole rows, not unrolled, applies the activation to the few
+        // outputs a lane holds there (4567 x 8192 x 256 FP16 with tanh 103 -> 85 us, 8192 x 8192 x 2048 354 -> 324).
+        // The lambda is forced inline: called, it would take the accumulators through memory.
         // Long K: the outputs bypass the caches' usual retention (they would displace the A and W panels the other
         // tiles of the die are re-reading: 8192 cubed 0.908 against 0.934 ms); short K: the next layer reads them
         // back soon and they are most of the traffic (8192 x 8192 x 1024: 0.162 against 0.175 ms the other way round).
         const bool stream_out = K >= 2048u && !g.ws;
-        auto turn = [&](auto es_c, auto mode_c) __attribute__((always_inline)) {
+        auto turn = [&](auto es_c, auto act_c) __attribute__((always_inline)) {
             constexpr int ES = decltype(es_c)::value;
-            constexpr int MODE = decltype(mode_c)::value;            // 0: cheap activations, 1: sigmoid / tanh, 2: partial sums
-            constexpr int PITCH = BW * ES + 16;                      // lanes 0-31 and 32-63 (four rows apart) on different banks
+            constexpr int ACT = decltype(act_c)::value;              // A_COUNT: partial sums
+            constexpr bool SLOW = ACT == A_SIGMOID || ACT == A_TANH;
+            constexpr int SS = SLOW ? 4 : ES;                   // bytes of an element while it waits in LDS
+            constexpr int PITCH = BW * SS + 16;                      // lanes 0-31 and 32-63 (four rows apart) on different banks
             constexpr int LPR = BW * ES / 16;                        // lanes that write one row
             constexpr int RPP = 64 / LPR;                            // rows per store instruction
             char *mine = reinterpret_cast<char *>(smem) + wave * (32 * PITCH);
@@ -920,59 +921,73 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int rl = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        const float pre = MODE == 2 ? acc[i][j][r] : fmaf(acc[i][j][r], wscale, bias[j]);
-                        const float v = MODE == 2 ? pre : MODE == 1 ? apply_act(pre, g.L.act) : apply_act_cheap(pre, g.L.act);
-                        char *dst = mine + rl * PITCH + (j * 32 + (lane & 31)) * ES;
-                        if constexpr (ES == 4) *reinterpret_cast<float *>(dst) = v;
+                        const float pre = ACT == A_COUNT ? acc[i][j][r] : fmaf(acc[i][j][r], wscale, bias[j]);
+                        const float v = SLOW ? pre : apply_act(pre, ACT);
+                        char *dst = mine + rl * PITCH + (j * 32 + (lane & 31)) * SS;
+                        if constexpr (SS == 4) *reinterpret_cast<float *>(dst) = v;
                         else *reinterpret_cast<uint16_t *>(dst) = f32_to_t16<F16T>(v);
                     }
-#pragma unroll
-                for (int p = 0; p < 32 / RPP; ++p) {
+                auto put = [&](int p) {
                     const int rl = p * RPP + lane / LPR, seg = lane % LPR;
-                    const uint4 v = *reinterpret_cast<const uint4 *>(mine + rl * PITCH + seg * 16);
+                    const char *src = mine + rl * PITCH + seg * (16 / ES) * SS;
+                    u32x4 vv;
+                    if constexpr (SLOW) {
+                        float e[16 / ES];
+#pragma unroll
+                        for (int x = 0; x < 16 / ES; ++x) e[x] = apply_act(reinterpret_cast<const float *>(src)[x], ACT);
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            if constexpr (ES == 4) vv[x] = __float_as_uint(e[x]);
+                            else vv[x] = (uint32_t)f32_to_t16<F16T>(e[2 * x]) | (uint32_t)f32_to_t16<F16T>(e[2 * x + 1]) << 16;
+                        }
+                    } else {
+                        const uint4 v = *reinterpret_cast<const uint4 *>(src);
+                        vv = u32x4{v.x, v.y, v.z, v.w};
+                    }
                     const uint32_t row = m0 + (wm * TM + i) * 32 + rl;
                     const uint32_t col = n0 + wn * BW + seg * (16 / ES);
                     if (row < M && col < N) {                        // N is a multiple of 16 / ES: a unit is all in or all out
                         u32x4 *dstp = reinterpret_cast<u32x4 *>(out + ((size_t)row * N + col) * ES);
-                        const u32x4 vv{v.x, v.y, v.z, v.w};
                         if (stream_out) __builtin_nontemporal_store(vv, dstp);
                         else *dstp = vv;
                     }
+                };
+                if constexpr (SLOW) {
+#pragma unroll 1
+                    for (int p = 0; p < 32 / RPP; ++p) put(p);
+                } else {
+#pragma unroll
+                    for (int p = 0; p < 32 / RPP; ++p) put(p);
                 }
             }
         };
-        const bool slow = g.L.act == A_SIGMOID || g.L.act == A_TANH;
         using E4 = std::integral_constant<int, 4>;
         using E2 = std::integral_constant<int, 2>;
-        if (g.ws) {
-            turn(E4{}, std::integral_constant<int, 2>{});
-        } else if (g.out_f32) {
-            if (slow) turn(E4{}, std::integral_constant<int, 1>{});
-            else turn(E4{}, std::integral_constant<int, 0>{});
-        } else {
-            if (slow) turn(E2{}, std::integral_constant<int, 1>{});
-            else turn(E2{}, std::integral_constant<int, 0>{});
-        }
+        if (g.ws) turn(E4{}, std::integral_constant<int, A_COUNT>{});
+        else if (g.out_f32) with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E4{}, act_c); });
+        else with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E2{}, act_c); });
         return;
     }
+    with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const uint32_t col = n0 + (wn * TN + j) * 32 + (lane & 31);
-        if (col >= N) continue;
-        const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
+        for (int j = 0; j < TN; ++j) {
+            const uint32_t col = n0 + (wn * TN + j) * 32 + (lane & 31);
+            if (col >= N) continue;
+            const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
+            for (int i = 0; i < TM; ++i) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (row >= M) continue;
-                const float v = apply_act(fmaf(acc[i][j][r], wscale, bias), g.L.act);
-                const size_t o = (size_t)row * N + col;
-                if (g.out_f32) reinterpret_cast<float *>(g.C)[o] = v;
-                else reinterpret_cast<uint16_t *>(g.C)[o] = f32_to_t16<F16T>(v);
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t row = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    if (row >= M) continue;
+                    const float v = apply_act(fmaf(acc[i][j][r], wscale, bias), decltype(act_c)::value);
+                    const size_t o = (size_t)row * N + col;
+                    if (g.out_f32) reinterpret_cast<float *>(g.C)[o] = v;
+                    else reinterpret_cast<uint16_t *>(g.C)[o] = f32_to_t16<F16T>(v);
+                }
             }
         }
-    }
+    });
 }
 
 // adds the partial sums of a split launch (K splits in split order; with split activations the sums of the second

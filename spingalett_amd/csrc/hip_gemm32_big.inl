@@ -161,38 +161,40 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32_big(const BigGemm32Args g)
         __syncthreads();
     }
 
-    auto store = [&](uint32_t m, uint32_t n, float v, float bias) {
-        const size_t o = (size_t)m * N + n;
-        if (g.ws) g.ws[(size_t)blockIdx.y * M * N + o] = v;
-        else g.C[o] = apply_act(v + bias, g.act);
-    };
     auto bias_of = [&](uint32_t n) { return elem_value_rt(g.bias_fmt, g.bias, n) * g.bscale; };
     // element e = 32 j + 16 i + r of a thread
     auto row_of = [&](uint32_t e) { return m0 + (wm * TM + (e >> 4 & 1u)) * 32u + 8u * (e >> 2 & 3u) + 4u * h + (e & 3u); };
     auto col_of = [&](uint32_t e) { return n0 + (wn * 2u + (e >> 5)) * 32u + q; };
     uint64_t again = 0;                                    // the elements whose sum is not finite
+    with_act(g.act, [&](auto act_c) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_c)::value;
 #pragma unroll
-    for (uint32_t j = 0; j < 2u; ++j) {
-        const uint32_t n = col_of(32u * j);
-        if (n >= N) continue;
-        const float bias = bias_of(n);
+        for (uint32_t j = 0; j < 2u; ++j) {
+            const uint32_t n = col_of(32u * j);
+            if (n >= N) continue;
+            const float bias = bias_of(n);
 #pragma unroll
-        for (uint32_t i = 0; i < (uint32_t)TM; ++i)
+            for (uint32_t i = 0; i < (uint32_t)TM; ++i)
 #pragma unroll
-            for (uint32_t r = 0; r < 16u; ++r) {
-                const uint32_t e = 32u * j + 16u * i + r, m = row_of(e);
-                if (m >= M) continue;
-                const float v = acc[i][j][r];
-                if (!(fabsf(v) < __builtin_inff())) again |= 1ull << e;
-                store(m, n, v, bias);
-            }
-    }
+                for (uint32_t r = 0; r < 16u; ++r) {
+                    const uint32_t e = 32u * j + 16u * i + r, m = row_of(e);
+                    if (m >= M) continue;
+                    const float v = acc[i][j][r];
+                    if (!(fabsf(v) < __builtin_inff())) again |= 1ull << e;
+                    const size_t o = (size_t)m * N + n;
+                    if (g.ws) g.ws[(size_t)blockIdx.y * M * N + o] = v;
+                    else g.C[o] = apply_act(v + bias, ACT);
+                }
+        }
+    });
     while (again) {
         const uint32_t e = (uint32_t)__builtin_ctzll(again), m = row_of(e), n = col_of(e);
         again &= again - 1u;
         const float *a = g.A + (size_t)m * K, *b = g.B + (size_t)n * K;
         float s = 0.0f;
         for (uint32_t k = kbeg; k < kend && s == s; ++k) s = fmaf(a[k], b[k], s);
-        store(m, n, s, bias_of(n));
+        const size_t o = (size_t)m * N + n;
+        if (g.ws) g.ws[(size_t)blockIdx.y * M * N + o] = s;
+        else g.C[o] = apply_act(s + bias_of(n), g.act);
     }
 }

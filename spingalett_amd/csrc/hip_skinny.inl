@@ -126,14 +126,13 @@ __device__ __forceinline__ void skinny_frag(const uint4 &v, int j, uint32_t (&f)
     }
 }
 
-// SLOW: the activation may be sigmoid or tanh.  Callers with many outputs per lane keep a copy of their loops for
-// those two: a switch over all activations behind every output is mostly their code, fetched for nothing.
-template <bool F16T, bool SLOW = true>
+// ACT: the layer's activation where it is known at compile time (with_act), or -1
+template <bool F16T, int ACT = -1>
 __device__ __forceinline__ void skinny_emit_biased(const SkinnyArgs &a, uint32_t c, uint32_t r, float accv, float bias)
 {
     const uint32_t m = a.mode_b ? r : c, n = a.mode_b ? c : r;
     const float pre = fmaf(accv, a.L.wscale, bias);
-    const float v = SLOW ? apply_act(pre, a.L.act) : apply_act_cheap(pre, a.L.act);
+    const float v = apply_act(pre, ACT < 0 ? a.L.act : ACT);
     const size_t o = (size_t)m * a.L.N + n;
     if (a.out_f32) reinterpret_cast<float *>(a.C)[o] = v;
     else reinterpret_cast<uint16_t *>(a.C)[o] = f32_to_t16<F16T>(v);
@@ -383,8 +382,8 @@ __global__ __launch_bounds__(64 * NWV) void sp_skinny16(const SkinnyArgs a)
         }
         return;
     }
-    auto emit = [&](auto slow_c) __attribute__((always_inline)) {
-        constexpr bool SLOW = decltype(slow_c)::value;
+    auto emit = [&](auto act_c) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_c)::value;
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const uint32_t r = row0 + rt * 32u + n31;
@@ -398,12 +397,11 @@ __global__ __launch_bounds__(64 * NWV) void sp_skinny16(const SkinnyArgs a)
                     const uint32_t c = cbase + ct * 32u + 8u * (q >> 2) + 4u * h + (q & 3);
                     if (c >= a.NC) continue;
                     const float bias = a.mode_b ? elem_value_rt(a.L.bias_fmt, a.L.bias, c) * a.L.bscale : bias_r;
-                    skinny_emit_biased<F16T, SLOW>(a, c, r, acc[rt][ct][q], bias);
+                    skinny_emit_biased<F16T, ACT>(a, c, r, acc[rt][ct][q], bias);
                 }
         }
     };
-    if (a.L.act == A_SIGMOID || a.L.act == A_TANH) emit(std::true_type{});
-    else emit(std::false_type{});
+    with_act(a.L.act, emit);
 }
 
 // Variant for a thin operand of at most NCP (8 or 16; the host uses 8) rows: the NW waves of a workgroup share one tile of 32

@@ -537,6 +537,29 @@ def test_large_fp32_layers_take_the_128_by_128_tile(S, O):
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_VEC
 
 
+@pytest.mark.parametrize("fmt,K,N,act,head,kernel", [
+    ("i8", 144, 4112, "tanh", True, "sp_gemm16"),            # an uneven round of large tiles and a short sum
+    ("i8", 144, 4112, "relu", True, "sp_gemm16"),
+    ("i4", 1056, 4128, "sigmoid", True, "sp_gemm16_big"),    # ... a sum too long for that
+    ("f16", 512, 4112, "sigmoid", True, "sp_gemm16"),
+    ("f16", 520, 4120, "sigmoid", True, "sp_gemm16_big"),      # 16-bit outputs through the FP32 staging of large tiles
+    ("f16", 144, 4112, "leaky_relu", True, "sp_gemm16_big"),
+    ("bf16", 640, 4116, "tanh", False, "sp_gemm16_big"),       # FP32 outputs, the last tiles of both kinds in part
+])
+def test_short_layers_of_uneven_rounds_of_large_tiles(S, O, fmt, K, N, act, head, kernel):
+    """306 large tiles on 256 compute units: which kernel takes the layer, and the epilogues with tanh and sigmoid of both."""
+    n = 4605
+    topo, acts = ([K, N, 24], [act, "none"]) if head else ([K, N], [act])
+    src = make_oracle_net(O, topo, acts, seed=K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    h = S.lib().spingalett_hip_handle(net)
+    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == kernel
+    X = np.random.default_rng(N).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    S.free_network(net)
+    assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_MFMA
+
+
 @pytest.mark.parametrize("n,K,N", [
     (4095, 520, 1000),     # 256 tiles of 128 x 128: rows of 64, a last tile of each kind in part, K 8 beyond its tiles
     (8321, 268, 897),      # rows of 128, no split
