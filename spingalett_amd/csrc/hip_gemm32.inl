@@ -97,14 +97,20 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32(const Gemm32Args g)
 
     const uint32_t col = n0 + wn * 32 + (lane & 31);
     if (col >= N) return;
-    const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
+    // (a copy of the loop per activation: 4096 x 512 x 784 with tanh 36.9 -> 35.5 us, with leaky ReLU 35.5 -> 34.0)
+    auto row_of = [&](int r) { return m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); };
+    if (g.ws) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t row = m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (row >= M) continue;
-        if (g.ws) g.ws[((size_t)blockIdx.y * M + row) * N + col] = acc[r];
-        else g.C[(size_t)row * N + col] = apply_act(acc[r] + bias, g.L.act);
+        for (int r = 0; r < 16; ++r)
+            if (row_of(r) < M) g.ws[((size_t)blockIdx.y * M + row_of(r)) * N + col] = acc[r];
+        return;
     }
+    const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
+    with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            if (row_of(r) < M) g.C[(size_t)row_of(r) * N + col] = apply_act(acc[r] + bias, decltype(act_c)::value);
+    });
 }
 
 // The same product where sp_gemm32_f32_big does not take it (training's forward, whose sums keep their order, and tiles that
@@ -206,19 +212,21 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32_128(const Gemm32Args g)
         __syncthreads();
     }
 
+    with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int jn = 0; jn < 2; ++jn) {
-        const uint32_t col = n0 + wn * 64 + jn * 32 + q;
-        if (col >= N) continue;
-        const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
+        for (int jn = 0; jn < 2; ++jn) {
+            const uint32_t col = n0 + wn * 64 + jn * 32 + q;
+            if (col >= N) continue;
+            const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (row < M) g.C[(size_t)row * N + col] = apply_act(acc[i][jn][r] + bias, g.L.act);
-            }
-    }
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                    if (row < M) g.C[(size_t)row * N + col] = apply_act(acc[i][jn][r] + bias, decltype(act_c)::value);
+                }
+        }
+    });
 }
 
 // What a training step wants besides the outputs of its last layer: their deltas (sp_train_out_delta's modes)

@@ -131,21 +131,29 @@ __global__ __launch_bounds__(256) void sp_train_gemm32(const TrGemmArgs g)
         __syncthreads();
     }
 
+    auto emit = [&](auto put) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-        const uint32_t col = n0 + (wn * TM + j) * 32 + (lane & 31);
-        if (col >= N) continue;
+        for (int j = 0; j < TM; ++j) {
+            const uint32_t col = n0 + (wn * TM + j) * 32 + (lane & 31);
+            if (col >= N) continue;
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t row = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (row >= M) continue;
-                const size_t o = (size_t)row * N + col;
-                if (g.ws) g.ws[(size_t)blockIdx.y * M * N + o] = acc[i][j][r];
-                else if (EPI == TR_EPI_DELTA) g.C[o] = acc[i][j][r] * act_derivative(g.aux[o], g.act);
-                else g.C[o] = g.scale * acc[i][j][r];
-            }
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t row = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    if (row < M) put((size_t)row * N + col, acc[i][j][r]);
+                }
+        }
+    };
+    if (g.ws) {
+        float *ws = g.ws + (size_t)blockIdx.y * M * N;
+        emit([&](size_t o, float v) { ws[o] = v; });
+    } else if constexpr (EPI == TR_EPI_DELTA) {
+        with_act(g.act, [&](auto act_c) __attribute__((always_inline)) {
+            emit([&](size_t o, float v) { g.C[o] = v * act_derivative(g.aux[o], decltype(act_c)::value); });
+        });
+    } else {
+        emit([&](size_t o, float v) { g.C[o] = g.scale * v; });
     }
 }
 
