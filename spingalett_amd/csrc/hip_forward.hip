@@ -9,7 +9,8 @@
 //                     through registers into 16-bit MFMAs, the thin one in LDS (_kw: thin side of <= 8 rows, K split
 //                     inside the workgroup)
 //   hip_gemm16.inl    sp_gemm16_big / sp_gemm16: larger batches: LDS-tiled dequant-to-16-bit MFMA GEMM, fused epilogue
-//   hip_gemm32.inl    sp_gemm32_f32: FP32 weights beyond 64 samples: FP32 MFMA GEMM
+//   hip_gemm32.inl    sp_gemm32_f32: FP32 weights beyond four samples: FP32 MFMA GEMM
+//   hip_gemm32_big.inl  sp_gemm32_f32_big: large FP32 forward products on BF16 parts
 //   sp_softmax_rows   per-sample softmax (Activation.c:5-21)
 //   sp_eval_*         loss and argmax of a labelled batch (SIMD.c:522-552, Training.c:421-435)
 //   hip_train.inl     the batched training step (included at the end)
@@ -960,15 +961,17 @@ uint32_t gemm16_splits(int fmt, uint32_t M, uint32_t N, uint32_t K, uint32_t *kp
 // last round is mostly empty; several of the single-stage kernel's smaller workgroups share a compute unit and one's
 // epilogue runs beside another's products.  A tanh or sigmoid per output lengthens the epilogue; 16-bit weights, which
 // reach the big kernel's LDS by DMA, shorten the rest.  Big against single-stage, input conversion included, tanh, INT4 /
-// INT8 / FP16: 4567 x 8192 x 448 96 / 84, 99 / 88, 100 / 96 us, 8192 x 4736 x 448 99 / 90, 101 / 97, 101 / 100, 4567 x 8192 x 768
-// 119 / 105, 124 / 118, 123 / 126, x 1024 136 / 126, 143 / 139, 142 / 152, x 1536 172 / 173, 183 / 189, 177 / -; a ReLU there
-// 4567 x 8192 x 448 71 / 65, 74 / 72, 72 / 81, 4567 x 4736 x 768 66 / 63, 68 / 65, 65 / 72, 4567 x 8192 x 1024 113 / 111, 118 / 123,
-// 112 / 139.  Full rounds are the big kernel's: 8192 x 8192 x 448 with tanh 133 / 144, 140 / 152, 145 / -.
+// INT8: 4567 x 8192 x 448 98 / 78, 100 / 90 us, 8192 x 4736 x 448 101 / 88, 103 / 97, 4567 x 8192 x 1024 139 / 123, 145 / 141 (x
+// 1536 even or lost); FP16 100 / 96 and 101 / 100 at 448, 123 / 126 at 768.  Without them a quarter of the rounds has to be
+// idle: leaky ReLU 4567 x 8192 x 448 67 / 62, 72 / 70, 4567 x 4736 x 448 47 / 44, 50 / 48, but 8192 x 4736 x 448 70 / 70, 74 / 77 and
+// 4567 x 8192 x 768 92 / 84, 98 / 102; FP16 never.  Full rounds are the big kernel's: 8192 x 8192 x 448 with tanh 133 / 144.
 uint32_t gemm16_shared_limit(int fmt, int act, uint32_t big_tiles)
 {
     const bool slow = act == A_TANH || act == A_SIGMOID, wide = fmt_bits(fmt) == 16;
-    if (big_tiles <= 256u || (big_tiles + 255u) / 256u * 1024u < 5u * big_tiles) return 0;
-    return slow ? (wide ? 512u : 1024u) : wide ? 0u : 768u;
+    const uint32_t slots = (big_tiles + 255u) / 256u * 256u;
+    if (big_tiles <= 256u || 4u * slots < 5u * big_tiles) return 0;
+    if (slow) return wide ? 512u : 1024u;
+    return wide || 10u * slots < 13u * big_tiles ? 0u : 512u;
 }
 
 // K splits of the single-stage kernel for rows that are not whole 16-byte units (always 64 x 64 tiles, element-wise
