@@ -683,8 +683,9 @@ Regime pick_regime(const sphip_net *net, uint32_t n, uint32_t flags)
 // by word, and every tile of such a layer waits for those loads (1030-1531-777-33 FP16 at 1333 samples: 107 us for each
 // of three layers, 9 to 15 padded).  So an input or hidden layer of such a width gets neurons without weights up to
 // the next whole unit (wide ones up to a multiple of 64, whole cache lines): zero rows and zero biases on the producing
-// side, zero columns on the consuming side, so that whatever activation(0) is adds nothing.  Not the output layer, whose
-// rows are the caller's, and not a hidden softmax, whose sum runs over its real neurons.
+// side, zero columns on the consuming side.  The kernels store something finite for a padded neuron whatever its inputs
+// are (layer_sum, tile_clear_padding), so that it adds nothing behind infinities and NaNs either.  Not the output layer, whose rows are the
+// caller's, and not a hidden softmax, whose sum runs over its real neurons.
 // Integer rows of eight codes' multiples (1000 INT8 codes) have kernels of their own, which are as good on small layers
 // and take the input as it is; hidden widths of that kind are padded in front of half a million weights and more, where
 // the streaming and DMA kernels, which want 16-byte rows, are the better ones.  FP32 rows stay as they are.
@@ -711,6 +712,7 @@ LayerArgs make_layer_args(const sphip_net *net, uint32_t l /*1-based layer*/, bo
     L.bias_fmt = net->prec;
     L.act = net->act[l - 1] == A_SOFTMAX ? A_NONE : net->act[l - 1];
     L.N = net->ptopo[l];
+    L.pad = net->ptopo[l] - net->topo[l];
     L.K = raw ? net->topo[l - 1] : net->ptopo[l - 1];
     return L;
 }

@@ -50,6 +50,25 @@ __device__ __forceinline__ uint32_t int_to_t16(int q)
     }
 }
 
+// What layer_sum() is to the tile kernels: a wave whose block of ROWS x COLS outputs from (r0, c0) on reaches into the
+// padding stores zeros over it behind its outputs.  (A select behind every output, or sums cleared in registers, costs
+// all tiles something: up to four vector registers, which at 2 x 2 tiles of 8-bit codes is a third of the resident waves; so
+// does a loop over the padded columns alone here.)
+template <int ROWS, int COLS>
+__device__ __forceinline__ void tile_clear_padding(const GemmArgs &g, uint32_t r0, uint32_t c0)
+{
+    const uint32_t N = g.L.N, real = N - g.L.pad;
+    if (g.L.pad == 0u || c0 + COLS <= real) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // the outputs' stores have arrived
+    for (uint32_t e = threadIdx.x & 63u; e < (uint32_t)(ROWS * COLS); e += 64u) {
+        const uint32_t row = r0 + e / COLS, col = c0 + e % COLS;
+        if (row >= g.M || col < real || col >= N) continue;
+        const size_t o = (size_t)row * N + col;
+        if (g.out_f32) reinterpret_cast<float *>(g.C)[o] = 0.0f;
+        else reinterpret_cast<uint16_t *>(g.C)[o] = 0;
+    }
+}
+
 // packed FP16 subtraction a - c (two lanes at once)
 __device__ __forceinline__ uint32_t h2_sub(uint32_t v, uint32_t c)
 {
@@ -386,6 +405,7 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
         }
     };
     with_act(g.L.act, emit);
+    tile_clear_padding<32 * TM, 32 * TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32);
 }
 
 // Small layers in one launch: a workgroup owns a 32 x 32 tile of the output, its eight waves split K in whole steps of
@@ -511,7 +531,6 @@ __global__ __launch_bounds__(512) void sp_gemm16_small(const GemmArgs g)
         part[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 33 + q] = HALVES == 2 ? fmaf(accl[r], kLoScale, acc[r]) : acc[r];
     __syncthreads();
     // the waves' sums in wave order, scale, bias, activation; 512 threads, two outputs each
-    const float wscale = g.L.wscale;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int e = t + 512 * i, row = e >> 5, col = e & 31;
@@ -519,7 +538,7 @@ __global__ __launch_bounds__(512) void sp_gemm16_small(const GemmArgs g)
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += part[w][row * 33 + col];
         if (m0 + row >= M || n0 + col >= N) continue;
-        v = apply_act(fmaf(v, wscale, elem_value_rt(g.L.bias_fmt, g.L.bias, n0 + col) * g.L.bscale), g.L.act);
+        v = apply_act(layer_sum(g.L, v, elem_value_rt(g.L.bias_fmt, g.L.bias, n0 + col) * g.L.bscale, n0 + col), g.L.act);
         const size_t o = (size_t)(m0 + row) * N + n0 + col;
         if (g.out_f32) reinterpret_cast<float *>(g.C)[o] = v;
         else if constexpr (HALVES == 2) {
@@ -966,6 +985,7 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
         if (g.ws) turn(E4{}, std::integral_constant<int, A_COUNT>{});
         else if (g.out_f32) with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E4{}, act_c); });
         else with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E2{}, act_c); });
+        if (!g.ws) tile_clear_padding<32 * TM, 32 * TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32);
         return;
     }
     with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) {
@@ -988,6 +1008,7 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
             }
         }
     });
+    tile_clear_padding<32 * TM, 32 * TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32);
 }
 
 // adds the partial sums of a split launch (K splits in split order; with split activations the sums of the second
@@ -1015,7 +1036,7 @@ __global__ __launch_bounds__(256) void sp_gemm16_reduce(const GemmArgs g, uint32
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col + i) * g.L.bscale;
-            v[i] = apply_act(fmaf(in[i], g.L.wscale, bias), g.L.act);
+            v[i] = apply_act(layer_sum(g.L, in[i], bias, col + i), g.L.act);
         }
         if (g.out_f32) {
             *reinterpret_cast<float4 *>(reinterpret_cast<float *>(g.C) + idx) = make_float4(v[0], v[1], v[2], v[3]);
@@ -1041,7 +1062,7 @@ __global__ __launch_bounds__(256) void sp_gemm16_reduce(const GemmArgs g, uint32
         }
         const uint32_t col = (uint32_t)(idx % g.L.N);
         const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
-        const float v = apply_act(fmaf(fmaf(low, kLoScale, sum), g.L.wscale, bias), g.L.act);
+        const float v = apply_act(layer_sum(g.L, fmaf(low, kLoScale, sum), bias, col), g.L.act);
         if (g.out_f32) reinterpret_cast<float *>(g.C)[idx] = v;
         else if (g.halves == 2) {
             uint16_t hi, lo;

@@ -13,7 +13,15 @@ struct LayerArgs {
     int bias_fmt;
     int act;               // activation applied in the epilogue (A_NONE for softmax layers)
     uint32_t N, K;         // out, in
+    uint32_t pad;          // the last of the N outputs that are padding, not neurons
 };
+
+// The sum of output n, before its activation.  A padded neuron's is zero, whatever its zero weights meet: an infinite
+// input would make a NaN of it (0 x inf), and the next layer's zero column NaNs of all its outputs.
+__device__ __forceinline__ float layer_sum(const LayerArgs &L, float acc, float bias, uint32_t n)
+{
+    return n + L.pad < L.N ? fmaf(acc, L.wscale, bias) : 0.0f;
+}
 
 // unpack one 16-byte chunk into its 128/bits unscaled float values
 template <int FMT>
@@ -141,7 +149,7 @@ __global__ __launch_bounds__(256) void sp_gemv(const LayerArgs L, const float *_
             const float bias = elem_value_rt(L.bias_fmt, L.bias, row) * L.bscale;
 #pragma unroll
             for (int b = 0; b < BT; ++b)
-                if (b < nb) y[(size_t)b * L.N + row] = apply_act(fmaf(acc[r][b], L.wscale, bias), L.act);
+                if (b < nb) y[(size_t)b * L.N + row] = apply_act(layer_sum(L, acc[r][b], bias, row), L.act);
         }
     }
 }
@@ -231,7 +239,7 @@ __global__ __launch_bounds__(256) void sp_gemv_words(const LayerArgs L, const fl
         const float bias = elem_value_rt(L.bias_fmt, L.bias, row) * L.bscale;
 #pragma unroll
         for (int b = 0; b < BT; ++b)
-            if (b < nb) y[(size_t)b * L.N + row] = apply_act(fmaf(acc[b], L.wscale, bias), L.act);
+            if (b < nb) y[(size_t)b * L.N + row] = apply_act(layer_sum(L, acc[b], bias, row), L.act);
     }
 }
 
@@ -262,7 +270,7 @@ __global__ __launch_bounds__(256) void sp_gemv_generic(const LayerArgs L, const 
         const float bias = elem_value_rt(L.bias_fmt, L.bias, row) * L.bscale;
 #pragma unroll
         for (int b = 0; b < BT; ++b)
-            if (b < nb) y[(size_t)b * L.N + row] = apply_act(fmaf(acc[b], L.wscale, bias), L.act);
+            if (b < nb) y[(size_t)b * L.N + row] = apply_act(layer_sum(L, acc[b], bias, row), L.act);
     }
 }
 
@@ -708,7 +716,7 @@ __device__ __forceinline__ void gemv_i8_specialised(const GemvI8Args &a)
             dot = 0.0f;
             for (uint32_t k = 0; k < K; ++k) dot = fmaf((float)int_code<FMT>(a.L.w, base + k), xs[k], dot);
         }
-        a.y[(size_t)g * N + nrow] = apply_act(fmaf(dot, a.L.wscale, bias), a.L.act);
+        a.y[(size_t)g * N + nrow] = apply_act(layer_sum(a.L, dot, bias, nrow), a.L.act);
     }
 }
 
@@ -904,7 +912,7 @@ __global__ __launch_bounds__(FQ ? 1024 : MT <= 4 ? 1024 : 256) void sp_gemv_i8mf
                 dot = 0.0f;
                 for (uint32_t k = 0; k < K; ++k) dot = fmaf((float)int_code<FMT>(a.L.w, base + k), xs[k], dot);
             }
-            a.y[(size_t)s0 * N + nrow] = apply_act(fmaf(dot, a.L.wscale, bias), a.L.act);
+            a.y[(size_t)s0 * N + nrow] = apply_act(layer_sum(a.L, dot, bias, nrow), a.L.act);
         }
     }
 }

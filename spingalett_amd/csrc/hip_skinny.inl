@@ -131,8 +131,7 @@ template <bool F16T, int ACT = -1>
 __device__ __forceinline__ void skinny_emit_biased(const SkinnyArgs &a, uint32_t c, uint32_t r, float accv, float bias)
 {
     const uint32_t m = a.mode_b ? r : c, n = a.mode_b ? c : r;
-    const float pre = fmaf(accv, a.L.wscale, bias);
-    const float v = apply_act(pre, ACT < 0 ? a.L.act : ACT);
+    const float v = apply_act(layer_sum(a.L, accv, bias, n), ACT < 0 ? a.L.act : ACT);
     const size_t o = (size_t)m * a.L.N + n;
     if (a.out_f32) reinterpret_cast<float *>(a.C)[o] = v;
     else reinterpret_cast<uint16_t *>(a.C)[o] = f32_to_t16<F16T>(v);
@@ -676,7 +675,7 @@ __global__ __launch_bounds__(256) void sp_skinny_reduce(const SkinnyArgs a, uint
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float bias = elem_value_rt(a.L.bias_fmt, a.L.bias, r + i) * a.L.bscale;
-            v[i] = apply_act(fmaf(in[i], a.L.wscale, bias), a.L.act);
+            v[i] = apply_act(layer_sum(a.L, in[i], bias, r + i), a.L.act);
         }
         const size_t o = (size_t)c * a.L.N + r;
         if (a.out_f32) {
@@ -704,7 +703,7 @@ __global__ __launch_bounds__(256) void sp_skinny_reduce(const SkinnyArgs a, uint
         const uint32_t c = (uint32_t)(idx / a.R), r = (uint32_t)(idx % a.R);
         const uint32_t m = a.mode_b ? r : c, n = a.mode_b ? c : r;
         const float bias = elem_value_rt(a.L.bias_fmt, a.L.bias, n) * a.L.bscale;
-        skinny_store<F16T>(a, (size_t)m * a.L.N + n, apply_act(fmaf(fmaf(low, kLoScale, sum), a.L.wscale, bias), a.L.act));
+        skinny_store<F16T>(a, (size_t)m * a.L.N + n, apply_act(layer_sum(a.L, fmaf(low, kLoScale, sum), bias, n), a.L.act));
     }
 }
 

@@ -16,6 +16,7 @@ agree 100 %.
 """
 import ctypes as C
 import os
+import tempfile
 
 import numpy as np
 import pytest
@@ -1336,6 +1337,64 @@ def test_padded_widths_leave_the_outputs_alone(S, O, fmt, topo, acts):
     twin = d.clone()
     assert np.array_equal(twin.forward(X[:300]), d.forward(X[:300]))
     twin.destroy()
+    S.free_network(net)
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
+@pytest.mark.parametrize("act", ["tanh", "sigmoid", "leaky_relu", "foo52"])
+@pytest.mark.parametrize("topo,sizes", [
+    ([777, 1030, 33], (1, 3, 5, 33, 260, 1500)),                   # vector, small, streaming and single-stage kernels
+    ([200, 37, 90, 9], (2, 64, 700)),                              # widths below one unit, thin layers
+    ([640, 4500, 2300, 10], (4, 8, 130, 2100)),                    # large tiles, K splits, a padded last column of tiles
+])
+def test_padded_widths_keep_infinities_and_nans_where_they_are(S, fmt, act, topo, sizes):
+    """A padded neuron sees the infinite input too: 0 x inf must not reach the outputs.  Single infinities of either sign,
+    and NaNs, in samples of their own, against FP64 on the decoded arrays.  (A zero code of a real neuron makes a NaN of an
+    infinity, as in the reference's FP32 sums: integer weights are drawn without zeros.)"""
+    rng = np.random.default_rng(len(topo) + topo[1])
+    levels = {"i8": 127, "i4": 7, "i2": 1}.get(fmt)
+    W, b = [], []
+    for l in range(len(topo) - 1):
+        w = rng.standard_normal((topo[l + 1], topo[l])) / np.sqrt(topo[l])
+        if levels:
+            top = np.abs(w).max()
+            q = np.rint(w / top * levels)
+            w = np.where(q == 0, np.where(w < 0, -1, 1), q) * (top / levels)
+            w.ravel()[0] = top                                     # the scale that the writer finds again
+        W.append(w.astype(F32)); b.append((rng.standard_normal(topo[l + 1]) * 0.1).astype(F32))
+    acts = [act] * (len(topo) - 2) + ["none"]
+    src = S.new_spingalett()
+    S.layer(src, topo[0])
+    for l, a in enumerate(acts):
+        S.layer(src, topo[l + 1], {"tanh": S.ACT_TANH, "sigmoid": S.ACT_SIGMOID, "leaky_relu": S.ACT_LEAKY_RELU,
+                                   "foo52": S.ACT_FOO52, "none": S.ACT_NONE}[a], S.WEIGHT_INITIALIZATION_NONE)
+        S.weights_view(src, l)[:] = W[l]
+        S.biases_view(src, l)[:] = b[l]
+    with tempfile.TemporaryDirectory() as d:
+        path = os.path.join(d, "net.nn")
+        prec = {"f16": S.PRECISION_FP16, "bf16": S.PRECISION_BFLOAT16, "i8": S.PRECISION_INT8, "i4": S.PRECISION_INT4,
+                "i2": S.PRECISION_INT2}[fmt]
+        S.save_spingalett(src, path, prec, do_not_save_optimizer=True)
+        net = S.load_spingalett(path)
+    S.free_network(src)
+    D = [(S.weights_view(net, l).astype(np.float64), S.biases_view(net, l).astype(np.float64)) for l in range(len(acts))]
+    f = {"tanh": np.tanh, "sigmoid": lambda z: 1 / (1 + np.exp(-z)), "leaky_relu": lambda z: np.where(z > 0, z, 0.01 * z),
+         "foo52": lambda z: np.where(z > 1, 1 + 0.01 * (z - 1), np.where(z < 0, 0.01 * z, z)), "none": lambda z: z}
+    X = rng.standard_normal((max(sizes), topo[0])).astype(F32)
+    X[0, 5] = np.inf
+    X[1::7, topo[0] - 1] = -np.inf
+    X[2::7, 3] = np.nan
+    with np.errstate(invalid="ignore", over="ignore"):
+        a = X.astype(np.float64)
+        for (w, c), name in zip(D, acts):
+            a = f[name](a @ w.T + c)
+    for n in sizes:
+        for split in ([False, True] if n > 4 else [False]):
+            assert S.lib().spingalett_set_net_activations(net, S.NET_ACTIVATIONS_SPLIT if split else S.NET_ACTIVATIONS_DEFAULT) == 0
+            got = S.forward_batch(net, X[:n])
+            assert _same_nonfinite(got, a[:n]), (n, split)
+            fin = np.isfinite(a[:n])
+            assert not fin.any() or rel_max_abs(got[fin], a[:n][fin]) <= (TOL_VEC if n <= 4 else TOL_MFMA), (n, split)
     S.free_network(net)
 
 
