@@ -504,22 +504,30 @@ static bool write_array(FILE *fp, const float *src, uint32_t n, PrecisionMode p,
 
 /* A file that exists is written over and cut to its new length at the end (also after a failed write), instead of being
  * emptied first: giving up its cached pages, many of them still waiting for the disk, and making as many new ones cost
- * more than writing them (a 3.7 MB file saved again and again: 1.0 ms to empty it, 0.2 ms to write it). */
-static FILE *open_for_overwrite(const char *name)
+ * more than writing them (a 3.7 MB file saved again and again: 1.0 ms to empty it, 0.2 ms to write it).  Until it has its
+ * length such a file has new arrays in front of old ones, which nothing else would tell from a whole file: its version is
+ * zero while it is written, which every loader refuses, and comes last (*held: it does). */
+static FILE *open_for_overwrite(const char *name, bool *held)
 {
+    struct stat st;
     const int fd = open(name, O_WRONLY | O_CREAT | O_CLOEXEC, 0666);
     FILE *fp = fd >= 0 ? fdopen(fd, "wb") : NULL;
     if (fd >= 0 && !fp) close(fd);
+    *held = fp && fstat(fd, &st) == 0 && S_ISREG(st.st_mode) && st.st_size > 0;
     return fp;
 }
 
-static bool close_at_length(FILE *fp)
+static bool close_at_length(FILE *fp, bool held)
 {
+    static const uint16_t version = SPINGALETT_FORMAT_VERSION;
     struct stat st;
     bool ok = fflush(fp) == 0;
     if (fstat(fileno(fp), &st) == 0 && S_ISREG(st.st_mode)) {
         const off_t end = ftello(fp);
-        if (end >= 0 && end < st.st_size && ftruncate(fileno(fp), end) != 0) ok = false;
+        bool cut = end >= 0;
+        if (cut && end < st.st_size) cut = ftruncate(fileno(fp), end) == 0;
+        if (held && (!cut || end < 2 || pwrite(fileno(fp), &version, 2, 0) != 2)) cut = false;
+        ok = ok && cut;
     }
     return fclose(fp) == 0 && ok;
 }
@@ -546,7 +554,8 @@ void save_spingalett_struct_arguments(SaveArgs args)
         sprintf(owned, "%s.nn", name);
         name = owned;
     }
-    FILE *fp = open_for_overwrite(name);
+    bool held = false;
+    FILE *fp = open_for_overwrite(name, &held);
     if (!fp) {
         sp_set_error(SPINGALETT_ERR_INVALID, "save: cannot open file for writing");
         free(owned);
@@ -556,7 +565,7 @@ void save_spingalett_struct_arguments(SaveArgs args)
     const uint8_t has_opt = args.do_not_save_optimizer ? 0 : 1;
     uint8_t head[32];
     size_t h = 0;
-    const uint16_t version = SPINGALETT_FORMAT_VERSION;
+    const uint16_t version = held ? 0u : SPINGALETT_FORMAT_VERSION;
     memcpy(head + h, &version, 2); h += 2;
     memcpy(head + h, &net->layers, 4); h += 4;
     head[h++] = (uint8_t)net->loss_func;
@@ -572,7 +581,7 @@ void save_spingalett_struct_arguments(SaveArgs args)
     if (!ok) {
         sp_set_error(SPINGALETT_ERR_INVALID, "save: failed to write header");
         sp_log(LOG_ERROR, "Failed to write file header to %s", name);
-        (void)close_at_length(fp);
+        (void)close_at_length(fp, held);
         free(owned);
         return;
     }
@@ -591,14 +600,14 @@ void save_spingalett_struct_arguments(SaveArgs args)
               && write_array(fp, net->opt_v_biases + bo, bcount, p, &scratch);
     }
     free(scratch);
-    if (!close_at_length(fp)) ok = false;
+    if (!close_at_length(fp, held)) ok = false;
     if (!ok) {
         sp_set_error(SPINGALETT_ERR_INVALID, "save: write error (disk full?)");
         sp_log(LOG_ERROR, "Write error saving to %s", name);
     } else {
         sp_log(LOG_INFO, "Network saved to %s", name);
         sp_log(LOG_INFO, "Save info: format=v%u, layers=%u, weights=%llu, biases=%llu, precision=%s, optimizer=%s",
-               (unsigned)version, net->layers, (unsigned long long)net->total_weights,
+               (unsigned)SPINGALETT_FORMAT_VERSION, net->layers, (unsigned long long)net->total_weights,
                (unsigned long long)net->total_biases, sp_precision_names[p], has_opt ? "ON" : "OFF");
     }
     free(owned);

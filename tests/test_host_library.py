@@ -442,3 +442,44 @@ def test_codecs_at_block_thread_and_piece_edges(S, O, tmp_path, count):
             assert np.array_equal(bits(S.weights_view(again, 0)), bits(want.W(0))), (fmt, mode)
             S.free_network(again)
         S.lib().spingalett_set_dequant_mode(S.DEQUANT_STRICT)
+
+
+@pytest.mark.parametrize("fmt", ["f32", "i8"])
+@pytest.mark.parametrize("killed", [True, False])
+def test_a_save_over_an_old_file_that_ends_halfway_does_not_load(S, O, fmt, killed, tmp_path):
+    """A process killed while it writes over a file (the autosave of a training that is stopped), or whose disk is full:
+    new arrays in front of old ones at the old length must not pass for a net.  The file size limit ends the write at
+    60 % of the file, with the signal's default action or as a failed write."""
+    import signal
+    import subprocess
+    import sys
+    path = str(tmp_path / "net.nn")
+    net = S.new_spingalett()
+    S.layer(net, 600)
+    S.layer(net, 500, S.ACT_RELU, S.WEIGHT_INITIALIZATION_HE)
+    S.layer(net, 700, S.ACT_TANH, S.WEIGHT_INITIALIZATION_HE)
+    S.save_spingalett(net, path, PREC[fmt], do_not_save_optimizer=True)
+    size = os.path.getsize(path)
+    code = (f"import sys, signal, resource; sys.path.insert(0, {ROOT!r}); import spingalett_amd as S; S.set_verbose(False)\n"
+            f"net = S.load_spingalett({path!r}); S.weights_view(net, 0)[:] *= 2\n"
+            f"signal.signal(signal.SIGXFSZ, signal.SIG_DFL if {killed} else signal.SIG_IGN)\n"
+            f"resource.setrlimit(resource.RLIMIT_CORE, (0, 0))\n"
+            f"resource.setrlimit(resource.RLIMIT_FSIZE, ({size * 6 // 10}, {size * 6 // 10}))\n"
+            f"S.save_spingalett(net, {path!r}, {PREC[fmt]}, do_not_save_optimizer=True)\n"
+            f"sys.exit(3 if S.last_error()[0] else 0)\n")
+    res = subprocess.run([sys.executable, "-c", code])
+    assert res.returncode == (-signal.SIGXFSZ if killed else 3)
+    S.clear_error()
+    back = S.load_spingalett(path)
+    if killed:
+        assert back is None and S.last_error() == (S.SPINGALETT_ERR_INVALID, "load: unsupported format version")
+    else:
+        assert S.last_error() == (S.SPINGALETT_ERR_INVALID, "load: file appears truncated or corrupt")
+        assert os.path.getsize(path) == size * 6 // 10
+        S.free_network(back)
+    S.clear_error()
+    S.save_spingalett(net, path, PREC[fmt], do_not_save_optimizer=True)             # and a whole one over what is left
+    again = S.load_spingalett(path)
+    assert again is not None and S.last_error()[0] == 0
+    S.free_network(again)
+    S.free_network(net)
