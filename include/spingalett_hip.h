@@ -99,6 +99,8 @@ SPHIP_API int  sphip_forward(sphip_net *net, const float *x, uint32_t n, float *
  * splits, FP16 copies of small integer layers) is laid out in one fixed array of SPHIP_NOALLOC_SCRATCH_BYTES that each
  * GPU holds from library load until the process ends; the call makes no device or pinned allocation and frees none.
  * A batch whose workspace exceeds the array is refused with an error that names both sizes (sphip_forward takes it).
+ * The workspace is counted at the widths of the topology; where the padded widths that 16-bit and integer nets of ragged
+ * widths run with need more, the batch runs in blocks of rows (sphip_forward's results for those blocks).
  * Nothing in the array needs clearing between calls: every kernel reads only what this call wrote.  All calls on one
  * GPU share the array, so two calls that overlap in time (from different threads) race; nets of more than 64 layers
  * are refused.  flags: SPHIP_FORCE_GEMM / SPHIP_FORCE_GEMV / SPHIP_BF16_ACTIVATIONS /

@@ -119,8 +119,9 @@ std::mutex g_init_mutex;
 // Workspace of sphip_forward_noalloc: one fixed array per GPU, held until the process ends.  Host code never uses the
 // array's name as an address: g_scratch_ptr[device] is what hipGetSymbolAddress returned with that device current.
 constexpr size_t kScratchBytes = SPHIP_NOALLOC_SCRATCH_BYTES;
+constexpr size_t kScratchRoom = kScratchBytes + (64u << 10);       // a row of padded widths where the widths themselves fit
 constexpr int kScratchDevices = 16;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchRoom];
 unsigned char *g_scratch_ptr[kScratchDevices] = {};
 
 // address of the scratch array on the current device (looked up once per device); caller holds g_init_mutex
@@ -1525,10 +1526,10 @@ struct WorkspaceNeed {
 };
 
 // an integer layer with at most 64 outputs streams the activations against an FP16 copy of its codes
-bool layer_wants_codes16(const sphip_net *net, uint32_t l /*1-based*/, uint32_t n)
+bool layer_wants_codes16(const sphip_net *net, const std::vector<uint32_t> &width, uint32_t l /*1-based*/, uint32_t n)
 {
     if (net->prec < I8) return false;
-    const ThinPlan tp = plan_thin(net->prec, n, net->ptopo[l], net->ptopo[l - 1]);
+    const ThinPlan tp = plan_thin(net->prec, n, width[l], width[l - 1]);
     return tp.use && tp.mode_b;
 }
 
@@ -1541,22 +1542,25 @@ uint32_t cat3_kp(uint32_t K) { return (K + 7u) & ~7u; }
 bool cat3_layer(uint32_t n, uint32_t N, uint32_t K) { return N >= 128u && 2.0 * (double)n * N * K >= 3e9; }
 
 // In a split-activation forward of a 16-bit or integer net every matrix-core layer writes one set of partial sums per
-// activation matrix (halves = 2)
-WorkspaceNeed workspace_need(const sphip_net *net, uint32_t n, uint32_t flags)
+// activation matrix (halves = 2).  width: the net's padded widths, which it runs with, or those it was made with.
+WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &width, uint32_t n, uint32_t flags)
 {
     WorkspaceNeed w{};
+    uint32_t widest = 0;
+    for (uint32_t l = 0; l < net->layers; ++l)
+        if (width[l] > widest) widest = width[l];
     const Regime reg = pick_regime(net, n, flags);
     const uint32_t halves = (flags & SPHIP_SPLIT_ACTIVATIONS) && reg == R_GEMM16 ? 2u : 1u;
-    w.act_floats = (uint64_t)n * net->max_width;
+    w.act_floats = (uint64_t)n * widest;
     for (uint32_t l = 1; l < net->layers; ++l)
-        if (net->act[l - 1] == A_SOFTMAX && (uint64_t)n * net->ptopo[l] > w.soft_floats) w.soft_floats = (uint64_t)n * net->ptopo[l];
+        if (net->act[l - 1] == A_SOFTMAX && (uint64_t)n * width[l] > w.soft_floats) w.soft_floats = (uint64_t)n * width[l];
     if (n <= 64 && net->prec >= I8) {
-        const uint64_t padded = (uint64_t)n * ((uint64_t)net->max_width + 4096u);
+        const uint64_t padded = (uint64_t)n * ((uint64_t)widest + 4096u);
         w.plane_bytes = padded * 4u;
         w.plane_recs = padded / 64u + 64u;
     }
     for (uint32_t l = 1; l < net->layers; ++l) {
-        const uint32_t N = net->ptopo[l], K = net->ptopo[l - 1];
+        const uint32_t N = width[l], K = width[l - 1];
         uint32_t kper = 0;
         uint64_t ws = 0;
         if (reg == R_CAT3 && cat3_layer(n, N, K)) {
@@ -1659,7 +1663,7 @@ int pad_layer(sphip_net *net, uint32_t l, bool weights, bool biases)
 // grows the net's own workspace to what n samples need
 int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
 {
-    const WorkspaceNeed need = workspace_need(net, n, flags);
+    const WorkspaceNeed need = workspace_need(net, net->ptopo, n, flags);
     if (need.cat_elems > net->cat_cap) {
         if (net->cat_buf) { HCHECK(hipFree(net->cat_buf)); net->cat_buf = nullptr; }
         net->cat_cap = 0;
@@ -1704,7 +1708,7 @@ int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
     }
     for (uint32_t l = 1; l < net->layers; ++l) {
         DevArray &wa = net->w(l - 1);
-        if (layer_wants_codes16(net, l, n) && !wa.codes16_valid && net->W[l - 1].uploaded) {
+        if (layer_wants_codes16(net, net->ptopo, l, n) && !wa.codes16_valid && net->W[l - 1].uploaded) {
             if (!wa.codes16) HCHECK(hipMalloc((void **)&wa.codes16, wa.count * sizeof(uint16_t)));
             launch_codes16(net->prec, wa.base, wa.codes16, wa.count);
             HCHECK(hipGetLastError());
@@ -2220,16 +2224,51 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
         std::lock_guard<std::mutex> lock(g_init_mutex);
         if (scratch_lookup(&base)) return 1;
     }
-    // lay the workspace out inside the scratch array, every piece at a multiple of 256 bytes
-    const WorkspaceNeed need = workspace_need(net, n, flags);
-    if (need.cat_elems)
+    // an integer layer with few outputs reads an FP16 copy of its codes: the net's own if an earlier call made one,
+    // else one made here, in the scratch array, on every call
+    // (only the matrix-core regime reads them: a forced vector forward or one of up to four samples never does)
+    const uint32_t fwd_flags = flags & (SPHIP_FORCE_GEMM | SPHIP_FORCE_GEMV | SPHIP_BF16_ACTIVATIONS | SPHIP_SPLIT_ACTIVATIONS);
+    const bool reads_codes = pick_regime(net, n, fwd_flags) == R_GEMM16;
+    // every piece of the workspace lies at a multiple of 256 bytes
+    auto room = [](uint64_t bytes) { return (size_t)((bytes + 255u) & ~(uint64_t)255u); };
+    auto pieces = [&](const WorkspaceNeed &w) {
+        return 2u * room(w.act_floats * sizeof(float)) + room(w.soft_floats * sizeof(float)) + room(w.plane_bytes) +
+               (w.plane_bytes ? room(w.plane_recs * sizeof(float)) + room(w.plane_recs * 4u * sizeof(int)) : 0u) +
+               room(w.split_floats * sizeof(float)) + room(w.cat_elems * sizeof(uint16_t));
+    };
+    auto all = [&](const std::vector<uint32_t> &width, const WorkspaceNeed &w) {
+        size_t bytes = pieces(w);
+        for (uint32_t l = 1; l < net->layers && reads_codes; ++l)
+            if (layer_wants_codes16(net, width, l, n) && !net->w(l - 1).codes16_valid)
+                bytes += room((uint64_t)width[l - 1] * width[l] * sizeof(uint16_t));
+        return bytes;
+    };
+    // A batch that fits at the widths of the caller's net is accepted, whatever the padding needs.
+    const WorkspaceNeed plain = workspace_need(net, net->topo, n, flags);
+    if (plain.cat_elems)
         for (uint32_t l = 1; l < net->layers; ++l)
             if (cat3_layer(n, net->ptopo[l], net->ptopo[l - 1]) && !net->w(l - 1).cat3_valid)
                 return fail_msg("sphip_forward_noalloc: the split mode of an FP32 net needs FP16 parts of its weights, which the first sphip_forward in that mode makes");
+    uint32_t rows = n;
+    WorkspaceNeed need = workspace_need(net, net->ptopo, rows, flags);
+    const size_t known = all(net->topo, plain);
+    if (known > kScratchBytes && all(net->ptopo, need) > kScratchBytes) {
+        snprintf(g_err, sizeof g_err, "sphip_forward_noalloc: %u samples of this net need %zu bytes of workspace, the fixed scratch array holds %zu",
+                 n, known, kScratchBytes);
+        return 1;
+    }
+    // Where the padded widths do need more, the batch runs in the fewest equal blocks of rows that fit, and without the
+    // copies of codes that do not (the tile kernels read the codes themselves).
+    for (uint32_t blocks = 2; pieces(need) > kScratchRoom && rows > 1u; ++blocks) {
+        rows = (n + blocks - 1u) / blocks;
+        if (rows > 4u) rows = (rows + 3u) & ~3u;             // the next block's rows start as aligned as the first one's
+        need = workspace_need(net, net->ptopo, rows, flags);
+    }
+    if (pieces(need) > kScratchRoom) return fail_msg("sphip_forward_noalloc: one row of this net does not fit the fixed scratch array");
     size_t used = 0;
     auto take = [&](uint64_t bytes) -> unsigned char * {
         unsigned char *p = base + used;
-        used += (size_t)((bytes + 255u) & ~(uint64_t)255u);
+        used += room(bytes);
         return p;
     };
     uint16_t *codes[kMaxLayers] = {};
@@ -2245,34 +2284,25 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
     wk.split_ws = reinterpret_cast<float *>(take(need.split_floats * sizeof(float)));
     wk.split_cap = need.split_floats;
     if (need.cat_elems) wk.cat = reinterpret_cast<uint16_t *>(take(need.cat_elems * sizeof(uint16_t)));
-    // an integer layer with few outputs reads an FP16 copy of its codes: the net's own if an earlier call made one,
-    // else one made here, in the scratch array, on every call
-    // (only the matrix-core regime reads them: a forced vector forward or one of up to four samples never does)
-    const uint32_t fwd_flags = flags & (SPHIP_FORCE_GEMM | SPHIP_FORCE_GEMV | SPHIP_BF16_ACTIVATIONS | SPHIP_SPLIT_ACTIVATIONS);
-    const bool reads_codes = pick_regime(net, n, fwd_flags) == R_GEMM16;
-    bool fresh[kMaxLayers] = {};
     for (uint32_t l = 1; l < net->layers; ++l) {
-        if (!reads_codes || !layer_wants_codes16(net, l, n)) continue;
+        if (!reads_codes || !layer_wants_codes16(net, net->ptopo, l, rows)) continue;
         const DevArray &wa = net->w(l - 1);
         if (wa.codes16_valid) { codes[l - 1] = wa.codes16; continue; }
+        if (used + room(wa.count * sizeof(uint16_t)) > kScratchRoom) continue;
         codes[l - 1] = reinterpret_cast<uint16_t *>(take(wa.count * sizeof(uint16_t)));
-        fresh[l - 1] = true;
+        launch_codes16(net->prec, wa.base, codes[l - 1], wa.count);
     }
     wk.codes16 = codes;
-    if (used > kScratchBytes) {
-        snprintf(g_err, sizeof g_err, "sphip_forward_noalloc: %u samples of this net need %zu bytes of workspace, the fixed scratch array holds %zu",
-                 n, used, kScratchBytes);
-        return 1;
-    }
     if (need.big_floats > need.split_floats && used + need.big_floats * sizeof(float) <= kScratchBytes) {
         wk.split_ws = reinterpret_cast<float *>(take(need.big_floats * sizeof(float)));
         wk.split_cap = need.big_floats;
     }
-    for (uint32_t l = 1; l < net->layers; ++l)
-        if (fresh[l - 1]) launch_codes16(net->prec, net->w(l - 1).base, codes[l - 1], net->w(l - 1).count);
     // the integer GEMV's quantise launch is never skipped here (that shortcut belongs to the layer timer)
     net->aq_valid_layer = 0;
-    return enqueue_forward(net, wk, d_x, n, d_y, fwd_flags, 0);
+    const uint32_t in_w = net->topo[0], out_w = net->topo[net->layers - 1];
+    for (uint32_t r0 = 0; r0 < n; r0 += rows)
+        if (enqueue_forward(net, wk, d_x + (size_t)r0 * in_w, n - r0 < rows ? n - r0 : rows, d_y + (size_t)r0 * out_w, fwd_flags, 0)) return 1;
+    return 0;
 }
 
 int sphip_forward_layers(sphip_net *net, const float *x, float *host_neurons)

@@ -123,3 +123,25 @@ def test_noalloc_forward_refuses_what_does_not_fit(S):
     assert np.array_equal(d_y2.to_numpy(F32, (100, 16)), net.forward(X))
     assert S.lib().sphip_forward_noalloc(net.h, None, 100, d_y2.ptr, 0) == 1          # argument check
     net.destroy()
+
+
+@pytest.mark.parametrize("fmt,topo,n,flags", [
+    ("f16", [65, 65, 65, 5], 120000, 0),                  # 59.5 MiB of activations, 65.9 at the padded widths: two blocks of rows
+    ("i2", [65, 65, 65, 5], 100000, 0),                   # 49.6 and 97.7 MiB (65 codes run as 128)
+    ("i2", [3, 1, 33, 2], 250001, 0),                     # widths below one unit, a batch that blocks do not divide
+    ("i8", [777, 1030, 515, 33], 4000, 128),              # split activations: partial sums of both matrices
+    ("i8", [16, 400001, 40, 10], 8, 0),                   # the FP16 copy of the codes does not fit: the tile kernel
+])
+def test_noalloc_forward_takes_what_fits_without_the_padding(S, fmt, topo, n, flags):
+    """What is accepted goes by the net's own widths; 2e-2 against sphip_forward like every 16-bit route against another
+    (a block of rows may take another kernel than the whole batch)."""
+    net = _net(S, fmt, topo, [S.ACT_TANH] * (len(topo) - 2) + [S.ACT_NONE], seed=sum(topo))
+    X = np.random.default_rng(n).standard_normal((n, topo[0])).astype(F32)
+    d_x = S.DeviceBuffer.from_numpy(X)
+    d_y = S.DeviceBuffer.from_numpy(np.full(n * topo[-1], np.nan, F32))
+    assert net.forward_noalloc(d_x, n, d_y, flags) == 0, S.lib().sphip_last_error_string()
+    S.synchronize()
+    got, want = d_y.to_numpy(F32, (n, topo[-1])), net.forward(X, flags)
+    assert np.isfinite(got).all()
+    assert np.max(np.abs(got - want)) <= 2e-2 * np.max(np.abs(want))
+    net.destroy()
