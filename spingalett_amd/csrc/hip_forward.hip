@@ -167,6 +167,7 @@ struct DecodeParams {
     float max_val;       // scale from the file
     float rel_scale;     // fl(max * fl(1/d))  (mode 1)
     int mode;            // 0 strict, 1 release
+    uint32_t cols, pcols;  // elements of a row, and of a row as it lies (padded_width)
     float lut[256];
 };
 
@@ -175,14 +176,15 @@ __global__ __launch_bounds__(256) void sp_decode(const DecodeParams p)
 {
     uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
     if (i >= p.n) return;
+    const uint64_t at = p.cols == p.pcols ? i : i / p.cols * p.pcols + i % p.cols;
     float v;
     if constexpr (FMT == F32 || FMT == F16 || FMT == BF16) {
-        v = elem_value<FMT>(p.codes, i);
+        v = elem_value<FMT>(p.codes, at);
     } else {
         if (!(p.max_val > 0.0f)) {
             v = 0.0f;
         } else {
-            int q = int_code<FMT>(p.codes, i);
+            int q = int_code<FMT>(p.codes, at);
             if (FMT == I2) v = __fmul_rn((float)q, p.max_val);                    // Serialize.c:285
             else if (p.mode == 1) v = __fmul_rn((float)q, p.rel_scale);
             else v = __fmul_rn(p.lut[q + (FMT == I8 ? 128 : 8)], p.max_val);      // Serialize.c:233,258
@@ -577,6 +579,7 @@ struct DevArray {
     uint8_t *base = nullptr;       // inside sphip_net::arrays, at a multiple of 256 bytes
     size_t bytes = 0;
     uint64_t count = 0;
+    uint64_t laid = 0;             // elements that lie at base: the uploaded ones, and zeros around them (padded_width)
     float max_val = 0.0f;
     bool uploaded = false;
     uint16_t *codes16 = nullptr;   // weights of a layer with few outputs: unscaled codes as FP16 (made on demand)
@@ -610,16 +613,19 @@ struct sphip_net {
     std::vector<uint32_t> topo;
     std::vector<uint8_t> act;
     int prec = 0;
-    std::vector<DevArray> W, B;    // [layers-1] as uploaded (W: zero rows behind it up to the padded outputs)
-    // Widths whose weight rows would not be whole 16-byte units run padded with zero weights (padded_width); PW / PB are
-    // the arrays of the layers this touches, base == nullptr where the uploaded ones serve.
-    uint8_t *arrays = nullptr;     // the one allocation behind every base
+    std::vector<DevArray> W, B;    // [layers-1] as uploaded, zeros behind them up to the padded outputs
+    // Widths whose weight rows would not be whole 16-byte units run padded with zero weights (padded_width); PW are the
+    // weights of the layers whose inputs that touches.  They lie on the device instead of W (base == nullptr there), but
+    // for the first layer, whose uploaded rows the vector kernels multiply with the caller's.
     std::vector<uint32_t> ptopo;
-    std::vector<DevArray> PW, PB;
+    std::vector<DevArray> PW;
+    uint8_t *arrays = nullptr;     // the one allocation behind every base, its size ...
+    size_t arrays_bytes = 0;
+    uint8_t *pad_stage = nullptr;  // ... and behind it the room through which uploaded rows reach PW
+    size_t pad_stage_bytes = 0;
 
     DevArray &w(uint32_t l) { return PW[l].base ? PW[l] : W[l]; }                    // what a forward multiplies with
     const DevArray &w(uint32_t l) const { return PW[l].base ? PW[l] : W[l]; }
-    const DevArray &b(uint32_t l) const { return PB[l].base ? PB[l] : B[l]; }
     // workspace, grown on demand
     uint64_t cap_elems = 0;        // capacity of each ping-pong buffer in FP32 elements
     void *buf[2] = {nullptr, nullptr};
@@ -705,7 +711,7 @@ uint32_t padded_width(int fmt, uint32_t w, uint32_t next, bool hidden)
 LayerArgs make_layer_args(const sphip_net *net, uint32_t l /*1-based layer*/, bool raw = false)
 {
     LayerArgs L{};
-    const DevArray &w = raw ? net->W[l - 1] : net->w(l - 1), &b = net->b(l - 1);
+    const DevArray &w = raw ? net->W[l - 1] : net->w(l - 1), &b = net->B[l - 1];
     L.w = w.base;
     L.bias = b.base;
     L.wscale = fmt_scale(net->prec, net->W[l - 1].max_val);
@@ -1634,29 +1640,43 @@ int make_cat3(DevArray &wa, uint32_t N, uint32_t K)
     return 0;
 }
 
-// The padded arrays of one layer from the uploaded ones (sp_pad_rows).  Enqueues only.
-int pad_layer(sphip_net *net, uint32_t l, bool weights, bool biases)
+// Rows r0 .. r0 + rows of a layer's weights, as uploaded, into its padded array, and zero rows behind the last one
+// (sp_pad_rows).  Enqueues only.
+int pad_rows(sphip_net *net, uint32_t l, const uint8_t *src, uint32_t r0, uint32_t rows)
 {
-    if (net->prec == F32) return 0;                        // (never padded)
     const uint32_t N = net->topo[l + 1], K = net->topo[l], Np = net->ptopo[l + 1], Kp = net->ptopo[l];
-    DevArray &pw = net->PW[l], &pb = net->PB[l];
-    auto go = [&](const DevArray &src, DevArray &dst, uint32_t rows, uint32_t cols, uint32_t prows, uint32_t pcols) {
-        const uint64_t words = (fmt_bytes(net->prec, (uint64_t)prows * pcols) + 3u) / 4u;
-        const uint32_t grid = (uint32_t)((words + 255u) / 256u);
-        uint32_t *out = reinterpret_cast<uint32_t *>(dst.base);
-        switch (fmt_bits(net->prec)) {
-        case 16: sp_pad_rows<16><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
-        case 8:  sp_pad_rows<8><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
-        case 4:  sp_pad_rows<4><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
-        default: sp_pad_rows<2><<<grid, 256, 0, g_stream>>>(src.base, out, rows, cols, pcols, words); break;
-        }
-    };
-    if (weights && pw.base) {
-        go(net->W[l], pw, N, K, Np, Kp);
-        pw.codes16_valid = pw.wide16_valid = pw.cat3_valid = false;
+    const uint64_t row_bytes = fmt_bytes(net->prec, Kp);                        // (a multiple of 16)
+    const uint64_t words = row_bytes / 4u * (r0 + rows == N ? Np - r0 : rows);
+    const uint32_t grid = (uint32_t)((words + 255u) / 256u);
+    uint32_t *out = reinterpret_cast<uint32_t *>(net->PW[l].base + row_bytes * r0);
+    switch (fmt_bits(net->prec)) {
+    case 16: sp_pad_rows<16><<<grid, 256, 0, g_stream>>>(src, out, rows, K, Kp, words); break;
+    case 8:  sp_pad_rows<8><<<grid, 256, 0, g_stream>>>(src, out, rows, K, Kp, words); break;
+    case 4:  sp_pad_rows<4><<<grid, 256, 0, g_stream>>>(src, out, rows, K, Kp, words); break;
+    default: sp_pad_rows<2><<<grid, 256, 0, g_stream>>>(src, out, rows, K, Kp, words); break;
     }
-    if (biases && pb.base) go(net->B[l], pb, 1, N, 1, Np);
     HCHECK(hipGetLastError());
+    return 0;
+}
+
+// A layer's weights to where they lie.  Layers behind a padded one go row by row through pad_stage, four rows at a time or
+// a multiple of that: the codes of four rows are whole bytes.
+int upload_weights(sphip_net *net, uint32_t l, const uint8_t *codes)
+{
+    const DevArray &a = net->W[l];
+    if (a.base) {
+        HCHECK(hipMemcpyAsync(a.base, codes, a.bytes, hipMemcpyHostToDevice, g_stream));
+        return net->PW[l].base ? pad_rows(net, l, a.base, 0, net->topo[l + 1]) : 0;
+    }
+    const uint32_t N = net->topo[l + 1], K = net->topo[l];
+    const uint64_t four = fmt_bytes(net->prec, 4ull * K);
+    const uint64_t step64 = net->pad_stage_bytes / four * 4u;
+    const uint32_t step = step64 < N ? (uint32_t)step64 : N;
+    for (uint32_t r0 = 0; r0 < N; r0 += step) {
+        const uint32_t rows = N - r0 < step ? N - r0 : step;
+        HCHECK(hipMemcpyAsync(net->pad_stage, codes + four * (r0 / 4u), fmt_bytes(net->prec, (uint64_t)rows * K), hipMemcpyHostToDevice, g_stream));
+        if (pad_rows(net, l, net->pad_stage, r0, rows)) return 1;
+    }
     return 0;
 }
 
@@ -1709,8 +1729,8 @@ int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
     for (uint32_t l = 1; l < net->layers; ++l) {
         DevArray &wa = net->w(l - 1);
         if (layer_wants_codes16(net, net->ptopo, l, n) && !wa.codes16_valid && net->W[l - 1].uploaded) {
-            if (!wa.codes16) HCHECK(hipMalloc((void **)&wa.codes16, wa.count * sizeof(uint16_t)));
-            launch_codes16(net->prec, wa.base, wa.codes16, wa.count);
+            if (!wa.codes16) HCHECK(hipMalloc((void **)&wa.codes16, wa.laid * sizeof(uint16_t)));
+            launch_codes16(net->prec, wa.base, wa.codes16, wa.laid);
             HCHECK(hipGetLastError());
             wa.codes16_valid = true;
         }
@@ -1927,7 +1947,6 @@ int sphip_create(const sphip_desc *desc, sphip_net **out)
     net->W.resize(desc->layers - 1);
     net->B.resize(desc->layers - 1);
     net->PW.resize(desc->layers - 1);
-    net->PB.resize(desc->layers - 1);
     net->codes16_ptrs.assign(desc->layers - 1, nullptr);
     for (uint32_t l = 0; l < desc->layers; ++l) {
         const bool hidden_softmax = l && net->act[l - 1] == A_SOFTMAX;
@@ -1940,32 +1959,44 @@ int sphip_create(const sphip_desc *desc, sphip_net **out)
     // All arrays in one allocation, each at a multiple of 256 bytes with 16 bytes of slack: vector loads of the last chunk
     // never leave it.  (A hipMalloc takes 10 to 100 us.)
     size_t at = 0;
-    auto place = [&](DevArray &a, uint64_t count, uint64_t room) {
-        a.count = count;
-        a.bytes = fmt_bytes(net->prec, count);
-        a.base = reinterpret_cast<uint8_t *>(at);
-        at += (fmt_bytes(net->prec, room) + 16u + 255u) & ~(size_t)255u;
-    };
     std::vector<DevArray *> placed;
+    auto place = [&](DevArray &a, uint64_t laid) {
+        a.laid = laid;
+        a.base = reinterpret_cast<uint8_t *>(at);
+        at += (fmt_bytes(net->prec, laid) + 16u + 255u) & ~(size_t)255u;
+        placed.push_back(&a);
+    };
+    bool padded = false;
     for (uint32_t l = 0; l + 1 < desc->layers; ++l) {
         const uint64_t K = net->topo[l], N = net->topo[l + 1], Kp = net->ptopo[l], Np = net->ptopo[l + 1];
-        place(net->W[l], K * N, K * Np);
-        place(net->B[l], N, N);
-        placed.insert(placed.end(), {&net->W[l], &net->B[l]});
-        if (Np != N || Kp != K) { place(net->PW[l], Kp * Np, Kp * Np); placed.push_back(&net->PW[l]); }
-        if (Np != N) { place(net->PB[l], Np, Np); placed.push_back(&net->PB[l]); }
+        DevArray &w = net->W[l], &b = net->B[l];
+        w.count = K * N;
+        w.bytes = fmt_bytes(net->prec, w.count);
+        b.count = N;
+        b.bytes = fmt_bytes(net->prec, b.count);
+        if (Kp == K || l == 0) place(w, K * Np);
+        if (Kp != K) place(net->PW[l], Kp * Np);
+        place(b, Np);
+        padded |= Np != N || Kp != K;
+        if (!w.base && l) {
+            // at most 4 MiB, at least four rows
+            const size_t four = fmt_bytes(net->prec, 4ull * K);
+            size_t stage = w.bytes + four < (4u << 20) ? w.bytes + four : (4u << 20);
+            if (stage < four) stage = four;
+            if (stage > net->pad_stage_bytes) net->pad_stage_bytes = stage;
+        }
     }
-    if (hipMalloc((void **)&net->arrays, at) != hipSuccess) {
+    net->arrays_bytes = at;
+    if (hipMalloc((void **)&net->arrays, at + net->pad_stage_bytes) != hipSuccess) {
         for (DevArray *a : placed) a->base = nullptr;
+        net->arrays = nullptr;
         sphip_destroy(net);
         return fail_msg("sphip_create: device allocation failed");
     }
     for (DevArray *a : placed) a->base = net->arrays + reinterpret_cast<size_t>(a->base);
-    for (uint32_t l = 0; l + 1 < desc->layers; ++l)
-        if (net->PB[l].base) {                              // zero rows behind the uploaded ones
-            const uint64_t floats = (fmt_bytes(net->prec, (uint64_t)net->topo[l] * net->ptopo[l + 1]) + 16u) / 4u;
-            sp_fill0<<<(uint32_t)((floats + 255u) / 256u), 256, 0, g_stream>>>(reinterpret_cast<float *>(net->W[l].base), floats);
-        }
+    net->pad_stage = net->arrays + at;
+    if (padded)                                             // the zeros around the arrays that are uploaded
+        sp_fill0<<<(uint32_t)((at / 4u + 255u) / 256u), 256, 0, g_stream>>>(reinterpret_cast<float *>(net->arrays), at / 4u);
     *out = net;
     return 0;
 }
@@ -1975,7 +2006,7 @@ void sphip_destroy(sphip_net *net)
     if (!net) return;
     if (g_stream) (void)hipStreamSynchronize(g_stream);
     train_free(net);
-    for (auto *arrays : {&net->W, &net->PW, &net->B, &net->PB})
+    for (auto *arrays : {&net->W, &net->PW, &net->B})
         for (auto &a : *arrays) {
             if (a.codes16) (void)hipFree(a.codes16);
             if (a.wide16) (void)hipFree(a.wide16);
@@ -2004,19 +2035,19 @@ void sphip_destroy(sphip_net *net)
 // The word the reduction leaves its result in sits behind the copy, in the same allocation.
 int make_wide(DevArray &wa)
 {
-    const size_t copy_bytes = (wa.count * sizeof(uint16_t) + 15u) & ~(size_t)15u;
+    const size_t copy_bytes = (wa.laid * sizeof(uint16_t) + 15u) & ~(size_t)15u;
     if (!wa.wide16) HCHECK(hipMalloc((void **)&wa.wide16, copy_bytes + 16u));
     uint32_t *word = reinterpret_cast<uint32_t *>(reinterpret_cast<uint8_t *>(wa.wide16) + copy_bytes);
     const uint16_t *src = reinterpret_cast<const uint16_t *>(wa.base);
     uint32_t top = 0;
     HCHECK(hipMemsetAsync(word, 0, sizeof(uint32_t), g_stream));
-    uint64_t blocks = (wa.count + 255) / 256;
+    uint64_t blocks = (wa.laid + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    sp_absmax_bf16<<<(uint32_t)blocks, 256, 0, g_stream>>>(src, wa.count, word);
+    sp_absmax_bf16<<<(uint32_t)blocks, 256, 0, g_stream>>>(src, wa.laid, word);
     HCHECK(hipMemcpyAsync(&top, word, sizeof(uint32_t), hipMemcpyDeviceToHost, g_stream));
     HCHECK(hipStreamSynchronize(g_stream));
     wa.wide_shift = top ? 14 - ((int)(top >> 7) - 127) : 0;       // largest magnitude = 1.m x 2^(e - 127)
-    sp_bf16_to_f16<<<(uint32_t)((wa.count + 255) / 256), 256, 0, g_stream>>>(src, wa.wide16, wa.count, wa.wide_shift);
+    sp_bf16_to_f16<<<(uint32_t)((wa.laid + 255) / 256), 256, 0, g_stream>>>(src, wa.wide16, wa.laid, wa.wide_shift);
     HCHECK(hipGetLastError());
     HCHECK(hipStreamSynchronize(g_stream));
     wa.wide16_valid = true;
@@ -2028,14 +2059,12 @@ int sphip_upload_array(sphip_net *net, uint32_t l, int which, const void *codes,
     if (!net || l + 1 >= net->layers || (which != 0 && which != 1) || !codes) return fail_msg("sphip_upload_array: invalid argument");
     DevArray &a = which == 0 ? net->W[l] : net->B[l];
     if (bytes != a.bytes) return fail_msg("sphip_upload_array: byte count does not match the array's serialized size");
-    HCHECK(hipMemcpyAsync(a.base, codes, bytes, hipMemcpyHostToDevice, g_stream));
+    if (which == 1) HCHECK(hipMemcpyAsync(a.base, codes, bytes, hipMemcpyHostToDevice, g_stream));
+    else if (upload_weights(net, l, static_cast<const uint8_t *>(codes))) return 1;
     HCHECK(hipStreamSynchronize(g_stream));
     a.max_val = max_val;
     a.uploaded = true;
-    a.codes16_valid = false;
-    a.wide16_valid = false;
-    a.cat3_valid = false;
-    if (pad_layer(net, l, which == 0, which == 1)) return 1;
+    for (DevArray *copies : {&a, which == 0 ? &net->PW[l] : &a}) copies->codes16_valid = copies->wide16_valid = copies->cat3_valid = false;
     if (which == 0 && net->prec == BF16 && make_wide(net->w(l))) return 1;
     return 0;
 }
@@ -2046,24 +2075,23 @@ int sphip_clone(const sphip_net *src, sphip_net **out)
     sphip_desc d{src->layers, src->topo.data(), src->act.data(), (uint8_t)src->prec};
     sphip_net *net = nullptr;
     if (sphip_create(&d, &net)) return 1;
-    for (uint32_t l = 0; l + 1 < src->layers; ++l) {
-        for (int which = 0; which < 4; ++which) {
-            const DevArray &s = which == 0 ? src->W[l] : which == 1 ? src->B[l] : which == 2 ? src->PW[l] : src->PB[l];
-            DevArray &t = which == 0 ? net->W[l] : which == 1 ? net->B[l] : which == 2 ? net->PW[l] : net->PB[l];
-            if (!s.base) continue;
-            hipError_t e = hipMemcpyAsync(t.base, s.base, s.bytes, hipMemcpyDeviceToDevice, g_stream);
-            if (e != hipSuccess) { sphip_destroy(net); return fail_hip("sphip_clone copy", e); }
+    hipError_t e = hipMemcpyAsync(net->arrays, src->arrays, src->arrays_bytes, hipMemcpyDeviceToDevice, g_stream);   // (the same layout)
+    for (uint32_t l = 0; l + 1 < src->layers && e == hipSuccess; ++l) {
+        for (int which = 0; which < 2; ++which) {
+            const DevArray &s = which == 0 ? src->W[l] : src->B[l];
+            DevArray &t = which == 0 ? net->W[l] : net->B[l];
             t.max_val = s.max_val;
             t.uploaded = s.uploaded;
-            if (s.wide16_valid) {
-                e = hipMalloc((void **)&t.wide16, ((s.count * sizeof(uint16_t) + 15u) & ~(size_t)15u) + 16u);
-                if (e == hipSuccess) e = hipMemcpyAsync(t.wide16, s.wide16, s.count * sizeof(uint16_t), hipMemcpyDeviceToDevice, g_stream);
-                if (e != hipSuccess) { sphip_destroy(net); return fail_hip("sphip_clone copy", e); }
-                t.wide_shift = s.wide_shift;
-                t.wide16_valid = true;
-            }
         }
+        const DevArray &s = src->w(l);
+        DevArray &t = net->w(l);
+        if (!s.wide16_valid) continue;
+        e = hipMalloc((void **)&t.wide16, ((s.laid * sizeof(uint16_t) + 15u) & ~(size_t)15u) + 16u);
+        if (e == hipSuccess) e = hipMemcpyAsync(t.wide16, s.wide16, s.laid * sizeof(uint16_t), hipMemcpyDeviceToDevice, g_stream);
+        t.wide_shift = s.wide_shift;
+        t.wide16_valid = e == hipSuccess;
     }
+    if (e != hipSuccess) { sphip_destroy(net); return fail_hip("sphip_clone copy", e); }
     HCHECK(hipStreamSynchronize(g_stream));
     *out = net;
     return 0;
@@ -2288,9 +2316,9 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
         if (!reads_codes || !layer_wants_codes16(net, net->ptopo, l, rows)) continue;
         const DevArray &wa = net->w(l - 1);
         if (wa.codes16_valid) { codes[l - 1] = wa.codes16; continue; }
-        if (used + room(wa.count * sizeof(uint16_t)) > kScratchRoom) continue;
-        codes[l - 1] = reinterpret_cast<uint16_t *>(take(wa.count * sizeof(uint16_t)));
-        launch_codes16(net->prec, wa.base, codes[l - 1], wa.count);
+        if (used + room(wa.laid * sizeof(uint16_t)) > kScratchRoom) continue;
+        codes[l - 1] = reinterpret_cast<uint16_t *>(take(wa.laid * sizeof(uint16_t)));
+        launch_codes16(net->prec, wa.base, codes[l - 1], wa.laid);
     }
     wk.codes16 = codes;
     if (need.big_floats > need.split_floats && used + need.big_floats * sizeof(float) <= kScratchBytes) {
@@ -2392,7 +2420,9 @@ int sphip_decode(sphip_net *net, uint32_t l, int which, int mode, float *host_ou
     float *d_out = nullptr;
     HCHECK(hipMalloc((void **)&d_out, a.count * sizeof(float)));
     DecodeParams p{};
-    p.codes = a.base;
+    p.codes = which == 0 && !a.base ? net->PW[l].base : a.base;
+    p.cols = which == 0 ? net->topo[l] : 1u;
+    p.pcols = which == 0 && !a.base ? net->ptopo[l] : p.cols;
     p.out = d_out;
     p.n = a.count;
     p.max_val = a.max_val;

@@ -111,6 +111,45 @@ def test_mid_size_random_net(S, O, fmt):
     S.free_network(net)
 
 
+@pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
+@pytest.mark.parametrize("topo", [[33, 7, 130, 1101, 5], [64, 3001, 1503, 8], [8, 6001, 5003, 3]])
+def test_layers_that_lie_padded_decode_as_uploaded(S, O, fmt, topo):
+    """Layers behind a padded width lie on the device with padded rows only, uploaded through a staging area in chunks of
+    whole bytes (several chunks for the larger nets); sphip_decode finds the elements again, in a clone too."""
+    src = make_oracle_net(O, topo, ["tanh"] * (len(topo) - 2) + ["none"], seed=topo[1])
+    blob = src.serialize(O.PREC[fmt])
+    ref = O.Net.parse(blob)
+    net = load(S, blob)
+    for l in range(len(topo) - 1):
+        assert np.array_equal(bits(S.hip_decode(net, l, 0)), bits(ref.W(l).ravel())), l
+        assert np.array_equal(bits(S.hip_decode(net, l, 1)), bits(ref.b(l))), l
+    d = S.DeviceNet(topo, [O.ACT["tanh"]] * (len(topo) - 2) + [O.ACT["none"]], O.PREC[fmt], handle=S.lib().spingalett_hip_handle(net))
+    d.owned = False
+    twin = d.clone()
+    X = np.random.default_rng(1).standard_normal((70, topo[0])).astype(F32)
+    assert np.array_equal(twin.forward(X), d.forward(X)) and np.array_equal(twin.forward(X[:3]), d.forward(X[:3]))
+    twin.destroy()
+    S.free_network(net)
+
+
+def test_padded_nets_hold_their_weights_once(S):
+    """Device memory of an FP16 net of ragged widths: one copy of the weights (two of the first layer's, whose rows the
+    vector kernels want as the caller has them), a few MiB of staging, and the padding itself."""
+    topo = [1030] + [4097] * 5 + [10]
+    weights = [np.ones(a * b, np.float16).view(np.uint16) for a, b in zip(topo, topo[1:])]
+    S.synchronize()
+    S.device_memory()
+    before, _ = S.device_memory()
+    net = S.DeviceNet(topo, [S.ACT_RELU] * 6, S.PRECISION_FP16)
+    for l, w in enumerate(weights):
+        net.upload(l, 0, w)
+        net.upload(l, 1, np.zeros(topo[l + 1], np.uint16))
+    after, _ = S.device_memory()
+    used, packed = before - after, sum(w.nbytes for w in weights) + weights[0].nbytes
+    net.destroy()
+    assert used <= 1.1 * packed + (16 << 20), (used, packed)
+
+
 def test_invalidate_switches_the_device_to_the_fp32_arrays(S):
     net = S.load_spingalett(os.path.join(GOLD, "tiny_i4.nn"))
     assert S.lib().spingalett_hip_precision(net) == S.PRECISION_INT4
