@@ -691,7 +691,7 @@ Regime pick_regime(const sphip_net *net, uint32_t n, uint32_t flags)
 // of three layers, 9 to 15 padded).  So an input or hidden layer of such a width gets neurons without weights up to
 // the next whole unit (wide ones up to a multiple of 64, whole cache lines): zero rows and zero biases on the producing
 // side, zero columns on the consuming side.  The kernels store something finite for a padded neuron whatever its inputs
-// are (layer_sum, tile_clear_padding), so that it adds nothing behind infinities and NaNs either.  Not the output layer, whose rows are the
+// are (layer_sum), so that it adds nothing behind infinities and NaNs either.  Not the output layer, whose rows are the
 // caller's, and not a hidden softmax, whose sum runs over its real neurons.
 // Integer rows of eight codes' multiples (1000 INT8 codes) have kernels of their own, which are as good on small layers
 // and take the input as it is; hidden widths of that kind are padded in front of half a million weights and more, where

@@ -50,25 +50,6 @@ __device__ __forceinline__ uint32_t int_to_t16(int q)
     }
 }
 
-// What layer_sum() is to the tile kernels: a wave whose block of ROWS x COLS outputs from (r0, c0) on reaches into the
-// padding stores zeros over it behind its outputs.  (A select behind every output, or sums cleared in registers, costs
-// all tiles something: up to four vector registers, which at 2 x 2 tiles of 8-bit codes is a third of the resident waves; so
-// does a loop over the padded columns alone here.)
-template <int ROWS, int COLS>
-__device__ __forceinline__ void tile_clear_padding(const GemmArgs &g, uint32_t r0, uint32_t c0)
-{
-    const uint32_t N = g.L.N, real = N - g.L.pad;
-    if (g.L.pad == 0u || c0 + COLS <= real) return;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // the outputs' stores have arrived
-    for (uint32_t e = threadIdx.x & 63u; e < (uint32_t)(ROWS * COLS); e += 64u) {
-        const uint32_t row = r0 + e / COLS, col = c0 + e % COLS;
-        if (row >= g.M || col < real || col >= N) continue;
-        const size_t o = (size_t)row * N + col;
-        if (g.out_f32) reinterpret_cast<float *>(g.C)[o] = 0.0f;
-        else reinterpret_cast<uint16_t *>(g.C)[o] = 0;
-    }
-}
-
 // packed FP16 subtraction a - c (two lanes at once)
 __device__ __forceinline__ uint32_t h2_sub(uint32_t v, uint32_t c)
 {
@@ -371,6 +352,11 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
                         const float v = apply_act(pre, ACT);
                         stage[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * SP + (lane & 31)] = f32_to_t16<F16T>(v);
                     }
+                    // padded neurons (layer_sum): only hidden layers of this path have any
+                    if (col + g.L.pad >= N) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) stage[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * SP + (lane & 31)] = 0;
+                    }
                     __builtin_amdgcn_wave_barrier();
 #pragma unroll
                     for (int p = 0; p < 2; ++p) {
@@ -405,7 +391,6 @@ __global__ __launch_bounds__(256) void sp_gemm16(const GemmArgs g)
         }
     };
     with_act(g.L.act, emit);
-    tile_clear_padding<32 * TM, 32 * TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32);
 }
 
 // Small layers in one launch: a workgroup owns a 32 x 32 tile of the output, its eight waves split K in whole steps of
@@ -946,6 +931,19 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
                         if constexpr (SS == 4) *reinterpret_cast<float *>(dst) = v;
                         else *reinterpret_cast<uint16_t *>(dst) = f32_to_t16<F16T>(v);
                     }
+                // padded neurons (layer_sum; a select behind every output costs all tiles more)
+                if (ACT != A_COUNT && g.L.pad != 0u) {
+#pragma unroll 1
+                    for (int j = 0; j < TN; ++j) {
+                        if (n0 + (wn * TN + j) * 32 + (lane & 31) + g.L.pad < N) continue;
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            char *dst = mine + (8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * PITCH + (j * 32 + (lane & 31)) * SS;
+                            if constexpr (SS == 4) *reinterpret_cast<float *>(dst) = 0.0f;
+                            else *reinterpret_cast<uint16_t *>(dst) = 0;
+                        }
+                    }
+                }
                 auto put = [&](int p) {
                     const int rl = p * RPP + lane / LPR, seg = lane % LPR;
                     const char *src = mine + rl * PITCH + seg * (16 / ES) * SS;
@@ -985,7 +983,6 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
         if (g.ws) turn(E4{}, std::integral_constant<int, A_COUNT>{});
         else if (g.out_f32) with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E4{}, act_c); });
         else with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E2{}, act_c); });
-        if (!g.ws) tile_clear_padding<32 * TM, 32 * TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32);
         return;
     }
     with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) {
@@ -1008,7 +1005,6 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
             }
         }
     });
-    tile_clear_padding<32 * TM, 32 * TN>(g, m0 + wm * TM * 32, n0 + wn * TN * 32);
 }
 
 // adds the partial sums of a split launch (K splits in split order; with split activations the sums of the second
