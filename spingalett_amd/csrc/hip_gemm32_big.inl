@@ -17,9 +17,14 @@ struct BigGemm32Args {
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// two floats as three BF16 parts each, h + m + l == x exactly (8 + 8 + 8 significant bits, each part the nearest one)
+// two floats as three BF16 parts each, h + m + l == 2^24 x exactly (8 + 8 + 8 significant bits, each part the nearest one).
+// The lowest bit of any FP32 number, 2^-149, is a normal BF16 number (from 2^-126 on) after the scaling: unscaled, operands
+// below 2^-110 kept fewer than 24 bits.
+constexpr float kPartScale = 0x1p24f, kPartSumScale = 0x1p-48f;
 __device__ __forceinline__ void bf16_parts2(float x, float y, uint32_t &h, uint32_t &m, uint32_t &l)
 {
+    x *= kPartScale;
+    y *= kPartScale;
     auto pack = [](float a, float b) {
         const bf16x2 v = {(__bf16)a, (__bf16)b};
         uint32_t u;
@@ -40,15 +45,16 @@ __device__ __forceinline__ void bf16_parts2(float x, float y, uint32_t &h, uint3
 // in 6 x 8 passes what v_mfma_f32_32x32x2_f32 does in 8 x 16, and rounds the accumulator 6 times per 16 k instead of 8:
 // the error against 64 bits is the smaller one at every size tried (relative, 2-norm, FP32 matrix cores -> here: 20000 x 512
 // x 784 5.1e-7 -> 4.3e-7, 4096 x 4096 x 4096 1.15e-6 -> 1.00e-6, 700 x 3000 x 3000 9.9e-7 -> 3.5e-7, 8192 x 16384 x 64 1.4e-7 ->
-// 1.1e-7).  Parts end at 2^-133, so operands below 2^-110 keep fewer than 24 bits.
+// 1.1e-7), and so it is for operands down to the smallest subnormal ones, which the splitting scales up.
 // Tile (64 TM) x 128 x 32, four waves of (32 TM) x 64; the FP32 elements of the next K tile are loaded while the matrix
 // cores work, split in registers on their way into LDS: [operand][part][row][32 k], the 16-byte units of a row XOR-ed with
 // row / 4, so that the 16 rows of a read cycle lie in different banks.  48 KB (TM = 2) and one stage: three workgroups
 // share a compute unit, and one's splitting runs beside another's products.  Bound by the matrix cores and the splitting's
-// vector instructions together: 4096 x 4096 x 4096 1070 -> 694 us (198 TFLOP/s of FP32 products, 1.19 PFLOP/s of BF16),
-// 20000 x 1000 x 512 221 -> 130, 2000 x 4096 x 4096 600 -> 359, 512 x 4096 x 4096 (split over K) 178 -> 106.
-// An operand with infinities (or beyond the largest BF16) has no such parts: an element whose sum comes out infinite or
-// NaN is formed again as a chain of FP32 products.
+// vector instructions together: 4096 x 4096 x 4096 1070 -> 732 us (188 TFLOP/s of FP32 products, 1.13 PFLOP/s of BF16),
+// 20000 x 1000 x 512 221 -> 124, 2000 x 4096 x 4096 600 -> 353, 512 x 4096 x 4096 (split over K) 178 -> 107.  (Of that the
+// scaling of the operands costs between -3 and 4 %: 723, 123, 364 and 110 us without it.)
+// Infinities and operands from 2^104 on have no such parts, sums from 2^80 on no room for their scale: an element whose sum
+// comes out infinite or NaN is formed again as a chain of FP32 products.
 template <int TM>
 __global__ __launch_bounds__(256) void sp_gemm32_f32_big(const BigGemm32Args g)
 {
@@ -182,8 +188,8 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32_big(const BigGemm32Args g)
                     const float v = acc[i][j][r];
                     if (!(fabsf(v) < __builtin_inff())) again |= 1ull << e;
                     const size_t o = (size_t)m * N + n;
-                    if (g.ws) g.ws[(size_t)blockIdx.y * M * N + o] = v;
-                    else g.C[o] = apply_act(v + bias, ACT);
+                    if (g.ws) g.ws[(size_t)blockIdx.y * M * N + o] = v * kPartSumScale;
+                    else g.C[o] = apply_act(fmaf(v, kPartSumScale, bias), ACT);
                 }
         }
     });

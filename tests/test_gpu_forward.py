@@ -584,6 +584,27 @@ def test_large_fp32_products_on_bf16_parts(S, O, n, K, N):
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 1e-5
 
 
+@pytest.mark.parametrize("x_exp,w_exp", [(-118, 40), (-122, 0), (-130, 60), (20, -125), (-60, -30), (101, -60), (110, -80), (60, 25)])
+def test_large_fp32_products_of_tiny_and_huge_operands_keep_their_bits(S, x_exp, w_exp):
+    """Operands down to subnormal ones have BF16 parts that hold all their bits, operands from 2^104 and sums from 2^80 on
+    are formed as FP32 chains.  Against 64 bits; the accumulator is rounded six times per 16 k, so the 2-norm of the error
+    is about 2^-24 sqrt(6 K / 16) of the result's, a fraction of it since the sums grow; four times that at most, where
+    parts that end at 2^-133 give 9e-6 of a result with operands of 2^-118.  (An FP32 chain is rounded K times.)"""
+    n, K, N = 700, 1000, 3000
+    rng = np.random.default_rng(x_exp + 200)
+    X = np.ldexp(rng.standard_normal((n, K)), x_exp).astype(F32)
+    W = np.ldexp(rng.standard_normal((N, K)), w_exp).astype(F32)
+    d = S.DeviceNet([K, N], [S.ACT_NONE], S.PRECISION_FLOAT32)
+    d.upload(0, 0, W.ravel())
+    d.upload(0, 1, np.zeros(N, F32))
+    assert S.lib().sphip_layer_kernel_name(d.h, 1, n, 0).decode() == "sp_gemm32_f32_big"
+    got = d.forward(X).astype(np.float64)
+    want = X.astype(np.float64) @ W.astype(np.float64).T
+    rounds = K if x_exp >= 104 or x_exp + w_exp >= 80 else 6 * K / 16
+    assert np.linalg.norm(got - want) <= 4 * 2.0 ** -24 * np.sqrt(rounds) * np.linalg.norm(want), np.linalg.norm(got - want) / np.linalg.norm(want)
+    d.destroy()
+
+
 def test_large_fp32_products_keep_infinities_and_nans(S):
     """Operands without BF16 parts (infinite, beyond the largest BF16, NaN), next to weights whose lower parts are zero."""
     n, K, N = 4096, 784, 640
