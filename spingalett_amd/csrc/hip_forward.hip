@@ -10,7 +10,7 @@
 //                     inside the workgroup)
 //   hip_gemm16.inl    sp_gemm16_big / sp_gemm16: larger batches: LDS-tiled dequant-to-16-bit MFMA GEMM, fused epilogue
 //   hip_gemm32.inl    sp_gemm32_f32: FP32 weights beyond four samples: FP32 MFMA GEMM
-//   hip_gemm32_big.inl  sp_gemm32_f32_big: large FP32 forward products on BF16 parts
+//   hip_gemm32_parts.inl  sp_gemm32_bf16_parts: large FP32 forward products on BF16 parts
 //   sp_softmax_rows   per-sample softmax (Activation.c:5-21)
 //   sp_eval_*         loss and argmax of a labelled batch (SIMD.c:522-552, Training.c:421-435)
 //   hip_train.inl     the batched training step (included at the end)
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(256) void sp_bf16_to_f16(const uint16_t *__restrict
 }
 
 #include "hip_gemm32.inl"
-#include "hip_gemm32_big.inl"
+#include "hip_gemm32_parts.inl"
 
 // ---------------------------------------------------------------------------
 // FP32 weights on the 16-bit matrix cores (split mode of an FP32 net beyond 64 samples).  With FP16 parts
@@ -1423,20 +1423,20 @@ void launch_gemm32_small(const Gemm32Args &g, uint32_t tile, const KSegments &se
     else sp_gemm32_small16<false><<<grid, 512, 0, g_stream>>>(g, seg, soft_out, tail);
 }
 
-// Whether a forward product takes sp_gemm32_f32_big: from 2 G multiply-adds on, where its tiles fill the chip with more than
+// Whether a forward product takes sp_gemm32_bf16_parts: from 2 G multiply-adds on, where its tiles fill the chip with more than
 // their own start-up (2048 x 1024 x 1024 42 against 49 us in the FP32 kernels, 4096 x 1000 x 1000 68 against 91, 10000 x 512 x
 // 784 71 against 88, 700 x 3000 x 3000 104 against 185; below: 2048 x 512 x 784 30 against 25, 1000 x 1024 x 1024 30 against 32),
 // unless more than a fifth of the tiles would be padding (20000 x 130 x 100 25 against 17 us).  Training's products stay in
 // the FP32 kernels and their order of sums: a run whose gradients nearly cancel multiplies a last-bit difference.
-bool gemm32_big_pays(uint32_t M, uint32_t N, uint32_t K)
+bool gemm32_parts_pay(uint32_t M, uint32_t N, uint32_t K)
 {
     const uint64_t rows = (M + 127ull) / 128u * 128u, cols = (N + 127ull) / 128u * 128u;
     return K >= 64u && 5u * (uint64_t)M * N >= 4u * rows * cols && (double)M * N * K >= 2e9;
 }
 
-// K splits of sp_gemm32_f32_big: two workgroups per compute unit where there are fewer tiles than compute units, at least
+// K splits of sp_gemm32_bf16_parts: two workgroups per compute unit where there are fewer tiles than compute units, at least
 // four K tiles each (512 x 4096 x 4096 106 us, 168 unsplit; three per compute unit 109; 700 x 3000 x 3000 104 / 143 / 109)
-uint32_t gemm32_big_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper)
+uint32_t gemm32_parts_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper)
 {
     const uint64_t tiles = (M + 127ull) / 128u * ((N + 127ull) / 128u);
     const uint32_t ktiles = (K + 31u) / 32u;
@@ -1452,12 +1452,12 @@ uint32_t gemm32_big_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper)
 // Tiles of 64 rows where those of 128 would be one on some compute units and two on others (256 to 383: twice as many are
 // still resident at once; 10000 x 512 x 784 82 -> 71 us, 4096 x 1000 x 1000 78 -> 68, but 512 tiles of 2000 x 4096 x 4096 359
 // -> 390), and for short sums, which are mostly load, split and store (8192 x 16384 x 64 230 -> 200 us)
-void launch_gemm32_big(const BigGemm32Args &g, uint32_t splits)
+void launch_gemm32_parts(const PartsGemm32Args &g, uint32_t splits)
 {
     const uint32_t cols = (g.N + 127u) / 128u;
     const uint64_t tiles = (g.M + 127ull) / 128u * cols;
-    if (splits == 1u && ((tiles >= 256u && tiles < 384u) || g.K <= 128u)) sp_gemm32_f32_big<1><<<(g.M + 63u) / 64u * cols, 256, 0, g_stream>>>(g);
-    else sp_gemm32_f32_big<2><<<dim3((g.M + 127u) / 128u * cols, splits), 256, 0, g_stream>>>(g);
+    if (splits == 1u && ((tiles >= 256u && tiles < 384u) || g.K <= 128u)) sp_gemm32_bf16_parts<1><<<(g.M + 63u) / 64u * cols, 256, 0, g_stream>>>(g);
+    else sp_gemm32_bf16_parts<2><<<dim3((g.M + 127u) / 128u * cols, splits), 256, 0, g_stream>>>(g);
 }
 
 // soft_out: the layer is a softmax layer whose normalised outputs belong there; returns true if they were written
@@ -1466,17 +1466,17 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
 {
     Gemm32Args g{L, A, C, nullptr, M, 0};
     const bool vec = L.K % 4u == 0 && (reinterpret_cast<uintptr_t>(A) & 15u) == 0 && (reinterpret_cast<uintptr_t>(L.w) & 15u) == 0;
-    if (!training && gemm32_big_pays(M, L.N, L.K)) {
-        BigGemm32Args b{};
-        uint32_t parts = gemm32_big_splits(M, L.N, L.K, &b.kper);
+    if (!training && gemm32_parts_pay(M, L.N, L.K)) {
+        PartsGemm32Args b{};
+        uint32_t parts = gemm32_parts_splits(M, L.N, L.K, &b.kper);
         if (parts > 1 && (uint64_t)parts * M * L.N > ws_floats) { parts = 1; b.kper = (L.K + 31u) / 32u * 32u; }
-        tl_route.name = "sp_gemm32_f32_big";
+        tl_route.name = "sp_gemm32_bf16_parts";
         if (tl_route.dry) return false;
         b.A = A; b.B = reinterpret_cast<const float *>(L.w); b.C = C; b.ws = parts > 1 ? ws : nullptr;
         b.M = M; b.N = L.N; b.K = L.K;
         b.vec = vec;
         b.bias = L.bias; b.bscale = L.bscale; b.bias_fmt = L.bias_fmt; b.act = L.act;
-        launch_gemm32_big(b, parts);
+        launch_gemm32_parts(b, parts);
         if (parts > 1) {
             g.ws = ws;
             sp_gemm32_reduce<<<(uint32_t)(((uint64_t)M * L.N + 255) / 256), 256, 0, g_stream>>>(g, parts);
@@ -1486,12 +1486,12 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
     // weights beyond the L2s (4 MB per XCD) and enough 128 x 128 tiles for two per compute unit: the larger tile
     if (vec && M >= 512u && (uint64_t)L.N * L.K * sizeof(float) > (4ull << 20) &&
         (uint64_t)((M + 127u) / 128u) * ((L.N + 127u) / 128u) >= 512u) {
-        tl_route.name = "sp_gemm32_f32_128";
+        tl_route.name = "sp_gemm32_f32_big";
         if (tl_route.dry) return false;
         constexpr size_t lds = 2 * 2 * 128 * 36 * sizeof(float);
-        static bool once = ((void)hipFuncSetAttribute((const void *)sp_gemm32_f32_128, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
+        static bool once = ((void)hipFuncSetAttribute((const void *)sp_gemm32_f32_big, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
         (void)once;
-        sp_gemm32_f32_128<<<((M + 127u) / 128u) * ((L.N + 127u) / 128u), 256, lds, g_stream>>>(g);
+        sp_gemm32_f32_big<<<((M + 127u) / 128u) * ((L.N + 127u) / 128u), 256, lds, g_stream>>>(g);
         return false;
     }
     uint32_t splits = gemm32_fwd_splits(M, L.N, L.K, &g.kper);
@@ -1527,7 +1527,7 @@ struct WorkspaceNeed {
     uint64_t plane_bytes;      // digit planes: 4 bytes per element (+ padding of the last chunk) ...
     uint64_t plane_recs;       // ... and one scale (+ four digit sums) per 64 elements
     uint64_t split_floats;
-    uint64_t big_floats;       // the partial sums that sp_gemm32_f32_big would like room for (it runs without them too)
+    uint64_t parts_floats;     // the partial sums that sp_gemm32_bf16_parts would like room for (it runs without them too)
     uint64_t cat_elems;        // split mode of an FP32 net: FP16 elements of the widest three-part layer input
 };
 
@@ -1583,8 +1583,8 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             if (reg == R_GEMV) continue;
             const uint32_t sp = gemm32_fwd_splits(n, N, K, &kper);
             if (sp > 1) ws = (uint64_t)sp * n * N;
-            const uint64_t big = gemm32_big_pays(n, N, K) ? gemm32_big_splits(n, N, K, &kper) : 1u;
-            if (big > 1 && big * n * N > w.big_floats) w.big_floats = big * n * N;
+            const uint64_t parts = gemm32_parts_pay(n, N, K) ? gemm32_parts_splits(n, N, K, &kper) : 1u;
+            if (parts > 1 && parts * n * N > w.parts_floats) w.parts_floats = parts * n * N;
         } else {
             const ThinPlan tp = plan_thin(net->prec, n, N, K);
             if (tp.use) {
@@ -1719,7 +1719,7 @@ int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
     }
     if (keep_layers && !net->layers_buf)
         HCHECK(hipMalloc((void **)&net->layers_buf, net->slots_total * sizeof(float)));
-    const uint64_t split_floats = need.big_floats > need.split_floats ? need.big_floats : need.split_floats;
+    const uint64_t split_floats = need.parts_floats > need.split_floats ? need.parts_floats : need.split_floats;
     if (split_floats > net->split_cap) {
         if (net->split_ws) { HCHECK(hipFree(net->split_ws)); net->split_ws = nullptr; }
         net->split_cap = 0;
@@ -2321,9 +2321,9 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
         launch_codes16(net->prec, wa.base, codes[l - 1], wa.laid);
     }
     wk.codes16 = codes;
-    if (need.big_floats > need.split_floats && used + need.big_floats * sizeof(float) <= kScratchBytes) {
-        wk.split_ws = reinterpret_cast<float *>(take(need.big_floats * sizeof(float)));
-        wk.split_cap = need.big_floats;
+    if (need.parts_floats > need.split_floats && used + need.parts_floats * sizeof(float) <= kScratchBytes) {
+        wk.split_ws = reinterpret_cast<float *>(take(need.parts_floats * sizeof(float)));
+        wk.split_cap = need.parts_floats;
     }
     // the integer GEMV's quantise launch is never skipped here (that shortcut belongs to the layer timer)
     net->aq_valid_layer = 0;

@@ -1,5 +1,5 @@
 // hip_gemm32.inl — the FP32 MFMA GEMM for FP32 weights beyond 64 samples (sp_gemm32_f32,
-// sp_gemm32_reduce; its large products: hip_gemm32_big.inl).  Part of hip_forward.hip's translation unit (included there, inside its unnamed
+// sp_gemm32_reduce; its large products: hip_gemm32_parts.inl).  Part of hip_forward.hip's translation unit (included there, inside its unnamed
 // namespace); not compiled on its own.
 
 // ---------------------------------------------------------------------------
@@ -113,14 +113,14 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32(const Gemm32Args g)
     });
 }
 
-// The same product where sp_gemm32_f32_big does not take it (training's forward, whose sums keep their order, and tiles that
+// The same product where sp_gemm32_bf16_parts does not take it (training's forward, whose sums keep their order, and tiles that
 // are mostly padding) and the weights exceed the L2s, at 512 samples and more: 128 x 128 x 32 tile (each wave
 // 64 x 64 = 2 x 2 accumulators), two LDS stages and one barrier per K tile, rows of 36 floats in LDS.  MFMA step
 // (j, t), t = 0 .. 3, of a K tile multiplies k = 8 j + 4 h + t on the lanes of half h for both operands alike (a sum
 // over k in any order), so that a lane reads the four k of four steps with one 16-byte LDS load.  Half the bytes per
 // flop of the 64 x 64 tile, through LDS and through the fabric (8192 x 4096 x 4096: 9.2 GB fetched per launch with
 // 64 x 64 tiles).  Rows are 16-byte aligned (K % 4 == 0); no K split.
-__global__ __launch_bounds__(256) void sp_gemm32_f32_128(const Gemm32Args g)
+__global__ __launch_bounds__(256) void sp_gemm32_f32_big(const Gemm32Args g)
 {
     constexpr int BM = 128, BN = 128, BK = 32, LD = 36, SIZE = BM * LD;
     extern __shared__ __attribute__((aligned(16))) float smem32[];

@@ -1,8 +1,8 @@
-// hip_gemm32_big.inl — FP32 forward products of 2 G multiply-adds and more on the BF16 matrix cores (sp_gemm32_f32_big).
+// hip_gemm32_parts.inl — FP32 forward products of 2 G multiply-adds and more on the BF16 matrix cores (sp_gemm32_bf16_parts).
 // Part of hip_forward.hip's translation unit (included there, inside its unnamed namespace, behind hip_gemm32.inl); not
 // compiled on its own.
 
-struct BigGemm32Args {
+struct PartsGemm32Args {
     const float *A, *B;    // [M][K], [N][K]
     float *C;              // [M][N]
     float *ws;             // [splits][M][N] partial sums when the grid splits K, else nullptr
@@ -56,7 +56,7 @@ __device__ __forceinline__ void bf16_parts2(float x, float y, uint32_t &h, uint3
 // Infinities and operands from 2^104 on have no such parts, sums from 2^80 on no room for their scale: an element whose sum
 // comes out infinite or NaN is formed again as a chain of FP32 products.
 template <int TM>
-__global__ __launch_bounds__(256) void sp_gemm32_f32_big(const BigGemm32Args g)
+__global__ __launch_bounds__(256) void sp_gemm32_bf16_parts(const PartsGemm32Args g)
 {
     constexpr uint32_t BM = 64 * TM, BN = 128, BK = 32;
     constexpr uint32_t PA = BM * BK, PB = BN * BK;        // 16-bit elements of one part of an operand

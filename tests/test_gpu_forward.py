@@ -523,16 +523,18 @@ def test_rows_that_are_not_whole_16_byte_units_split_k_at_few_samples(S, O, fmt,
     assert rel_max_abs(fine, want) <= 2e-5
 
 
-def test_large_fp32_layers_take_the_128_by_128_tile(S, O):
-    """FP32 weights beyond the L2s at 512 samples and more: the two-stage 128 x 128 kernel (ragged M, N and a K that is
-    not a whole number of tiles), the layer behind it the 64 x 64 one; FP32 bar against the float64 forward."""
-    topo, acts, n = [1000, 1100, 300], ["tanh", "none"], 8195
-    src = make_oracle_net(O, topo, acts, seed=12, bias_std=0.1)
+@pytest.mark.parametrize("act", ["sigmoid", "relu", "tanh", "leaky_relu", "foo52", "none"])
+@pytest.mark.parametrize("n,K,N", [(515, 132, 16390), (512, 128, 16384), (700, 68, 16300)])
+def test_large_fp32_layers_take_the_128_by_128_tile(S, O, n, K, N, act):
+    """FP32 weights beyond the L2s at 512 samples and more, too few multiply-adds for the BF16 parts: the two-stage
+    128 x 128 kernel (ragged M, N and a K that is not a whole number of tiles) with every epilogue, the layer behind it
+    and 500 samples the 64 x 64 one; FP32 bar against the float64 forward."""
+    src = make_oracle_net(O, [K, N, 40], [act, "none"], seed=12, bias_std=0.1)
     _, ref, net = quantized_pair(O, S, src, "f32")
     h = S.lib().spingalett_hip_handle(net)
     assert [S.lib().sphip_layer_kernel_name(h, l, n, 0).decode() for l in (1, 2)] == ["sp_gemm32_f32_big", "sp_gemm32_f32"]
     assert S.lib().sphip_layer_kernel_name(h, 1, 500, 0).decode() == "sp_gemm32_f32"
-    X = np.random.default_rng(8).standard_normal((n, topo[0])).astype(F32)
+    X = np.random.default_rng(8).standard_normal((n, K)).astype(F32)
     got = S.forward_batch(net, X)
     S.free_network(net)
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_VEC
@@ -577,7 +579,7 @@ def test_large_fp32_products_on_bf16_parts(S, O, n, K, N):
     src = make_oracle_net(O, [K, N], ["none"], seed=n + K, bias_std=0.1)
     _, ref, net = quantized_pair(O, S, src, "f32")
     h = S.lib().spingalett_hip_handle(net)
-    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm32_f32_big"
+    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm32_bf16_parts"
     X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
     got = S.forward_batch(net, X)
     S.free_network(net)
@@ -597,7 +599,7 @@ def test_large_fp32_products_of_tiny_and_huge_operands_keep_their_bits(S, x_exp,
     d = S.DeviceNet([K, N], [S.ACT_NONE], S.PRECISION_FLOAT32)
     d.upload(0, 0, W.ravel())
     d.upload(0, 1, np.zeros(N, F32))
-    assert S.lib().sphip_layer_kernel_name(d.h, 1, n, 0).decode() == "sp_gemm32_f32_big"
+    assert S.lib().sphip_layer_kernel_name(d.h, 1, n, 0).decode() == "sp_gemm32_bf16_parts"
     got = d.forward(X).astype(np.float64)
     want = X.astype(np.float64) @ W.astype(np.float64).T
     rounds = K if x_exp >= 104 or x_exp + w_exp >= 80 else 6 * K / 16
@@ -627,7 +629,7 @@ def test_large_fp32_products_keep_infinities_and_nans(S):
     S.biases_view(net, 0)[:] = b
     got = S.forward_batch(net, X)
     h = S.lib().spingalett_hip_handle(net)
-    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm32_f32_big"
+    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm32_bf16_parts"
     S.free_network(net)
     with np.errstate(invalid="ignore"):
         want = X.astype(np.float64) @ W.astype(np.float64).T + b

@@ -96,6 +96,31 @@ OPT_CASES = [
 ]
 
 
+def test_gradients_of_a_large_layer_match_float64():
+    """Weights beyond the L2s (1000 x 1052, 4.2 MB) and 512 tiles of 128 x 128: the forward product of this step is
+    sp_gemm32_f32_big's, in one order of sums however many multiply-adds it has (the inference forward's kernel on BF16
+    parts is not used).  One SGD step of size 1 on a mean of squared differences, against float64."""
+    n, topo = 8100, [1052, 1000, 3]
+    rng = np.random.default_rng(5)
+    W = [(rng.standard_normal((b, a)) / np.sqrt(a)).astype(np.float32) for a, b in zip(topo, topo[1:])]
+    d = S.DeviceNet(topo, [S.ACT_TANH, S.ACT_NONE], S.PRECISION_FLOAT32)
+    for l, w in enumerate(W):
+        d.upload(l, 0, w.ravel())
+        d.upload(l, 1, np.zeros(topo[l + 1], np.float32))
+    X = rng.standard_normal((n, topo[0])).astype(np.float32)
+    T = rng.standard_normal((n, topo[-1])).astype(np.float32)
+    d.train_begin()
+    d.train_step(X, T, step_args(0, 0, lr=1.0))
+    a = np.tanh(X.astype(np.float64) @ W[0].T.astype(np.float64))
+    delta = a @ W[1].T.astype(np.float64) - T
+    hidden = (delta @ W[1].astype(np.float64)) * (1 - a * a)
+    for l, (g, x) in enumerate([(hidden, X.astype(np.float64)), (delta, a)]):
+        grad = g.T @ x / n
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_GW, l).reshape(grad.shape), grad) <= TOL, l
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_W, l).reshape(grad.shape), W[l] - grad) <= TOL, l
+    d.destroy()
+
+
 @pytest.mark.parametrize("opt,kw", OPT_CASES)
 def test_four_steps_of_each_optimizer_match_oracle(opt, kw):
     topo, acts, loss, n = [30, 70, 40, 6], ["tanh", "leaky_relu", "softmax"], 1, 96
