@@ -1498,7 +1498,7 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
     KSegments seg;
     const uint32_t small = gemm32_small_tile(M, L.N, L.K, vec, &seg);
     if (small) {
-        tl_route.name = "sp_gemm32_small";
+        tl_route.name = small == 16u ? "sp_gemm32_small16" : "sp_gemm32_small";
         if (tl_route.dry) return false;
         const bool soft = soft_out && L.N <= small;
         launch_gemm32_small(g, small, seg, soft ? soft_out : nullptr, DeltaTail{});

@@ -653,10 +653,10 @@ def test_fp32_nets_leave_the_vector_kernel_beyond_four_samples(S, O):
     h = S.lib().spingalett_hip_handle(net)
     # (512 x 784 at these batch sizes: the one-launch kernel for small layers; at 4096 samples the tiled one)
     assert [S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() for n in (1, 4, 5, 64, 65, 4096)] == \
-        ["sp_gemv", "sp_gemv", "sp_gemm32_small", "sp_gemm32_small", "sp_gemm32_small", "sp_gemm32_f32"]
+        ["sp_gemv", "sp_gemv", "sp_gemm32_small16", "sp_gemm32_small16", "sp_gemm32_small16", "sp_gemm32_f32"]
     # the 1000 -> 10 head: a workgroup per row, up to eight samples (layers of at most 64 outputs)
     assert [S.lib().sphip_layer_kernel_name(h, 3, n, 0).decode() for n in (1, 4, 5, 8, 9)] == \
-        ["sp_gemv_words"] * 4 + ["sp_gemm32_small"]
+        ["sp_gemv_words"] * 4 + ["sp_gemm32_small16"]
     X = np.random.default_rng(3).random((4096, topo[0]), dtype=F32)
     want = ref.forward_batch_f64(X)
     for n in (4, 5, 8, 9, 33, 64, 300, 4096):
@@ -1421,14 +1421,14 @@ def test_padded_widths_keep_infinities_and_nans_where_they_are(S, fmt, act, topo
     S.free_network(net)
 
 
-@pytest.mark.parametrize("N,K,n", [
-    (16, 16, 5), (17, 33, 16), (1, 3, 9), (512, 784, 64), (300, 2000, 33),      # 16 x 16 tiles: whole and partial steps, few rows
-    (233, 1038, 64), (65, 1, 40), (90, 1023, 100), (31, 1026, 17),               # ... rows that start anywhere
-    (1000, 512, 128), (1024, 1024, 128), (65, 1024, 1365),                       # ... at their bound, and 32 x 32 tiles beyond it
-    (500, 1000, 512), (512, 1020, 1024),
+@pytest.mark.parametrize("N,K,n,tile", [
+    (16, 16, 5, 16), (17, 33, 16, 16), (1, 3, 9, 16), (512, 784, 64, 16), (300, 2000, 33, 16),   # 16 x 16 tiles: whole and partial steps, few rows
+    (233, 1038, 64, 16), (65, 1, 40, 16), (90, 1023, 100, 16), (31, 1026, 17, 16),               # ... rows that start anywhere
+    (1000, 512, 128, 16), (1024, 1024, 128, 16), (65, 1024, 1365, 32),                           # ... at their bound, and 32 x 32 tiles beyond it
+    (500, 1000, 512, 32), (512, 1020, 1024, 32),
 ])
 @pytest.mark.parametrize("act", ["tanh", "softmax"])
-def test_small_fp32_layers_run_in_one_launch(S, O, N, K, n, act):
+def test_small_fp32_layers_run_in_one_launch(S, O, N, K, n, tile, act):
     """Small FP32 layers whose workgroups split K among their waves; a softmax of at most a tile's width in the same
     launch, wider ones by the row kernel.  1e-4 against the float64 forward, like every FP32 path."""
     src = make_oracle_net(O, [K, N], [act], seed=N + K, bias_std=0.1)
@@ -1439,4 +1439,4 @@ def test_small_fp32_layers_run_in_one_launch(S, O, N, K, n, act):
     S.free_network(net)
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_VEC
     if N > 64 or n > 8:
-        assert name == "sp_gemm32_small"
+        assert name == ("sp_gemm32_small16" if tile == 16 else "sp_gemm32_small")
