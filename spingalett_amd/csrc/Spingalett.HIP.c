@@ -425,12 +425,15 @@ void train_struct_arguments(TrainArgs args)
     const uint32_t in_sz = net->topology[0], out_sz = net->topology[net->layers - 1];
     uint32_t *order = NULL, *orders = NULL;
     float *bx = NULL, *bt = NULL;
-    /* One launch covers the epochs up to the next one that something on the host looks at: at most about 50 ms of them
-     * (5000 cycles and a quarter of a cycle per weight and sample for a step), and 64 K shuffled sample numbers. */
+    /* One launch covers the epochs up to the next one that something on the host looks at, or a part of one epoch: at most
+     * about 50 ms of steps (5000 cycles and a quarter of a cycle per weight and sample for each), and 64 K shuffled sample
+     * numbers of several epochs. */
     const uint64_t steps_per_epoch = ((uint64_t)sample_count + eff_batch - 1u) / eff_batch;
-    uint64_t tiny_epochs = 120000000u / (5000u + net->total_weights * eff_batch / 4u) / steps_per_epoch;
+    const uint64_t launch_steps = 120000000u / (5000u + net->total_weights * eff_batch / 4u) + 1u;
+    uint64_t tiny_epochs = launch_steps / steps_per_epoch;
     if (small && tiny_epochs > 65536u / sample_count) tiny_epochs = 65536u / sample_count;
     if (tiny_epochs < 1u) tiny_epochs = 1u;
+    const uint32_t tiny_samples = launch_steps < steps_per_epoch ? (uint32_t)launch_steps * eff_batch : sample_count;
     if (small) {
         order = (uint32_t *)malloc((size_t)sample_count * sizeof(uint32_t));
         if (tiny) {
@@ -474,20 +477,28 @@ void train_struct_arguments(TrainArgs args)
                 sp_shuffle_indices(order, sample_count);
                 memcpy(orders + (size_t)e * sample_count, order, (size_t)sample_count * sizeof(uint32_t));
             }
-            const sp_tiny_run run = {
-                .weights = net->weights, .biases = net->biases, .m_weights = net->opt_m_weights, .m_biases = net->opt_m_biases,
-                .v_weights = net->opt_v_weights, .v_biases = net->opt_v_biases, .g_weights = net->grad_weights,
-                .g_biases = net->grad_biases, .x = args.inputs, .t = args.targets, .samples = sample_count, .batch = eff_batch,
-                .epochs = count, .order = orders, .order_room = (uint32_t)tiny_epochs * sample_count, .first = begin == 1u,
-                .args = &ta, .total_loss = need_loss ? &total_error : NULL,
-            };
-            failed = sp_train_tiny_run(sn->dev, &run) != 0;
-            sn->opt_loaded = true;
-            for (uint64_t s = 0; s < steps_per_epoch * count; ++s) {
-                net->time_step++;
-                ta.beta1_pow_t *= args.beta1;
-                ta.beta2_pow_t *= args.beta2;
+            double loss = 0.0;
+            for (uint32_t start = 0, part; start < sample_count && !failed; start += part) {
+                part = sample_count - start < tiny_samples ? sample_count - start : tiny_samples;
+                double part_loss = 0.0;
+                const sp_tiny_run run = {
+                    .weights = net->weights, .biases = net->biases, .m_weights = net->opt_m_weights, .m_biases = net->opt_m_biases,
+                    .v_weights = net->opt_v_weights, .v_biases = net->opt_v_biases, .g_weights = net->grad_weights,
+                    .g_biases = net->grad_biases, .x = args.inputs, .t = args.targets, .samples = sample_count, .batch = eff_batch,
+                    .epochs = count, .start = start, .count = part, .order = orders ? orders + start : NULL,
+                    .order_room = (uint32_t)tiny_epochs * sample_count, .first = begin == 1u && start == 0u, .args = &ta,
+                    .total_loss = need_loss ? &part_loss : NULL,
+                };
+                failed = sp_train_tiny_run(sn->dev, &run) != 0;
+                sn->opt_loaded = true;
+                loss += part_loss;
+                for (uint64_t s = 0; s < ((uint64_t)part + eff_batch - 1u) / eff_batch * count; ++s) {
+                    net->time_step++;
+                    ta.beta1_pow_t *= args.beta1;
+                    ta.beta2_pow_t *= args.beta2;
+                }
             }
+            total_error = (float)loss;
         } else if (per_sample) {
             for (uint32_t s = 0; s < sample_count && !failed; ++s) {
                 float loss = 0.0f;

@@ -453,11 +453,14 @@ int sp_train_tiny_run(sphip_net *net, const sp_tiny_run *r)
     TinyPlan p;
     if (!tiny_plan(net->layers, net->topo.data(), r->samples, r->batch, r->order != nullptr, &p))
         return fail_msg("sp_train_tiny_run: the net does not fit");
+    // (an epoch whose samples fit LDS is never too long for a launch: its steps are a few ten thousand at most)
+    if (r->count != r->samples && (p.x_lds || r->epochs != 1u || r->start % r->batch || (uint64_t)r->start + r->count > r->samples))
+        return fail_msg("sp_train_tiny_run: not a part of one epoch");
     TinyArgs &a = p.a;
     const uint32_t n_in = net->topo[0], n_out = net->topo[net->layers - 1];
     const uint64_t total = (uint64_t)a.total_w + a.total_b;
     const uint64_t xf = (uint64_t)r->samples * n_in, tf = (uint64_t)r->samples * n_out;
-    const uint64_t of = r->order ? (uint64_t)r->epochs * r->samples : 0;
+    const uint64_t of = r->order ? (uint64_t)r->epochs * r->count : 0;
     // pinned: loss (two floats) | results (4 arrays) | state (3 arrays) | order | samples | targets
     const uint64_t in_at = 2u + 4u * total, ord_at = in_at + 3u * total, data_at = ord_at + (r->order ? r->order_room : 0u);
     if (of > data_at - ord_at) return fail_msg("sp_train_tiny_run: more sample numbers than announced");
@@ -481,8 +484,9 @@ int sp_train_tiny_run(sphip_net *net, const sp_tiny_run *r)
     }
     a.in = r->first ? pin + in_at : pin + 2;
     a.out = pin + 2;
-    a.x = p.x_lds ? pin + data_at : net->stage_x;
-    a.t = p.x_lds ? pin + data_at + xf : net->stage_y;
+    const uint64_t skip = r->order ? 0u : r->start;          // (an order names samples of the whole set)
+    a.x = p.x_lds ? pin + data_at : net->stage_x + skip * n_in;
+    a.t = p.x_lds ? pin + data_at + xf : net->stage_y + skip * n_out;
     if (r->order) {
         memcpy(pin + ord_at, r->order, of * 4u);
         a.order = reinterpret_cast<const uint32_t *>(pin + ord_at);
@@ -494,7 +498,7 @@ int sp_train_tiny_run(sphip_net *net, const sp_tiny_run *r)
         net->W[l].cat3_valid = false;
     }
     a.dmW = ts->mW; a.dvW = ts->vW; a.dmB = ts->mB; a.dvB = ts->vB; a.dgW = ts->gW; a.dgB = ts->gB;
-    a.samples = r->samples;
+    a.samples = r->count;
     a.batch = r->batch;
     a.epochs = r->epochs;
     a.opt = opt_args(*r->args);
@@ -517,11 +521,7 @@ int sp_train_tiny_run(sphip_net *net, const sp_tiny_run *r)
     memcpy(r->v_biases, o + 2u * total + a.total_w, (size_t)a.total_b * 4u);
     memcpy(r->g_weights, o + 3u * total, (size_t)a.total_w * 4u);
     memcpy(r->g_biases, o + 3u * total + a.total_w, (size_t)a.total_b * 4u);
-    if (r->total_loss) {
-        double sum;
-        memcpy(&sum, pin, sizeof sum);
-        *r->total_loss = (float)sum;
-    }
+    if (r->total_loss) memcpy(r->total_loss, pin, sizeof(double));
     return 0;
 }
 

@@ -19,12 +19,14 @@ typedef struct {
     float *weights, *biases, *m_weights, *m_biases, *v_weights, *v_biases, *g_weights, *g_biases;
     const float *x, *t;              /* [samples][width], host memory */
     uint32_t samples, batch, epochs;
-    const uint32_t *order;           /* [epochs][samples] which sample comes when, or NULL: as they lie */
+    uint32_t start, count;           /* which of an epoch's places this run covers: all of them, or whole batches of one
+                                        epoch that is too long for a launch */
+    const uint32_t *order;           /* [epochs][count] which sample comes when, or NULL: as they lie */
     uint32_t order_room;             /* entries that any part of this training passes in order at most */
     bool first;                      /* first part of a training: arrays and samples go to the device (later parts go on
                                         from where the last one ended) */
     const sphip_train_args *args;    /* beta*_pow_t: before the first step */
-    float *total_loss;               /* sum of the last epoch's losses, or NULL */
+    double *total_loss;              /* sum of the losses of the last epoch's places covered here, or NULL */
 } sp_tiny_run;
 
 /* A build of the C side alone (the host sanitizer's) has neither: weak there, checked before use. */

@@ -532,6 +532,33 @@ def test_small_nets_match_the_oracle(topo, acts, loss, n, batch, epochs, opt, kw
     S.free_network(net)
 
 
+def test_an_epoch_of_many_steps_runs_in_several_launches():
+    """60,000 updates of a small net, one per sample, are three launches; without momentum four trainings over a quarter
+    of the samples each are the same updates, bit for bit.  A shuffled order of equal samples is no order at all."""
+    n = 60000
+    rng = np.random.default_rng(2)
+    X = rng.uniform(-1, 1, (n, 2)).astype(np.float32)
+    T = (X[:, :1] * X[:, 1:] > 0).astype(np.float32)
+    kw = dict(learning_rate=0.05, weight_decay=1e-4)
+    W = []
+    for parts in (1, 4):
+        net, _ = public_net([2, 8, 1], ["tanh", "sigmoid"], 0, seed=4)
+        for p in range(parts):
+            S.train(net, X[p * n // parts:(p + 1) * n // parts], T[p * n // parts:(p + 1) * n // parts], 1, S.STRATEGY_SAMPLE, S.OPTIMIZER_SGD, **kw)
+        W.append([S.weights_view(net, l).copy() for l in (0, 1)] + [S.biases_view(net, l).copy() for l in (0, 1)])
+        assert S.last_error()[0] == S.SPINGALETT_OK, S.last_error()
+        S.free_network(net)
+    assert all(np.array_equal(a, b) for a, b in zip(*W)) and np.isfinite(W[0][0]).all()
+    X[:], T[:] = X[0], T[0]
+    W = []
+    for strategy in (S.STRATEGY_SAMPLE, S.STRATEGY_SMALL_BATCH):
+        net, _ = public_net([2, 8, 1], ["tanh", "sigmoid"], 0, seed=4)
+        S.train(net, X[:30001], T[:30001], 1, strategy, S.OPTIMIZER_SGD, batch_size=1, learning_rate=0.05)
+        W.append([S.weights_view(net, l).copy() for l in (0, 1)])
+        S.free_network(net)
+    assert all(np.array_equal(a, b) for a, b in zip(*W))
+
+
 @pytest.mark.parametrize("topo,acts,loss,n", [
     ([784, 512, 1000, 10], ["relu", "relu", "softmax"], 1, 64),          # small products, deltas and grouped updates throughout
     ([100, 333, 70, 17], ["tanh", "sigmoid", "softmax"], 0, 9),          # unaligned rows, a head wider than a 16 x 16 tile

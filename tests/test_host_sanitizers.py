@@ -21,3 +21,16 @@ def test_host_sources_under_address_and_ub_sanitizers():
                          text=True, env=env, timeout=600)
     assert run.returncode == 0, run.stdout[-4000:]
     assert "host_sanitize:" in run.stdout and "refused" in run.stdout, run.stdout[-2000:]
+
+
+def test_trainings_of_small_nets_are_cut_into_short_launches():
+    """`make train_runs`: train() with stand-ins that check every launch's share of the steps and their order; an epoch
+    longer than about 50 ms is cut too."""
+    res = subprocess.run(["make", "-C", CSRC, "-B", "train_runs"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout
+    env = dict(os.environ)
+    env.pop("LD_PRELOAD", None)
+    run = subprocess.run([os.path.join(CSRC, "build", "host_train_runs")], stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                         text=True, env=env, timeout=300)
+    assert run.returncode == 0, run.stdout[-4000:]
+    assert "1000000 samples" in run.stdout
