@@ -619,9 +619,8 @@ struct sphip_net {
     // for the first layer, whose uploaded rows the vector kernels multiply with the caller's.
     std::vector<uint32_t> ptopo;
     std::vector<DevArray> PW;
-    uint8_t *arrays = nullptr;     // the one allocation behind every base, its size ...
-    size_t arrays_bytes = 0;
-    uint8_t *pad_stage = nullptr;  // ... and behind it the room through which uploaded rows reach PW
+    uint8_t *arrays = nullptr;     // the one allocation behind every base
+    uint8_t *pad_stage = nullptr;  // ... and behind them the room through which uploaded rows reach PW
     size_t pad_stage_bytes = 0;
 
     DevArray &w(uint32_t l) { return PW[l].base ? PW[l] : W[l]; }                    // what a forward multiplies with
@@ -1986,7 +1985,6 @@ int sphip_create(const sphip_desc *desc, sphip_net **out)
             if (stage > net->pad_stage_bytes) net->pad_stage_bytes = stage;
         }
     }
-    net->arrays_bytes = at;
     if (hipMalloc((void **)&net->arrays, at + net->pad_stage_bytes) != hipSuccess) {
         for (DevArray *a : placed) a->base = nullptr;
         net->arrays = nullptr;
@@ -2075,11 +2073,13 @@ int sphip_clone(const sphip_net *src, sphip_net **out)
     sphip_desc d{src->layers, src->topo.data(), src->act.data(), (uint8_t)src->prec};
     sphip_net *net = nullptr;
     if (sphip_create(&d, &net)) return 1;
-    hipError_t e = hipMemcpyAsync(net->arrays, src->arrays, src->arrays_bytes, hipMemcpyDeviceToDevice, g_stream);   // (the same layout)
+    hipError_t e = hipSuccess;
     for (uint32_t l = 0; l + 1 < src->layers && e == hipSuccess; ++l) {
-        for (int which = 0; which < 2; ++which) {
-            const DevArray &s = which == 0 ? src->W[l] : src->B[l];
-            DevArray &t = which == 0 ? net->W[l] : net->B[l];
+        // (array by array: a profile's copy of known size is the largest one's)
+        for (int which = 0; which < 3; ++which) {
+            const DevArray &s = which == 0 ? src->W[l] : which == 1 ? src->B[l] : src->PW[l];
+            DevArray &t = which == 0 ? net->W[l] : which == 1 ? net->B[l] : net->PW[l];
+            if (s.base && e == hipSuccess) e = hipMemcpyAsync(t.base, s.base, fmt_bytes(src->prec, s.laid), hipMemcpyDeviceToDevice, g_stream);
             t.max_val = s.max_val;
             t.uploaded = s.uploaded;
         }
