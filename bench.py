@@ -189,6 +189,18 @@ def load_traffic():
 PROFILED_TRAFFIC = load_traffic()
 
 
+def matrix_peak(prec, kernel):
+    """FLOP/s of products that the matrix cores could do at most in the way this kernel does them: sp_gemm32_bf16_parts
+    forms an FP32 product as six BF16 ones, the other kernels of FP32 weights use the FP32 matrix instructions."""
+    if kernel == "sp_gemm32_bf16_parts":
+        return MFMA16_PEAK / 6.0
+    return FP32_PEAK if prec == S.PRECISION_FLOAT32 else MFMA16_PEAK
+
+
+def layer_kernel(copies, topo, n):
+    return S.lib().sphip_layer_kernel_name(copies[0].h, dominant_layer(topo), n, 0).decode()
+
+
 def dominant_layer(topo):
     return 1 + int(np.argmax([topo[l] * topo[l + 1] for l in range(len(topo) - 1)]))
 
@@ -210,7 +222,7 @@ def roofline_for(copies, topo, prec, n, iters):
     K, N = topo[l - 1], topo[l]
     same = [i for i in range(1, len(topo)) if (topo[i - 1], topo[i]) == (K, N)]
     ms = float(np.mean([timed_layer(copies, i, n, iters) for i in same]))
-    kernel = S.lib().sphip_layer_kernel_name(copies[0].h, l, n, 0).decode()
+    kernel = layer_kernel(copies, topo, n)
     # a batch that runs in blocks of rows launches the layer's kernel once per block: ms (and traffic) are those of
     # all of them together, the layer's share of one forward
     rows = S.lib().sphip_batch_block_rows(copies[0].h, n, 0)
@@ -227,7 +239,7 @@ def roofline_for(copies, topo, prec, n, iters):
                     traffic=traffic, kernel=kernel, layer=l, shape=[n, N, K], avg_ms=ms, launches=launches)
     fl = 2.0 * n * K * N
     ach = fl / (ms * 1e-3)
-    peak = FP32_PEAK if prec == S.PRECISION_FLOAT32 else MFMA16_PEAK
+    peak = matrix_peak(prec, kernel)
     return dict(bound="mfma", achieved=ach / 1e12, peak=peak / 1e12, unit="TFLOP/s", frac=ach / peak,
                 traffic=traffic, kernel=kernel, layer=l, shape=[n, N, K], avg_ms=ms, launches=launches)
 
@@ -309,7 +321,7 @@ def run_workload(name, batches, steps, warmup, want_output=False, cpu_budget_s=0
         row = dict(workload=name, format=PREC_NAMES[prec], batch=n, steps=k, ms_per_step=ms_wall, ms_per_step_events=ms_ev,
                    samples_per_s=n / (ms_wall * 1e-3),
                    hbm_frac=algorithmic_bytes(topo, prec, n) / (ms_ev * 1e-3) / HBM_PEAK,
-                   mfma_frac=fl / (ms_ev * 1e-3) / (FP32_PEAK if prec == S.PRECISION_FLOAT32 else MFMA16_PEAK),
+                   mfma_frac=fl / (ms_ev * 1e-3) / matrix_peak(prec, layer_kernel(copies, topo, n)),
                    copies=len(copies), finite=bool(np.isfinite(y).all()))
         if n in cfg.get("roofline_batches", batches):
             row["roofline"] = roofline_for(copies, topo, prec, n, 20 if n >= 1024 else 200)
