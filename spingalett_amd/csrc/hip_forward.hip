@@ -718,7 +718,7 @@ LayerArgs make_layer_args(const sphip_net *net, uint32_t l /*1-based layer*/, bo
     L.bias_fmt = net->prec;
     L.act = net->act[l - 1] == A_SOFTMAX ? A_NONE : net->act[l - 1];
     L.N = net->ptopo[l];
-    L.pad = net->ptopo[l] - net->topo[l];
+    L.pad = (uint16_t)(net->ptopo[l] - net->topo[l]);                          // (at most 63)
     L.K = raw ? net->topo[l - 1] : net->ptopo[l - 1];
     return L;
 }

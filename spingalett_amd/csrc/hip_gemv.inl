@@ -11,10 +11,13 @@ struct LayerArgs {
     float wscale;          // folded weight scale
     float bscale;          // folded bias scale
     int bias_fmt;
-    int act;               // activation applied in the epilogue (A_NONE for softmax layers)
+    uint16_t act;          // activation applied in the epilogue (A_NONE for softmax layers)
+    uint16_t pad;          // the last of the N outputs that are padding, not neurons
     uint32_t N, K;         // out, in
-    uint32_t pad;          // the last of the N outputs that are padding, not neurons
 };
+// The vector kernels' arguments fill one 64-byte line: a second one is another miss before the first load (64-827-31 BF16
+// at four samples 11.5 -> 11.7 us).
+static_assert(sizeof(LayerArgs) == 40, "");
 
 // The sum of output n, before its activation.  A padded neuron's is zero, whatever its zero weights meet: an infinite
 // input would make a NaN of it (0 x inf), and the next layer's zero column NaNs of all its outputs.
