@@ -88,7 +88,8 @@ SPHIP_API int  sphip_upload_array(sphip_net *net, uint32_t l, int which,
  *   [n][topology[last]], FP32.  n <= 4 runs the vector (GEMV) kernels in FP32-grade
  *   arithmetic (integer weights: exact integer dot products on the INT8 matrix
  *   cores); larger n runs the matrix-core kernels with 16-bit activations.  FP32
- *   weights always compute in FP32 (vector kernels up to n = 64). */
+ *   weights compute in FP32 or with FP32's bits (vector kernels up to n = 4, FP32
+ *   matrix instructions, large products as products of BF16 parts). */
 SPHIP_API int  sphip_forward(sphip_net *net, const float *x, uint32_t n, float *y,
                              uint32_t flags);
 /* sphip_forward for callers that cannot allocate (code under HIP graph capture, tight serving loops, harnesses
