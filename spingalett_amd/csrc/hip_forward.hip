@@ -1251,17 +1251,17 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         if (tl_route.dry) return;
         if (bm == 128u) {
             // 128-row tiles (gemm16_tile_rows)
-            constexpr size_t lds = 2 * (128 + 256) * 64 * sizeof(uint16_t);
-            auto kern = sp_gemm16_big<FMT, F16T, 2, 4, 2, 2>;
+            constexpr size_t lds = BigTile<FMT, 4>::LDS;
+            auto kern = sp_gemm16_big<FMT, F16T, 4>;
             static bool once = ((void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
             (void)once;
-            kern<<<grid, 512, lds, g_stream>>>(g);
+            kern<<<grid, 256, lds, g_stream>>>(g);
         } else {
-            constexpr size_t lds = 2 * (256 + 256) * 64 * sizeof(uint16_t);
-            auto kern = sp_gemm16_big<FMT, F16T, 2, 4, 4, 2>;
+            constexpr size_t lds = BigTile<FMT, 8>::LDS;
+            auto kern = sp_gemm16_big<FMT, F16T, 8>;
             static bool once = ((void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
             (void)once;
-            kern<<<grid, 512, lds, g_stream>>>(g);
+            kern<<<grid, 256, lds, g_stream>>>(g);
         }
         if (g.ws) {
             const uint64_t total = (uint64_t)M * L.N;

@@ -558,63 +558,140 @@ __device__ __forceinline__ void ds_read128(u32x4 &dst, uint32_t addr)
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
 
-// reads CNT fragments 4 KiB apart (32 tile rows of 128 bytes) starting at addr + BASE
+// 16 bytes per lane from scalar base + 32-bit lane offset + immediate.  Inline assembly: the compiler's
+// wait-count bookkeeping does not see the load, the caller waits with s_waitcnt vmcnt before using dst.
+template <int OFF>
+__device__ __forceinline__ void load16_async(u32x4 &dst, uint32_t voff, const void *sbase)
+{
+    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(dst) : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
+}
+
+// reads CNT fragments 2 KiB apart (16 tile rows of 128 bytes) starting at addr + BASE
 template <int BASE, int CNT, int I = 0>
 __device__ __forceinline__ void frag_reads(u32x4 *dst, uint32_t addr)
 {
     if constexpr (I < CNT) {
-        ds_read128<BASE + I * 4096>(dst[I], addr);
+        ds_read128<BASE + I * 2048>(dst[I], addr);
         frag_reads<BASE, CNT, I + 1>(dst, addr);
     }
 }
 
 // ---------------------------------------------------------------------------
-// Large-tile variant of the 16-bit MFMA GEMM (rows 16-byte aligned).  WM x WN waves,
-// each TM x TN tiles of 32x32; BK = 64.  A K that is not a multiple of 64 leaves a
-// partial K tile, which is processed first: its lanes past the end of a row fetch the
-// row's element k0 instead (always inside the array) and overwrite what they fetched
-// with zeros once it has landed.
-//   * LDS rows hold 64 elements = eight 16-byte chunks, unpadded; chunk c of row
-//     r sits at position c ^ ((r >> 1) & 7).  A 128-bit fragment read is served 16
-//     lanes (16 consecutive rows, 256 bytes = all 64 banks) per cycle: rows of equal
-//     parity share a 128-byte half, and r >> 1 gives those eight rows eight
-//     different chunk positions.
-//   * 16-bit operands (activations always, BF16/FP16 weights) go from global
-//     memory straight into LDS (global_load_lds_dwordx4: each wave fills 1 KiB =
-//     8 tile rows per instruction); which global chunk a lane fetches carries the
-//     swizzle.  Integer weights pass through registers to be unpacked.
-//   * two LDS stages: tile kt+1 is in flight while tile kt feeds the MFMAs; one
-//     barrier per K tile.
-template <int FMT, bool F16T, int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
+// Large-tile variant of the 16-bit MFMA GEMM (rows 16-byte aligned): 256 x 256 tiles (RM = 8) or 128 x 256 (RM = 4), four
+// waves of RM x 8 tiles of 16 x 16, BK = 64.
+//
+// On this data the part is at its power limit, not at an issue limit: matrix instructions alone, operands in registers, run
+// at 1.98 PFLOP/s as v_mfma_f32_16x16x32 and at 1.73 as 32x32x16 (half the accumulator traffic per product), and what LDS
+// reads and loads add to the time of 8192 x 8192 x 8192 is nearly additive (0.58 ms without either, 0.18 and 0.14 for
+// eight waves of 128 x 64).  So: the small instruction; as much of the tile per wave as the registers hold, which is
+// 128 x 128 with one wave per SIMD (128 instead of 192 KiB of fragment reads per K tile); neighbouring products share an
+// operand.  8192 x 8192 x 8192 FP16 0.870 -> 0.771 ms (1.43 PFLOP/s; 32 x 32 x 16 in eight waves before, whose 16 x 16 x 32
+// form took 0.82), 4096 x 8192 x 8192 INT8 0.465 -> 0.408, INT4 0.449 -> 0.377, INT2 0.395 -> 0.356, 2000 x 4096 x 12288 on
+// RM = 4 0.198 -> 0.167 ms.  Sums of a few hundred gain little (8192 x 8192 x 512 98 -> 95 us): a tile's prologue takes 2.4 us,
+// its epilogue 8, in which all compute units write at once (4 TB/s).  FP32 outputs of sums of 256, written 4 waves instead
+// of 8 at a time, lose 2-7 % (4096 x 4096 x 256 26.1 -> 27.5 us).
+//
+// The accumulators are accumulation registers by number (mfma_acc, acc_read): left to the compiler, 256 of them next to the
+// fragments are spilled.  Nothing else here lives in those registers (the first statement claims all of them, and the
+// vector registers suffice for the rest).
+//
+// One wave per SIMD has nobody to hide behind, so the loop is straight-line code with everything asked for ahead:
+//   * A K tile is RM quads of sixteen products (four row tiles x four column tiles).  Consecutive quads share one of their
+//     two sets of four fragments, the other was requested a quad earlier.
+//   * 16-bit operands (activations always, BF16/FP16 weights) go from global memory straight into LDS
+//     (global_load_lds_dwordx4: each wave fills 1 KiB = 8 tile rows per instruction), one instruction behind every fourth
+//     product; which global chunk a lane fetches carries the swizzle.  Integer weights come as packed codes, three
+//     tiles ahead, and are unpacked through registers a step per product (w_step).
+//   * Two LDS stages (RM = 4: three).  The barrier comes when the last fragments of a tile are in registers, two quads (one)
+//     before its products end: the next tile's first fragments and the loads that overwrite this tile's stage go
+//     out behind those products.
+//   * LDS rows hold 64 elements = eight 16-byte chunks, unpadded; chunk c of row r sits at position c ^ ((r >> 1) & 7).  A
+//     128-bit fragment read is served 16 lanes (16 consecutive rows, 256 bytes = all 64 banks) per cycle: rows of equal
+//     parity share a 128-byte half, and r >> 1 gives those eight rows eight different chunk positions.
+// A K that is not a multiple of 64 leaves a partial K tile, which is processed first: its lanes past the end of a row fetch
+// the row's element k0 instead (always inside the array) and overwrite what they fetched with zeros once it has landed.
+// ---------------------------------------------------------------------------
+// accumulation registers ACC .. ACC + 3 += a . b (16 rows of a, 16 columns of b, 32 k)
+template <bool F16T, int ACC>
+__device__ __forceinline__ void mfma_acc(const u32x4 &a, const u32x4 &b)
 {
-    constexpr int NT = 64 * WM * WN, NWAVES = WM * WN;
-    constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 64;
+    if constexpr (F16T) asm volatile("v_mfma_f32_16x16x32_f16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(ACC), "n"(ACC + 3));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(a), "v"(b), "n"(ACC), "n"(ACC + 3));
+}
+
+template <int R>
+__device__ __forceinline__ float acc_read()
+{
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(v) : "n"(R));
+    return v;
+}
+
+template <int R>
+__device__ __forceinline__ void acc_zero()
+{
+    asm volatile("v_accvgpr_write_b32 a[%0], 0" ::"n"(R));
+}
+
+#define SP_ACC10(d) "a" #d "0", "a" #d "1", "a" #d "2", "a" #d "3", "a" #d "4", "a" #d "5", "a" #d "6", "a" #d "7", "a" #d "8", "a" #d "9"
+#define SP_ACC128                                                                                                      \
+    "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", SP_ACC10(1), SP_ACC10(2), SP_ACC10(3), SP_ACC10(4),    \
+        SP_ACC10(5), SP_ACC10(6), SP_ACC10(7), SP_ACC10(8), SP_ACC10(9), SP_ACC10(10), SP_ACC10(11), "a120", "a121",   \
+        "a122", "a123", "a124", "a125", "a126", "a127"
+#define SP_ACC256                                                                                                      \
+    SP_ACC128, "a128", "a129", SP_ACC10(13), SP_ACC10(14), SP_ACC10(15), SP_ACC10(16), SP_ACC10(17), SP_ACC10(18),     \
+        SP_ACC10(19), SP_ACC10(20), SP_ACC10(21), SP_ACC10(22), SP_ACC10(23), SP_ACC10(24), "a250", "a251", "a252",    \
+        "a253", "a254", "a255"
+
+// two FP32 values below 65520 in magnitude (they round to at most 65504), as f32_to_f16_sat converts them
+__device__ __forceinline__ uint32_t pack_f16_small(float a, float b)
+{
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 h = {(_Float16)a, (_Float16)b};
+    uint32_t r;
+    __builtin_memcpy(&r, &h, 4);
+    return r;
+}
+
+// LDS stages (three where they fit), bytes of packed codes per K tile (integer formats), bytes of LDS
+template <int FMT, int RM>
+struct BigTile {
+    static constexpr int NSTAGE = RM == 8 || FMT == I8 ? 2 : 3;
+    static constexpr int W_AT = 32 * RM * 128, STAGE = W_AT + 256 * 128;      // the weights' part of a stage, a stage
+    static constexpr int CODES = fmt_bits(FMT) == 16 ? 0 : 256 * 64 * fmt_bits(FMT) / 8;
+    static constexpr int LDS = NSTAGE * STAGE + 2 * CODES;
+};
+
+template <int FMT, bool F16T, int RM>
+__global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
+{
+    static_assert(RM == 8 || RM == 4, "");
+    constexpr int BM = 32 * RM, BN = 256, BK = 64;
+    using B = BigTile<FMT, RM>;
+    constexpr int NSTAGE = B::NSTAGE, W_AT = B::W_AT, STAGE = B::STAGE, CODES = B::CODES;
     constexpr int bits = fmt_bits(FMT);
     constexpr bool W_DIRECT = (FMT == BF16 || FMT == F16);
-    constexpr int A_ISSUES = BM * 8 / NT;               // 16-byte chunks per thread and tile
-    constexpr int W_ISSUES = BN * 8 / NT;
+    constexpr int A_DMA = BM / 32, DMA = A_DMA + (W_DIRECT ? BN / 32 : 0);     // load instructions per wave and tile
     constexpr int EPL = 128 / bits;                     // weight elements per 16-byte global load
     constexpr int CPL = EPL / 8;                        // LDS chunks produced per global load
-    constexpr int W_LOADS = W_DIRECT ? 1 : (BN * BK / EPL + NT - 1) / NT;
+    constexpr int W_LOADS = W_DIRECT ? 1 : BN * BK / EPL / 256;
+    constexpr int PW = 16 / bits;                       // packed pairs per 32-bit word of codes (integer formats)
 
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-    uint16_t *As = smem;                                // [2][BM][64]
-    uint16_t *Ws = smem + 2 * BM * BK;                  // [2][BN][64]
+    if constexpr (RM == 8) asm volatile("" ::: SP_ACC256);
+    else asm volatile("" ::: SP_ACC128);
 
     const uint32_t M = g.M, N = g.L.N, K = g.L.K;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = wave / WN, wn = wave % WN;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
 
     // Tile order: each XCD (workgroup id mod 8) gets a contiguous run of tiles; inside the run, 8 row tiles x 4
     // column tiles are consecutive so that the 32 workgroups an XCD runs at once share A rows and W rows in its L2.
-    // (A workgroup that walks over several tiles instead, one workgroup per compute unit, was measured: no faster,
-    // and the longer live ranges cost the integer formats register spills.)
     const uint32_t tiles_n = (N + BN - 1) / BN, tiles_m = (M + BM - 1) / BM;
-    const uint32_t ntiles = tiles_m * tiles_n;
-    uint32_t m0 = 0, n0 = 0;
-    auto place = [&](uint32_t bid) {
-        const uint32_t per = ntiles / 8u;
+    uint32_t m0, n0;
+    {
+        const uint32_t ntiles = tiles_m * tiles_n, per = ntiles / 8u;
+        uint32_t bid = blockIdx.x;
         if (bid < per * 8u) bid = (bid & 7u) * per + (bid >> 3);
         constexpr uint32_t GM = 8;
         const uint32_t group = bid / (GM * tiles_n);
@@ -623,218 +700,7 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
         const uint32_t in = bid - group * GM * tiles_n;
         m0 = (first + in % rows) * BM;
         n0 = (in / rows) * BN;
-    };
-
-    f32x16 acc[TM][TN];
-
-    // LDS-DMA sources: a uniform base (advanced per K tile on the scalar unit) plus a fixed 32-bit
-    // byte offset per lane and issue, and LDS destinations derived from a scalar wave index: the main
-    // loop then issues its loads without any vector-ALU instruction, which would otherwise queue
-    // behind the other wave's MFMAs
-    const int wave_s = __builtin_amdgcn_readfirstlane(wave);
-    // Only the first wave of each SIMD (waves 0 .. NWAVES/2-1, which the issue arbiter serves first)
-    // issues the loads, for itself and for wave + NWAVES/2: a wave stalls while the address unit takes
-    // its load, and the other wave of the SIMD keeps the MFMA pipe fed meanwhile.
-    // (four-wave workgroups have one wave per SIMD: every wave loads its own share)
-    constexpr int HALF = NWAVES > 4 ? NWAVES / 2 : NWAVES;      // loader waves
-    constexpr int PER = NWAVES / HALF;                            // shares a loader wave issues
-    constexpr int A_DUTY = PER * A_ISSUES, W_DUTY = W_DIRECT ? PER * W_ISSUES : 1;
-    uint32_t a_voff[A_DUTY], w_voff[W_DUTY];
-    auto lane_offsets = [&]() {
-#pragma unroll
-        for (int d = 0; d < A_DUTY; ++d) {
-            const int i = d / PER, wv = (wave & (HALF - 1)) + (d % PER) * HALF;
-            const int ci = (i * NWAVES + wv) * 64 + lane, row = ci >> 3, pos = ci & 7;
-            const uint32_t m = m0 + row < M ? m0 + row : M - 1;
-            a_voff[d] = (uint32_t)(((size_t)m * K + ((pos ^ ((row >> 1) & 7)) << 3)) * 2u);
-        }
-        if constexpr (W_DIRECT) {
-#pragma unroll
-            for (int d = 0; d < W_DUTY; ++d) {
-                const int i = d / PER, wv = (wave & (HALF - 1)) + (d % PER) * HALF;
-                const int ci = (i * NWAVES + wv) * 64 + lane, row = ci >> 3, pos = ci & 7;
-                const uint32_t n = n0 + row < N ? n0 + row : N - 1;
-                w_voff[d] = (uint32_t)(((size_t)n * K + ((pos ^ ((row >> 1) & 7)) << 3)) * 2u);
-            }
-        }
-    };
-    // which 8 elements of a 64-element tile row this lane fetches: the same for every load it issues, because
-    // the rows of two of its loads are a multiple of 16 apart
-    static_assert(NWAVES % 2 == 0 && HALF % 2 == 0, "the swizzle of a lane's loads must not depend on the load");
-    const uint32_t kchunk = (uint32_t)((lane & 7) ^ ((((wave & (HALF - 1)) * 8 + (lane >> 3)) >> 1) & 7)) << 3;
-    const char *a_base = reinterpret_cast<const char *>(g.A + (size_t)(blockIdx.y / g.ksplits) * g.M * g.L.K);
-    const char *w_base = reinterpret_cast<const char *>(g.L.w);
-    const size_t w_row_bytes = (size_t)K * bits / 8u;
-    uint4 rw[W_LOADS];
-    const uint32_t lds_a = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)As + (uint32_t)(wave_s & (HALF - 1)) * 1024u;
-    const uint32_t lds_w = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)Ws + (uint32_t)(wave_s & (HALF - 1)) * 1024u;
-    const bool loader = wave_s < HALF;
-    // the idx-th load instruction of a loader wave's tile (A first, then W); idx is a constant once
-    // the caller's loops are unrolled
-    constexpr int DMA_TOTAL = A_DUTY + (W_DIRECT ? W_DUTY : 0);
-    auto issue_one = [&](int buf, uint32_t k0, int idx) {
-        if (!loader) return;
-#pragma unroll
-        for (int d = 0; d < A_DUTY; ++d)
-            if (d == idx)
-                lds_dma16(lds_a + (uint32_t)(buf * BM * BK * 2 + ((d / PER) * NWAVES + (d % PER) * HALF) * 1024), a_voff[d],
-                          a_base + (size_t)k0 * 2u);
-        if constexpr (W_DIRECT) {
-#pragma unroll
-            for (int d = 0; d < W_DUTY; ++d)
-                if (A_DUTY + d == idx)
-                    lds_dma16(lds_w + (uint32_t)(buf * BN * BK * 2 + ((d / PER) * NWAVES + (d % PER) * HALF) * 1024), w_voff[d],
-                              w_base + (size_t)k0 * 2u);
-        }
-    };
-    auto issue_direct = [&](int buf, uint32_t k0) {            // the whole tile at once (prologue)
-#pragma unroll
-        for (int idx = 0; idx < DMA_TOTAL; ++idx) issue_one(buf, k0, idx);
-    };
-    auto load_w_regs = [&](uint32_t k0) {
-        if constexpr (!W_DIRECT) {
-            constexpr int LPR = BK / EPL;
-#pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) {
-                const int c = t + NT * i, row = c / LPR, kc = c % LPR;
-                const uint32_t n = n0 + row < N ? n0 + row : N - 1;
-                if (row < BN)
-                    rw[i] = *reinterpret_cast<const uint4 *>(g.L.w + (size_t)n * w_row_bytes + (size_t)(k0 + kc * EPL) * bits / 8u);
-            }
-        }
-    };
-    // The partial K tile at k0 (prologue only).  Rows are whole 16-byte units, so a 16-byte piece lies entirely
-    // inside a row or entirely past its end; code 0 decodes to 0.
-    auto load_w_regs_tail = [&](uint32_t k0) {
-        if constexpr (!W_DIRECT) {
-            constexpr int LPR = BK / EPL;
-#pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) {
-                const int c = t + NT * i, row = c / LPR, kc = c % LPR;
-                const uint32_t n = n0 + row < N ? n0 + row : N - 1;
-                if (row >= BN) continue;
-                if (k0 + kc * EPL < K)
-                    rw[i] = *reinterpret_cast<const uint4 *>(g.L.w + (size_t)n * w_row_bytes + (size_t)(k0 + kc * EPL) * bits / 8u);
-                else
-                    rw[i] = make_uint4(0u, 0u, 0u, 0u);
-            }
-        }
-    };
-    auto issue_tail = [&](uint32_t k0) {                       // into stage 0
-        if (!loader) return;
-        const uint32_t back = k0 + kchunk < K ? 0u : kchunk * 2u;
-#pragma unroll
-        for (int d = 0; d < A_DUTY; ++d)
-            lds_dma16(lds_a + (uint32_t)(((d / PER) * NWAVES + (d % PER) * HALF) * 1024), a_voff[d] - back, a_base + (size_t)k0 * 2u);
-        if constexpr (W_DIRECT) {
-#pragma unroll
-            for (int d = 0; d < W_DUTY; ++d)
-                lds_dma16(lds_w + (uint32_t)(((d / PER) * NWAVES + (d % PER) * HALF) * 1024), w_voff[d] - back, w_base + (size_t)k0 * 2u);
-        }
-    };
-    auto zero_tail = [&](uint32_t k0) {                        // after the loads of issue_tail have landed
-        if (!loader || k0 + kchunk < K) return;
-        const uint32_t mine = (uint32_t)(wave & (HALF - 1)) * 1024u + (uint32_t)lane * 16u;
-#pragma unroll
-        for (int d = 0; d < A_DUTY; ++d)
-            *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(As) + mine + ((d / PER) * NWAVES + (d % PER) * HALF) * 1024) =
-                make_uint4(0u, 0u, 0u, 0u);
-        if constexpr (W_DIRECT) {
-#pragma unroll
-            for (int d = 0; d < W_DUTY; ++d)
-                *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(Ws) + mine + ((d / PER) * NWAVES + (d % PER) * HALF) * 1024) =
-                    make_uint4(0u, 0u, 0u, 0u);
-        }
-    };
-    auto store_w_regs = [&](int buf) {
-        if constexpr (!W_DIRECT) {
-            constexpr int LPR = BK / EPL;
-            constexpr int PW = 16 / bits;
-#pragma unroll
-            for (int i = 0; i < W_LOADS; ++i) {
-                const int c = t + NT * i, row = c / LPR, kc = c % LPR;
-                if (row >= BN) continue;
-                const uint32_t w[4] = {rw[i].x, rw[i].y, rw[i].z, rw[i].w};
-                uint32_t o[4 * PW];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) unpack_word16<FMT, F16T>(w[q], o + q * PW);
-                uint16_t *rowp = Ws + buf * BN * BK + row * BK;
-#pragma unroll
-                for (int v = 0; v < CPL; ++v) {
-                    const int chunk = kc * CPL + v;
-                    *reinterpret_cast<uint4 *>(rowp + ((chunk ^ ((row >> 1) & 7)) << 3)) =
-                        make_uint4(o[4 * v], o[4 * v + 1], o[4 * v + 2], o[4 * v + 3]);
-                }
-            }
-        }
-    };
-
-    // ---- main loop -----------------------------------------------------------
-    // Fragment reads are issued as explicit ds_read_b128 with manual lgkmcnt waits:
-    // the compiler would otherwise drain every pending LDS-DMA load before the first
-    // LDS read of an iteration and serialise load and compute.  Reads of k-step s+1
-    // are in flight while the MFMAs of k-step s run.
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)smem;
-    const int h = lane >> 5, l7 = (lane >> 1) & 7;
-    uint32_t va[4], vw[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        const uint32_t xo = (uint32_t)(((2 * ks + h) ^ l7) << 4);
-        va[ks] = lds0 + (uint32_t)((wm * TM * 32 + (lane & 31)) * 128) + xo;
-        vw[ks] = lds0 + (uint32_t)(2 * BM * BK * 2) + (uint32_t)((wn * TN * 32 + (lane & 31)) * 128) + xo;
     }
-    u32x4 fa[2][TM], fb[2][TN];
-
-    // A loader wave slips one load instruction behind each of the first MFMAs of k-steps 0..2: the
-    // matrix pipe is busy for eight passes after every issue, and the address unit takes the load meanwhile.
-    constexpr int DPS = (DMA_TOTAL + 2) / 3;              // load instructions per k-step
-    auto stage = [&](auto cur_c, bool more, uint32_t knext) {
-        constexpr int CUR = decltype(cur_c)::value;
-        if (more) load_w_regs(knext);
-        frag_reads<CUR * BM * BK * 2, TM>(fa[0], va[0]);
-        frag_reads<CUR * BN * BK * 2, TN>(fb[0], vw[0]);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int cs = ks & 1;
-            if (ks < 3) {
-                frag_reads<CUR * BM * BK * 2, TM>(fa[cs ^ 1], va[ks + 1]);
-                frag_reads<CUR * BN * BK * 2, TN>(fb[cs ^ 1], vw[ks + 1]);
-                asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TM + TN));
-            } else {
-                asm volatile("s_waitcnt lgkmcnt(0)");
-            }
-#pragma unroll
-            for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(fa[cs][i]));
-#pragma unroll
-            for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(fb[cs][j]));
-            __builtin_amdgcn_sched_barrier(0);          // keep the MFMA group between its wait and the next reads
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    if constexpr (F16T) {
-                        f16x8 a, b;
-                        __builtin_memcpy(&a, &fa[cs][i], 16);
-                        __builtin_memcpy(&b, &fb[cs][j], 16);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc[i][j], 0, 0, 0);
-                    } else {
-                        bf16x8 a, b;
-                        __builtin_memcpy(&a, &fa[cs][i], 16);
-                        __builtin_memcpy(&b, &fb[cs][j], 16);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[i][j], 0, 0, 0);
-                    }
-                    if (more && ks < 3 && i * TN + j < DPS) {
-                        __builtin_amdgcn_sched_barrier(0);
-                        issue_one(CUR ^ 1, knext, ks * DPS + i * TN + j);
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (more) store_w_regs(CUR ^ 1);
-        asm volatile("s_waitcnt vmcnt(0)");         // this wave's share of the next stage has landed
-        __syncthreads();                             // ... and everybody's; the current stage is free again
-    };
 
     // grid y splits K for problems with too few tiles to fill the chip
     const uint32_t kbeg = g.kper ? (blockIdx.y % g.ksplits) * g.kper : 0u;
@@ -843,168 +709,526 @@ __global__ __launch_bounds__(64 * WM * WN) void sp_gemm16_big(const GemmArgs g)
     const uint32_t tail = (kend - kbeg) % BK;              // only the last K split can have one
     // tile 0 is the partial tile if there is one; tile s >= 1 then starts at kbeg + (s - 1) * BK
     const uint32_t kshift = tail ? (uint32_t)BK : 0u;
-    place(blockIdx.x);
-    lane_offsets();
+    auto k_of = [&](uint32_t s) { return kbeg + s * BK - kshift; };
+
+    // LDS-DMA sources: a uniform base (advanced per K tile on the scalar unit) plus a fixed 32-bit byte offset per lane and
+    // load.  A lane fetches the same eight of a tile row's 64 elements in every load: the rows of two of its loads are a
+    // multiple of 32 apart.
+    const uint32_t kchunk = (uint32_t)((lane & 7) ^ (((wave * 8 + (lane >> 3)) >> 1) & 7)) << 3;
+    uint32_t a_voff[A_DMA], w_voff[W_DIRECT ? BN / 32 : W_LOADS];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < A_DMA; ++i) {
+        const uint32_t m = m0 + (i * 4 + wave) * 8 + (lane >> 3);
+        a_voff[i] = (uint32_t)(((size_t)(m < M ? m : M - 1) * K + kchunk) * 2u);
+    }
+    if constexpr (W_DIRECT) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    if (tail) {
-        const uint32_t kt0 = kend - tail;
-        issue_tail(kt0);
-        load_w_regs_tail(kt0);
-        store_w_regs(0);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        zero_tail(kt0);
+        for (int i = 0; i < BN / 32; ++i) {
+            const uint32_t n = n0 + (i * 4 + wave) * 8 + (lane >> 3);
+            w_voff[i] = (uint32_t)(((size_t)(n < N ? n : N - 1) * K + kchunk) * 2u);
+        }
     } else {
-        issue_direct(0, kbeg);
-        load_w_regs(kbeg);
-        store_w_regs(0);
-        asm volatile("s_waitcnt vmcnt(0)");
+#pragma unroll
+        for (int i = 0; i < W_LOADS; ++i) {
+            constexpr int LPR = BK / EPL;                   // loads per tile row
+            const int c = t + 256 * i;
+            const uint32_t n = n0 + c / LPR;
+            w_voff[i] = (uint32_t)((size_t)(n < N ? n : N - 1) * ((size_t)K * bits / 8u) + (size_t)(c % LPR) * 16u);
+        }
     }
+    const char *const a_base = reinterpret_cast<const char *>(g.A + (size_t)(blockIdx.y / g.ksplits) * M * K);
+    const char *const w_base = reinterpret_cast<const char *>(g.L.w);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t *)smem;
+    // the idx-th load instruction of this wave's share of the tile at k0 (A first, then W); idx is a constant once unrolled
+    auto dma_at = [&](uint32_t stage, const char *a_at, const char *w_at, uint32_t back, int idx) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < A_DMA; ++i)
+            if (i == idx) lds_dma16(stage + (uint32_t)(i * 4096), a_voff[i] - back, a_at);
+        if constexpr (W_DIRECT) {
+#pragma unroll
+            for (int i = 0; i < BN / 32; ++i)
+                if (A_DMA + i == idx) lds_dma16(stage + (uint32_t)(W_AT + i * 4096), w_voff[i] - back, w_at);
+        }
+    };
+    const uint32_t lds_w = lds0 + (uint32_t)wave * 1024u;   // where this wave's share of a stage begins
+    auto dma = [&](uint32_t stage, uint32_t k0, uint32_t back, int idx) __attribute__((always_inline)) {
+        dma_at(lds_w + stage, a_base + (size_t)k0 * 2u, w_base + (W_DIRECT ? (size_t)k0 * 2u : 0u), back, idx);
+    };
+    // Integer weights: the packed codes of a tile go to LDS too, a thread's 16-byte pieces to a place of its own, which only
+    // that thread reads.  (Loaded into registers two tiles ahead they would be copied while still on their way: the compiler
+    // does not see these loads.)
+    const uint32_t codes0 = (uint32_t)(NSTAGE * STAGE);
+    auto dma_codes = [&](uint32_t buf, uint32_t k0, bool clip) __attribute__((always_inline)) {
+        if constexpr (!W_DIRECT) {
+#pragma unroll
+            for (int i = 0; i < W_LOADS; ++i) {
+                constexpr int LPR = BK / EPL;
+                const uint32_t piece = (uint32_t)((t + 256 * i) % LPR);
+                const uint32_t back = clip && k0 + piece * EPL >= K ? piece * 16u : 0u;      // past its row: the row's start of the tile
+                lds_dma16(lds0 + codes0 + buf + (uint32_t)(i * 4 + wave) * 1024u, w_voff[i] - back, w_base + (size_t)k0 * bits / 8u);
+            }
+        }
+    };
+    u32x4 rw[W_LOADS];                                      // this thread's codes of the tile that is unpacked
+    auto read_codes = [&](uint32_t buf) __attribute__((always_inline)) {
+        if constexpr (!W_DIRECT) {
+#pragma unroll
+            for (int i = 0; i < W_LOADS; ++i) ds_read128<0>(rw[i], lds0 + codes0 + buf + (uint32_t)(t + 256 * i) * 16u);
+        }
+    };
+    auto pin_codes = [&]() __attribute__((always_inline)) {
+        if constexpr (!W_DIRECT) {
+#pragma unroll
+            for (int i = 0; i < W_LOADS; ++i) asm volatile("" : "+v"(rw[i]));
+        }
+    };
+    constexpr int CREADS = W_DIRECT ? 0 : W_LOADS;
+    // Step s of 64 that unpack rw into the stage at `stage`: eight chunks of eight codes, eight steps each (INT2: two chunks
+    // in sixteen), at most three vector instructions a step, so that a step fits behind a product.
+    uint32_t up[8];
+    auto w_step = [&](uint32_t stage, int s) __attribute__((always_inline)) {
+        if constexpr (!W_DIRECT) {
+            constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
+            constexpr int LPR = BK / EPL;
+            const int c = s >> 3, p = s & 7;                 // chunk of this thread, step of it
+            const int i = c / CPL, v = c % CPL;              // its load, its chunk of that load
+            auto put = [&](int chunk_of_load, uint32_t o0, uint32_t o1, uint32_t o2, uint32_t o3) __attribute__((always_inline)) {
+                const int cc = t + 256 * i, row = cc / LPR, chunk = (cc % LPR) * CPL + chunk_of_load;
+                char *const at = reinterpret_cast<char *>(smem) + stage + W_AT + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4);
+                *reinterpret_cast<uint4 *>(at) = make_uint4(o0, o1, o2, o3);
+            };
+            if constexpr (!F16T) {
+                (void)LO; (void)HI;
+                if (p == 0) {
+#pragma unroll
+                    for (int q = 0; q < 4 / PW; ++q) unpack_word16<FMT, F16T>(rw[i][v * (4 / PW) + q], up + q * PW);
+                    put(v, up[0], up[1], up[2], up[3]);
+                }
+            } else if constexpr (FMT == I8) {
+                if (p < 4) {
+                    const uint32_t w = rw[i][2 * v + (p >> 1)];
+                    up[p] = h2_sub((((p & 1) ? w >> 8 : w) & 0x00FF00FFu) ^ 0x64806480u, 0x64806480u);
+                } else if (p == 4) {
+                    up[4] = __builtin_amdgcn_perm(up[1], up[0], LO);
+                    up[5] = __builtin_amdgcn_perm(up[1], up[0], HI);
+                } else if (p == 5) {
+                    up[6] = __builtin_amdgcn_perm(up[3], up[2], LO);
+                    up[7] = __builtin_amdgcn_perm(up[3], up[2], HI);
+                } else if (p == 6) {
+                    put(v, up[4], up[5], up[6], up[7]);
+                }
+            } else if constexpr (FMT == I4) {
+                const uint32_t w = rw[i][v];
+                if (p == 0) up[0] = h2_sub((w & 0x000F000Fu) ^ 0x64086408u, 0x64086408u);
+                else if (p == 1) up[1] = h2_sub((w & 0x00F000F0u) ^ 0x54805480u, 0x54805480u);
+                else if (p == 2) up[2] = h2_sub(((w >> 8) & 0x000F000Fu) ^ 0x64086408u, 0x64086408u);
+                else if (p == 3) up[3] = h2_sub(((w >> 8) & 0x00F000F0u) ^ 0x54805480u, 0x54805480u);
+                else if (p == 4) {
+                    up[4] = __builtin_amdgcn_perm(up[1], up[0], LO);
+                    up[5] = __builtin_amdgcn_perm(up[3], up[2], LO);
+                } else if (p == 5) {
+                    up[6] = __builtin_amdgcn_perm(up[1], up[0], HI);
+                    up[7] = __builtin_amdgcn_perm(up[3], up[2], HI);
+                } else if (p == 6) {
+                    put(v, up[4], up[5], up[6], up[7]);
+                }
+            } else if constexpr (FMT == I2) {
+                const uint32_t w = rw[i][v >> 1], y = w >> 10;
+                const int p2 = s & 15;
+                if (p2 == 0) up[0] = h2_sub((w & 0x00030003u) ^ 0x64026402u, 0x64026402u);
+                else if (p2 == 1) up[1] = h2_sub((w & 0x000C000Cu) ^ 0x5C085C08u, 0x5C085C08u);
+                else if (p2 == 2) up[2] = h2_sub((w & 0x00300030u) ^ 0x54205420u, 0x54205420u);
+                else if (p2 == 3) up[3] = h2_sub((w & 0x00C000C0u) ^ 0x4C804C80u, 0x4C804C80u);
+                else if (p2 == 4) up[4] = h2_sub((w & 0x03000300u) ^ 0x46004600u, 0x46004600u);
+                else if (p2 == 5) up[5] = h2_sub((y & 0x00030003u) ^ 0x64026402u, 0x64026402u);
+                else if (p2 == 6) up[6] = h2_sub((y & 0x000C000Cu) ^ 0x5C085C08u, 0x5C085C08u);
+                else if (p2 == 7) up[7] = h2_sub((y & 0x00300030u) ^ 0x54205420u, 0x54205420u);
+                else if (p2 == 9)
+                    put(v & ~1, __builtin_amdgcn_perm(up[1], up[0], LO), __builtin_amdgcn_perm(up[3], up[2], LO),
+                        __builtin_amdgcn_perm(up[5], up[4], LO), __builtin_amdgcn_perm(up[7], up[6], LO));
+                else if (p2 == 11)
+                    put(v | 1, __builtin_amdgcn_perm(up[1], up[0], HI), __builtin_amdgcn_perm(up[3], up[2], HI),
+                        __builtin_amdgcn_perm(up[5], up[4], HI), __builtin_amdgcn_perm(up[7], up[6], HI));
+            }
+        }
+    };
+
+    // ---- fragments -------------------------------------------------------------
+    // Explicit ds_read_b128 with manual lgkmcnt waits: the compiler would otherwise drain every pending LDS-DMA load before
+    // the first LDS read of an iteration and serialise load and compute.
+    const int q4 = lane >> 4, l15 = lane & 15;
+    uint32_t va[2], vw[2];                                  // of k-step 0 and 1 in the current stage
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        const uint32_t xo = (uint32_t)(((4 * ks + q4) ^ ((lane >> 1) & 7)) << 4);
+        va[ks] = lds0 + (uint32_t)((wm * (BM / 2) + l15) * 128) + xo;
+        vw[ks] = lds0 + W_AT + (uint32_t)((wn * 128 + l15) * 128) + xo;
+    }
+    u32x4 alo[4], ahi[4], blo[4], bhi[4];
+    auto pin = [&](u32x4 (&d)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(d[i]));
+    };
+    // sixteen products: row tiles AI .. AI + 3, column tiles BJ .. BJ + 3, hook(s) behind product s.  The weights are the
+    // first operand, so that a lane ends with four neighbouring outputs of one sample.
+    auto quad = [&](const u32x4 (&a)[4], const u32x4 (&b)[4], auto ai_c, auto bj_c, auto &&hook) __attribute__((always_inline)) {
+        constexpr int AI = decltype(ai_c)::value, BJ = decltype(bj_c)::value;
+        static_for<16>([&](auto s_c) __attribute__((always_inline)) {
+            constexpr int s = decltype(s_c)::value, i = s >> 2, j = (i & 1) ? 3 - (s & 3) : (s & 3);
+            mfma_acc<F16T, ((AI + i) * 8 + BJ + j) * 4>(b[j], a[i]);
+            hook(s);
+        });
+    };
+    using T0 = std::integral_constant<int, 0>;
+    using T4 = std::integral_constant<int, 4>;
+
+    // ---- prologue ----------------------------------------------------------------
+    const uint32_t bcol = n0 + (uint32_t)t;
+    const float my_bias = bcol < N && !g.ws ? elem_value_rt(g.L.bias_fmt, g.L.bias, bcol) * g.L.bscale : 0.0f;
+    const uint32_t k0 = tail ? kend - tail : kbeg;
+    const bool past = k0 + kchunk >= K && tail;             // this lane's pieces of the partial tile lie past their rows
+#pragma unroll
+    for (int idx = 0; idx < DMA; ++idx) dma(0, k0, past ? kchunk * 2u : 0u, idx);
+    dma_codes(0, k0, true);
+    if (1 < ktiles) dma_codes(CODES, k_of(1), false);
+    // the loads that the tiles before the first would have issued: of tile 1, and with three stages the first ones of tile 2
+    constexpr int AFTER = RM == 8 ? 2 : 1;                  // quads of a tile behind its barrier
+    constexpr int FIRST = AFTER * 4 < DMA ? AFTER * 4 : DMA;  // loads that go out there, four a quad
+    auto early_loads = [&]() __attribute__((always_inline)) {
+        if (1 < ktiles) {
+#pragma unroll
+            for (int idx = 0; idx < (NSTAGE == 2 ? FIRST : DMA); ++idx) dma(STAGE, k_of(1), 0u, idx);
+        }
+        if constexpr (NSTAGE == 3) {
+            if (2 < ktiles) {
+#pragma unroll
+                for (int idx = 0; idx < FIRST; ++idx) dma(2 * STAGE, k_of(2), 0u, idx);
+            }
+        }
+    };
+    // (three stages of packed codes: only behind the codes of tile 2, which the first barrier waits for)
+    constexpr bool EARLY = W_DIRECT || NSTAGE == 2;
+    if constexpr (EARLY) early_loads();
+    static_for<RM * 32>([&](auto r) __attribute__((always_inline)) { acc_zero<decltype(r)::value>(); });
+    if (EARLY && ktiles >= NSTAGE) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NSTAGE == 2 ? FIRST : DMA + FIRST) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (past) {
+#pragma unroll
+        for (int i = 0; i < A_DMA; ++i)
+            *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(smem) + (i * 4 + wave) * 1024 + lane * 16) = make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (W_DIRECT) {
+#pragma unroll
+            for (int i = 0; i < BN / 32; ++i)
+                *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(smem) + W_AT + (i * 4 + wave) * 1024 + lane * 16) = make_uint4(0u, 0u, 0u, 0u);
+        }
+    }
+    if constexpr (!W_DIRECT) {
+        constexpr int LPR = BK / EPL;
+        read_codes(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        pin_codes();
+        if (2 < ktiles) dma_codes(0, k_of(2), false);
+#pragma unroll
+        for (int i = 0; i < W_LOADS; ++i)
+            if (k0 + ((t + 256 * i) % LPR) * EPL >= K) rw[i] = u32x4{0u, 0u, 0u, 0u};        // (code 0 decodes to 0)
+        static_for<64>([&](auto s) __attribute__((always_inline)) { w_step(0, decltype(s)::value); });
+    }
+    if constexpr (!EARLY) early_loads();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+
+    // ---- main loop -----------------------------------------------------------------
+    // Stages as byte offsets: cur (this tile), nxt (the next one), fill (being loaded: NSTAGE - 1 tiles on).
+    uint32_t cur = 0, nxt = STAGE, fill = (NSTAGE - 1) * STAGE;
+    uint32_t code_buf = CODES;                              // the codes of the next tile
+    frag_reads<0, 4>(alo, va[0]);
+    frag_reads<0, 4>(blo, vw[0]);
+    // the tile whose loads are going out, kt + NSTAGE - 1 before a tile's barrier and kt + NSTAGE behind it
+    uint32_t to = lds_w + fill;
+    const char *a_at = a_base + (size_t)k_of(NSTAGE - 1) * 2u, *w_at = w_base + (W_DIRECT ? (size_t)k_of(NSTAGE - 1) * 2u : 0u);
+    // One tile.  KIND 2: there is a tile kt + NSTAGE, whose loads begin behind the barrier, where this tile's stage is free, and
+    // are finished in the next iteration's first quads; 1: the last loads are finished; 0: none are left.  (A branch around
+    // each load instead: 0.85 against 0.81 ms on 8192 cubed.)
+    auto tile = [&](auto kind_c, uint32_t kt) __attribute__((always_inline)) {
+        constexpr int KIND = decltype(kind_c)::value;
+        auto finish_loads = [&](int first) __attribute__((always_inline)) {
+            return [&, first](int s) __attribute__((always_inline)) {
+                if (KIND >= 1 && s % 4 == 3 && first + s / 4 < DMA) dma_at(to, a_at, w_at, 0u, first + s / 4);
+            };
+        };
+        auto begin_loads = [&](int first) __attribute__((always_inline)) {
+            return [&, first](int s) __attribute__((always_inline)) {
+                if (KIND == 2 && s % 4 == 3 && first + s / 4 < FIRST) dma_at(to, a_at, w_at, 0u, first + s / 4);
+            };
+        };
+        auto unpack = [&](int first) __attribute__((always_inline)) {
+            return [&, first](int s) __attribute__((always_inline)) {
+                if constexpr (!W_DIRECT && (KIND >= 1 || NSTAGE == 3)) {       // (else there is no next tile)
+                    w_step(nxt, first + s);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+        };
+        auto swap_stage = [&]() __attribute__((always_inline)) {
+            // this wave's share of the next tile has landed, its fragments of this one are in registers ...
+            if constexpr (NSTAGE == 3 && KIND >= 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(DMA) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();                   // ... and everybody's
+            asm volatile("" ::: "memory");
+            if constexpr (KIND == 2) {
+                if constexpr (!W_DIRECT) dma_codes(code_buf, NSTAGE == 3 || kt + 3 < ktiles ? k_of(kt + 3) : 0u, false);
+                to = lds_w + cur;
+                a_at = a_base + (size_t)k_of(kt + NSTAGE) * 2u;
+                if constexpr (W_DIRECT) w_at = w_base + (size_t)k_of(kt + NSTAGE) * 2u;
+            }
+            code_buf ^= (uint32_t)CODES;
+            const uint32_t step = nxt - cur;                // (wraps around)
+            va[0] += step; va[1] += step; vw[0] += step; vw[1] += step;
+        };
+        if constexpr (RM == 8) {
+            frag_reads<8192, 4>(bhi, vw[0]);
+            asm volatile("s_waitcnt lgkmcnt(4)");
+            pin(alo); pin(blo);
+            quad(alo, blo, T0{}, T0{}, finish_loads(FIRST));
+            frag_reads<8192, 4>(ahi, va[0]);
+            read_codes(code_buf);
+            asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(4 + CREADS));
+            pin(bhi);
+            quad(alo, bhi, T0{}, T4{}, finish_loads(FIRST + 4));
+            frag_reads<0, 4>(alo, va[1]);
+            asm volatile("s_waitcnt lgkmcnt(4)");
+            pin(ahi);
+            pin_codes();
+            quad(ahi, bhi, T4{}, T4{}, unpack(0));
+            frag_reads<8192, 4>(bhi, vw[1]);
+            asm volatile("s_waitcnt lgkmcnt(4)");
+            pin(alo);
+            quad(ahi, blo, T4{}, T0{}, unpack(16));
+            frag_reads<0, 4>(blo, vw[1]);
+            asm volatile("s_waitcnt lgkmcnt(4)");
+            pin(bhi);
+            quad(alo, bhi, T0{}, T4{}, unpack(32));
+            frag_reads<8192, 4>(ahi, va[1]);
+            asm volatile("s_waitcnt lgkmcnt(4)");
+            pin(blo);
+            quad(alo, blo, T0{}, T0{}, unpack(48));
+            swap_stage();
+            pin(ahi);
+            frag_reads<0, 4>(alo, va[0]);
+            quad(ahi, blo, T4{}, T0{}, begin_loads(0));
+            frag_reads<0, 4>(blo, vw[0]);
+            quad(ahi, bhi, T4{}, T4{}, begin_loads(4));
+        } else {
+            // (alo: k-step 0, ahi: k-step 1)
+            frag_reads<8192, 4>(bhi, vw[0]);
+            read_codes(code_buf);
+            asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(4 + CREADS));
+            pin(alo); pin(blo);
+            quad(alo, blo, T0{}, T0{}, finish_loads(FIRST));
+            frag_reads<0, 4>(ahi, va[1]);
+            frag_reads<0, 4>(blo, vw[1]);
+            asm volatile("s_waitcnt lgkmcnt(8)");
+            pin(bhi);
+            pin_codes();
+            quad(alo, bhi, T0{}, T4{}, [&](int s) __attribute__((always_inline)) {
+                finish_loads(FIRST + 4)(s);
+                unpack(0)(2 * s);
+                unpack(1)(2 * s);
+            });
+            frag_reads<8192, 4>(bhi, vw[1]);
+            asm volatile("s_waitcnt lgkmcnt(4)");
+            pin(ahi); pin(blo);
+            quad(ahi, blo, T0{}, T0{}, [&](int s) __attribute__((always_inline)) {
+                unpack(32)(2 * s);
+                unpack(33)(2 * s);
+            });
+            swap_stage();
+            pin(bhi);
+            frag_reads<0, 4>(alo, va[0]);
+            frag_reads<0, 4>(blo, vw[0]);
+            quad(ahi, bhi, T0{}, T4{}, begin_loads(0));
+        }
+        if constexpr (NSTAGE == 2) {
+            const uint32_t was = cur;
+            cur = nxt;
+            nxt = fill = was;
+        } else {
+            const uint32_t was = cur;
+            cur = nxt;
+            nxt = fill;
+            fill = was;
+        }
+    };
+    uint32_t kt = 0;
+    for (; kt + NSTAGE < ktiles; ++kt) tile(std::integral_constant<int, 2>{}, kt);
+    if (kt + NSTAGE - 1 < ktiles) tile(std::integral_constant<int, 1>{}, kt++);
+    for (; kt < ktiles; ++kt) tile(std::integral_constant<int, 0>{}, kt);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");      // the last fragments asked for; the last products
+    pin(alo); pin(blo);
     __syncthreads();
-    for (uint32_t kt = 0; kt < ktiles; kt += 2) {
-        stage(std::integral_constant<int, 0>{}, kt + 1 < ktiles, kbeg + (kt + 1) * BK - kshift);
-        if (kt + 1 < ktiles) stage(std::integral_constant<int, 1>{}, kt + 2 < ktiles, kbeg + (kt + 2) * BK - kshift);
-    }
-    // partial sums of a K split whose rows are not whole 16-byte units: one element per lane and store
-    if (g.ws && (N % 4u != 0 || (reinterpret_cast<uintptr_t>(g.ws) & 15u) != 0)) {
+
+    // ---- epilogue ------------------------------------------------------------------
+    // Lane (l15, q4) holds outputs 4 q4 .. 4 q4 + 3 of each column tile for sample l15 of each row tile.
+    const uint32_t mrow = m0 + wm * (BM / 2), ncol = n0 + wn * 128;
+    float *const bias_lds = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + 4 * 16 * (128 * 4 + 16));
+    bias_lds[t] = my_bias;
+    __syncthreads();
+    float4 bias[8];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const uint32_t col = n0 + (wn * TN + j) * 32 + (lane & 31);
-            if (col >= N) continue;
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t row = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    if (row < M) g.ws[((size_t)blockIdx.y * M + row) * N + col] = acc[i][j][r];
-                }
-        }
-        return;
-    }
+    for (int j = 0; j < 8; ++j) bias[j] = *reinterpret_cast<const float4 *>(bias_lds + wn * 128 + j * 16 + 4 * q4);
     const float wscale = g.L.wscale;
-    // Output rows that are whole 16-byte units: a wave turns its 32 x (32 TN) block of each row tile around in LDS
-    // (the stages are free after the loop's last barrier; every wave has a region of its own, so no barrier is
-    // needed) and writes whole rows of the block, 16 bytes per lane, instead of one element per lane.
-    // The partial sums of a K split go the same way into the workspace, unscaled, as FP32.
-    const uint32_t esz = g.out_f32 ? 4u : 2u;
-    if (g.ws || (((size_t)N * esz) % 16u == 0 && (reinterpret_cast<uintptr_t>(g.C) & 15u) == 0)) {
-        constexpr int BW = 32 * TN;                                  // columns of a wave's block
-        float bias[TN];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const uint32_t col = n0 + (wn * TN + j) * 32 + (lane & 31);
-            bias[j] = (col < N && !g.ws) ? elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale : 0.0f;
-        }
-        char *const out = g.ws ? reinterpret_cast<char *>(g.ws + (size_t)blockIdx.y * M * N) : reinterpret_cast<char *>(g.C);
-        // Every activation has its own copy of the loops (with_act).  Sigmoid and tanh are kept out of the unrolled ones
-        // over a lane's 16 TM TN outputs, where their code takes longer to fetch than to run: the sums wait in LDS as
-        // FP32, and the loop that reads them back and stores whole rows, not unrolled, applies the activation to the few
-        // outputs a lane holds there (4567 x 8192 x 256 FP16 with tanh 103 -> 85 us, 8192 x 8192 x 2048 354 -> 324).
-        // The lambda is forced inline: called, it would take the accumulators through memory.
-        // Long K: the outputs bypass the caches' usual retention (they would displace the A and W panels the other
-        // tiles of the die are re-reading: 8192 cubed 0.908 against 0.934 ms); short K: the next layer reads them
-        // back soon and they are most of the traffic (8192 x 8192 x 1024: 0.162 against 0.175 ms the other way round).
-        const bool stream_out = K >= 2048u && !g.ws;
-        auto turn = [&](auto es_c, auto act_c) __attribute__((always_inline)) {
-            constexpr int ES = decltype(es_c)::value;
-            constexpr int ACT = decltype(act_c)::value;              // A_COUNT: partial sums
-            constexpr bool SLOW = ACT == A_SIGMOID || ACT == A_TANH;
-            constexpr int SS = SLOW ? 4 : ES;                   // bytes of an element while it waits in LDS
-            constexpr int PITCH = BW * SS + 16;                      // lanes 0-31 and 32-63 (four rows apart) on different banks
-            constexpr int LPR = BW * ES / 16;                        // lanes that write one row
-            constexpr int RPP = 64 / LPR;                            // rows per store instruction
-            char *mine = reinterpret_cast<char *>(smem) + wave * (32 * PITCH);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int rl = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        const float pre = ACT == A_COUNT ? acc[i][j][r] : fmaf(acc[i][j][r], wscale, bias[j]);
-                        const float v = SLOW ? pre : apply_act(pre, ACT);
-                        char *dst = mine + rl * PITCH + (j * 32 + (lane & 31)) * SS;
-                        if constexpr (SS == 4) *reinterpret_cast<float *>(dst) = v;
-                        else *reinterpret_cast<uint16_t *>(dst) = f32_to_t16<F16T>(v);
-                    }
-                // padded neurons (layer_sum; a select behind every output costs all tiles more)
-                if (ACT != A_COUNT && g.L.pad != 0u) {
+    const uint32_t pad = g.L.pad;
+    // A wave turns the 16 x 128 block of each row tile around in LDS (the stages are free after the loop; every wave has a
+    // region of its own, so no barrier is needed) and writes whole rows of the block, 16 bytes per lane (rows that are not
+    // whole 16-byte units: element by element).  The partial sums of a K split go the same way into the workspace, unscaled,
+    // as FP32.
+    const bool f32_out = g.ws || g.out_f32;
+    char *const out = g.ws ? reinterpret_cast<char *>(g.ws + (size_t)blockIdx.y * M * N) : reinterpret_cast<char *>(g.C);
+    const bool rows16 = ((size_t)N * (f32_out ? 4u : 2u)) % 16u == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+    // Long K: the outputs bypass the caches' usual retention (they would displace the A and W panels the other
+    // tiles of the die are re-reading: 8192 cubed 0.908 against 0.934 ms); short K: the next layer reads them
+    // back soon and they are most of the traffic (8192 x 8192 x 1024: 0.162 against 0.175 ms the other way round).
+    const bool stream_out = K >= 2048u && !g.ws;
+    char *const mine = reinterpret_cast<char *>(smem) + wave * (16 * (128 * 4 + 16));
+    // Activations: one uniform branch per row tile to a copy of the code over a lane's 32 outputs.  Sigmoid and tanh are kept
+    // out of that unrolled code, where theirs takes longer to fetch than to run: the sums wait in LDS as FP32, and the
+    // loop that reads them back and stores whole rows, not unrolled, applies them (4567 x 8192 x 256 FP16 with tanh 103 -> 85
+    // us, 8192 x 8192 x 2048 354 -> 324).  The same loop converts FP16 blocks with outputs that saturate, infinities or NaNs,
+    // which the packed conversion does not know, and stores rows that are not whole 16-byte units.
+    const bool late = !g.ws && (g.L.act == A_SIGMOID || g.L.act == A_TANH);
+    // (the lambdas are forced inline: called, they would take what they capture through memory)
+    auto turn = [&](auto es_c) __attribute__((always_inline)) {
+        constexpr int ES = decltype(es_c)::value;                    // bytes of an element of the output
+        constexpr int EPS = 16 / ES;                                 // elements of a 16-byte store
+        constexpr int LPR = 128 / EPS, RPP = 64 / LPR;               // lanes that write one row, rows per store instruction
+        const int rl0 = lane / LPR, c0 = lane % LPR * EPS;
+        auto store = [&](int i, int p, u32x4 vv) __attribute__((always_inline)) {
+            const uint32_t row = mrow + i * 16 + p * RPP + rl0, col = ncol + c0;
+            if (row >= M || col >= N) return;                        // N is a multiple of EPS: a unit is all in or all out
+            u32x4 *dstp = reinterpret_cast<u32x4 *>(out + ((size_t)row * N + col) * ES);
+            if (stream_out) __builtin_nontemporal_store(vv, dstp);
+            else *dstp = vv;
+        };
+        constexpr int PUTS = 16 / RPP;
+        u32x4 held[PUTS];                                            // rows on their way from LDS to memory
+        bool pending = false;
+        // row tile i from LDS, where it waits as FP32
+        auto finish_rows = [&](int i) __attribute__((always_inline)) {
 #pragma unroll 1
-                    for (int j = 0; j < TN; ++j) {
-                        if (n0 + (wn * TN + j) * 32 + (lane & 31) + g.L.pad < N) continue;
+            for (int p = 0; p < 16 / RPP; ++p) {
+                float e[EPS];
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            char *dst = mine + (8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * PITCH + (j * 32 + (lane & 31)) * SS;
-                            if constexpr (SS == 4) *reinterpret_cast<float *>(dst) = 0.0f;
-                            else *reinterpret_cast<uint16_t *>(dst) = 0;
-                        }
+                for (int x = 0; x < EPS; x += 4) {
+                    const float4 f = *reinterpret_cast<const float4 *>(mine + (p * RPP + rl0) * (128 * 4 + 16) + (c0 + x) * 4);
+                    e[x] = f.x; e[x + 1] = f.y; e[x + 2] = f.z; e[x + 3] = f.w;
+                }
+                if (late) {
+#pragma unroll
+                    for (int x = 0; x < EPS; ++x) {
+                        e[x] = g.L.act == A_TANH ? apply_act(e[x], A_TANH) : apply_act(e[x], A_SIGMOID);
+                        if (ncol + c0 + x + pad >= N) e[x] = 0.0f;       // padded neurons (layer_sum)
                     }
                 }
-                auto put = [&](int p) {
-                    const int rl = p * RPP + lane / LPR, seg = lane % LPR;
-                    const char *src = mine + rl * PITCH + seg * (16 / ES) * SS;
+                if (rows16) {
                     u32x4 vv;
-                    if constexpr (SLOW) {
-                        float e[16 / ES];
 #pragma unroll
-                        for (int x = 0; x < 16 / ES; ++x) e[x] = apply_act(reinterpret_cast<const float *>(src)[x], ACT);
-#pragma unroll
-                        for (int x = 0; x < 4; ++x) {
-                            if constexpr (ES == 4) vv[x] = __float_as_uint(e[x]);
-                            else vv[x] = (uint32_t)f32_to_t16<F16T>(e[2 * x]) | (uint32_t)f32_to_t16<F16T>(e[2 * x + 1]) << 16;
-                        }
-                    } else {
-                        const uint4 v = *reinterpret_cast<const uint4 *>(src);
-                        vv = u32x4{v.x, v.y, v.z, v.w};
+                    for (int x = 0; x < 4; ++x) {
+                        if constexpr (ES == 4) vv[x] = __float_as_uint(e[x]);
+                        else vv[x] = (uint32_t)f32_to_t16<F16T>(e[2 * x]) | (uint32_t)f32_to_t16<F16T>(e[2 * x + 1]) << 16;
                     }
-                    const uint32_t row = m0 + (wm * TM + i) * 32 + rl;
-                    const uint32_t col = n0 + wn * BW + seg * (16 / ES);
-                    if (row < M && col < N) {                        // N is a multiple of 16 / ES: a unit is all in or all out
-                        u32x4 *dstp = reinterpret_cast<u32x4 *>(out + ((size_t)row * N + col) * ES);
-                        if (stream_out) __builtin_nontemporal_store(vv, dstp);
-                        else *dstp = vv;
-                    }
-                };
-                if constexpr (SLOW) {
-#pragma unroll 1
-                    for (int p = 0; p < 32 / RPP; ++p) put(p);
+                    store(i, p, vv);
                 } else {
+                    const uint32_t row = mrow + i * 16 + p * RPP + rl0;
 #pragma unroll
-                    for (int p = 0; p < 32 / RPP; ++p) put(p);
+                    for (int x = 0; x < EPS; ++x) {
+                        const uint32_t col = ncol + c0 + x;
+                        if (row >= M || col >= N) continue;
+                        const size_t o = (size_t)row * N + col;
+                        if constexpr (ES == 4) reinterpret_cast<float *>(out)[o] = e[x];
+                        else reinterpret_cast<uint16_t *>(out)[o] = f32_to_t16<F16T>(e[x]);
+                    }
                 }
             }
         };
-        using E4 = std::integral_constant<int, 4>;
-        using E2 = std::integral_constant<int, 2>;
-        if (g.ws) turn(E4{}, std::integral_constant<int, A_COUNT>{});
-        else if (g.out_f32) with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E4{}, act_c); });
-        else with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) { turn(E2{}, act_c); });
-        return;
-    }
-    with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) {
+        static_for<RM>([&](auto i_c) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_c)::value;
+            float v[32];
+            static_for<32>([&](auto e_c) __attribute__((always_inline)) {
+                constexpr int e = decltype(e_c)::value;
+                v[e] = acc_read<i * 32 + e>();
+            });
+            if (!g.ws) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const uint32_t col = n0 + (wn * TN + j) * 32 + (lane & 31);
-            if (col >= N) continue;
-            const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col) * g.L.bscale;
+                for (int e = 0; e < 32; ++e) {
+                    const float4 b = bias[e >> 2];
+                    v[e] = fmaf(v[e], wscale, (e & 3) == 0 ? b.x : (e & 3) == 1 ? b.y : (e & 3) == 2 ? b.z : b.w);
+                }
+                auto each = [&](auto act_c) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {
+                    for (int e = 0; e < 32; ++e) v[e] = decltype(act_c)::value == A_LEAKY ? fmaxf(v[e], 0.01f * v[e]) : apply_act(v[e], decltype(act_c)::value);
+                };
+                if (g.L.act == A_RELU) each(std::integral_constant<int, A_RELU>{});
+                else if (g.L.act == A_LEAKY) each(std::integral_constant<int, A_LEAKY>{});
+                else if (g.L.act == A_FOO52) each(std::integral_constant<int, A_FOO52>{});
+                // padded neurons (only hidden layers of this path have any)
+                if (!late && pad != 0u && ncol + 128u + pad > N) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const uint32_t row = m0 + (wm * TM + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    if (row >= M) continue;
-                    const float v = apply_act(fmaf(acc[i][j][r], wscale, bias), decltype(act_c)::value);
-                    const size_t o = (size_t)row * N + col;
-                    if (g.out_f32) reinterpret_cast<float *>(g.C)[o] = v;
-                    else reinterpret_cast<uint16_t *>(g.C)[o] = f32_to_t16<F16T>(v);
+                    for (int e = 0; e < 32; ++e)
+                        if (ncol + (e >> 2) * 16 + 4 * q4 + (e & 3) + pad >= N) v[e] = 0.0f;
                 }
             }
+            bool plain = rows16 && !late;
+            if constexpr (ES == 2 && F16T) {
+                float top = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 32; ++e) top = __builtin_elementwise_maximum(top, __builtin_fabsf(v[e]));
+                plain = plain && __all(top < 65520.0f);
+            }
+            // the row tile before this one, whose rows were asked for back from LDS before this one's arithmetic
+            if (pending) {
+#pragma unroll
+                for (int p = 0; p < PUTS; ++p) store(i - 1, p, held[p]);
+            }
+            pending = plain;
+            if (ES == 2 && plain) {
+                constexpr int PITCH = 128 * 2 + 16;                  // rows on different banks
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    uint2 d;
+                    if constexpr (F16T) {
+                        d = make_uint2(pack_f16_small(v[4 * j], v[4 * j + 1]), pack_f16_small(v[4 * j + 2], v[4 * j + 3]));
+                    } else {
+                        d = make_uint2((uint32_t)f32_to_t16<false>(v[4 * j]) | (uint32_t)f32_to_t16<false>(v[4 * j + 1]) << 16,
+                                       (uint32_t)f32_to_t16<false>(v[4 * j + 2]) | (uint32_t)f32_to_t16<false>(v[4 * j + 3]) << 16);
+                    }
+                    *reinterpret_cast<uint2 *>(mine + l15 * PITCH + j * 32 + q4 * 8) = d;
+                }
+            } else {
+                constexpr int PITCH = 128 * 4 + 16;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    *reinterpret_cast<float4 *>(mine + l15 * PITCH + j * 64 + q4 * 16) = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (plain) {
+#pragma unroll
+                for (int p = 0; p < PUTS; ++p) {
+                    const uint4 w = *reinterpret_cast<const uint4 *>(mine + (p * RPP + rl0) * (128 * ES + 16) + c0 * ES);
+                    held[p] = u32x4{w.x, w.y, w.z, w.w};
+                }
+            } else {
+                finish_rows(i);
+            }
+            __builtin_amdgcn_wave_barrier();
+        });
+        if (pending) {
+#pragma unroll
+            for (int p = 0; p < PUTS; ++p) store(RM - 1, p, held[p]);
         }
-    });
+    };
+    if (f32_out) turn(std::integral_constant<int, 4>{});
+    else turn(std::integral_constant<int, 2>{});
 }
 
 // adds the partial sums of a split launch (K splits in split order; with split activations the sums of the second

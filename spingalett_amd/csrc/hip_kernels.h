@@ -123,9 +123,8 @@ __device__ __forceinline__ float act_derivative(float a, int act)
 }
 
 // f(integral_constant<int, ACT>): a copy of an epilogue for each activation.  Behind every output of a lane, in an unrolled
-// loop, a switch over the activations is a chain of branches and code fetched for nothing (sp_gemm16_big's 128 outputs:
-// 100 KB of it where two of the six have a transcendental function, branches alone where none has: one FP16 layer with a
-// leaky ReLU 4567 x 8192 x 256 66 -> 56 us, 8192 x 8192 x 1024 180 -> 174).
+// loop, a switch over the activations is a chain of branches and code fetched for nothing (FP32 layers 4096 x 512 x 784 with
+// tanh 36.9 -> 35.5 us, 2048 x 1000 x 512 with a leaky ReLU 25.8 -> 24.3).
 template <class F>
 __device__ __forceinline__ void with_act(int act, F &&f)
 {

@@ -144,14 +144,6 @@ __device__ __forceinline__ void skinny_emit(const SkinnyArgs &a, uint32_t c, uin
     skinny_emit_biased<F16T>(a, c, r, accv, bias);
 }
 
-// 16 bytes per lane from scalar base + 32-bit lane offset + immediate.  Inline assembly: the compiler's
-// wait-count bookkeeping does not see the load, the caller waits with s_waitcnt vmcnt before using dst.
-template <int OFF>
-__device__ __forceinline__ void load16_async(u32x4 &dst, uint32_t voff, const void *sbase)
-{
-    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(dst) : "v"(voff), "s"(sbase), "n"(OFF) : "memory");
-}
-
 template <int FMT, bool F16T, int RT, int CT, int NWV>
 __global__ __launch_bounds__(64 * NWV) void sp_skinny16(const SkinnyArgs a)
 {

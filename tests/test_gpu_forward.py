@@ -563,6 +563,56 @@ def test_short_layers_of_uneven_rounds_of_large_tiles(S, O, fmt, K, N, act, head
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_MFMA
 
 
+@pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
+@pytest.mark.parametrize("n,K,N", [
+    (4096, 128, 4096), (4095, 144, 4088), (3841, 192, 4096),    # two and three K tiles, whole and in part: prologue and drain only
+    (4090, 320, 4086),                                           # rows of FP32 outputs that are not whole 16-byte units
+    (100, 4224, 1023), (100, 3200, 1536),                        # 128-row tiles, K splits of which the last is short
+])
+def test_large_tiles_at_the_edges_of_their_pipeline(S, O, fmt, n, K, N):
+    """sp_gemm16_big where its loop is hardly entered, behind partial K tiles and on both tile heights, FP32 outputs, against
+    the float64 forward.  (FP16 inputs: 2^-11 of each, at random over K terms.)"""
+    src = make_oracle_net(O, [K, N], ["none"], seed=n + K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    h = S.lib().spingalett_hip_handle(net)
+    name = S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode()
+    assert name == "sp_gemm16_big" or n == 100 or (fmt, K) in (("i4", 144), ("i2", 144)), name       # (rows that are not whole units)
+    X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    S.free_network(net)
+    assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 2e-3
+
+
+def test_large_tiles_saturate_and_keep_infinities_block_by_block(S):
+    """FP16 outputs of sp_gemm16_big: finite sums beyond +-65504 saturate, infinities and NaNs stay and only their own
+    samples have them, in row tiles that hold ordinary samples too."""
+    n, K, N = 4605, 144, 4112
+    rng = np.random.default_rng(5)
+    W = (rng.standard_normal((N, K)) * 0.1).astype(np.float16)
+    W[:, 3] = 1.0
+    V = np.zeros((8, N), np.float16)
+    V[np.arange(8), np.arange(8) * 513] = 1.0                    # each output of the net is one neuron of the large layer
+    X = rng.standard_normal((n, K)).astype(F32)
+    X[17, 3], X[4600, 3] = 65504.0, -65504.0
+    X[17, 4:] *= 3000.0                                          # sums on both sides of 65504
+    X[33, 3], X[1000, 3], X[4604, 7] = np.inf, -np.inf, np.nan
+    d = S.DeviceNet([K, N, 8], [S.ACT_NONE, S.ACT_NONE], S.PRECISION_FP16)
+    for l, a in ((0, W), (1, V)):
+        d.upload(l, 0, a.ravel().view(np.uint8))
+        d.upload(l, 1, np.zeros(a.shape[0], np.float16).view(np.uint8))
+    assert S.lib().sphip_layer_kernel_name(d.h, 1, n, 0).decode() == "sp_gemm16_big"
+    got = d.forward(X)
+    d.destroy()
+    odd = [33, 1000, 4604]
+    assert not np.isfinite(got[odd]).any()                       # (0 x inf in the second layer)
+    keep = np.setdiff1d(np.arange(n), odd)
+    sums = X[keep].astype(np.float16).astype(np.float64) @ W[::513][:8].astype(np.float64).T
+    want = np.clip(sums, -65504.0, 65504.0)
+    # one rounding to FP16, and FP32 sums of 144 terms of up to 65504 before it
+    assert np.all(np.abs(got[keep] - want) <= 2.0 ** -11 * np.abs(want) + 1e-5 * np.abs(X[keep]).max(axis=1, keepdims=True))
+    assert 0 < np.sum(got[17] == 65504.0) < 8
+
+
 @pytest.mark.parametrize("n,K,N", [
     (4095, 520, 1000),     # 256 tiles of 128 x 128: rows of 64, a last tile of each kind in part, K 8 beyond its tiles
     (8321, 268, 897),      # rows of 128, no split
