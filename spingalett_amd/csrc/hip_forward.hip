@@ -1018,7 +1018,9 @@ struct ThinPlan {
     int nw;                // waves per workgroup in that case (4 or 8)
     uint32_t R, NC;        // streamed rows, thin rows
     int rt, ct;
-    int nwv;               // waves per workgroup of sp_skinny16
+    int nwv;               // waves per workgroup of sp_skinny16_regs
+    bool regs;             // sp_skinny16_regs instead of sp_skinny16
+    int st;                // sixteens of samples per workgroup of sp_skinny16
     uint32_t splits, kper, row_blocks, cblocks;
 };
 
@@ -1032,8 +1034,36 @@ struct ThinPlan {
 // against 57 us at 256 samples).
 uint32_t thin_max_samples(int fmt, uint32_t N, uint32_t K)
 {
+    if (K <= 1024u) return 64u;
     if ((uint64_t)N * K * (uint64_t)fmt_bits(fmt) / 8u <= (8ull << 20)) return 256u;
     return fmt_bits(fmt) == 16 ? 64u : fmt == I8 ? 128u : 256u;
+}
+
+// codes of K in a chunk of sp_skinny16 (ThinFmt)
+uint32_t thin_chunk(int fmt) { return fmt == I4 || fmt == I2 ? ThinFmt<I4>::BK : ThinFmt<I8>::BK; }
+static_assert(ThinFmt<I2>::BK == ThinFmt<I4>::BK && ThinFmt<F16>::BK == ThinFmt<I8>::BK && ThinFmt<BF16>::BK == ThinFmt<I8>::BK, "thin_chunk");
+
+// K splits of sp_skinny16: what costs least by the times measured for it (us): a chunk on st sixteens of samples, or its weights
+// at the rate at which the chip reads them; the start and end of a workgroup, of which a compute unit holds one; the second
+// launch that adds the parts.
+uint32_t thin_splits(int fmt, int st, uint32_t wgs, uint32_t chunks, uint64_t outputs)
+{
+    const bool narrow = fmt == I2 || fmt == I4;
+    const float products = narrow ? 0.55f + 0.20f * st : 0.35f + 0.11f * st;
+    const float bytes = 16.0f * (float)thin_chunk(fmt) * (float)fmt_bits(fmt);           // 128 rows of a chunk
+    uint32_t best = 1;
+    float least = 0.0f;
+    for (uint32_t s = 1; s <= 16u && (s == 1u || 2u * s <= chunks); ++s) {
+        const float at_once = wgs * s < 256u ? (float)(wgs * s) : 256.0f;
+        const float chunk = fmaxf(products, at_once * bytes / 5.5e6f);
+        const float t = (float)((wgs * s + 255u) / 256u) * ((float)((chunks + s - 1) / s) * chunk + 3.5f) +
+                        (s > 1u ? 3.2f + (float)s * (float)outputs * 1e-6f : 0.0f);
+        if (s == 1u || t < least) {
+            best = s;
+            least = t;
+        }
+    }
+    return best;
 }
 
 // mode_b streams 16-bit activations (fmt = the activation type), mode a the weights
@@ -1088,6 +1118,23 @@ ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K)
         p.splits = (chunks + cps - 1) / cps;
         return p;
     }
+    // sp_skinny16: workgroups of 128 rows by up to 64 samples.  More of them than compute units with several blocks of samples
+    // would read the samples' chunks from L2 twice as often as the 256 rows of sp_skinny16_regs do (INT2 at 256 samples:
+    // 16384 x 2048 35 against 27 us, 16384 x 8192 84 against 70; at 100 samples 16384 x 8192 48.5 against 45.7, but x 4096 29.6
+    // against 31.8; from 8192 rows down never).
+    const uint32_t blocks = (p.R + 127u) / 128u * ((p.NC + 63u) / 64u);
+    p.regs = p.mode_b || ((fmt == I4 || fmt == I2) && p.NC > 64u && (blocks > 256u || (blocks == 256u && K >= 8192u)));
+    if (!p.regs) {
+        p.cblocks = (p.NC + 63u) / 64u;
+        p.st = (int)(((p.NC + p.cblocks - 1u) / p.cblocks + 15u) / 16u);
+        p.row_blocks = (p.R + 127u) / 128u;
+        const uint32_t bk = thin_chunk(fmt), chunks = (K + bk - 1) / bk;
+        p.splits = thin_splits(fmt, p.st, p.row_blocks * p.cblocks, chunks, (uint64_t)p.NC * p.R);
+        const uint32_t cps = (chunks + p.splits - 1) / p.splits;
+        p.kper = cps * bk;
+        p.splits = (chunks + cps - 1) / cps;
+        return p;
+    }
     p.ct = p.NC <= 32 ? 1 : 2;
     p.cblocks = (p.NC + 32u * p.ct - 1) / (32u * p.ct);
     // Waves per workgroup, and the number of workgroups the K split aims at.  Every workgroup fetches the thin block
@@ -1118,11 +1165,23 @@ void launch_thin_inst(const SkinnyArgs &a, const ThinPlan &p)
 {
     if (tl_route.dry) return;
     constexpr size_t lds = 2 * 32 * CT * SkinnyFmt<SFMT>::PITCH;
-    auto kern = sp_skinny16<SFMT, F16T, RT, CT, NWV>;
+    auto kern = sp_skinny16_regs<SFMT, F16T, RT, CT, NWV>;
     static bool once = ((void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
     (void)once;
     const uint32_t gx = p.cblocks > 1 ? (p.row_blocks + 7u) / 8u * 8u * p.cblocks : p.row_blocks;
     kern<<<dim3(gx, p.splits * a.halves, 1), 64 * NWV, lds, g_stream>>>(a);
+}
+
+template <int FMT, bool F16T, int ST>
+void launch_thin_dma(const SkinnyArgs &a, const ThinPlan &p)
+{
+    if (tl_route.dry) return;
+    constexpr size_t lds = ThinFmt<FMT>::template Tile<ST>::LDS;
+    auto kern = sp_skinny16<FMT, F16T, ST>;
+    static bool once = ((void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
+    (void)once;
+    const uint32_t gx = p.cblocks > 1 ? (p.row_blocks + 7u) / 8u * 8u * p.cblocks : p.row_blocks;
+    kern<<<dim3(gx, p.splits * a.halves, 1), 512, lds, g_stream>>>(a);
 }
 
 template <int SFMT, bool F16T, int NCP, int NW>
@@ -1155,10 +1214,19 @@ void launch_thin(SkinnyArgs a, const ThinPlan &p)
         } else {
             launch_thin_kw<SFMT, F16T, 8, 4>(a, p);
         }
-    } else if (p.nwv == 8) {
-        if (p.ct == 2) launch_thin_inst<SFMT, F16T, 1, 2, 8>(a, p); else launch_thin_inst<SFMT, F16T, 1, 1, 8>(a, p);
-    } else {
-        if (p.ct == 2) launch_thin_inst<SFMT, F16T, 1, 2>(a, p); else launch_thin_inst<SFMT, F16T, 1, 1>(a, p);
+    } else if (!p.regs) {
+        if (p.st == 1) launch_thin_dma<SFMT, F16T, 1>(a, p);
+        else if (p.st == 2) launch_thin_dma<SFMT, F16T, 2>(a, p);
+        else if (p.st == 3) launch_thin_dma<SFMT, F16T, 3>(a, p);
+        else launch_thin_dma<SFMT, F16T, 4>(a, p);
+    } else if constexpr (SFMT == I4 || SFMT == I2) {
+        launch_thin_inst<SFMT, F16T, 1, 2, 8>(a, p);
+    } else if constexpr (SFMT == F16 || SFMT == BF16) {
+        if (p.nwv == 8) {
+            if (p.ct == 2) launch_thin_inst<SFMT, F16T, 1, 2, 8>(a, p); else launch_thin_inst<SFMT, F16T, 1, 1, 8>(a, p);
+        } else {
+            if (p.ct == 2) launch_thin_inst<SFMT, F16T, 1, 2>(a, p); else launch_thin_inst<SFMT, F16T, 1, 1>(a, p);
+        }
     }
     if (a.ws && !tl_route.dry) {
         const uint64_t total = (uint64_t)a.NC * a.R;
@@ -1214,7 +1282,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         SkinnyArgs a{};
         a.halves = halves; a.half_elems = (uint64_t)M * L.K;
         a.L = L; a.C = C; a.ws = ctx.ws; a.R = tp.R; a.NC = tp.NC; a.row_blocks = tp.row_blocks; a.cblocks = tp.cblocks; a.kper = tp.kper; a.out_f32 = out_f32; a.mode_b = tp.mode_b ? 1 : 0;
-        tl_route.name = tp.kw ? "sp_skinny16_kw" : "sp_skinny16";
+        tl_route.name = tp.kw ? "sp_skinny16_kw" : tp.regs ? "sp_skinny16_regs" : "sp_skinny16";
         if (tp.mode_b) {
             if (ctx.soft_out && tp.kw && tp.splits == 1 && halves == 1) {
                 a.soft_out = ctx.soft_out;

@@ -8,6 +8,7 @@
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 struct GemmArgs {
     LayerArgs L;
@@ -1231,6 +1232,25 @@ __global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
     else turn(std::integral_constant<int, 2>{});
 }
 
+// The parts of four neighbouring sums, `stride` float4 apart: the first `splits` added in order into sum, the others into low.
+// Four are on their way at a time: one after the other, each is a round trip to memory (four parts of 50 x 8192 sums 4.9 ->
+// RED us, sixteen of 50 x 1000 7.4 -> RED2).
+__device__ __forceinline__ void add_parts(const float4 *at, uint64_t stride, uint32_t splits, uint32_t parts, float4 &sum, float4 &low)
+{
+    sum = low = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (uint32_t p0 = 0; p0 < parts; p0 += 4u) {
+        float4 v[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) v[i] = at[(p0 + i < parts ? p0 + i : p0) * stride];
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+            if (p0 + i >= parts) continue;
+            float4 &to = p0 + i < splits ? sum : low;
+            to.x += v[i].x; to.y += v[i].y; to.z += v[i].z; to.w += v[i].w;
+        }
+    }
+}
+
 // adds the partial sums of a split launch (K splits in split order; with split activations the sums of the second
 // matrix, scaled by 2^-11, after those of the first) and applies scale, bias and activation; a thread takes four
 // neighbouring columns (VEC: N a multiple of four, workspace and C 16-byte aligned) or one.  16-bit outputs of a
@@ -1243,20 +1263,18 @@ __global__ __launch_bounds__(256) void sp_gemm16_reduce(const GemmArgs g, uint32
     if constexpr (VEC) {
         const uint64_t idx = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * 4u;
         if (idx >= total) return;
-        float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f), low = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (uint32_t sp = 0; sp < parts; ++sp) {
-            const float4 v = *reinterpret_cast<const float4 *>(g.ws + (uint64_t)sp * total + idx);
-            if (sp < splits) { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; }
-            else { low.x += v.x; low.y += v.y; low.z += v.z; low.w += v.w; }
-        }
         const uint32_t col = (uint32_t)(idx % g.L.N);
+        float bias[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bias[i] = elem_value_rt(g.L.bias_fmt, g.L.bias, col + i) * g.L.bscale;
+        float4 sum, low;
+        add_parts(reinterpret_cast<const float4 *>(g.ws + idx), total / 4u, splits, parts, sum, low);
         const float in[4] = {fmaf(low.x, kLoScale, sum.x), fmaf(low.y, kLoScale, sum.y), fmaf(low.z, kLoScale, sum.z),
                              fmaf(low.w, kLoScale, sum.w)};
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, col + i) * g.L.bscale;
-            v[i] = apply_act(layer_sum(g.L, in[i], bias, col + i), g.L.act);
+            v[i] = apply_act(layer_sum(g.L, in[i], bias[i], col + i), g.L.act);
         }
         if (g.out_f32) {
             *reinterpret_cast<float4 *>(reinterpret_cast<float *>(g.C) + idx) = make_float4(v[0], v[1], v[2], v[3]);

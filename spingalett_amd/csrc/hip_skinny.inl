@@ -145,7 +145,7 @@ __device__ __forceinline__ void skinny_emit(const SkinnyArgs &a, uint32_t c, uin
 }
 
 template <int FMT, bool F16T, int RT, int CT, int NWV>
-__global__ __launch_bounds__(64 * NWV) void sp_skinny16(const SkinnyArgs a)
+__global__ __launch_bounds__(64 * NWV) void sp_skinny16_regs(const SkinnyArgs a)
 {
     using F = SkinnyFmt<FMT>;
     constexpr int EPL = F::EPL, LPC = F::LPC, BKC = F::BKC, STEPS = F::STEPS, PITCH = F::PITCH;
@@ -395,11 +395,384 @@ __global__ __launch_bounds__(64 * NWV) void sp_skinny16(const SkinnyArgs a)
     with_act(a.L.act, emit);
 }
 
+// ---------------------------------------------------------------------------
+// Layers of 9 .. 256 samples whose weights are streamed: everything through LDS by DMA
+// ---------------------------------------------------------------------------
+// A workgroup of eight waves owns 128 weight rows x 16 ST samples (ST <= 4) x a share of K (grid y), in chunks of BK.  Wave
+// (g, w): rows 32 w .. 32 w + 31, the g-th half of every chunk's k; the halves' sums meet in LDS at the end.
+//
+// The kernel before spent 1.35 us per chunk of 256 INT2 codes on 64 samples (8192 x 8192: 8 chunks a workgroup) where the matrix
+// cores need 0.45: its loads alone take 0.8 (a lane reads 16 bytes of a weight row of its own, so that four lanes touch four
+// lines, and half of each line of the samples at a time), its arithmetic alone 0.95 (unpacking and reordering samples
+// next to the products of one wave per SIMD), and two waves per SIMD with loads like these gain nothing.  Here
+//   * every load is global_load_lds_dwordx4 of whole 64- to 512-byte pieces of rows, NSTAGE - 1 chunks ahead, counted with
+//     vmcnt; one barrier per chunk;
+//   * samples stay in their own order; the codes are put in order as they are unpacked (unpack_word16);
+//   * the two waves of a SIMD work on different halves of the same chunk, so that the second wave costs no loads.
+// MEASURED
+// LDS: a row of a chunk is whole, unpadded, its 16-byte pieces permuted by the row (swz) so that the sixteen rows of a
+// fragment read lie on different banks.  Lane (l15, q4) of a wave takes, of row l15 of a tile, the k-quarter q4 of its half
+// chunk: which k an operation sums does not matter as long as both operands agree.
+template <int FMT>
+struct ThinFmt {
+    static constexpr int bits = fmt_bits(FMT);
+    static constexpr int BK = FMT == I2 || FMT == I4 ? 256 : 128;
+    static constexpr int EPL = 128 / bits;                      // codes of a 16-byte piece
+    static constexpr int TROW = BK * 2, WROW = BK * bits / 8;   // bytes of a chunk's row
+    static constexpr int KQ = BK / 8;                           // k of a lane and chunk: its quarter of its half
+    template <int ST>
+    struct Tile {
+        static constexpr int W_AT = ST * 16 * TROW, STAGE = W_AT + 128 * WROW;
+        static constexpr int NSTAGE = 4 * STAGE <= 160 * 1024 ? 4 : 3;
+        static constexpr int T_DMA = (ST * 16 * TROW / 1024 + 7) / 8, W_DMA = 128 * WROW / 8192;    // load instructions per wave and chunk
+        static constexpr int LDS = NSTAGE * STAGE;
+    };
+};
+
+// Position of piece p in row r of ROW bytes, and the piece at a position.  A row covers ROW / 256 of the banks' 256 bytes: rows
+// that share them get different positions for the same piece, and the lanes of a fragment read that are served together
+// (sixteen of them, rows 4 .. 11 of one k-quarter beside rows 0 .. 3 and 12 .. 15 of the one before) too: their pieces may
+// differ in the lowest two bits of the sixteen positions only, so that of 512-byte rows, where a quarter is four pieces, they
+// trade places with the two above them.
+template <int ROW>
+__device__ __forceinline__ uint32_t thin_mask(uint32_t r)
+{
+    return ROW >= 256 ? r & 15u : ROW == 128 ? (r >> 1) & 7u : (r >> 2) & 3u;
+}
+__device__ __forceinline__ uint32_t thin_trade(uint32_t p) { return (p & ~15u) | (p & 3u) << 2 | ((p >> 2) & 3u); }
+template <int ROW>
+__device__ __forceinline__ uint32_t thin_pos(uint32_t r, uint32_t p) { return (ROW == 512 ? thin_trade(p) : p) ^ thin_mask<ROW>(r); }
+template <int ROW>
+__device__ __forceinline__ uint32_t thin_piece(uint32_t r, uint32_t pos)
+{
+    const uint32_t p = pos ^ thin_mask<ROW>(r);
+    return ROW == 512 ? thin_trade(p) : p;
+}
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+template <int OFF>
+__device__ __forceinline__ void ds_read64(u32x2 &dst, uint32_t addr)
+{
+    asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
+}
+
+template <int FMT, bool F16T, int ST>
+__global__ __launch_bounds__(512) void sp_skinny16(const SkinnyArgs a)
+{
+    using F = ThinFmt<FMT>;
+    using T = typename F::template Tile<ST>;
+    constexpr int BK = F::BK, EPL = F::EPL, TROW = F::TROW, WROW = F::WROW, KQ = F::KQ, bits = F::bits;
+    constexpr int STAGE = T::STAGE, W_AT = T::W_AT, NSTAGE = T::NSTAGE, T_DMA = T::T_DMA, W_DMA = T::W_DMA;
+    constexpr bool W16 = bits == 16;
+    extern __shared__ __attribute__((aligned(16))) uint8_t sk_lds[];
+
+    const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const uint32_t l15 = lane & 15u, q4 = lane >> 4, w = wave & 3u, g = wave >> 2;
+    const uint32_t K = a.L.K;
+    // (row block, sample block) as in sp_skinny16_regs
+    uint32_t rblk = blockIdx.x, cblk = 0;
+    if (a.cblocks > 1) {
+        const uint32_t per = 8u * a.cblocks, group = blockIdx.x / per, rem = blockIdx.x % per;
+        rblk = group * 8u + (rem & 7u);
+        cblk = rem >> 3;
+        if (rblk >= a.row_blocks) return;                 // padding of the last group
+    }
+    const uint32_t row0 = rblk * 128u, cbase = cblk * (16u * ST);
+    const uint16_t *const thin = a.thin + (size_t)(blockIdx.y / a.ksplits) * a.half_elems;
+    const uint32_t kbeg = (blockIdx.y % a.ksplits) * a.kper;
+    const uint32_t kend = kbeg + a.kper < K ? kbeg + a.kper : K;
+    const uint32_t nchunks = (kend - kbeg + BK - 1) / BK;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)sk_lds;
+
+    // This wave's load instructions: 1 KiB of LDS each, instruction i of wave v fills bytes 1024 (8 i + v) + 16 lane of the
+    // samples' or the weights' part.  Lane offsets (32-bit: the host checks that both operands span less than 4 GiB), and the
+    // k of the piece in its chunk.
+    uint32_t t_off[T_DMA], w_off[W_DMA], t_k[T_DMA], w_k[W_DMA];
+#pragma unroll
+    for (int i = 0; i < T_DMA; ++i) {
+        const uint32_t at = (8u * i + wave) * 1024u + lane * 16u, r = at / TROW, p = thin_piece<TROW>(r, at % TROW / 16u);
+        const uint32_t c = cbase + r < a.NC ? cbase + r : a.NC - 1u;
+        t_k[i] = p * 8u;
+        t_off[i] = (uint32_t)(((size_t)c * K + t_k[i]) * 2u);
+    }
+#pragma unroll
+    for (int i = 0; i < W_DMA; ++i) {
+        const uint32_t at = (8u * i + wave) * 1024u + lane * 16u, r = at / WROW, p = thin_piece<WROW>(r, at % WROW / 16u);
+        const uint32_t n = row0 + r < a.R ? row0 + r : a.R - 1u;
+        w_k[i] = p * EPL;
+        w_off[i] = (uint32_t)((size_t)n * ((size_t)K * bits / 8u) + p * 16u);
+    }
+    constexpr bool T_FULL = ST * 16 * TROW % 8192 == 0;     // every wave has T_DMA of them (else the later waves have one less)
+    const bool t_last = T_FULL || (8u * (T_DMA - 1) + wave) * 1024u < (uint32_t)(ST * 16 * TROW);
+    auto load = [&](uint32_t stage, uint32_t ch) __attribute__((always_inline)) {
+        const uint32_t k0 = kbeg + ch * BK;
+        const uint32_t to = lds0 + stage + wave * 1024u;
+        const uint8_t *const tb = reinterpret_cast<const uint8_t *>(thin) + (size_t)k0 * 2u;
+        const uint8_t *const wb = a.stream + (size_t)k0 * bits / 8u;
+        if (k0 + BK <= kend) {
+#pragma unroll
+            for (int i = 0; i < W_DMA; ++i) lds_dma16(to + (uint32_t)(W_AT + i * 8192), w_off[i], wb);
+#pragma unroll
+            for (int i = 0; i < T_DMA; ++i)
+                if (i < T_DMA - 1 || t_last) lds_dma16(to + (uint32_t)(i * 8192), t_off[i], tb);
+        } else {
+            // the partial chunk at the end of K: pieces past the end of their row come from the chunk's start
+#pragma unroll
+            for (int i = 0; i < W_DMA; ++i) lds_dma16(to + (uint32_t)(W_AT + i * 8192), k0 + w_k[i] < kend ? w_off[i] : w_off[i] - w_k[i] * bits / 8u, wb);
+#pragma unroll
+            for (int i = 0; i < T_DMA; ++i)
+                if (i < T_DMA - 1 || t_last) lds_dma16(to + (uint32_t)(i * 8192), k0 + t_k[i] < kend ? t_off[i] : t_off[i] - t_k[i] * 2u, tb);
+        }
+    };
+    // ... and are cleared once they have landed (packed codes need not be: they meet samples that are zero)
+    auto clear_tail = [&](uint32_t stage, uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < T_DMA; ++i)
+            if ((i < T_DMA - 1 || t_last) && k0 + t_k[i] >= kend)
+                *reinterpret_cast<uint4 *>(sk_lds + stage + (8u * i + wave) * 1024u + lane * 16u) = make_uint4(0u, 0u, 0u, 0u);
+        if constexpr (W16) {
+#pragma unroll
+            for (int i = 0; i < W_DMA; ++i)
+                if (k0 + w_k[i] >= kend)
+                    *reinterpret_cast<uint4 *>(sk_lds + stage + W_AT + (8u * i + wave) * 1024u + lane * 16u) = make_uint4(0u, 0u, 0u, 0u);
+        }
+    };
+
+    f32x4 acc[2][ST];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int s = 0; s < ST; ++s)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[j][s][r] = 0.0f;
+
+    // LDS addresses of this lane in stage 0: its codes, and its samples' pieces of each step of eight k
+    constexpr int STEPS = KQ / 8, CW = KQ * bits / 32;      // steps, 32-bit words of codes per row tile
+    const uint32_t k_lane = g * (BK / 2) + q4 * KQ;         // first k of this lane in a chunk
+    uint32_t c_addr[W16 ? 2 : 1], t_addr[STEPS];
+    const uint32_t wr = w * 32u + l15;                      // (row 16 further on: the same position)
+#pragma unroll
+    for (int p = 0; p < (W16 ? 2 : 1); ++p)
+        c_addr[p] = lds0 + W_AT + wr * WROW + thin_pos<WROW>(wr, k_lane / EPL + p) * 16u + (k_lane % EPL) * bits / 8u;
+#pragma unroll
+    for (int e = 0; e < STEPS; ++e) t_addr[e] = lds0 + l15 * TROW + thin_pos<TROW>(l15, k_lane / 8u + e) * 16u;
+
+    // One chunk.  LDS reads are explicit, with lgkmcnt waits: the samples of a step are asked for a step ahead, while the
+    // codes of this one are unpacked (the compiler would ask for them right before the products).
+    auto compute = [&](uint32_t stage) __attribute__((always_inline)) {
+        u32x4 cw[2][W16 ? 2 : 1];
+        u32x2 c2[2];
+        u32x4 tf[2][ST];
+        auto samples = [&](auto e_c) __attribute__((always_inline)) {
+            constexpr int e = decltype(e_c)::value;
+            static_for<ST>([&](auto s_c) __attribute__((always_inline)) {
+                ds_read128<decltype(s_c)::value * 16 * TROW>(tf[e & 1][decltype(s_c)::value], t_addr[e] + stage);
+            });
+        };
+        if constexpr (FMT == I2) {
+            ds_read64<0>(c2[0], c_addr[0] + stage);
+            ds_read64<16 * WROW>(c2[1], c_addr[0] + stage);
+        } else {
+#pragma unroll
+            for (int p = 0; p < (W16 ? 2 : 1); ++p) {
+                ds_read128<0>(cw[0][p], c_addr[p] + stage);
+                ds_read128<16 * WROW>(cw[1][p], c_addr[p] + stage);
+            }
+        }
+        samples(std::integral_constant<int, 0>{});
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(ST));
+        uint32_t code[2][CW];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if constexpr (FMT == I2) {
+                asm volatile("" : "+v"(c2[j]));
+                code[j][0] = c2[j].x;
+                code[j][1] = c2[j].y;
+            } else {
+#pragma unroll
+                for (int p = 0; p < (W16 ? 2 : 1); ++p) {
+                    asm volatile("" : "+v"(cw[j][p]));
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) code[j][4 * p + x] = cw[j][p][x];
+                }
+            }
+        }
+        // Codes to FP16 (as unpack_word16), in eight pieces a step of at most four vector instructions: piece k of step n takes
+        // row tile k / 4.  INT2: a word is two steps, its fields are formed one step ahead.
+        u32x4 wf[2][2];                                     // [step & 1][row tile]
+        uint32_t fld[2][2][8];                              // [word & 1][row tile]: pairs of fields
+        auto piece = [&](auto n_c, auto k_c) __attribute__((always_inline)) {
+            constexpr int n = decltype(n_c)::value, j = decltype(k_c)::value >> 2, q = decltype(k_c)::value & 3;
+            constexpr uint32_t LO = 0x05040100u, HI = 0x07060302u;
+            if constexpr (W16) {
+                wf[n & 1][j][q] = code[j][4 * n + q];
+            } else if constexpr (FMT == I2) {
+                constexpr int word = n >> 1;
+                // the first step of a chunk forms all fields of its word, step 2 m + 1 the first half of the next word's,
+                // step 2 m + 2 the second
+                auto form = [&](auto w_c, auto f_c) __attribute__((always_inline)) {
+                    constexpr int w2 = decltype(w_c)::value, f = decltype(f_c)::value;
+                    constexpr uint32_t mask = f == 0 || f == 5 ? 0x00030003u : f == 1 || f == 6 ? 0x000C000Cu : f == 2 || f == 7 ? 0x00300030u : f == 3 ? 0x00C000C0u : 0x03000300u;
+                    constexpr uint32_t bias = f == 0 || f == 5 ? 0x64026402u : f == 1 || f == 6 ? 0x5C085C08u : f == 2 || f == 7 ? 0x54205420u : f == 3 ? 0x4C804C80u : 0x46004600u;
+                    const uint32_t x = f > 4 ? code[j][w2] >> 10 : code[j][w2];
+                    fld[w2 & 1][j][f] = h2_sub((x & mask) ^ bias, bias);
+                };
+                if constexpr (n == 0) {
+                    form(std::integral_constant<int, 0>{}, std::integral_constant<int, 2 * q>{});
+                    form(std::integral_constant<int, 0>{}, std::integral_constant<int, 2 * q + 1>{});
+                } else if constexpr (n % 2 == 0) {
+                    form(std::integral_constant<int, word>{}, std::integral_constant<int, 4 + q>{});
+                }
+                if constexpr (n % 2 == 0) {
+                    // (the fields of pair q: 2 q and 2 q + 1, both here by now)
+                    constexpr int pq = q;
+                    wf[0][j][pq] = __builtin_amdgcn_perm(fld[word & 1][j][2 * pq + 1], fld[word & 1][j][2 * pq], LO);
+                } else {
+                    wf[1][j][q] = __builtin_amdgcn_perm(fld[word & 1][j][2 * q + 1], fld[word & 1][j][2 * q], HI);
+                    if constexpr (n + 1 < STEPS) form(std::integral_constant<int, word + 1>{}, std::integral_constant<int, q>{});
+                }
+            } else {
+                // fields 0 1 | 2 3 of eight codes, then the four pairs in order
+                uint32_t(&m)[8] = fld[0][j];
+                if constexpr (q < 2) {
+                    const uint32_t w = FMT == I8 ? code[j][2 * n + q] : q ? code[j][n] >> 8 : code[j][n];
+                    if constexpr (FMT == I8) {
+                        m[2 * q] = h2_sub((w & 0x00FF00FFu) ^ 0x64806480u, 0x64806480u);
+                        m[2 * q + 1] = h2_sub(((w >> 8) & 0x00FF00FFu) ^ 0x64806480u, 0x64806480u);
+                    } else {
+                        m[2 * q] = h2_sub((w & 0x000F000Fu) ^ 0x64086408u, 0x64086408u);
+                        m[2 * q + 1] = h2_sub((w & 0x00F000F0u) ^ 0x54805480u, 0x54805480u);
+                    }
+                } else if constexpr (FMT == I8) {
+                    wf[n & 1][j][2 * (q - 2)] = __builtin_amdgcn_perm(m[2 * (q - 2) + 1], m[2 * (q - 2)], LO);
+                    wf[n & 1][j][2 * (q - 2) + 1] = __builtin_amdgcn_perm(m[2 * (q - 2) + 1], m[2 * (q - 2)], HI);
+                } else {
+                    wf[n & 1][j][2 * (q - 2)] = __builtin_amdgcn_perm(m[1], m[0], q == 2 ? LO : HI);
+                    wf[n & 1][j][2 * (q - 2) + 1] = __builtin_amdgcn_perm(m[3], m[2], q == 2 ? LO : HI);
+                }
+            }
+        };
+        static_for<8>([&](auto k_c) __attribute__((always_inline)) { piece(std::integral_constant<int, 0>{}, k_c); });
+        static_for<STEPS>([&](auto e_c) __attribute__((always_inline)) {
+            constexpr int e = decltype(e_c)::value;
+            if constexpr (e + 1 < STEPS) samples(std::integral_constant<int, e + 1>{});
+            asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(e + 1 < STEPS ? ST : 0));
+#pragma unroll
+            for (int s = 0; s < ST; ++s) asm volatile("" : "+v"(tf[e & 1][s]));
+            __builtin_amdgcn_sched_barrier(0);
+            // The next step's codes are unpacked between this one's products.  (Both waves of a SIMD do the same at the same
+            // time: one after the other, the times of unpacking and products add up, MS.)
+            static_for<2 * ST>([&](auto x_c) __attribute__((always_inline)) {
+                constexpr int x = decltype(x_c)::value, j = x / ST, s = x % ST;
+                if constexpr (F16T) {
+                    f16x8 av, bv;
+                    __builtin_memcpy(&av, &wf[e & 1][j], 16);
+                    __builtin_memcpy(&bv, &tf[e & 1][s], 16);
+                    acc[j][s] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, acc[j][s], 0, 0, 0);
+                } else {
+                    bf16x8 av, bv;
+                    __builtin_memcpy(&av, &wf[e & 1][j], 16);
+                    __builtin_memcpy(&bv, &tf[e & 1][s], 16);
+                    acc[j][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[j][s], 0, 0, 0);
+                }
+                if constexpr (e + 1 < STEPS) {
+                    constexpr int from = x * 8 / (2 * ST), to = (x + 1) * 8 / (2 * ST);
+                    static_for<to - from>([&](auto d_c) __attribute__((always_inline)) {
+                        piece(std::integral_constant<int, e + 1>{}, std::integral_constant<int, from + decltype(d_c)::value>{});
+                    });
+                    if constexpr (!W16) __builtin_amdgcn_sched_barrier(0);
+                }
+            });
+        });
+    };
+
+    // ---- chunks ------------------------------------------------------------------
+    // Chunk c sits in stage c % NSTAGE.  Loads of chunk c + NSTAGE - 1 go out behind the barrier of chunk c, which every wave
+    // reaches when it is done with chunk c - 1.
+    constexpr int PER = T_DMA + W_DMA;                      // loads of a wave and chunk (one less where !t_last)
+#pragma unroll
+    for (int c = 0; c < NSTAGE - 1; ++c)
+        if ((uint32_t)c < nchunks) {
+            if (c) __builtin_amdgcn_s_barrier();            // (every wave's loads of a chunk before anybody's of the next)
+            load((uint32_t)(c * STAGE), (uint32_t)c);
+        }
+    uint32_t stage = 0, fill = (NSTAGE - 1) * STAGE;
+    for (uint32_t c = 0; c < nchunks; ++c) {
+        // chunk c has landed when only the loads of the chunks behind it are on their way (and this wave's
+        // fragments of the chunk before are in registers)
+        if (c + NSTAGE - 2 < nchunks) {
+            if (t_last) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NSTAGE - 2) * PER) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NSTAGE - 2) * (PER - 1)) : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        }
+        if (kbeg + (c + 1) * BK > kend) {
+            clear_tail(stage, kbeg + c * BK);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (c + NSTAGE - 1 < nchunks) load(fill, c + NSTAGE - 1);
+        compute(stage);
+        asm volatile("" ::: "memory");
+        fill = stage;
+        stage = stage == (NSTAGE - 1) * STAGE ? 0u : stage + STAGE;
+    }
+    __syncthreads();
+
+    // ---- the two halves meet: a wave keeps row tile g and gives the other away --------
+    f32x4 *const ex = reinterpret_cast<f32x4 *>(sk_lds) + (size_t)w * (2 * ST * 64) + lane;
+#pragma unroll
+    for (int s = 0; s < ST; ++s) ex[((g ^ 1u) * ST + s) * 64u] = g ? acc[0][s] : acc[1][s];
+    __syncthreads();
+    f32x4 sum[ST];
+#pragma unroll
+    for (int s = 0; s < ST; ++s) {
+        const f32x4 other = ex[(g * ST + s) * 64u];
+        sum[s] = g ? other + acc[1][s] : acc[0][s] + other;    // (first half + second half)
+    }
+
+    // lane (l15, q4): rows 4 q4 .. 4 q4 + 3 of the tile, samples l15 of each sample tile
+    const uint32_t r0 = row0 + w * 32u + g * 16u + 4u * q4;
+    if (r0 >= a.R) return;
+    if (a.ws) {
+        const bool whole = a.R % 4u == 0 && (reinterpret_cast<uintptr_t>(a.ws) & 15u) == 0;
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+            const uint32_t c = cbase + s * 16u + l15;
+            if (c >= a.NC) continue;
+            float *const dst = a.ws + ((size_t)blockIdx.y * a.NC + c) * a.R + r0;
+            if (whole) {
+                *reinterpret_cast<f32x4 *>(dst) = sum[s];
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (r0 + r < a.R) dst[r] = sum[s][r];
+            }
+        }
+        return;
+    }
+    float bias[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bias[r] = elem_value_rt(a.L.bias_fmt, a.L.bias, r0 + r < a.R ? r0 + r : a.R - 1u) * a.L.bscale;
+    with_act(a.L.act, [&](auto act_c) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_c)::value;
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+            const uint32_t c = cbase + s * 16u + l15;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (c < a.NC && r0 + r < a.R) skinny_emit_biased<F16T, ACT>(a, c, r0 + r, sum[s][r], bias[r]);
+        }
+    });
+}
+
 // Variant for a thin operand of at most NCP (8 or 16; the host uses 8) rows: the NW waves of a workgroup share one tile of 32
 // streamed rows and split K among themselves (wave w takes chunks w, w + NW, ...), so that a layer with many streamed
 // rows needs no K split across workgroups, no partial sums in memory and no second launch.  Each wave stages its own
 // thin chunks in its own LDS region (no workgroup barrier in the loop); the NW accumulator tiles meet in LDS at the
-// end and are added in wave order.  Loads and their bookkeeping are those of sp_skinny16.
+// end and are added in wave order.  Loads and their bookkeeping are those of sp_skinny16_regs.
 template <int FMT, bool F16T, int NCP, int NW>
 __global__ __launch_bounds__(64 * NW) void sp_skinny16_kw(const SkinnyArgs a)
 {
@@ -654,20 +1027,18 @@ __global__ __launch_bounds__(256) void sp_skinny_reduce(const SkinnyArgs a, uint
     if constexpr (VEC) {
         const uint64_t idx = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * 4u;
         if (idx >= total) return;
-        float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f), low = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (uint32_t sp = 0; sp < parts; ++sp) {
-            const float4 v = *reinterpret_cast<const float4 *>(a.ws + (uint64_t)sp * total + idx);
-            if (sp < splits) { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; }
-            else { low.x += v.x; low.y += v.y; low.z += v.z; low.w += v.w; }
-        }
         const uint32_t c = (uint32_t)(idx / a.R), r = (uint32_t)(idx % a.R);
+        float bias[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bias[i] = elem_value_rt(a.L.bias_fmt, a.L.bias, r + i) * a.L.bscale;
+        float4 sum, low;
+        add_parts(reinterpret_cast<const float4 *>(a.ws + idx), total / 4u, splits, parts, sum, low);
         const float in[4] = {fmaf(low.x, kLoScale, sum.x), fmaf(low.y, kLoScale, sum.y), fmaf(low.z, kLoScale, sum.z),
                              fmaf(low.w, kLoScale, sum.w)};
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float bias = elem_value_rt(a.L.bias_fmt, a.L.bias, r + i) * a.L.bscale;
-            v[i] = apply_act(layer_sum(a.L, in[i], bias, r + i), a.L.act);
+            v[i] = apply_act(layer_sum(a.L, in[i], bias[i], r + i), a.L.act);
         }
         const size_t o = (size_t)c * a.L.N + r;
         if (a.out_f32) {

@@ -583,6 +583,25 @@ def test_large_tiles_at_the_edges_of_their_pipeline(S, O, fmt, n, K, N):
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 2e-3
 
 
+@pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
+@pytest.mark.parametrize("n,K,N", [
+    (9, 2112, 1031), (17, 4160, 130), (33, 2176, 2050), (48, 2560, 126), (64, 2112, 4099),   # one to four sixteens of samples, K
+    (65, 8256, 1000), (129, 2496, 1155), (256, 2048, 2047), (200, 2112, 16300),              # splits whose last chunk is partial,
+])                                                                                            # rows that end inside a tile
+def test_streamed_weights_at_the_edges_of_their_tiles(S, O, fmt, n, K, N):
+    """sp_skinny16 (and what takes these layers where it does not) against the float64 forward.  (FP16 inputs: 2^-12 of each, at
+    random over K terms.)"""
+    src = make_oracle_net(O, [K, N], ["none"], seed=n + K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    h = S.lib().spingalett_hip_handle(net)
+    name = S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode()
+    assert name == "sp_skinny16" or n > 64, name
+    X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    S.free_network(net)
+    assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 2e-3
+
+
 def test_large_tiles_saturate_and_keep_infinities_block_by_block(S):
     """FP16 outputs of sp_gemm16_big: finite sums beyond +-65504 saturate, infinities and NaNs stay and only their own
     samples have them, in row tiles that hold ordinary samples too."""
