@@ -196,27 +196,10 @@ __global__ __launch_bounds__(256) void sp_decode(const DecodeParams p)
 // ---------------------------------------------------------------------------
 // softmax over rows (Activation.c:5-21); one wave per row
 // ---------------------------------------------------------------------------
-// out_kind: 0 FP32, 1 BF16, 2 FP16, 3 split FP16 (hi, and (v - hi) 2^11 rows * width elements further on)
-__global__ __launch_bounds__(256) void sp_softmax_rows(const float *__restrict__ in, void *__restrict__ out,
-                                                       int out_kind, uint32_t rows, uint32_t width)
+// put(i, value i) for the row at p, by the lanes of one wave
+template <class Put>
+__device__ __forceinline__ void softmax_row(const float *__restrict__ p, uint32_t width, int lane, Put &&put)
 {
-    const int lane = threadIdx.x & 63;
-    const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float *p = in + (size_t)row * width;
-    auto put = [&](uint32_t i, float v) {
-        const size_t o = (size_t)row * width + i;
-        if (out_kind == 0) reinterpret_cast<float *>(out)[o] = v;
-        else if (out_kind == 1) reinterpret_cast<uint16_t *>(out)[o] = f32_to_bf16_rne(v);
-        else if (out_kind == 2) reinterpret_cast<uint16_t *>(out)[o] = f32_to_f16_sat(v);
-        else {
-            const uint16_t hi = f32_to_f16_sat(v);
-            _Float16 hh;
-            __builtin_memcpy(&hh, &hi, 2);
-            reinterpret_cast<uint16_t *>(out)[o] = hi;
-            reinterpret_cast<uint16_t *>(out)[(size_t)rows * width + o] = f32_to_f16_sat((v - (float)hh) * 2048.0f);
-        }
-    };
     constexpr int R = 16;                       // rows up to 1024 wide stay in registers: one batch of loads
     if (width <= (uint32_t)R * kWave) {
         float v[R];
@@ -254,6 +237,28 @@ __global__ __launch_bounds__(256) void sp_softmax_rows(const float *__restrict__
     s = wave_sum(s);
     const float inv = s > 0.0f ? 1.0f / s : 1.0f;
     for (uint32_t i = lane; i < width; i += kWave) put(i, expf(p[i] - m) * inv);
+}
+
+// out_kind: 0 FP32, 1 BF16, 2 FP16, 3 split FP16 (hi, and (v - hi) 2^11 rows * width elements further on)
+__global__ __launch_bounds__(256) void sp_softmax_rows(const float *__restrict__ in, void *__restrict__ out,
+                                                       int out_kind, uint32_t rows, uint32_t width)
+{
+    const int lane = threadIdx.x & 63;
+    const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    softmax_row(in + (size_t)row * width, width, lane, [&](uint32_t i, float v) {
+        const size_t o = (size_t)row * width + i;
+        if (out_kind == 0) reinterpret_cast<float *>(out)[o] = v;
+        else if (out_kind == 1) reinterpret_cast<uint16_t *>(out)[o] = f32_to_bf16_rne(v);
+        else if (out_kind == 2) reinterpret_cast<uint16_t *>(out)[o] = f32_to_f16_sat(v);
+        else {
+            const uint16_t hi = f32_to_f16_sat(v);
+            _Float16 hh;
+            __builtin_memcpy(&hh, &hi, 2);
+            reinterpret_cast<uint16_t *>(out)[o] = hi;
+            reinterpret_cast<uint16_t *>(out)[(size_t)rows * width + o] = f32_to_f16_sat((v - (float)hh) * 2048.0f);
+        }
+    });
 }
 
 // FP32 -> 16-bit activations for the first GEMM layer
@@ -481,6 +486,50 @@ __global__ __launch_bounds__(256) void sp_pack_layers(const PackArgs a)
     if (s >= a.count) return;
     for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < a.len[s]; i += gridDim.x * 256u)
         a.dst[a.dst_off[s] + i] = a.src[a.src_off[s] + i];
+}
+
+// The end of a single-sample forward in one launch of one workgroup: the softmax of the last layer, if it has one, the
+// gathering of up to 16 layer slots into pinned host memory, and the sequence number that the host polls (sp_signal_host).
+// Three launches before, each of which begins when the one before has ended: 784-512-1000-10 INT8 30.4 -> 27.2 us a call.  One
+// compute unit gathers 16384 values in about the time of a launch; longer nets keep the three.
+struct GatherArgs {
+    PackArgs p;
+    uint32_t total;        // values to gather
+    const float *logits;   // of the last layer, whose softmax is the last slot; nullptr: no softmax here
+    uint32_t *flag;
+    uint32_t seq;
+};
+constexpr uint32_t kGatherMost = 16384u;
+
+__global__ __launch_bounds__(1024) void sp_gather_host(const GatherArgs a)
+{
+    const uint32_t t = threadIdx.x, last = a.p.count - 1u;
+    const uint32_t end = a.logits ? a.p.dst_off[last] : a.total;
+    if (t >= 960u) {
+        // the last wave
+        if (a.logits)
+            softmax_row(a.logits, a.p.len[last], (int)(t - 960u), [&](uint32_t i, float v) { a.p.dst[end + i] = v; });
+    } else {
+        for (uint32_t base = 0; base < end; base += 4u * 960u) {
+            float v[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) {
+                const uint32_t i = base + j * 960u + t;
+                uint32_t at = 0;
+                for (uint32_t s = 0; s < a.p.count; ++s)
+                    if (i >= a.p.dst_off[s]) at = a.p.src_off[s] + (i - a.p.dst_off[s]);
+                v[j] = i < end ? a.p.src[at] : 0.0f;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) {
+                const uint32_t i = base + j * 960u + t;
+                if (i < end) a.p.dst[i] = v[j];
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // this wave's values are written ...
+    __syncthreads();                                        // ... and everybody's
+    if (t == 0) __hip_atomic_store(a.flag, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The last launch of a single-sample forward: a sequence number into pinned host memory, system scope, behind the
@@ -1827,8 +1876,10 @@ int check_uploaded(const sphip_net *net)
 // only_layer != 0 restricts the launch to the main kernel of that layer.
 // keep (n == 1): every layer's output goes to its slot of layers_buf, d_x must be slot 0 and d_y the last slot.
 int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint32_t n, float *d_y, uint32_t flags,
-                    uint32_t only_layer, bool keep = false)
+                    uint32_t only_layer, bool keep = false, const float **logits = nullptr)
 {
+    // logits: the caller applies the softmax of the last layer; set to where its logits are, nullptr if there is none to apply
+    if (logits) *logits = nullptr;
     const Regime reg = pick_regime(net, n, flags);
     // split activations: two FP16 matrices between the layers, whatever else the flags say
     const bool split = (flags & SPHIP_SPLIT_ACTIVATIONS) && reg == R_GEMM16;
@@ -1929,7 +1980,9 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
                 launch_gemm16(wide ? (int)F16 : net->prec, L, (const uint16_t *)in, main_out, n, out_f32, ctx);
             }
         }
-        if (softmax && !only_layer && !soft_done) {
+        if (softmax && !only_layer && !soft_done && is_last && logits) {
+            *logits = wk.soft_tmp;
+        } else if (softmax && !only_layer && !soft_done) {
             const int kind = (reg == R_GEMM16 && !is_last) ? (split ? 3 : f16t ? 2 : 1) : 0;
             sp_softmax_rows<<<(n + 3) / 4, 256, 0, g_stream>>>(wk.soft_tmp, dst, kind, n, net->topo[l]);
         }
@@ -2169,14 +2222,18 @@ int sphip_clone(const sphip_net *src, sphip_net **out)
 // memory: a last one-wave launch stores the call's sequence number into a pinned word and the host polls it (the
 // runtime's own wait costs several microseconds after the last kernel has ended).  Bounded: after about 50 ms
 // without the number the stream is waited for in the ordinary way, which also reports a failed kernel.
-static int wait_for_small_results(sphip_net *net)
+static int next_signal(sphip_net *net, uint32_t *seq)
 {
     if (!net->pin_flag) {
         HCHECK(hipHostMalloc((void **)&net->pin_flag, 64, hipHostMallocDefault));
         *net->pin_flag = 0;
     }
-    const uint32_t seq = ++net->flag_seq ? net->flag_seq : ++net->flag_seq;     // never 0
-    sp_signal_host<<<1, 64, 0, g_stream>>>(net->pin_flag, seq);
+    *seq = ++net->flag_seq ? net->flag_seq : ++net->flag_seq;     // never 0
+    return 0;
+}
+
+static int wait_for_signal(sphip_net *net, uint32_t seq)
+{
     HCHECK(hipGetLastError());
     const volatile uint32_t *flag = net->pin_flag;
     const auto t0 = std::chrono::steady_clock::now();
@@ -2187,6 +2244,14 @@ static int wait_for_small_results(sphip_net *net)
     }
     HCHECK(hipStreamSynchronize(g_stream));
     return 0;
+}
+
+static int wait_for_small_results(sphip_net *net)
+{
+    uint32_t seq = 0;
+    if (next_signal(net, &seq)) return 1;
+    sp_signal_host<<<1, 64, 0, g_stream>>>(net->pin_flag, seq);
+    return wait_for_signal(net, seq);
 }
 
 // Small host inputs travel through a pinned staging buffer and a copy kernel; small outputs are
@@ -2411,7 +2476,9 @@ int sphip_forward_layers(sphip_net *net, const float *x, float *host_neurons)
     if (grow_pinned(&net->pin_out, &net->pin_out_cap, net->total_neurons)) return 1;
     memcpy(net->pin_in, x, (size_t)net->topo[0] * sizeof(float));
     sp_copy32<<<(net->topo[0] + 255) / 256, 256, 0, g_stream>>>(net->pin_in, net->layers_buf, net->topo[0]);
-    if (enqueue_forward(net, net->workspace(), net->layers_buf, 1, net->layers_buf + net->slot_off[last], 0, 0, true)) return 1;
+    const bool one_launch = net->layers <= 16u && net->total_neurons <= kGatherMost;
+    const float *logits = nullptr;
+    if (enqueue_forward(net, net->workspace(), net->layers_buf, 1, net->layers_buf + net->slot_off[last], 0, 0, true, one_launch ? &logits : nullptr)) return 1;
     // all slots, densely packed, straight into pinned memory
     uint32_t dense = 0;
     for (uint32_t l0 = 0; l0 < net->layers; l0 += 16) {
@@ -2427,11 +2494,18 @@ int sphip_forward_layers(sphip_net *net, const float *x, float *host_neurons)
             dense += net->topo[l0 + i];
             if (pa.len[i] > widest) widest = pa.len[i];
         }
+        if (one_launch) {
+            uint32_t seq = 0;
+            if (next_signal(net, &seq)) return 1;
+            sp_gather_host<<<1, 1024, 0, g_stream>>>(GatherArgs{pa, dense, logits, net->pin_flag, seq});
+            if (wait_for_signal(net, seq)) return 1;
+            break;
+        }
         uint32_t gx = (widest + 255) / 256;
         if (gx > 64) gx = 64;
         sp_pack_layers<<<dim3(gx, pa.count), 256, 0, g_stream>>>(pa);
     }
-    if (wait_for_small_results(net)) return 1;
+    if (!one_launch && wait_for_small_results(net)) return 1;
     memcpy(host_neurons, net->pin_out, net->total_neurons * sizeof(float));
     return 0;
 }
