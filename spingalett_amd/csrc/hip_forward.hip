@@ -2311,7 +2311,7 @@ static int upload_from_host(void *dst, const void *src, size_t bytes)
         if (i >= kStageSlots) HCHECK(hipEventSynchronize(g_upload.ev[slot]));         // its last transfer has left the chunk
         const char *s = static_cast<const char *>(src) + off;
         char *d = static_cast<char *>(g_upload.buf[slot]);
-        const size_t part = (len / kStageThreads + 4095) & ~(size_t)4095;
+        const size_t part = (len / kStageThreads + 4096) & ~(size_t)4095;
         std::thread helpers[kStageThreads - 1];
         int started = 0;
         for (int t = 1; t < kStageThreads; ++t) {

@@ -1509,3 +1509,14 @@ def test_small_fp32_layers_run_in_one_launch(S, O, N, K, n, tile, act):
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= TOL_VEC
     if N > 64 or n > 8:
         assert name == ("sp_gemm32_small16" if tile == 16 else "sp_gemm32_small")
+
+
+@pytest.mark.parametrize("nbytes", [(16 << 20) - 1, 16 << 20, (16 << 20) + 1, (17 << 20) + 17, (35 << 20) + 4])
+def test_large_uploads_arrive_whole(S, nbytes):
+    """Uploads through the ring of chunks, at and off its multiples and the helpers' pages, several in a row."""
+    rng = np.random.default_rng(nbytes)
+    dst = S.DeviceBuffer(nbytes + 4)
+    for shift in (0, 4, 0):
+        a = rng.integers(0, 256, nbytes, dtype=np.uint8)
+        assert S.lib().sphip_memcpy_h2d(dst.ptr.value + shift, a.ctypes.data, nbytes) == 0
+        assert np.array_equal(dst.to_numpy(np.uint8, nbytes + 4)[shift:shift + nbytes], a)
