@@ -27,6 +27,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <new>
 #include <thread>
@@ -2273,27 +2274,32 @@ static int grow_pinned(float **p, uint64_t *cap, uint64_t need)
 // here; copied by a few threads into a ring of pinned chunks, each handed to the copy engine as soon as it is full,
 // the host-side copy and the transfer overlap.  Like hipMemcpyAsync from pageable memory, the call returns when
 // all of src has been read; the transfers themselves are ordered on g_stream.
+//
+// With a `landed`, the transfers run on a stream of their own, and landed(upto) is called after each chunk: what it
+// enqueues on g_stream may read the first upto bytes of dst and runs beside the transfers that follow.  The ways without a
+// ring call it once.
 namespace {
 constexpr size_t kStageChunk = 8u << 20;
 constexpr int kStageSlots = 3, kStageThreads = 4;
 struct UploadRing {
     void *buf[kStageSlots] = {};
-    hipEvent_t ev[kStageSlots] = {};
+    hipEvent_t ev[kStageSlots] = {}, start = nullptr;
+    hipStream_t side = nullptr;
     bool ready = false;
     std::mutex mu;
 } g_upload;
 }  // namespace
 
-static int upload_from_host(void *dst, const void *src, size_t bytes)
+static int upload_from_host(void *dst, const void *src, size_t bytes, const std::function<int(size_t)> &landed = {})
 {
     if (bytes < 2 * kStageChunk) {
         HCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
-        return 0;
+        return landed ? landed(bytes) : 0;
     }
     hipPointerAttribute_t attr{};
     if (hipPointerGetAttributes(&attr, src) == hipSuccess && attr.type != hipMemoryTypeUnregistered) {
         HCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));      // pinned already
-        return 0;
+        return landed ? landed(bytes) : 0;
     }
     (void)hipGetLastError();                                   // an unknown pointer leaves an error behind
     std::lock_guard<std::mutex> lock(g_upload.mu);
@@ -2302,7 +2308,14 @@ static int upload_from_host(void *dst, const void *src, size_t bytes)
             HCHECK(hipHostMalloc(&g_upload.buf[i], kStageChunk, hipHostMallocDefault));
             HCHECK(hipEventCreateWithFlags(&g_upload.ev[i], hipEventDisableTiming));
         }
+        HCHECK(hipEventCreateWithFlags(&g_upload.start, hipEventDisableTiming));
+        HCHECK(hipStreamCreateWithFlags(&g_upload.side, hipStreamNonBlocking));
         g_upload.ready = true;
+    }
+    const hipStream_t stream = landed ? g_upload.side : g_stream;
+    if (landed) {
+        HCHECK(hipEventRecord(g_upload.start, g_stream));     // what is still reading dst
+        HCHECK(hipStreamWaitEvent(stream, g_upload.start, 0));
     }
     size_t off = 0;
     for (int i = 0; off < bytes; ++i, off += kStageChunk) {
@@ -2322,11 +2335,58 @@ static int upload_from_host(void *dst, const void *src, size_t bytes)
         }
         memcpy(d, s, len < part ? len : part);
         for (int t = 0; t < started; ++t) helpers[t].join();
-        HCHECK(hipMemcpyAsync(static_cast<char *>(dst) + off, d, len, hipMemcpyHostToDevice, g_stream));
-        HCHECK(hipEventRecord(g_upload.ev[slot], g_stream));
+        HCHECK(hipMemcpyAsync(static_cast<char *>(dst) + off, d, len, hipMemcpyHostToDevice, stream));
+        HCHECK(hipEventRecord(g_upload.ev[slot], stream));
+        if (landed) {
+            HCHECK(hipStreamWaitEvent(g_stream, g_upload.ev[slot], 0));
+            if (landed(off + len)) { (void)hipStreamSynchronize(stream); return 1; }
+        }
     }
     // the ring may be reused by the next call right away: its events order that
     return 0;
+}
+
+// Rows per block when a batch comes from the host and its layers run over the rows that have landed while the others are
+// under way, 0 if they wait for all of them.  Only where the layers are the shorter part by far, so that running them in
+// smaller blocks costs nothing: per value of a sample the bus takes 0.085 ns, a multiply-add of FP32 layers at 100 TFLOP/s
+// 0.00002 ns; the line lies at half of that.  A block is what one chunk holds, in whole tiles of 256 rows, and 2048 at
+// least (10000 samples of 784-512-1000-10 FP32 from the host 955 -> 865 us, 20000 1780 -> 1575; 20000 of 784-128-10 1570
+// -> 1455); a rest of fewer than kLastRows joins the block before it, so that no few rows take a path for few rows.
+static const uint32_t kLastRows = 512;
+static uint32_t landing_rows(const sphip_net *net, uint32_t n, uint32_t flags)
+{
+    const uint32_t in_w = net->topo[0];
+    if ((flags & SPHIP_WHOLE_BATCH) || (uint64_t)n * in_w * sizeof(float) < 2u * kStageChunk) return 0;
+    if (pick_regime(net, n, flags) == R_GEMV || batch_block_rows(net, n, flags) < n) return 0;
+    uint64_t macs = 0;
+    for (uint32_t l = 1; l < net->layers; ++l) macs += (uint64_t)net->topo[l - 1] * net->topo[l];
+    if (macs > 2000ull * in_w) return 0;
+    uint32_t rows = (uint32_t)(kStageChunk / sizeof(float) / in_w / 256u * 256u);
+    if (rows < 2048u) rows = 2048u;
+    return rows + kLastRows <= n ? rows : 0;
+}
+
+// x from the host to net->stage_x and through all layers into d_y
+static int enqueue_forward_from_host(sphip_net *net, const float *x, uint32_t n, float *d_y, uint32_t flags)
+{
+    const uint32_t rows = landing_rows(net, n, flags), in_w = net->topo[0], out_w = net->topo[net->layers - 1];
+    const size_t row_bytes = (size_t)in_w * sizeof(float);
+    if (!rows) {
+        if (upload_from_host(net->stage_x, x, n * row_bytes)) return 1;
+        return enqueue_forward_batch(net, net->stage_x, n, d_y, flags, 0);
+    }
+    const uint32_t last = (n - kLastRows) % rows + kLastRows;
+    if (reserve(net, rows, false, flags) || reserve(net, last, false, flags)) return 1;
+    uint32_t r0 = 0;
+    return upload_from_host(net->stage_x, x, n * row_bytes, [&](size_t upto) {
+        while (r0 < n) {
+            const uint32_t m = n - r0 < rows + kLastRows ? n - r0 : rows;
+            if ((r0 + m) * row_bytes > upto) break;
+            if (enqueue_forward(net, net->workspace(), net->stage_x + (size_t)r0 * in_w, m, d_y + (size_t)r0 * out_w, flags, 0)) return 1;
+            r0 += m;
+        }
+        return 0;
+    });
 }
 
 int sphip_forward(sphip_net *net, const float *x, uint32_t n, float *y, uint32_t flags)
@@ -2338,7 +2398,7 @@ int sphip_forward(sphip_net *net, const float *x, uint32_t n, float *y, uint32_t
     const uint64_t in_cnt = (uint64_t)n * net->topo[0], out_cnt = (uint64_t)n * net->topo[net->layers - 1];
     const float *d_x = x;
     float *d_y = y;
-    bool y_pinned = false;
+    bool y_pinned = false, x_large = false;
     if (!(flags & SPHIP_X_ON_DEVICE)) {
         if (grow(&net->stage_x, &net->stage_x_cap, in_cnt)) return 1;
         if (in_cnt <= kSmallIn) {
@@ -2346,7 +2406,7 @@ int sphip_forward(sphip_net *net, const float *x, uint32_t n, float *y, uint32_t
             memcpy(net->pin_in, x, in_cnt * sizeof(float));
             sp_copy32<<<(uint32_t)((in_cnt + 255) / 256), 256, 0, g_stream>>>(net->pin_in, net->stage_x, in_cnt);
         } else {
-            if (upload_from_host(net->stage_x, x, in_cnt * sizeof(float))) return 1;
+            x_large = true;
         }
         d_x = net->stage_x;
     }
@@ -2360,7 +2420,7 @@ int sphip_forward(sphip_net *net, const float *x, uint32_t n, float *y, uint32_t
             d_y = net->stage_y;
         }
     }
-    if (enqueue_forward_batch(net, d_x, n, d_y, fwd_flags, 0)) return 1;
+    if (x_large ? enqueue_forward_from_host(net, x, n, d_y, fwd_flags) : enqueue_forward_batch(net, d_x, n, d_y, fwd_flags, 0)) return 1;
     if (!(flags & SPHIP_Y_ON_DEVICE)) {
         if (y_pinned) {
             if (wait_for_small_results(net)) return 1;
@@ -2531,14 +2591,13 @@ int sphip_evaluate(sphip_net *net, const float *x, const float *targets, uint32_
     uint32_t *d_hit = d_pred + n;
     double *d_tot = reinterpret_cast<double *>((reinterpret_cast<uintptr_t>(d_hit + n) + 7u) & ~(uintptr_t)7u);
     uint32_t *d_hits = reinterpret_cast<uint32_t *>(d_tot + 1);
-    const float *d_x = x;
-    if (!on_dev) {
+    if (on_dev) {
+        if (enqueue_forward_batch(net, x, n, d_y, fwd_flags, 0)) return 1;
+    } else {
         if (grow(&net->stage_x, &net->stage_x_cap, in_cnt)) return 1;
-        if (upload_from_host(net->stage_x, x, in_cnt * sizeof(float))) return 1;
-        HCHECK(hipMemcpyAsync(d_t, targets, out_cnt * sizeof(float), hipMemcpyHostToDevice, g_stream));
-        d_x = net->stage_x;
+        if (upload_from_host(d_t, targets, out_cnt * sizeof(float))) return 1;
+        if (enqueue_forward_from_host(net, x, n, d_y, fwd_flags)) return 1;
     }
-    if (enqueue_forward_batch(net, d_x, n, d_y, fwd_flags, 0)) return 1;
     EvalArgs a{d_y, on_dev ? targets : d_t, d_loss, d_pred, d_hit, n, width, loss_func,
                net->act[net->layers - 2] == A_SIGMOID ? 1 : 0};
     sp_eval_rows<<<(n + 3) / 4, 256, 0, g_stream>>>(a);

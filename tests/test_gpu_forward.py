@@ -1520,3 +1520,25 @@ def test_large_uploads_arrive_whole(S, nbytes):
         a = rng.integers(0, 256, nbytes, dtype=np.uint8)
         assert S.lib().sphip_memcpy_h2d(dst.ptr.value + shift, a.ctypes.data, nbytes) == 0
         assert np.array_equal(dst.to_numpy(np.uint8, nbytes + 4)[shift:shift + nbytes], a)
+
+
+@pytest.mark.parametrize("fmt", ["f32", "f16", "i8"])
+@pytest.mark.parametrize("topo,n", [([784, 96, 33], 5350), ([784, 96, 33], 8193), ([2100, 40, 10], 2049), ([2100, 40, 10], 6145)])
+def test_layers_over_the_rows_that_have_landed(S, O, fmt, topo, n):
+    """Batches whose upload is followed block by block: the first size of a block and of an upload in chunks, a last block of
+    one row more than a whole one, sizes that leave whole blocks.  A row's result does not depend on the block it is in, up to
+    the order of a K split's sums: two orders of K products differ by at most K 2^-24 of the sum of their magnitudes (784
+    of them: 5e-5), and 16-bit activations may round the other way once per layer."""
+    src = make_oracle_net(O, topo, ["relu", "softmax"], seed=74, loss=1)
+    _, _, net = quantized_pair(O, S, src, fmt)
+    X = np.random.default_rng(75).random((n, topo[0])).astype(F32)
+    got = S.forward_batch(net, X)
+    want = sphip_forward(S, net, X, S.SPHIP_WHOLE_BATCH)
+    assert rel_max_abs(got, want) <= (TOL_VEC if fmt == "f32" else 2.0 ** -9)
+    T = np.eye(topo[-1], dtype=F32)[np.arange(n) % topo[-1]]
+    total, pred, correct = S.evaluate_batch(net, X, T)
+    loss = O.batch_loss(got, T, 1, O.ACT["softmax"])
+    assert abs(total - loss) <= 2e-5 * abs(loss)
+    assert np.array_equal(pred, O.argmax_rows(got))
+    assert correct == int((O.argmax_rows(got) == O.argmax_rows(T)).sum())
+    S.free_network(net)
