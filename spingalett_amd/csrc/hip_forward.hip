@@ -9,7 +9,8 @@
 //                     through registers into 16-bit MFMAs, the thin one in LDS (_kw: thin side of <= 8 rows, K split
 //                     inside the workgroup)
 //   hip_gemm16.inl    sp_gemm16_big / sp_gemm16: larger batches: LDS-tiled dequant-to-16-bit MFMA GEMM, fused epilogue
-//   hip_gemm32.inl    sp_gemm32_f32: FP32 weights beyond four samples: FP32 MFMA GEMM
+//   hip_gemm32.inl    FP32 weights beyond four samples: FP32 MFMA GEMMs of small layers, unaligned rows, large weights
+//   hip_tile32.inl    sp_gemm32_f32: the FP32 MFMA GEMM of the other layers and of training's backward
 //   hip_gemm32_parts.inl  sp_gemm32_bf16_parts: large FP32 forward products on BF16 parts
 //   sp_softmax_rows   per-sample softmax (Activation.c:5-21)
 //   sp_eval_*         loss and argmax of a labelled batch (SIMD.c:522-552, Training.c:421-435)
@@ -326,6 +327,7 @@ __global__ __launch_bounds__(256) void sp_bf16_to_f16(const uint16_t *__restrict
 }
 
 #include "hip_gemm32.inl"
+#include "hip_tile32.inl"
 #include "hip_gemm32_parts.inl"
 
 // ---------------------------------------------------------------------------
@@ -1502,13 +1504,6 @@ uint32_t gemm32_fwd_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper)
 // 48 against 43 us.  Up to 64 K splits instead of 16 gave 32 us on the first and cost other thin layers 10 us.)
 bool f32_thin_vector(const LayerArgs &L, uint32_t n) { return L.N <= 64u && n <= 8u; }
 
-// Unused dynamic LDS for the 64 x 64 FP32 forward kernel when the grid is several times what the chip holds: with
-// 32 KB per workgroup five of them share a compute unit instead of eight, and a product of thousands of tiles runs
-// 3-5 % faster (20000 x 1000 x 512: 221 -> 210 us standalone, 227 -> 220 us in the training step; 20000 x 512 x 784:
-// 179 -> 175 us; more padding, four per compute unit: the same).  The training products with their other operand
-// layouts lose by it (235 -> 240 us, and 48 -> 53 us where K is 10 and memory decides).  `own`: the kernel's static LDS.
-size_t gemm32_lds_pad(uint64_t workgroups, size_t own) { return workgroups >= 2048u && own < (32u << 10) ? (32u << 10) - own : 0; }
-
 // Tile of sp_gemm32_small (32) or sp_gemm32_small16 for a layer that would otherwise need a K split and a second launch (or a handful of
 // workgroups), 0 where the other kernels are the faster ones: 32 x 32 tiles up to 512 of them and K = 1024 (measured
 // against the split path: 256 x 512 x 784 8 against 12 us, 1024 x 512 x 784 17 against 20 us, 1024 x 1024 x 1024 42 against 32 us); 16 x 16 tiles where the 32 x 32
@@ -1625,10 +1620,13 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
     if (splits > 1) g.ws = ws;
     tl_route.name = "sp_gemm32_f32";
     if (tl_route.dry) return false;
-    const dim3 grid(((M + 63) / 64) * ((L.N + 63) / 64), splits);
-    const size_t pad = gemm32_lds_pad((uint64_t)grid.x * grid.y, 17u << 10);
-    if (vec) sp_gemm32_f32<true><<<grid, 256, pad, g_stream>>>(g);
-    else sp_gemm32_f32<false><<<grid, 256, pad, g_stream>>>(g);
+    if (gemm32_tile_takes(A, L.w, L.K, L.K)) {
+        const Tile32Args t{A, reinterpret_cast<const float *>(L.w), C, g.ws, nullptr, L.bias, L.bias_fmt, L.bscale,
+                           M, L.N, L.K, L.K, L.K, g.kper, L.act, 1.0f};
+        launch_gemm32_tile<T32_LAYER, false, false>(t, splits);
+    } else {
+        sp_gemm32_f32_any<<<dim3(((M + 63) / 64) * ((L.N + 63) / 64), splits), 256, 0, g_stream>>>(g);
+    }
     if (splits > 1 && soft_out && L.N <= 64u) {
         sp_gemm32_reduce_softmax<<<(M + 15u) / 16u, 256, 0, g_stream>>>(g, splits, soft_out);
         return true;

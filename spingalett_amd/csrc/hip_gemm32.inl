@@ -1,5 +1,5 @@
-// hip_gemm32.inl — the FP32 MFMA GEMM for FP32 weights beyond 64 samples (sp_gemm32_f32,
-// sp_gemm32_reduce; its large products: hip_gemm32_parts.inl).  Part of hip_forward.hip's translation unit (included there, inside its unnamed
+// hip_gemm32.inl — FP32 MFMA GEMMs for FP32 weights (sp_gemm32_f32_any, sp_gemm32_f32_big, the small layers' kernels and
+// sp_gemm32_reduce; aligned rows: hip_tile32.inl, large products: hip_gemm32_parts.inl).  Part of hip_forward.hip's translation unit (included there, inside its unnamed
 // namespace); not compiled on its own.
 
 // ---------------------------------------------------------------------------
@@ -14,12 +14,11 @@ struct Gemm32Args {
     uint32_t kper;         // k range of one split (multiple of 32)
 };
 
-// 64 x 64 x 32 tile, one 32 x 32 MFMA accumulator per wave.  The next K tile is fetched into
-// registers while the current one is multiplied from LDS; small problems split K over grid y
-// (a layer of this path is often a few dozen tiles only) and a second launch adds the parts.
-// VEC: rows are 16-byte aligned (K % 4 == 0) and are read as float4.
-template <bool VEC>
-__global__ __launch_bounds__(256) void sp_gemm32_f32(const Gemm32Args g)
+// Rows that are not whole 16-byte units, read element by element: 64 x 64 x 32 tile, one 32 x 32 MFMA accumulator per wave.
+// The next K tile is fetched into registers while the current one is multiplied from LDS; small problems split K over grid y
+// (a layer of this path is often a few dozen tiles only) and a second launch adds the parts.  (Whole units: sp_gemm32_f32 in
+// hip_tile32.inl, with the same order of sums.)
+__global__ __launch_bounds__(256) void sp_gemm32_f32_any(const Gemm32Args g)
 {
     constexpr int BM = 64, BN = 64, BK = 32, LDK = BK + 1;
     __shared__ float As[BM * LDK];
@@ -52,23 +51,15 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32(const Gemm32Args g)
             const int p = t + 256 * i, row = p >> 3;
             const uint32_t k = k0 + (uint32_t)(p & 7) * 4u;
             const uint32_t m = m0 + row, n = n0 + row;
-            if constexpr (VEC) {
-                const bool kin = k < kend;                       // whole pieces: K and the split are multiples of 4
-                const float4 va = *reinterpret_cast<const float4 *>(g.A + (size_t)(m < M ? m : M - 1) * K + (kin ? k : 0u));
-                const float4 vw = *reinterpret_cast<const float4 *>(Wf + (size_t)(n < N ? n : N - 1) * K + (kin ? k : 0u));
-                ra[i] = (kin && m < M) ? va : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                rw[i] = (kin && n < N) ? vw : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            } else {
-                float a4[4], w4[4];
+            float a4[4], w4[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const bool kin = k + e < kend;
-                    a4[e] = (kin && m < M) ? g.A[(size_t)m * K + k + e] : 0.0f;
-                    w4[e] = (kin && n < N) ? Wf[(size_t)n * K + k + e] : 0.0f;
-                }
-                ra[i] = make_float4(a4[0], a4[1], a4[2], a4[3]);
-                rw[i] = make_float4(w4[0], w4[1], w4[2], w4[3]);
+            for (int e = 0; e < 4; ++e) {
+                const bool kin = k + e < kend;
+                a4[e] = (kin && m < M) ? g.A[(size_t)m * K + k + e] : 0.0f;
+                w4[e] = (kin && n < N) ? Wf[(size_t)n * K + k + e] : 0.0f;
             }
+            ra[i] = make_float4(a4[0], a4[1], a4[2], a4[3]);
+            rw[i] = make_float4(w4[0], w4[1], w4[2], w4[3]);
         }
     };
     auto stash = [&]() {

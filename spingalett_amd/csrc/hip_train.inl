@@ -25,16 +25,14 @@ struct TrGemmArgs {
     int vecA, vecB;        // operand may be read as float4 (leading dimension and base 16-byte aligned)
 };
 
-// C[m][n] = sum_k A(m, k) B(n, k) on the FP32 matrix cores.  Tile (64 TM) x (64 TM) x 32, four waves in a
-// 2 x 2 grid, TM x TM 32 x 32 accumulators per wave (TM is fixed to 1 below).  Each operand is either k-contiguous (element (r, k) at
-// r * ld + k; LDS tile [row][33]) or row-contiguous (element (r, k) at k * ld + r; LDS tile [k][64 TM + 32]):
-// the hidden deltas read the weights row-contiguous, the gradients read both operands so.  Both LDS layouts
+// C[m][n] = sum_k A(m, k) B(n, k) where an operand's rows are not whole 16-byte units (else sp_gemm32_f32 of hip_tile32.inl, with
+// the same order of sums), through registers.  Tile 64 x 64 x 32, four waves in a 2 x 2 grid.  Each operand is either
+// k-contiguous (element (r, k) at r * ld + k; LDS tile [row][33]) or row-contiguous (element (r, k) at k * ld + r; LDS tile
+// [k][96]): the hidden deltas read the weights row-contiguous, the gradients read both operands so.  Both LDS layouts
 // are conflict-free for the matrix-core operand reads (lane -> row, half-wave -> k).
 template <bool AMC, bool BMC, int EPI>
 __global__ __launch_bounds__(256) void sp_train_gemm32(const TrGemmArgs g)
 {
-    // TM = 2 (128 x 128 tiles) was measured on the 784-512-1000-10 net at batch 20000: 255 us against 227 us for the
-    // 20000 x 512 x 1000 product (628 large tiles fill 256 compute units unevenly), no gain on the gradient products.
     constexpr int TM = 1;
     constexpr int BM = 64 * TM, BN = 64 * TM, BK = 32, LDK = BK + 1, LDM = BM + 32;
     constexpr int TILE = BK * LDM > BM * LDK ? BK * LDM : BM * LDK;
@@ -724,6 +722,11 @@ void set_vec(TrGemmArgs &g)
     g.vecB = g.ldb % 4u == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15u) == 0;
 }
 
+Tile32Args tile32_args(const TrGemmArgs &g)
+{
+    return {g.A, g.B, g.C, g.ws, g.aux, nullptr, F32, 1.0f, g.M, g.N, g.K, g.lda, g.ldb, g.kper, g.act, g.scale};
+}
+
 // Hidden deltas: one launch of sp_train_delta_small for batches of up to 512 samples and 2048 tiles of 16 x 16 (wider tiles
 // as there are more of them than the chip takes at once), else the tiled kernel with its K split.
 void launch_train_delta(TrGemmArgs g, float *ws, uint64_t ws_floats)
@@ -742,7 +745,10 @@ void launch_train_delta(TrGemmArgs g, float *ws, uint64_t ws_floats)
     if (splits > 1 && (uint64_t)splits * g.M * g.N > ws_floats) { splits = 1; g.kper = (g.K + 31u) / 32u * 32u; }
     g.ws = splits > 1 ? ws : nullptr;
     set_vec(g);
-    sp_train_gemm32<false, true, TR_EPI_DELTA><<<dim3(((g.M + 63) / 64) * ((g.N + 63) / 64), splits), 256, 0, g_stream>>>(g);
+    if (gemm32_tile_takes(g.A, g.B, g.lda, g.ldb))
+        launch_gemm32_tile<T32_DELTA, false, true>(tile32_args(g), splits);
+    else
+        sp_train_gemm32<false, true, TR_EPI_DELTA><<<dim3(((g.M + 63) / 64) * ((g.N + 63) / 64), splits), 256, 0, g_stream>>>(g);
     if (splits > 1) sp_train_delta_reduce<<<(uint32_t)(((uint64_t)g.M * g.N + 255) / 256), 256, 0, g_stream>>>(g, splits);
 }
 
@@ -850,7 +856,10 @@ void train_gradients(sphip_net *net, const float *d_x, uint32_t n, const sphip_t
         g.ws = ts->ws;
         const uint32_t splits = gemm32_splits(g.M, g.N, g.K, &g.kper);
         set_vec(g);
-        sp_train_gemm32<true, true, TR_EPI_SCALE><<<dim3(((g.M + 63) / 64) * ((g.N + 63) / 64), splits), 256, 0, g_stream>>>(g);
+        if (gemm32_tile_takes(g.A, g.B, g.lda, g.ldb))
+            launch_gemm32_tile<T32_SCALE, true, true>(tile32_args(g), splits);
+        else
+            sp_train_gemm32<true, true, TR_EPI_SCALE><<<dim3(((g.M + 63) / 64) * ((g.N + 63) / 64), splits), 256, 0, g_stream>>>(g);
         opt.W = reinterpret_cast<float *>(net->W[l].base);
         opt.g = ts->gW + ts->woff[l]; opt.m = ts->mW + ts->woff[l]; opt.v = ts->vW + ts->woff[l];
         const uint64_t total = (uint64_t)g.M * g.N;

@@ -83,6 +83,38 @@ def test_gradients_match_oracle(topo, hidden, out_act, loss, n):
     d.destroy()
 
 
+@pytest.mark.parametrize("topo,n", [
+    ([64, 68, 4, 8], 513),           # rows of four floats, one K tile and a cut one; batches beyond the small kernels
+    ([36, 132, 260, 12], 1057),      # a column of four beside 64 and 128; an odd and an even number of K tiles, tails of 1, 4 and 12
+    ([100, 520, 128, 64], 2016),     # whole tiles only in the last product
+    ([32, 252, 1000, 12], 8256),     # tiles of 64 x 128, the last of them with 104 columns
+    ([64, 1000, 96, 4], 16385),      # ... and with one row
+])
+def test_products_of_aligned_layers_match_float64(topo, n):
+    """Forward, hidden deltas and gradients at the edges of the aligned FP32 kernel's tiles, K ranges and splits."""
+    rng = np.random.default_rng(n)
+    W = [(rng.standard_normal((b, a)) / np.sqrt(a)).astype(np.float32) for a, b in zip(topo, topo[1:])]
+    B = [(0.1 * rng.standard_normal(b)).astype(np.float32) for b in topo[1:]]
+    d = S.DeviceNet(topo, [S.ACT_TANH] * (len(W) - 1) + [S.ACT_NONE], S.PRECISION_FLOAT32)
+    for l, (w, b) in enumerate(zip(W, B)):
+        d.upload(l, 0, w.ravel())
+        d.upload(l, 1, b)
+    X = rng.standard_normal((n, topo[0])).astype(np.float32)
+    T = rng.standard_normal((n, topo[-1])).astype(np.float32)
+    d.train_begin()
+    d.train_step(X, T, step_args(-1, 0))
+    a = [X.astype(np.float64)]
+    for l, (w, b) in enumerate(zip(W, B)):
+        z = a[-1] @ w.T.astype(np.float64) + b
+        a.append(np.tanh(z) if l + 1 < len(W) else z)
+    delta = a[-1] - T
+    for l in reversed(range(len(W))):
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_GW, l).reshape(W[l].shape), delta.T @ a[l] / n) <= TOL, l
+        assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_GB, l), delta.sum(0) / n) <= TOL, l
+        delta = (delta @ W[l].astype(np.float64)) * (1 - a[l] * a[l])
+    d.destroy()
+
+
 OPT_CASES = [
     (S.OPTIMIZER_SGD, {}),
     (S.OPTIMIZER_SGD, {"weight_decay": 0.3}),
