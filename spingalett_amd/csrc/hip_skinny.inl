@@ -409,7 +409,7 @@ __global__ __launch_bounds__(64 * NWV) void sp_skinny16_regs(const SkinnyArgs a)
 //     vmcnt; one barrier per chunk;
 //   * samples stay in their own order; the codes are put in order as they are unpacked (unpack_word16);
 //   * the two waves of a SIMD work on different halves of the same chunk, so that the second wave costs no loads.
-// MEASURED
+// 8192 x 8192 INT2 at 20 samples 14.5 -> 10.2 us, at 50 15.9 -> 14.2, the reducing launch not counted.
 // LDS: a row of a chunk is whole, unpadded, its 16-byte pieces permuted by the row (swz) so that the sixteen rows of a
 // fragment read lie on different banks.  Lane (l15, q4) of a wave takes, of row l15 of a tile, the k-quarter q4 of its half
 // chunk: which k an operation sums does not matter as long as both operands agree.
