@@ -224,13 +224,13 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32(const Tile32Args g)
     }
 }
 
-// One launch of it: both operands at multiples of 16 bytes, rows of multiples of four floats, and offsets within a tile of 32
-// bits (gemm32_tile_takes()).  64 x 128 tiles where that leaves four per compute unit: 20000 x 512 x 1000 by the weights
+// One launch of it: both operands at multiples of 16 bytes, rows of multiples of four floats, and byte offsets within a tile, of
+// up to 128 rows, that 32 bits hold (gemm32_tile_takes()).  64 x 128 tiles where that leaves four per compute unit: 20000 x 512 x 1000 by the weights
 // 185 us against 191 with 64 x 64, 20000 x 512 x 784 forward 151 against 160, but 4096 x 512 x 784 35.4 against 34.0; the gradient
 // products, which are cut to about four 64 x 64 tiles per unit, 183 against 173 (512 x 784 x 20000).
 bool gemm32_tile_takes(const void *a, const void *b, uint32_t lda, uint32_t ldb)
 {
-    auto fits = [](const void *p, uint32_t ld) { return ld % 4u == 0 && ld <= (1u << 24) && (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+    auto fits = [](const void *p, uint32_t ld) { return ld % 4u == 0 && ld <= (1u << 23) && (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     return fits(a, lda) && fits(b, ldb);
 }
 
