@@ -2319,7 +2319,7 @@ static int upload_from_host(void *dst, const void *src, size_t bytes, const std:
     for (int i = 0; off < bytes; ++i, off += kStageChunk) {
         const int slot = i % kStageSlots;
         const size_t len = bytes - off < kStageChunk ? bytes - off : kStageChunk;
-        if (i >= kStageSlots) HCHECK(hipEventSynchronize(g_upload.ev[slot]));         // its last transfer has left the chunk
+        HCHECK(hipEventSynchronize(g_upload.ev[slot]));         // its last transfer, of this call or the one before, has left the chunk
         const char *s = static_cast<const char *>(src) + off;
         char *d = static_cast<char *>(g_upload.buf[slot]);
         const size_t part = (len / kStageThreads + 4096) & ~(size_t)4095;
@@ -2340,7 +2340,6 @@ static int upload_from_host(void *dst, const void *src, size_t bytes, const std:
             if (landed(off + len)) { (void)hipStreamSynchronize(stream); return 1; }
         }
     }
-    // the ring may be reused by the next call right away: its events order that
     return 0;
 }
 

@@ -1542,3 +1542,18 @@ def test_layers_over_the_rows_that_have_landed(S, O, fmt, topo, n):
     assert np.array_equal(pred, O.argmax_rows(got))
     assert correct == int((O.argmax_rows(got) == O.argmax_rows(T)).sum())
     S.free_network(net)
+
+
+def test_uploads_in_a_row_do_not_share_a_chunk(S, O):
+    """Targets of four chunks, then samples of two: the samples' first chunk goes where the targets' last one lay."""
+    topo, n = [512, 24, 1000], 8192
+    src = make_oracle_net(O, topo, ["relu", "none"], seed=76)
+    _, _, net = quantized_pair(O, S, src, "f32")
+    rng = np.random.default_rng(77)
+    X = rng.random((n, topo[0]), dtype=F32)
+    T = rng.random((n, topo[-1]), dtype=F32) + F32(8)
+    want = float(((S.forward_batch(net, X).astype(np.float64) - T) ** 2).sum())
+    for _ in range(3):
+        total, _, _ = S.evaluate_batch(net, X, T)
+        assert abs(total - want) <= 2e-5 * abs(want)
+    S.free_network(net)
