@@ -662,7 +662,7 @@ __global__ __launch_bounds__(512) void sp_skinny16(const SkinnyArgs a)
             for (int s = 0; s < ST; ++s) asm volatile("" : "+v"(tf[e & 1][s]));
             __builtin_amdgcn_sched_barrier(0);
             // The next step's codes are unpacked between this one's products.  (Both waves of a SIMD do the same at the same
-            // time: one after the other, the times of unpacking and products add up, MS.)
+            // time: one after the other, the times of unpacking and products add up.)
             static_for<2 * ST>([&](auto x_c) __attribute__((always_inline)) {
                 constexpr int x = decltype(x_c)::value, j = x / ST, s = x % ST;
                 if constexpr (F16T) {
