@@ -493,8 +493,10 @@ __global__ __launch_bounds__(256) void sp_pack_layers(const PackArgs a)
 
 // The end of a single-sample forward in one launch of one workgroup: the softmax of the last layer, if it has one, the
 // gathering of up to 16 layer slots into pinned host memory, and the sequence number that the host polls (sp_signal_host).
-// Three launches before, each of which begins when the one before has ended: 784-512-1000-10 INT8 30.4 -> 27.2 us a call.  One
-// compute unit gathers 16384 values in about the time of a launch; longer nets keep the three.
+// Three launches before, each of which begins when the one before has ended: 784-512-1000-10 INT8 30.4 -> 27.2 us a call.  Up
+// to 3840 values are one round of loads of one workgroup; with more of them a second round costs what a launch does, and a
+// net without a softmax saves one only (INT2 nets of 4440 values 30.7 -> 33.1 us, of 4535 27.6 -> 29.2), so longer nets keep the
+// three.
 struct GatherArgs {
     PackArgs p;
     uint32_t total;        // values to gather
@@ -502,7 +504,7 @@ struct GatherArgs {
     uint32_t *flag;
     uint32_t seq;
 };
-constexpr uint32_t kGatherMost = 16384u;
+constexpr uint32_t kGatherMost = 3840u;
 
 __global__ __launch_bounds__(1024) void sp_gather_host(const GatherArgs a)
 {

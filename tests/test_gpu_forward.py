@@ -1557,3 +1557,21 @@ def test_uploads_in_a_row_do_not_share_a_chunk(S, O):
         total, _, _ = S.evaluate_batch(net, X, T)
         assert abs(total - want) <= 2e-5 * abs(want)
     S.free_network(net)
+
+
+@pytest.mark.parametrize("topo", [[1200, 1630, 1010], [1200, 1631, 1010], [1200, 2640], [1200, 2641], [65] * 16, [65] * 17])
+@pytest.mark.parametrize("last", ["softmax", "none"])
+def test_single_sample_ends_on_both_sides_of_one_launch(S, O, topo, last):
+    """3840 values and 16 layers are gathered by one workgroup, more by the launches before it; the call is repeated."""
+    src = make_oracle_net(O, topo, ["tanh"] * (len(topo) - 2) + [last], seed=79, init="xavier")
+    _, ref, net = quantized_pair(O, S, src, "f16")
+    rng = np.random.default_rng(80)
+    for _ in range(3):
+        x = rng.standard_normal(topo[0]).astype(F32)
+        y = S.forward(net, x)
+        assert rel_max_abs(y, ref.forward_batch(x[None])[0]) <= TOL_VEC
+        v = S.neurons_view(net)
+        assert np.array_equal(v[:topo[0]], x) and np.array_equal(v[-topo[-1]:], y)
+        hidden = np.tanh(ref.W(0).astype(np.float64) @ x + ref.b(0)) if len(topo) > 2 else y
+        assert rel_max_abs(v[topo[0]:topo[0] + topo[1]], hidden) <= TOL_VEC
+    S.free_network(net)
