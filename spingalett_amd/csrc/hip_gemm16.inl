@@ -1125,11 +1125,17 @@ __global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
                     e[x] = f.x; e[x + 1] = f.y; e[x + 2] = f.z; e[x + 3] = f.w;
                 }
                 if (late) {
+                    // (one branch for all of them: one wave per SIMD hides an exponential only behind another's)
+                    if (g.L.act == A_TANH) {
 #pragma unroll
-                    for (int x = 0; x < EPS; ++x) {
-                        e[x] = g.L.act == A_TANH ? apply_act(e[x], A_TANH) : apply_act(e[x], A_SIGMOID);
-                        if (ncol + c0 + x + pad >= N) e[x] = 0.0f;       // padded neurons (layer_sum)
+                        for (int x = 0; x < EPS; ++x) e[x] = apply_act(e[x], A_TANH);
+                    } else {
+#pragma unroll
+                        for (int x = 0; x < EPS; ++x) e[x] = apply_act(e[x], A_SIGMOID);
                     }
+#pragma unroll
+                    for (int x = 0; x < EPS; ++x)
+                        if (ncol + c0 + x + pad >= N) e[x] = 0.0f;       // padded neurons (layer_sum)
                 }
                 if (rows16) {
                     u32x4 vv;
