@@ -51,7 +51,12 @@ typedef struct {
 /* A batch whose 16-bit activation buffers would exceed the memory-side cache (more than 128 MiB per buffer) runs as
  * equal blocks of rows, all layers per block (at most 64 MiB per buffer, a multiple of 256 rows), so that the layer
  * boundaries stay in that cache; the workspace is sized for a block.  Rows are independent, the outputs are the whole
- * batch's.  This flag runs the whole batch layer by layer instead (benchmark comparisons). */
+ * batch's.
+ * Inputs of 16 MiB and more in pageable host memory, of a net whose layers take less time than their transfer, run as
+ * blocks of rows too, each as soon as it has landed.  Which arithmetic an FP32 layer uses (FP32 matrix instructions, BF16
+ * parts, the FP16 parts of split mode) follows the whole batch's size there as well; tiles and K splits, and with them
+ * the order of the FP32 sums, follow the block's.
+ * This flag runs the whole batch layer by layer instead, after its transfer (benchmark comparisons). */
 #define SPHIP_WHOLE_BATCH 64u
 /* Split activations on the matrix-core path (5 samples and more; any 16-bit or integer weight format): between the
  * layers every activation travels as two FP16 numbers, hi = the value rounded to FP16 and lo = (value - hi) 2^11, about
@@ -192,8 +197,9 @@ SPHIP_API int  sphip_time_layer(sphip_net *const *nets, int count, uint32_t laye
 /* `iters` training steps on device-resident inputs and targets, timed like sphip_time_forward. */
 SPHIP_API int  sphip_time_train_step(sphip_net *net, const float *d_x, const float *d_targets, uint32_t n,
                                      const sphip_train_args *args, int iters, float *ms);
-/* Rows per pass of a forward of n samples with these flags: n, or the block size when the batch runs in blocks of rows
- * (SPHIP_WHOLE_BATCH has the rule); every layer kernel is then launched once per block. */
+/* Rows per pass of a forward of n samples on the device with these flags: n, or the block size when the batch runs in
+ * blocks of rows (SPHIP_WHOLE_BATCH has the rule); every layer kernel is then launched once per block.  (Blocks of rows
+ * that are still on their way from the host are not meant.) */
 SPHIP_API uint32_t sphip_batch_block_rows(sphip_net *net, uint32_t n, uint32_t flags);
 /* Name of the main kernel that a forward of n samples with these flags runs for the given layer (1..layers-1):
  * the library's routing evaluated without launching anything. */

@@ -1575,12 +1575,14 @@ void launch_gemm32_parts(const PartsGemm32Args &g, uint32_t splits)
 }
 
 // soft_out: the layer is a softmax layer whose normalised outputs belong there; returns true if they were written
-// (a split-K layer of at most 64 outputs: the reduction does it), false if C holds the logits
-bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, float *ws, uint64_t ws_floats, float *soft_out, bool training = false)
+// (a split-K layer of at most 64 outputs: the reduction does it), false if C holds the logits.  batch: samples of the caller's
+// batch, of which M are multiplied here
+bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, float *ws, uint64_t ws_floats, float *soft_out, uint32_t batch,
+                   bool training = false)
 {
     Gemm32Args g{L, A, C, nullptr, M, 0};
     const bool vec = L.K % 4u == 0 && (reinterpret_cast<uintptr_t>(A) & 15u) == 0 && (reinterpret_cast<uintptr_t>(L.w) & 15u) == 0;
-    if (!training && gemm32_parts_pay(M, L.N, L.K)) {
+    if (!training && gemm32_parts_pay(batch, L.N, L.K)) {
         PartsGemm32Args b{};
         uint32_t parts = gemm32_parts_splits(M, L.N, L.K, &b.kper);
         if (parts > 1 && (uint64_t)parts * M * L.N > ws_floats) { parts = 1; b.kper = (L.K + 31u) / 32u * 32u; }
@@ -1666,8 +1668,10 @@ bool cat3_layer(uint32_t n, uint32_t N, uint32_t K) { return N >= 128u && 2.0 * 
 
 // In a split-activation forward of a 16-bit or integer net every matrix-core layer writes one set of partial sums per
 // activation matrix (halves = 2).  width: the net's padded widths, which it runs with, or those it was made with.
-WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &width, uint32_t n, uint32_t flags)
+// batch: samples of the caller's batch, by which the arithmetic of FP32 nets is chosen, when n is a part of them (0: n is all).
+WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &width, uint32_t n, uint32_t flags, uint32_t batch = 0)
 {
+    if (!batch) batch = n;
     WorkspaceNeed w{};
     uint32_t widest = 0;
     for (uint32_t l = 0; l < net->layers; ++l)
@@ -1686,7 +1690,7 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
         const uint32_t N = width[l], K = width[l - 1];
         uint32_t kper = 0;
         uint64_t ws = 0;
-        if (reg == R_CAT3 && cat3_layer(n, N, K)) {
+        if (reg == R_CAT3 && cat3_layer(batch, N, K)) {
             const uint32_t K3 = 3u * cat3_kp(K);
             if ((uint64_t)n * K3 > w.cat_elems) w.cat_elems = (uint64_t)n * K3;
             const ThinPlan tp = plan_thin(F16, n, N, K3);
@@ -1700,7 +1704,7 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             if (reg == R_GEMV) continue;
             const uint32_t sp = gemm32_fwd_splits(n, N, K, &kper);
             if (sp > 1) ws = (uint64_t)sp * n * N;
-            const uint64_t parts = gemm32_parts_pay(n, N, K) ? gemm32_parts_splits(n, N, K, &kper) : 1u;
+            const uint64_t parts = gemm32_parts_pay(batch, N, K) ? gemm32_parts_splits(n, N, K, &kper) : 1u;
             if (parts > 1 && parts * n * N > w.parts_floats) w.parts_floats = parts * n * N;
         } else {
             const ThinPlan tp = plan_thin(net->prec, n, N, K);
@@ -1797,10 +1801,11 @@ int upload_weights(sphip_net *net, uint32_t l, const uint8_t *codes)
     return 0;
 }
 
-// grows the net's own workspace to what n samples need
-int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
+// grows the net's own workspace to what n samples, of a batch of `batch` (0: all of it), need
+int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0, uint32_t batch = 0)
 {
-    const WorkspaceNeed need = workspace_need(net, net->ptopo, n, flags);
+    if (!batch) batch = n;
+    const WorkspaceNeed need = workspace_need(net, net->ptopo, n, flags, batch);
     if (need.cat_elems > net->cat_cap) {
         if (net->cat_buf) { HCHECK(hipFree(net->cat_buf)); net->cat_buf = nullptr; }
         net->cat_cap = 0;
@@ -1809,7 +1814,7 @@ int reserve(sphip_net *net, uint32_t n, bool keep_layers, uint32_t flags = 0)
     }
     if (need.cat_elems)
         for (uint32_t l = 1; l < net->layers; ++l)
-            if (cat3_layer(n, net->ptopo[l], net->ptopo[l - 1]) && !net->w(l - 1).cat3_valid && net->W[l - 1].uploaded &&
+            if (cat3_layer(batch, net->ptopo[l], net->ptopo[l - 1]) && !net->w(l - 1).cat3_valid && net->W[l - 1].uploaded &&
                 make_cat3(net->w(l - 1), net->ptopo[l], net->ptopo[l - 1])) return 1;
     if (need.act_floats > net->cap_elems) {
         for (int i = 0; i < 2; ++i) {
@@ -1876,9 +1881,11 @@ int check_uploaded(const sphip_net *net)
 // Enqueues every kernel of one forward.  d_x, d_y are device pointers.
 // only_layer != 0 restricts the launch to the main kernel of that layer.
 // keep (n == 1): every layer's output goes to its slot of layers_buf, d_x must be slot 0 and d_y the last slot.
+// batch: samples of the caller's batch, of which these are n (0: all of it).
 int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint32_t n, float *d_y, uint32_t flags,
-                    uint32_t only_layer, bool keep = false, const float **logits = nullptr)
+                    uint32_t only_layer, bool keep = false, const float **logits = nullptr, uint32_t batch = 0)
 {
+    if (!batch) batch = n;
     // logits: the caller applies the softmax of the last layer; set to where its logits are, nullptr if there is none to apply
     if (logits) *logits = nullptr;
     const Regime reg = pick_regime(net, n, flags);
@@ -1925,7 +1932,7 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
             L.w = reinterpret_cast<const uint8_t *>(wa.wide16);
             L.wscale = ldexpf(L.wscale, -wa.wide_shift);
         }
-        const bool cat3 = reg == R_CAT3 && cat3_layer(n, L.N, L.K);
+        const bool cat3 = reg == R_CAT3 && cat3_layer(batch, L.N, L.K);
         if (cat3) {
             if (!wa.cat3_valid) return fail_msg("sphip: the FP16 parts of this net's FP32 weights were not made (split mode)");
             L.w = reinterpret_cast<const uint8_t *>(wa.cat3);
@@ -1948,7 +1955,7 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
                 launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n, false);
             else if (reg == R_GEMM32 || (reg == R_CAT3 && !cat3))
                 soft_done = launch_gemm32(L, (const float *)in, (float *)main_out, n, wk.split_ws, wk.split_cap,
-                                          softmax && !only_layer ? (float *)dst : nullptr);
+                                          softmax && !only_layer ? (float *)dst : nullptr, batch);
             else if (cat3) {
                 // (timing one layer includes the conversion of its input)
                 const uint32_t K = net->ptopo[l - 1], Kp = cat3_kp(K);
@@ -2375,13 +2382,14 @@ static int enqueue_forward_from_host(sphip_net *net, const float *x, uint32_t n,
         return enqueue_forward_batch(net, net->stage_x, n, d_y, flags, 0);
     }
     const uint32_t last = (n - kLastRows) % rows + kLastRows;
-    if (reserve(net, rows, false, flags) || reserve(net, last, false, flags)) return 1;
+    if (reserve(net, rows, false, flags, n) || reserve(net, last, false, flags, n)) return 1;
     uint32_t r0 = 0;
     return upload_from_host(net->stage_x, x, n * row_bytes, [&](size_t upto) {
         while (r0 < n) {
             const uint32_t m = n - r0 < rows + kLastRows ? n - r0 : rows;
             if ((r0 + m) * row_bytes > upto) break;
-            if (enqueue_forward(net, net->workspace(), net->stage_x + (size_t)r0 * in_w, m, d_y + (size_t)r0 * out_w, flags, 0)) return 1;
+            if (enqueue_forward(net, net->workspace(), net->stage_x + (size_t)r0 * in_w, m, d_y + (size_t)r0 * out_w, flags, 0, false, nullptr, n))
+                return 1;
             r0 += m;
         }
         return 0;
@@ -2762,12 +2770,12 @@ const char *sphip_layer_kernel_name(sphip_net *net, uint32_t layer, uint32_t n, 
         break;
     case R_GEMM32:
         if (f32_thin_vector(L, n)) launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false);
-        else (void)launch_gemm32(L, aligned_ptr, nullptr, n, nullptr, ~0ull, nullptr);
+        else (void)launch_gemm32(L, aligned_ptr, nullptr, n, nullptr, ~0ull, nullptr, n);
         break;
     case R_CAT3: {
         if (!cat3_layer(n, L.N, L.K)) {
             if (f32_thin_vector(L, n)) launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false);
-            else (void)launch_gemm32(L, aligned_ptr, nullptr, n, nullptr, ~0ull, nullptr);
+            else (void)launch_gemm32(L, aligned_ptr, nullptr, n, nullptr, ~0ull, nullptr, n);
             break;
         }
         LayerArgs L3 = L;

@@ -1046,7 +1046,7 @@ int sphip_train_step(sphip_net *net, const float *x, const float *targets, uint3
         }
         bool soft_done = false;
         if (vector) launch_gemv(net->prec, net->workspace(), L, in, main_out, n, false);
-        else soft_done = launch_gemm32(L, in, main_out, n, net->split_ws, net->split_cap, softmax ? ts->act[l] : nullptr, true);
+        else soft_done = launch_gemm32(L, in, main_out, n, net->split_ws, net->split_cap, softmax ? ts->act[l] : nullptr, n, true);
         if (softmax && !soft_done) sp_softmax_rows<<<(n + 3) / 4, 256, 0, g_stream>>>(net->soft_tmp, ts->act[l], 0, n, net->topo[l]);
         in = ts->act[l];
     }

@@ -1544,6 +1544,22 @@ def test_layers_over_the_rows_that_have_landed(S, O, fmt, topo, n):
     S.free_network(net)
 
 
+def test_landed_blocks_keep_the_arithmetic_of_the_whole_batch(S, O):
+    """10,000 samples make this layer one for the BF16 parts, and for the FP16 parts in split mode, whose inputs saturate at
+    65504; the rows of a block that has landed are too few for either."""
+    topo, n = [784, 512], 10000
+    src = make_oracle_net(O, topo, ["none"], seed=81)
+    _, ref, net = quantized_pair(O, S, src, "f32")
+    X = np.random.default_rng(82).standard_normal((n, topo[0])).astype(F32)
+    true = ref.forward_batch_f64(X)
+    got, whole = (np.linalg.norm(sphip_forward(S, net, X, f).astype(np.float64) - true) for f in (0, S.SPHIP_WHOLE_BATCH))
+    assert got <= 1.2 * whole
+    X[5000, 7] = 1e6
+    got, whole = (sphip_forward(S, net, X, S.SPHIP_SPLIT_ACTIVATIONS | f) for f in (0, S.SPHIP_WHOLE_BATCH))
+    assert rel_max_abs(got, whole) <= TOL_VEC
+    S.free_network(net)
+
+
 def test_uploads_in_a_row_do_not_share_a_chunk(S, O):
     """Targets of four chunks, then samples of two: the samples' first chunk goes where the targets' last one lay."""
     topo, n = [512, 24, 1000], 8192
