@@ -2297,18 +2297,21 @@ struct UploadRing {
 } g_upload;
 }  // namespace
 
+// host memory that the copy engine reads as it is
+static bool host_registered(const void *src)
+{
+    hipPointerAttribute_t attr{};
+    if (hipPointerGetAttributes(&attr, src) == hipSuccess && attr.type != hipMemoryTypeUnregistered) return true;
+    (void)hipGetLastError();                                   // an unknown pointer leaves an error behind
+    return false;
+}
+
 static int upload_from_host(void *dst, const void *src, size_t bytes, const std::function<int(size_t)> &landed = {})
 {
-    if (bytes < 2 * kStageChunk) {
+    if (bytes < 2 * kStageChunk || host_registered(src)) {
         HCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
         return landed ? landed(bytes) : 0;
     }
-    hipPointerAttribute_t attr{};
-    if (hipPointerGetAttributes(&attr, src) == hipSuccess && attr.type != hipMemoryTypeUnregistered) {
-        HCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));      // pinned already
-        return landed ? landed(bytes) : 0;
-    }
-    (void)hipGetLastError();                                   // an unknown pointer leaves an error behind
     std::lock_guard<std::mutex> lock(g_upload.mu);
     if (!g_upload.ready) {
         for (int i = 0; i < kStageSlots; ++i) {
@@ -2359,10 +2362,10 @@ static int upload_from_host(void *dst, const void *src, size_t bytes, const std:
 // least (10000 samples of 784-512-1000-10 FP32 from the host 955 -> 865 us, 20000 1780 -> 1575; 20000 of 784-128-10 1570
 // -> 1455); a rest of fewer than kLastRows joins the block before it, so that no few rows take a path for few rows.
 static const uint32_t kLastRows = 512;
-static uint32_t landing_rows(const sphip_net *net, uint32_t n, uint32_t flags)
+static uint32_t landing_rows(const sphip_net *net, const float *x, uint32_t n, uint32_t flags)
 {
     const uint32_t in_w = net->topo[0];
-    if ((flags & SPHIP_WHOLE_BATCH) || (uint64_t)n * in_w * sizeof(float) < 2u * kStageChunk) return 0;
+    if ((flags & SPHIP_WHOLE_BATCH) || (uint64_t)n * in_w * sizeof(float) < 2u * kStageChunk || host_registered(x)) return 0;
     if (pick_regime(net, n, flags) == R_GEMV || batch_block_rows(net, n, flags) < n) return 0;
     uint64_t macs = 0;
     for (uint32_t l = 1; l < net->layers; ++l) macs += (uint64_t)net->topo[l - 1] * net->topo[l];
@@ -2375,7 +2378,7 @@ static uint32_t landing_rows(const sphip_net *net, uint32_t n, uint32_t flags)
 // x from the host to net->stage_x and through all layers into d_y
 static int enqueue_forward_from_host(sphip_net *net, const float *x, uint32_t n, float *d_y, uint32_t flags)
 {
-    const uint32_t rows = landing_rows(net, n, flags), in_w = net->topo[0], out_w = net->topo[net->layers - 1];
+    const uint32_t rows = landing_rows(net, x, n, flags), in_w = net->topo[0], out_w = net->topo[net->layers - 1];
     const size_t row_bytes = (size_t)in_w * sizeof(float);
     if (!rows) {
         if (upload_from_host(net->stage_x, x, n * row_bytes)) return 1;

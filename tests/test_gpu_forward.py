@@ -1560,6 +1560,27 @@ def test_landed_blocks_keep_the_arithmetic_of_the_whole_batch(S, O):
     S.free_network(net)
 
 
+def test_pinned_batches_run_whole(S, O):
+    """Memory that the copy engine reads as it is arrives in one piece: bit for bit the whole batch's outputs (whose 784 sums
+    the blocks of a pageable batch cut differently)."""
+    topo, n = [784, 512], 10000
+    src = make_oracle_net(O, topo, ["none"], seed=83)
+    _, _, net = quantized_pair(O, S, src, "f32")
+    X = np.random.default_rng(84).random((n, topo[0]), dtype=F32)
+    whole = sphip_forward(S, net, X, S.SPHIP_WHOLE_BATCH)
+    with open("/proc/self/maps") as f:
+        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))      # (the one the library runs on)
+    at = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(at), C.c_size_t(X.nbytes), 0) == 0
+    pinned = np.frombuffer((C.c_float * X.size).from_address(at.value), dtype=F32).reshape(X.shape)
+    pinned[:] = X
+    got = sphip_forward(S, net, pinned, 0)
+    assert hip.hipHostFree(at) == 0
+    assert np.array_equal(got, whole)
+    assert not np.array_equal(sphip_forward(S, net, X, 0), whole)
+    S.free_network(net)
+
+
 def test_uploads_in_a_row_do_not_share_a_chunk(S, O):
     """Targets of four chunks, then samples of two: the samples' first chunk goes where the targets' last one lay."""
     topo, n = [512, 24, 1000], 8192
