@@ -1175,7 +1175,8 @@ ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K)
     // sp_skinny16: workgroups of 128 rows by up to 64 samples.  More of them than compute units with several blocks of samples
     // would read the samples' chunks from L2 twice as often as the 256 rows of sp_skinny16_regs do (INT2 at 256 samples:
     // 16384 x 2048 35 against 27 us, 16384 x 8192 84 against 70; at 100 samples 16384 x 8192 48.5 against 45.7, but x 4096 29.6
-    // against 31.8; from 8192 rows down never).
+    // against 31.8).  Exactly as many as compute units, which is 8065 to 8192 rows at 193 to 256 samples, from K = 8192 on:
+    // 8192 x 8192 INT2 44.3 against 42.5, INT4 45.3 against 47.6, 8192 x 16384 76 against 68 and 80 against 79; fewer never.
     const uint32_t blocks = (p.R + 127u) / 128u * ((p.NC + 63u) / 64u);
     p.regs = p.mode_b || ((fmt == I4 || fmt == I2) && p.NC > 64u && (blocks > 256u || (blocks == 256u && K >= 8192u)));
     if (!p.regs) {
@@ -1192,14 +1193,13 @@ ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K)
     p.ct = p.NC <= 32 ? 1 : 2;
     p.cblocks = (p.NC + 32u * p.ct - 1) / (32u * p.ct);
     // Waves per workgroup, and the number of workgroups the K split aims at.  Every workgroup fetches the thin block
-    // of its K share once, so eight waves (256 streamed rows) halve that traffic; they pay from 16384 streamed rows,
-    // or from 8192 with several blocks of thin rows (16384 x 16384 INT4: 38.7 / 50.4 / 83 us at 32 / 64 / 128 samples
-    // against 42.2 / 57.0 / 124; 8192 x 8192 INT2 at 256 samples 45 against 53 us), four waves stay better on smaller
-    // layers (8192 x 8192 INT8 at 64 samples 27.3 against 29.0 us).  One workgroup per compute unit is the target:
+    // of its K share once, so eight waves (256 streamed rows) halve that traffic; they pay from 16384 streamed rows, and
+    // with several blocks of thin rows (8192 x 8192 INT2 at 256 samples 45 against 53 us, 8100 rows 42.6 against 50.2), four
+    // waves stay better on smaller layers (8192 x 8192 INT8 at 64 samples 27.3 against 29.0 us).  One workgroup per compute unit is the target:
     // twice as many K splits write twice the partial sums (16384 x 16384 INT4 at 64 samples 67 us, 8192 x 8192 INT8
     // 38 us), half as many leave compute units idle (74 us).  Two row tiles per wave were slower wherever tried.
     p.rt = 1;
-    p.nwv = (p.R >= 16384u || (p.R >= 8192u && p.cblocks > 1u)) ? 8 : 4;
+    p.nwv = (p.R >= 16384u || p.cblocks > 1u) ? 8 : 4;
     const uint32_t target = 256u;
     p.row_blocks = (p.R + 32u * p.nwv * p.rt - 1) / (32u * p.nwv * p.rt);
     const uint32_t chunks = (K + bkc - 1) / bkc;

@@ -1522,6 +1522,23 @@ def test_large_uploads_arrive_whole(S, nbytes):
         assert np.array_equal(dst.to_numpy(np.uint8, nbytes + 4)[shift:shift + nbytes], a)
 
 
+@pytest.mark.parametrize("fmt", ["i4", "i2"])
+def test_streamed_rows_a_little_below_8192_take_no_longer(S, fmt):
+    """sp_skinny16_regs at 256 samples: workgroups of 256 rows, and planned as such where the rows are fewer than 8192 too
+    (planned as 128 rows each, every other workgroup had none and the others twice the K: 1.4 times as long; now even)."""
+    n, K = 256, 8192
+    us = {}
+    for N in (8100, 8192):
+        net, W, b = _decoded_layer(S, fmt, N, K, seed=N)
+        assert S.lib().sphip_layer_kernel_name(net.h, 1, n, 0).decode() == "sp_skinny16_regs"
+        X = np.random.default_rng(N).standard_normal((n, K)).astype(F32)
+        pre = X.astype(np.float64) @ W.T + b
+        assert rel_max_abs(net.forward(X), np.where(pre > 0, pre, 0.01 * pre)) <= 1e-3
+        us[N] = min(S.time_layer([net], 1, n, 100) for _ in range(5))
+        net.destroy()
+    assert us[8100] <= 1.2 * us[8192]
+
+
 @pytest.mark.parametrize("fmt", ["f32", "f16", "i8"])
 @pytest.mark.parametrize("topo,n", [([784, 96, 33], 5350), ([784, 96, 33], 8193), ([2100, 40, 10], 2049), ([2100, 40, 10], 6145)])
 def test_layers_over_the_rows_that_have_landed(S, O, fmt, topo, n):
