@@ -483,6 +483,13 @@ __global__ __launch_bounds__(512) void sp_skinny16(const SkinnyArgs a)
     const uint32_t kbeg = (blockIdx.y % a.ksplits) * a.kper;
     const uint32_t kend = kbeg + a.kper < K ? kbeg + a.kper : K;
     const uint32_t nchunks = (kend - kbeg + BK - 1) / BK;
+    // Neighbouring row blocks begin at different chunks: where rows are a large power of two of bytes long, the same chunk of
+    // all rows lies in a few of the memory's channels, and workgroups that all begin at the first one move over the channels
+    // together (cold weights: 16384 x 16384 INT4 at 8 samples 44 -> 33 us, INT8 at 16 76 -> 53, 16384 x 8192 INT8 42 -> 32,
+    // 32768 x 8192 FP16 157 -> 92; other rows even).  With several blocks of samples their chunks, of which a die then
+    // reads many at once, cost more than that (16384 x 16384 INT8 at 100 samples 88 -> 104 us).
+    const uint32_t turn = a.cblocks > 1 ? 0u : rblk % nchunks;
+    auto turned = [&](uint32_t c) { return c + turn >= nchunks ? c + turn - nchunks : c + turn; };
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)sk_lds;
 
     // This wave's load instructions: 1 KiB of LDS each, instruction i of wave v fills bytes 1024 (8 i + v) + 16 lane of the
@@ -688,14 +695,14 @@ __global__ __launch_bounds__(512) void sp_skinny16(const SkinnyArgs a)
     };
 
     // ---- chunks ------------------------------------------------------------------
-    // Chunk c sits in stage c % NSTAGE.  Loads of chunk c + NSTAGE - 1 go out behind the barrier of chunk c, which every wave
+    // The c-th chunk, turned(c), sits in stage c % NSTAGE.  Loads of chunk c + NSTAGE - 1 go out behind the barrier of chunk c, which every wave
     // reaches when it is done with chunk c - 1.
     constexpr int PER = T_DMA + W_DMA;                      // loads of a wave and chunk (one less where !t_last)
 #pragma unroll
     for (int c = 0; c < NSTAGE - 1; ++c)
         if ((uint32_t)c < nchunks) {
             if (c) __builtin_amdgcn_s_barrier();            // (every wave's loads of a chunk before anybody's of the next)
-            load((uint32_t)(c * STAGE), (uint32_t)c);
+            load((uint32_t)(c * STAGE), turned((uint32_t)c));
         }
     uint32_t stage = 0, fill = (NSTAGE - 1) * STAGE;
     for (uint32_t c = 0; c < nchunks; ++c) {
@@ -707,13 +714,13 @@ __global__ __launch_bounds__(512) void sp_skinny16(const SkinnyArgs a)
         } else {
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         }
-        if (kbeg + (c + 1) * BK > kend) {
-            clear_tail(stage, kbeg + c * BK);
+        if (kbeg + (turned(c) + 1) * BK > kend) {
+            clear_tail(stage, kbeg + turned(c) * BK);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (c + NSTAGE - 1 < nchunks) load(fill, c + NSTAGE - 1);
+        if (c + NSTAGE - 1 < nchunks) load(fill, turned(c + NSTAGE - 1));
         compute(stage);
         asm volatile("" ::: "memory");
         fill = stage;

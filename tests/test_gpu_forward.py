@@ -1539,6 +1539,23 @@ def test_streamed_rows_a_little_below_8192_take_no_longer(S, fmt):
     assert us[8100] <= 1.2 * us[8192]
 
 
+def test_streamed_rows_of_8_kib_take_no_longer_than_others(S):
+    """sp_skinny16 on rows that are a power of two of bytes long: read in step, they lay in a few of the memory's channels
+    (16384 x 16384 INT4 1.35 times as long as 16384 x 15872; now even).  Weights larger than the memory-side cache."""
+    n, N, us = 16, 16384, {}
+    for K in (15872, 16384):
+        rng = np.random.default_rng(K)
+        nets = [S.DeviceNet([K, N], [S.ACT_RELU], S.PRECISION_INT4) for _ in range(4)]
+        for net in nets:
+            net.upload(0, 0, rng.integers(0, 256, N * K // 2, dtype=np.uint8), 0.01)
+            net.upload(0, 1, rng.integers(0, 256, N // 2, dtype=np.uint8), 0.1)
+        assert S.lib().sphip_layer_kernel_name(nets[0].h, 1, n, 0).decode() == "sp_skinny16"
+        us[K] = min(S.time_layer(nets, 1, n, 100) for _ in range(5))
+        for net in nets:
+            net.destroy()
+    assert us[16384] <= 1.15 * us[15872]
+
+
 @pytest.mark.parametrize("fmt", ["f32", "f16", "i8"])
 @pytest.mark.parametrize("topo,n", [([784, 96, 33], 5350), ([784, 96, 33], 8193), ([2100, 40, 10], 2049), ([2100, 40, 10], 6145)])
 def test_layers_over_the_rows_that_have_landed(S, O, fmt, topo, n):
