@@ -1099,15 +1099,15 @@ static_assert(ThinFmt<I2>::BK == ThinFmt<I4>::BK && ThinFmt<F16>::BK == ThinFmt<
 
 // K splits of sp_skinny16: what costs least by the times measured for it (us): a chunk on st sixteens of samples, or its weights
 // at the rate at which the chip reads them; the start and end of a workgroup, of which a compute unit holds one; the second
-// launch that adds the parts.
-uint32_t thin_splits(int fmt, int st, uint32_t wgs, uint32_t chunks, uint64_t outputs)
+// launch that adds the parts.  At most most_sums of them: what the caller's workspace holds.
+uint32_t thin_splits(int fmt, int st, uint32_t wgs, uint32_t chunks, uint64_t outputs, uint64_t most_sums)
 {
     const bool narrow = fmt == I2 || fmt == I4;
     const float products = narrow ? 0.55f + 0.20f * st : 0.35f + 0.11f * st;
     const float bytes = 16.0f * (float)thin_chunk(fmt) * (float)fmt_bits(fmt);           // 128 rows of a chunk
     uint32_t best = 1;
     float least = 0.0f;
-    for (uint32_t s = 1; s <= 16u && (s == 1u || 2u * s <= chunks); ++s) {
+    for (uint32_t s = 1; s <= 16u && (s == 1u || (2u * s <= chunks && s * outputs <= most_sums)); ++s) {
         const float at_once = wgs * s < 256u ? (float)(wgs * s) : 256.0f;
         const float chunk = fmaxf(products, at_once * bytes / 5.5e6f);
         const float t = (float)((wgs * s + 255u) / 256u) * ((float)((chunks + s - 1) / s) * chunk + 3.5f) +
@@ -1120,8 +1120,8 @@ uint32_t thin_splits(int fmt, int st, uint32_t wgs, uint32_t chunks, uint64_t ou
     return best;
 }
 
-// mode_b streams 16-bit activations (fmt = the activation type), mode a the weights
-ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K)
+// mode_b streams 16-bit activations (fmt = the activation type), mode a the weights.  most_sums: thin_splits().
+ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K, uint64_t most_sums = ~0ull)
 {
     ThinPlan p{};
     if (N <= 64 && K % 8u == 0 && M >= 1) {
@@ -1184,7 +1184,7 @@ ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K)
         p.st = (int)(((p.NC + p.cblocks - 1u) / p.cblocks + 15u) / 16u);
         p.row_blocks = (p.R + 127u) / 128u;
         const uint32_t bk = thin_chunk(fmt), chunks = (K + bk - 1) / bk;
-        p.splits = thin_splits(fmt, p.st, p.row_blocks * p.cblocks, chunks, (uint64_t)p.NC * p.R);
+        p.splits = thin_splits(fmt, p.st, p.row_blocks * p.cblocks, chunks, (uint64_t)p.NC * p.R, most_sums);
         const uint32_t cps = (chunks + p.splits - 1) / p.splits;
         p.kper = cps * bk;
         p.splits = (chunks + cps - 1) / cps;
@@ -1330,7 +1330,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         else sp_gemm16_small<FMT, F16T, false><<<grid, 512, 0, g_stream>>>(g);
         return;
     }
-    const ThinPlan tp = plan_thin(FMT, M, L.N, L.K);
+    const ThinPlan tp = plan_thin(FMT, M, L.N, L.K, ctx.ws_floats / halves);
     if (tp.use && !single && (!tp.mode_b || ctx.w16) &&
         ((tp.splits == 1 && halves == 1) || (uint64_t)tp.splits * halves * tp.NC * tp.R <= ctx.ws_floats)) {
         SkinnyArgs a{};
@@ -1646,6 +1646,7 @@ struct WorkspaceNeed {
     uint64_t plane_bytes;      // digit planes: 4 bytes per element (+ padding of the last chunk) ...
     uint64_t plane_recs;       // ... and one scale (+ four digit sums) per 64 elements
     uint64_t split_floats;
+    uint64_t split_least;      // what of it no layer can do without (sp_skinny16 cuts K into as many parts as there is room for)
     uint64_t parts_floats;     // the partial sums that sp_gemm32_bf16_parts would like room for (it runs without them too)
     uint64_t cat_elems;        // split mode of an FP32 net: FP16 elements of the widest three-part layer input
 };
@@ -1689,13 +1690,14 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
     for (uint32_t l = 1; l < net->layers; ++l) {
         const uint32_t N = width[l], K = width[l - 1];
         uint32_t kper = 0;
-        uint64_t ws = 0;
+        uint64_t ws = 0, spare = 0;
         if (reg == R_CAT3 && cat3_layer(batch, N, K)) {
             const uint32_t K3 = 3u * cat3_kp(K);
             if ((uint64_t)n * K3 > w.cat_elems) w.cat_elems = (uint64_t)n * K3;
             const ThinPlan tp = plan_thin(F16, n, N, K3);
             if (tp.use) {
                 if (tp.splits > 1) ws = (uint64_t)tp.splits * tp.NC * tp.R;
+                if (!tp.kw && !tp.regs) spare = ws;
             } else {
                 const uint32_t sp = gemm16_splits(F16, n, N, K3, &kper);
                 if (sp > 1) ws = (uint64_t)sp * n * N;
@@ -1710,6 +1712,7 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             const ThinPlan tp = plan_thin(net->prec, n, N, K);
             if (tp.use) {
                 if (tp.splits > 1 || halves > 1) ws = (uint64_t)tp.splits * halves * tp.NC * tp.R;
+                if (!tp.kw && !tp.regs) spare = ws - (halves > 1 ? (uint64_t)halves * tp.NC * tp.R : 0u);
             } else {
                 const uint32_t sp = gemm16_splits(net->prec, n, N, K, &kper);
                 if (sp > 1 || halves > 1) ws = (uint64_t)sp * halves * n * N;
@@ -1723,9 +1726,10 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
         }
         if (reg == R_GEMM16 && l == 1 && K != net->topo[0] && gemm16_small_layer(n, N, K, halves)) {
             const uint32_t rs = gemm16_ragged_splits(n, N, K, &kper);
-            if ((uint64_t)rs * halves * n * N > ws) ws = (uint64_t)rs * halves * n * N;
+            if ((uint64_t)rs * halves * n * N > ws) { ws = (uint64_t)rs * halves * n * N; spare = 0; }
         }
         if (ws > w.split_floats) w.split_floats = ws;
+        if (ws - spare > w.split_least) w.split_least = ws - spare;
     }
     return w;
 }
@@ -2467,6 +2471,7 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
                (w.plane_bytes ? room(w.plane_recs * sizeof(float)) + room(w.plane_recs * 4u * sizeof(int)) : 0u) +
                room(w.split_floats * sizeof(float)) + room(w.cat_elems * sizeof(uint16_t));
     };
+    auto least = [](WorkspaceNeed w) { w.split_floats = w.split_least; return w; };
     auto all = [&](const std::vector<uint32_t> &width, const WorkspaceNeed &w) {
         size_t bytes = pieces(w);
         for (uint32_t l = 1; l < net->layers && reads_codes; ++l)
@@ -2482,18 +2487,24 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
                 return fail_msg("sphip_forward_noalloc: the split mode of an FP32 net needs FP16 parts of its weights, which the first sphip_forward in that mode makes");
     uint32_t rows = n;
     WorkspaceNeed need = workspace_need(net, net->ptopo, rows, flags);
-    const size_t known = all(net->topo, plain);
-    if (known > kScratchBytes && all(net->ptopo, need) > kScratchBytes) {
+    const size_t known = all(net->topo, least(plain));
+    if (known > kScratchBytes && all(net->ptopo, least(need)) > kScratchBytes) {
         snprintf(g_err, sizeof g_err, "sphip_forward_noalloc: %u samples of this net need %zu bytes of workspace, the fixed scratch array holds %zu",
                  n, known, kScratchBytes);
         return 1;
     }
     // Where the padded widths do need more, the batch runs in the fewest equal blocks of rows that fit, and without the
     // copies of codes that do not (the tile kernels read the codes themselves).
-    for (uint32_t blocks = 2; pieces(need) > kScratchRoom && rows > 1u; ++blocks) {
+    for (uint32_t blocks = 2; pieces(least(need)) > kScratchRoom && rows > 1u; ++blocks) {
         rows = (n + blocks - 1u) / blocks;
         if (rows > 4u) rows = (rows + 3u) & ~3u;             // the next block's rows start as aligned as the first one's
         need = workspace_need(net, net->ptopo, rows, flags);
+    }
+    // Partial sums of sp_skinny16 take what the rest leaves.
+    const size_t total = all(net->ptopo, need);
+    if (total > kScratchRoom) {
+        const uint64_t over = (total - kScratchRoom + 255u) / 256u * (256u / sizeof(float));
+        need.split_floats = need.split_floats > need.split_least + over ? need.split_floats - over : need.split_least;
     }
     if (pieces(need) > kScratchRoom) return fail_msg("sphip_forward_noalloc: one row of this net does not fit the fixed scratch array");
     size_t used = 0;

@@ -125,6 +125,26 @@ def test_noalloc_forward_refuses_what_does_not_fit(S):
     net.destroy()
 
 
+@pytest.mark.parametrize("topo,n,flags", [
+    ([25600, 3072], 256, 0),          # five parts are 65.0 MiB in all, four 62.0
+    ([32768, 3072], 200, 0),          # 68.8
+    ([32768, 640, 16], 224, 128),     # split activations: parts of both matrices
+])
+def test_noalloc_forward_cuts_k_into_as_many_parts_as_fit(S, topo, n, flags):
+    """sp_skinny16 would rather have more partial sums than the scratch array holds; fewer do too.  (Another cut of K, another
+    order of FP32 sums: 1e-4.)"""
+    net = _net(S, "i2", topo, [S.ACT_RELU] * (len(topo) - 1), seed=sum(topo))
+    assert S.lib().sphip_layer_kernel_name(net.h, 1, n, flags).decode() == "sp_skinny16"
+    X = np.random.default_rng(n).standard_normal((n, topo[0])).astype(F32)
+    d_x = S.DeviceBuffer.from_numpy(X)
+    d_y = S.DeviceBuffer.from_numpy(np.full(n * topo[-1], np.nan, F32))
+    assert net.forward_noalloc(d_x, n, d_y, flags) == 0, S.lib().sphip_last_error_string()
+    S.synchronize()
+    got, want = d_y.to_numpy(F32, (n, topo[-1])), net.forward(X, flags)
+    assert np.abs(got - want).max() <= 1e-4 * np.abs(want).max()
+    net.destroy()
+
+
 @pytest.mark.parametrize("fmt,topo,n,flags", [
     ("f16", [65, 65, 65, 5], 120000, 0),                  # 59.5 MiB of activations, 65.9 at the padded widths: two blocks of rows
     ("i2", [65, 65, 65, 5], 100000, 0),                   # 49.6 and 97.7 MiB (65 codes run as 128)
