@@ -228,6 +228,8 @@ __global__ __launch_bounds__(256) void sp_gemm32_f32(const Tile32Args g)
 // up to 128 rows, that 32 bits hold (gemm32_tile_takes()).  64 x 128 tiles where that leaves four per compute unit: 20000 x 512 x 1000 by the weights
 // 185 us against 191 with 64 x 64, 20000 x 512 x 784 forward 151 against 160, but 4096 x 512 x 784 35.4 against 34.0; the gradient
 // products, which are cut to about four 64 x 64 tiles per unit, 183 against 173 (512 x 784 x 20000).
+// And where the second half of the last tile is not mostly padding: 70000 x 10 x 512 86 us against 54, x 160 x 168 75 / 58, x 320 x 84
+// 68 / 58, 20000 x 576 x 164 60 / 52, x 960 x 96 52 / 47, x 1088 x 84 even.
 bool gemm32_tile_takes(const void *a, const void *b, uint32_t lda, uint32_t ldb)
 {
     auto fits = [](const void *p, uint32_t ld) { return ld % 4u == 0 && ld <= (1u << 23) && (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
@@ -237,9 +239,13 @@ bool gemm32_tile_takes(const void *a, const void *b, uint32_t lda, uint32_t ldb)
 template <int EPI, bool AMC, bool BMC>
 void launch_gemm32_tile(const Tile32Args &g, uint32_t splits)
 {
-    const uint32_t rows = (g.M + 63u) / 64u, wide = (g.N + 127u) / 128u;
-    if (EPI != T32_SCALE && (uint64_t)rows * wide >= 1024u)
-        sp_gemm32_f32<EPI, AMC, BMC, 2><<<dim3(rows * wide, splits), 256, 2u * (64u + 128u) * 32u * sizeof(float), g_stream>>>(g);
-    else
-        sp_gemm32_f32<EPI, AMC, BMC, 1><<<dim3(rows * ((g.N + 63u) / 64u), splits), 256, 2u * (64u + 64u) * 32u * sizeof(float), g_stream>>>(g);
+    const uint32_t rows = (g.M + 63u) / 64u, cols = (g.N + 63u) / 64u;
+    if constexpr (EPI != T32_SCALE) {
+        const uint32_t wide = (cols + 1u) / 2u;
+        if ((uint64_t)rows * wide >= 1024u && (cols % 2u == 0 || cols >= 17u)) {
+            sp_gemm32_f32<EPI, AMC, BMC, 2><<<dim3(rows * wide, splits), 256, 2u * (64u + 128u) * 32u * sizeof(float), g_stream>>>(g);
+            return;
+        }
+    }
+    sp_gemm32_f32<EPI, AMC, BMC, 1><<<dim3(rows * cols, splits), 256, 2u * (64u + 64u) * 32u * sizeof(float), g_stream>>>(g);
 }
