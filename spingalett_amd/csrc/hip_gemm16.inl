@@ -590,7 +590,7 @@ __device__ __forceinline__ void frag_reads(u32x4 *dst, uint32_t addr)
 // form took 0.82), 4096 x 8192 x 8192 INT8 0.465 -> 0.408, INT4 0.449 -> 0.377, INT2 0.395 -> 0.356, 2000 x 4096 x 12288 on
 // RM = 4 0.198 -> 0.167 ms.  Sums of a few hundred gain little (8192 x 8192 x 512 98 -> 95 us): a tile's prologue takes 2.4 us,
 // its epilogue 8, in which all compute units write at once (4 TB/s).  FP32 outputs of sums of 256, written 4 waves instead
-// of 8 at a time, lose 2-7 % (4096 x 4096 x 256 26.1 -> 27.5 us).
+// of 8 at a time, lose 3-5 % (4096 x 4096 x 256 24.6 -> 25.3 us FP16, 25.5 -> 26.8 INT8; x 1024 48.5 -> 45.4).
 //
 // The accumulators are accumulation registers by number (mfma_acc, acc_read): left to the compiler, 256 of them next to the
 // fragments are spilled.  Nothing else here lives in those registers (the first statement claims all of them, and the
@@ -660,7 +660,8 @@ struct BigTile {
     static constexpr int NSTAGE = RM == 8 || FMT == I8 ? 2 : 3;
     static constexpr int W_AT = 32 * RM * 128, STAGE = W_AT + 256 * 128;      // the weights' part of a stage, a stage
     static constexpr int CODES = fmt_bits(FMT) == 16 ? 0 : 256 * 64 * fmt_bits(FMT) / 8;
-    static constexpr int LDS = NSTAGE * STAGE + 2 * CODES;
+    static constexpr int TURN = 64 * (128 * 4 + 16);        // of a wave in the epilogue: four row tiles as FP32
+    static constexpr int LOOP = NSTAGE * STAGE + 2 * CODES, END = 4 * TURN + 256 * 4, LDS = LOOP > END ? LOOP : END;
 };
 
 template <int FMT, bool F16T, int RM>
@@ -1072,7 +1073,7 @@ __global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
     // ---- epilogue ------------------------------------------------------------------
     // Lane (l15, q4) holds outputs 4 q4 .. 4 q4 + 3 of each column tile for sample l15 of each row tile.
     const uint32_t mrow = m0 + wm * (BM / 2), ncol = n0 + wn * 128;
-    float *const bias_lds = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + 4 * 16 * (128 * 4 + 16));
+    float *const bias_lds = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + 4 * B::TURN);
     bias_lds[t] = my_bias;
     __syncthreads();
     float4 bias[8];
@@ -1091,12 +1092,14 @@ __global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
     // tiles of the die are re-reading: 8192 cubed 0.908 against 0.934 ms); short K: the next layer reads them
     // back soon and they are most of the traffic (8192 x 8192 x 1024: 0.162 against 0.175 ms the other way round).
     const bool stream_out = K >= 2048u && !g.ws;
-    char *const mine = reinterpret_cast<char *>(smem) + wave * (16 * (128 * 4 + 16));
+    char *const mine = reinterpret_cast<char *>(smem) + wave * B::TURN;
     // Activations: one uniform branch per row tile to a copy of the code over a lane's 32 outputs.  Sigmoid and tanh are kept
-    // out of that unrolled code, where theirs takes longer to fetch than to run: the sums wait in LDS as FP32, and the
-    // loop that reads them back and stores whole rows, not unrolled, applies them (4567 x 8192 x 256 FP16 with tanh 103 -> 85
-    // us, 8192 x 8192 x 2048 354 -> 324).  The same loop converts FP16 blocks with outputs that saturate, infinities or NaNs,
-    // which the packed conversion does not know, and stores rows that are not whole 16-byte units.
+    // out of that unrolled code, where theirs takes longer to fetch than to run: the scaled sums of four row tiles go to LDS
+    // as FP32, and one loop, not unrolled, reads them back sixteen a lane, applies the activation and stores whole rows (a loop
+    // per row tile, eight copies of it, read and stored in turn: 8192 x 8192 x 448 FP16 and a head with sigmoid 213 -> 185 us, with
+    // tanh 239 -> 208, and with tanh_straight, one straight line for the sixteen, as a sigmoid).  150 cycles a value of a lane,
+    // what the instructions take.  The same loop does FP16 row tiles with outputs that saturate, infinities or NaNs, which the
+    // packed conversion does not know, and rows that are not whole 16-byte units.
     const bool late = !g.ws && (g.L.act == A_SIGMOID || g.L.act == A_TANH);
     // (the lambdas are forced inline: called, they would take what they capture through memory)
     auto turn = [&](auto es_c) __attribute__((always_inline)) {
@@ -1112,58 +1115,11 @@ __global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
             else *dstp = vv;
         };
         constexpr int PUTS = 16 / RPP;
-        u32x4 held[PUTS];                                            // rows on their way from LDS to memory
-        bool pending = false;
-        // row tile i from LDS, where it waits as FP32
-        auto finish_rows = [&](int i) __attribute__((always_inline)) {
-#pragma unroll 1
-            for (int p = 0; p < 16 / RPP; ++p) {
-                float e[EPS];
-#pragma unroll
-                for (int x = 0; x < EPS; x += 4) {
-                    const float4 f = *reinterpret_cast<const float4 *>(mine + (p * RPP + rl0) * (128 * 4 + 16) + (c0 + x) * 4);
-                    e[x] = f.x; e[x + 1] = f.y; e[x + 2] = f.z; e[x + 3] = f.w;
-                }
-                if (late) {
-                    // (one branch for all of them: one wave per SIMD hides an exponential only behind another's)
-                    if (g.L.act == A_TANH) {
-#pragma unroll
-                        for (int x = 0; x < EPS; ++x) e[x] = apply_act(e[x], A_TANH);
-                    } else {
-#pragma unroll
-                        for (int x = 0; x < EPS; ++x) e[x] = apply_act(e[x], A_SIGMOID);
-                    }
-#pragma unroll
-                    for (int x = 0; x < EPS; ++x)
-                        if (ncol + c0 + x + pad >= N) e[x] = 0.0f;       // padded neurons (layer_sum)
-                }
-                if (rows16) {
-                    u32x4 vv;
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        if constexpr (ES == 4) vv[x] = __float_as_uint(e[x]);
-                        else vv[x] = (uint32_t)f32_to_t16<F16T>(e[2 * x]) | (uint32_t)f32_to_t16<F16T>(e[2 * x + 1]) << 16;
-                    }
-                    store(i, p, vv);
-                } else {
-                    const uint32_t row = mrow + i * 16 + p * RPP + rl0;
-#pragma unroll
-                    for (int x = 0; x < EPS; ++x) {
-                        const uint32_t col = ncol + c0 + x;
-                        if (row >= M || col >= N) continue;
-                        const size_t o = (size_t)row * N + col;
-                        if constexpr (ES == 4) reinterpret_cast<float *>(out)[o] = e[x];
-                        else reinterpret_cast<uint16_t *>(out)[o] = f32_to_t16<F16T>(e[x]);
-                    }
-                }
-            }
-        };
-        static_for<RM>([&](auto i_c) __attribute__((always_inline)) {
-            constexpr int i = decltype(i_c)::value;
-            float v[32];
+        // the sums of row tile i, scaled and with their bias
+        auto sums = [&](auto i_c, float (&v)[32]) __attribute__((always_inline)) {
             static_for<32>([&](auto e_c) __attribute__((always_inline)) {
                 constexpr int e = decltype(e_c)::value;
-                v[e] = acc_read<i * 32 + e>();
+                v[e] = acc_read<decltype(i_c)::value * 32 + e>();
             });
             if (!g.ws) {
 #pragma unroll
@@ -1171,67 +1127,155 @@ __global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
                     const float4 b = bias[e >> 2];
                     v[e] = fmaf(v[e], wscale, (e & 3) == 0 ? b.x : (e & 3) == 1 ? b.y : (e & 3) == 2 ? b.z : b.w);
                 }
-                auto each = [&](auto act_c) __attribute__((always_inline)) {
+            }
+        };
+        uint32_t todo = late || !rows16 ? (1u << RM) - 1u : 0u;      // row tiles for the loop below
+        if (!todo) {
+            u32x4 held[PUTS];                                        // rows on their way from LDS to memory
+            bool pending = false;
+            static_for<RM>([&](auto i_c) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_c)::value;
+                float v[32];
+                sums(i_c, v);
+                if (!g.ws) {
+                    auto each = [&](auto act_c) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int e = 0; e < 32; ++e) v[e] = decltype(act_c)::value == A_LEAKY ? fmaxf(v[e], 0.01f * v[e]) : apply_act(v[e], decltype(act_c)::value);
-                };
-                if (g.L.act == A_RELU) each(std::integral_constant<int, A_RELU>{});
-                else if (g.L.act == A_LEAKY) each(std::integral_constant<int, A_LEAKY>{});
-                else if (g.L.act == A_FOO52) each(std::integral_constant<int, A_FOO52>{});
-                // padded neurons (only hidden layers of this path have any)
-                if (!late && pad != 0u && ncol + 128u + pad > N) {
+                        for (int e = 0; e < 32; ++e) v[e] = decltype(act_c)::value == A_LEAKY ? fmaxf(v[e], 0.01f * v[e]) : apply_act(v[e], decltype(act_c)::value);
+                    };
+                    if (g.L.act == A_RELU) each(std::integral_constant<int, A_RELU>{});
+                    else if (g.L.act == A_LEAKY) each(std::integral_constant<int, A_LEAKY>{});
+                    else if (g.L.act == A_FOO52) each(std::integral_constant<int, A_FOO52>{});
+                    // padded neurons (only hidden layers of this path have any)
+                    if (pad != 0u && ncol + 128u + pad > N) {
 #pragma unroll
-                    for (int e = 0; e < 32; ++e)
-                        if (ncol + (e >> 2) * 16 + 4 * q4 + (e & 3) + pad >= N) v[e] = 0.0f;
+                        for (int e = 0; e < 32; ++e)
+                            if (ncol + (e >> 2) * 16 + 4 * q4 + (e & 3) + pad >= N) v[e] = 0.0f;
+                    }
                 }
-            }
-            bool plain = rows16 && !late;
-            if constexpr (ES == 2 && F16T) {
-                float top = 0.0f;
+                bool plain = true;
+                if constexpr (ES == 2 && F16T) {
+                    float top = 0.0f;
 #pragma unroll
-                for (int e = 0; e < 32; ++e) top = __builtin_elementwise_maximum(top, __builtin_fabsf(v[e]));
-                plain = plain && __all(top < 65520.0f);
-            }
-            // the row tile before this one, whose rows were asked for back from LDS before this one's arithmetic
+                    for (int e = 0; e < 32; ++e) top = __builtin_elementwise_maximum(top, __builtin_fabsf(v[e]));
+                    plain = __all(top < 65520.0f);
+                }
+                // the row tile before this one, whose rows were asked for back from LDS before this one's arithmetic
+                if (pending) {
+#pragma unroll
+                    for (int p = 0; p < PUTS; ++p) store(i - 1, p, held[p]);
+                }
+                pending = plain;
+                if (plain) {
+                    constexpr int PITCH = 128 * ES + 16;             // rows on different banks
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        if constexpr (ES == 4) {
+                            *reinterpret_cast<float4 *>(mine + l15 * PITCH + j * 64 + q4 * 16) = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+                        } else {
+                            uint2 d;
+                            if constexpr (F16T) {
+                                d = make_uint2(pack_f16_small(v[4 * j], v[4 * j + 1]), pack_f16_small(v[4 * j + 2], v[4 * j + 3]));
+                            } else {
+                                d = make_uint2((uint32_t)f32_to_t16<false>(v[4 * j]) | (uint32_t)f32_to_t16<false>(v[4 * j + 1]) << 16,
+                                               (uint32_t)f32_to_t16<false>(v[4 * j + 2]) | (uint32_t)f32_to_t16<false>(v[4 * j + 3]) << 16);
+                            }
+                            *reinterpret_cast<uint2 *>(mine + l15 * PITCH + j * 32 + q4 * 8) = d;
+                        }
+                    }
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int p = 0; p < PUTS; ++p) {
+                        const uint4 w = *reinterpret_cast<const uint4 *>(mine + (p * RPP + rl0) * PITCH + c0 * ES);
+                        held[p] = u32x4{w.x, w.y, w.z, w.w};
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                } else {
+                    todo |= 1u << i;
+                }
+            });
             if (pending) {
 #pragma unroll
-                for (int p = 0; p < PUTS; ++p) store(i - 1, p, held[p]);
+                for (int p = 0; p < PUTS; ++p) store(RM - 1, p, held[p]);
             }
-            pending = plain;
-            if (ES == 2 && plain) {
-                constexpr int PITCH = 128 * 2 + 16;                  // rows on different banks
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    uint2 d;
-                    if constexpr (F16T) {
-                        d = make_uint2(pack_f16_small(v[4 * j], v[4 * j + 1]), pack_f16_small(v[4 * j + 2], v[4 * j + 3]));
-                    } else {
-                        d = make_uint2((uint32_t)f32_to_t16<false>(v[4 * j]) | (uint32_t)f32_to_t16<false>(v[4 * j + 1]) << 16,
-                                       (uint32_t)f32_to_t16<false>(v[4 * j + 2]) | (uint32_t)f32_to_t16<false>(v[4 * j + 3]) << 16);
-                    }
-                    *reinterpret_cast<uint2 *>(mine + l15 * PITCH + j * 32 + q4 * 8) = d;
-                }
-            } else {
-                constexpr int PITCH = 128 * 4 + 16;
+        }
+        constexpr int PITCH = 128 * 4 + 16;
+        constexpr int PASSES = 4 * PUTS, GO = 16 / EPS;              // store instructions of four row tiles, of one turn of the loop
+#pragma unroll 1
+        for (int four = 0; four < RM; four += 4) {
+            if (!(todo >> four & 15u)) continue;
+            static_for<RM>([&](auto i_c) __attribute__((always_inline)) {
+                constexpr int i = decltype(i_c)::value;
+                if (four != (i & ~3)) return;
+                float v[32];
+                sums(i_c, v);
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    *reinterpret_cast<float4 *>(mine + l15 * PITCH + j * 64 + q4 * 16) = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
-            }
+                    *reinterpret_cast<float4 *>(mine + ((i & 3) * 16 + l15) * PITCH + j * 64 + q4 * 16) = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+            });
             __builtin_amdgcn_wave_barrier();
-            if (plain) {
+            // Element x of a lane in the turn at p.  Rows of whole units: of store instruction x / EPS.  Others: 64 neighbouring
+            // lanes store 64 neighbouring outputs (16 bytes of a row per lane, stored one element after the other, took
+            // 4090 x 4086 x 320 FP16 with FP32 outputs 42 us instead of 34).
+            auto row_of = [&](int x) __attribute__((always_inline)) { return rows16 ? x / EPS * RPP + rl0 : x >> 1; };
+            auto col_of = [&](int x) __attribute__((always_inline)) { return rows16 ? c0 + x % EPS : (x & 1) * 64 + lane; };
+            float next[16];
+            auto ask = [&](int p) __attribute__((always_inline)) {
+                if (rows16) {
 #pragma unroll
-                for (int p = 0; p < PUTS; ++p) {
-                    const uint4 w = *reinterpret_cast<const uint4 *>(mine + (p * RPP + rl0) * (128 * ES + 16) + c0 * ES);
-                    held[p] = u32x4{w.x, w.y, w.z, w.w};
+                    for (int x = 0; x < 16; x += 4) {
+                        const float4 f = *reinterpret_cast<const float4 *>(mine + (p * RPP + row_of(x)) * PITCH + col_of(x) * 4);
+                        next[x] = f.x; next[x + 1] = f.y; next[x + 2] = f.z; next[x + 3] = f.w;
+                    }
+                } else {
+#pragma unroll
+                    for (int x = 0; x < 16; ++x) next[x] = *reinterpret_cast<const float *>(mine + (p * RPP + row_of(x)) * PITCH + col_of(x) * 4);
                 }
-            } else {
-                finish_rows(i);
+            };
+            ask(0);
+#pragma unroll 1
+            for (int p = 0; p < PASSES; p += GO) {
+                float e[16];
+#pragma unroll
+                for (int x = 0; x < 16; ++x) e[x] = next[x];
+                if (p + GO < PASSES) ask(p + GO);
+                const int i = four + p / PUTS;
+                if (!(todo >> i & 1u)) continue;
+                // (one branch for all of them: one wave per SIMD hides an exponential only behind another's)
+                if (!g.ws) {
+                    with_act(g.L.act, [&](auto act_c) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int x = 0; x < 16; ++x) e[x] = decltype(act_c)::value == A_TANH ? tanh_straight(e[x]) : apply_act(e[x], decltype(act_c)::value);
+                    });
+                    if (pad != 0u && ncol + 128u + pad > N) {        // padded neurons
+#pragma unroll
+                        for (int x = 0; x < 16; ++x)
+                            if (ncol + col_of(x) + pad >= N) e[x] = 0.0f;
+                    }
+                }
+                if (rows16) {
+#pragma unroll
+                    for (int k = 0; k < GO; ++k) {
+                        const float *const o = e + k * EPS;
+                        u32x4 vv;
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            if constexpr (ES == 4) vv[x] = __float_as_uint(o[x]);
+                            else vv[x] = (uint32_t)f32_to_t16<F16T>(o[2 * x]) | (uint32_t)f32_to_t16<F16T>(o[2 * x + 1]) << 16;
+                        }
+                        store(i, p % PUTS + k, vv);
+                    }
+                } else {
+#pragma unroll
+                    for (int x = 0; x < 16; ++x) {
+                        const uint32_t row = mrow + four * 16 + p * RPP + row_of(x), col = ncol + col_of(x);
+                        if (row >= M || col >= N) continue;
+                        const size_t at = (size_t)row * N + col;
+                        if constexpr (ES == 4) reinterpret_cast<float *>(out)[at] = e[x];
+                        else reinterpret_cast<uint16_t *>(out)[at] = f32_to_t16<F16T>(e[x]);
+                    }
+                }
             }
             __builtin_amdgcn_wave_barrier();
-        });
-        if (pending) {
-#pragma unroll
-            for (int p = 0; p < PUTS; ++p) store(RM - 1, p, held[p]);
         }
     };
     if (f32_out) turn(std::integral_constant<int, 4>{});

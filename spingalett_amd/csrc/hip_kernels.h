@@ -108,6 +108,19 @@ __device__ __forceinline__ float apply_act(float x, int act)
     }
 }
 
+// tanhf's result without its branch, for code in which one wave has to hide the latency of its values behind each other: the
+// library's function takes arguments below and above 0.625 apart by execution masks, one value after the other.  The first call
+// is known to be a near one, which leaves so little on either side that the compiler does both and chooses.
+__device__ __forceinline__ float tanh_straight(float x)
+{
+    const bool near = __builtin_fabsf(x) < 0.625f;
+    const float a = near ? x : 0.0f;
+    __builtin_assume(__builtin_fabsf(a) < 0.625f);
+    const float p = tanhf(a);
+    if (near) return p;
+    return tanhf(x);
+}
+
 // derivative of an activation as a function of its output (Activation.c:40-56, SIMD.c:90-188)
 __device__ __forceinline__ float act_derivative(float a, int act)
 {

@@ -576,7 +576,9 @@ def test_large_tiles_at_the_edges_of_their_pipeline(S, O, fmt, n, K, N):
     _, ref, net = quantized_pair(O, S, src, fmt)
     h = S.lib().spingalett_hip_handle(net)
     name = S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode()
-    assert name == "sp_gemm16_big" or n == 100 or (fmt, K) in (("i4", 144), ("i2", 144)), name       # (rows that are not whole units)
+    # (rows of 144 packed codes are not whole units; integer layers of few samples are streamed)
+    want = "sp_skinny16" if n == 100 and fmt in ("i8", "i4", "i2") else "sp_gemm16" if (fmt, K) in (("i4", 144), ("i2", 144)) else "sp_gemm16_big"
+    assert name == want
     X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
     got = S.forward_batch(net, X)
     S.free_network(net)
@@ -595,11 +597,34 @@ def test_streamed_weights_at_the_edges_of_their_tiles(S, O, fmt, n, K, N):
     _, ref, net = quantized_pair(O, S, src, fmt)
     h = S.lib().spingalett_hip_handle(net)
     name = S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode()
-    assert name == "sp_skinny16" or n > 64, name
+    packed, wide = fmt in ("i4", "i2"), fmt in ("f16", "bf16")
+    want = {65: "sp_gemm16_big" if wide else "sp_skinny16", 200: "sp_skinny16_regs" if packed else "sp_gemm16"}.get(n, "sp_skinny16")
+    assert name == want
     X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
     got = S.forward_batch(net, X)
     S.free_network(net)
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 2e-3
+
+
+@pytest.mark.parametrize("fmt,n,K,N,act", [
+    ("f16", 4095, 576, 4088, "tanh"), ("i8", 4090, 576, 4086, "sigmoid"),      # whole units, and rows that are not
+    ("i2", 4090, 640, 4086, "tanh"), ("bf16", 3900, 528, 4083, "sigmoid"),
+    ("bf16", 1000, 128, 8190, "tanh"), ("f16", 1000, 320, 8184, "sigmoid"),    # 128-row tiles
+    ("i4", 100, 192, 49160, "tanh"),
+])
+def test_large_tiles_with_sigmoid_and_tanh(S, O, fmt, n, K, N, act):
+    """The late activations of sp_gemm16_big, once with the layer as the last one (FP32 outputs) and once in front of a small
+    one (16-bit outputs, padded widths), against the float64 forward.  A sigmoid or tanh passes at most its argument's error on;
+    the 16-bit output adds 2^-9 of at most 1 (BF16), at random over the head's N terms."""
+    for topo, acts in (([K, N], [act]), ([K, N, 24], [act, "none"])):
+        src = make_oracle_net(O, topo, acts, seed=n + K + N, bias_std=0.1)
+        _, ref, net = quantized_pair(O, S, src, fmt)
+        h = S.lib().spingalett_hip_handle(net)
+        assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm16_big"
+        X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
+        got = S.forward_batch(net, X)
+        S.free_network(net)
+        assert rel_max_abs(got, ref.forward_batch_f64(X)) <= (8e-3 if fmt == "bf16" else 2e-3)
 
 
 def test_large_tiles_saturate_and_keep_infinities_block_by_block(S):
