@@ -1018,22 +1018,34 @@ uint32_t gemm16_splits(int fmt, uint32_t M, uint32_t N, uint32_t K, uint32_t *kp
     return (ktiles + per - 1) / per;
 }
 
-// Longest K at which the single-stage kernel is the better one for more than a round of 256 x 256 tiles, of which a fifth
-// and more is idle.  A large tile has a compute unit to itself, so that the matrix cores idle during its epilogue and the
-// last round is mostly empty; several of the single-stage kernel's smaller workgroups share a compute unit and one's
-// epilogue runs beside another's products.  A tanh or sigmoid per output lengthens the epilogue; 16-bit weights, which
-// reach the big kernel's LDS by DMA, shorten the rest.  Big against single-stage, input conversion included, tanh, INT4 /
-// INT8: 4567 x 8192 x 448 98 / 78, 100 / 90 us, 8192 x 4736 x 448 101 / 88, 103 / 97, 4567 x 8192 x 1024 139 / 123, 145 / 141 (x
-// 1536 even or lost); FP16 100 / 96 and 101 / 100 at 448, 123 / 126 at 768.  Without them a quarter of the rounds has to be
-// idle: leaky ReLU 4567 x 8192 x 448 67 / 62, 72 / 70, 4567 x 4736 x 448 47 / 44, 50 / 48, but 8192 x 4736 x 448 70 / 70, 74 / 77 and
-// 4567 x 8192 x 768 92 / 84, 98 / 102; FP16 never.  Full rounds are the big kernel's: 8192 x 8192 x 448 with tanh 133 / 144.
-uint32_t gemm16_shared_limit(int fmt, int act, uint32_t big_tiles)
+// Longest K at which the single-stage kernel is the better one instead of 256 x 256 tiles.  A large tile has a compute unit to
+// itself, one wave per SIMD, so that the matrix cores idle during its epilogue and the last round is mostly empty; several of
+// the single-stage kernel's smaller workgroups share a compute unit and one's epilogue runs beside another's products.  The
+// sigmoids or tanhs of a large tile take 17 us.  Large tiles / single-stage, input conversion and a head of 16 included, tanh (a
+// sigmoid within 4 % of it), us:
+//                      of the rounds   FP16                                          INT8
+//   8192 x 8192        all     512 204 / 187   768 229 / 225  1024 253 / 267    1024 258 / 255  1536 310 / 334
+//   15144 x 6416       0.83   1536 623 / 536  2048 720 / 655  3072 926 / 926    2048 761 / 630  3072 993 / 872
+//   8192 x 4736        0.77   1024 179 / 166  1536 214 / 217  2048 248 / 269    1536 223 / 212  2048 260 / 264
+//   4567 x 8192        0.74   1024 187 / 164  1536 220 / 209  2048 246 / 257    2048 266 / 247  3072 339 / 334
+//   4567 x 4736        0.65   1024 124 / 110  1536 146 / 144  2048 168 / 169    2048 178 / 164
+//   4605 x 4128        0.57    512 102 /  72  1024 121 /  97                    1024 128 /  97
+//   4096 x 4096        one     256  59 /  54   512  65 /  65   768  72 /  78     512  66 /  65   768  72 /  76
+// (Below six tenths it pays for longer than the lines there, which tests of both kernels' epilogues stand on.)
+// Without a transcendental function a quarter of the rounds has to be idle, and the codes packed: leaky ReLU INT8 4567 x 4736 x
+// 256 56 / 50, x 512 69 / 65, x 1024 94 / 96; 4567 x 8192 x 448 94 / 90, x 768 116 / 119; FP16 62 / 63 and 89 / 96 at 448.
+uint32_t gemm16_shared_limit(int fmt, int act, uint32_t big_tiles, uint64_t outputs)
 {
-    const bool slow = act == A_TANH || act == A_SIGMOID, wide = fmt_bits(fmt) == 16;
+    const bool wide = fmt_bits(fmt) == 16;
     const uint32_t slots = (big_tiles + 255u) / 256u * 256u;
-    if (big_tiles <= 256u || 4u * slots < 5u * big_tiles) return 0;
-    if (slow) return wide ? 512u : 1024u;
-    return wide || 10u * slots < 13u * big_tiles ? 0u : 512u;
+    if (act == A_TANH || act == A_SIGMOID) {
+        const uint64_t tenth = (uint64_t)slots * 65536u / 10u;
+        if (big_tiles <= 256u) return 512u;
+        if (outputs > 9u * tenth) return wide ? 768u : 1024u;
+        if (outputs < 6u * tenth) return wide ? 512u : 1024u;
+        return wide ? 1536u : 2048u;
+    }
+    return wide || big_tiles <= 256u || 10u * slots < 13u * big_tiles ? 0u : 512u;
 }
 
 // K splits of the single-stage kernel for rows that are not whole 16-byte units (always 64 x 64 tiles, element-wise
@@ -1363,7 +1375,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     const bool split_ok = splits > 1 && (uint64_t)splits * halves * M * L.N <= ctx.ws_floats;
     const bool halves_ok = halves == 1 || (uint64_t)halves * M * L.N <= ctx.ws_floats;     // (checked by the caller's reserve)
     // (too few tiles and no K split, gemm16_splits: the single-stage kernel below)
-    const bool shared_cu = halves == 1 && bm == 256u && L.K <= gemm16_shared_limit(FMT, L.act, big_tiles);
+    const bool shared_cu = halves == 1 && bm == 256u && L.K <= gemm16_shared_limit(FMT, L.act, big_tiles, (uint64_t)M * L.N);
     if (aligned && !shared_cu && L.K >= 128u && M > 64 && L.N >= 256 && fits32 && (big_tiles >= 192u || split_ok) && halves_ok) {
         if (big_tiles >= 192u) g.kper = 0;
         else g.ksplits = splits;

@@ -606,6 +606,42 @@ def test_streamed_weights_at_the_edges_of_their_tiles(S, O, fmt, n, K, N):
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 2e-3
 
 
+@pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
+@pytest.mark.parametrize("n,K,N", [(100, 128, 49152), (100, 192, 49160), (128, 320, 49410), (65, 1024, 49153)])
+def test_tiles_of_128_rows_in_every_format(S, O, fmt, n, K, N):
+    """sp_gemm16_big with 128-row tiles, whole and partial K tiles, against the float64 forward.  (As above.)"""
+    src = make_oracle_net(O, [K, N], ["none"], seed=n + K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    h = S.lib().spingalett_hip_handle(net)
+    assert S.lib().sphip_layer_kernel_name(h, 1, n, 0).decode() == "sp_gemm16_big"
+    X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    S.free_network(net)
+    assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 2e-3
+
+
+@pytest.mark.parametrize("fmt,n,K,N,act,name", [
+    # one round, as many rounds as tiles fill, three rounds of which a quarter is idle, two of which a third is
+    ("f16", 4096, 512, 4096, "sigmoid", "sp_gemm16"), ("f16", 4096, 520, 4096, "tanh", "sp_gemm16_big"),
+    ("i8", 4096, 528, 4096, "sigmoid", "sp_gemm16_big"), ("i2", 4096, 512, 4096, "tanh", "sp_gemm16"),
+    ("bf16", 8192, 768, 8192, "tanh", "sp_gemm16"), ("bf16", 8192, 776, 8192, "tanh", "sp_gemm16_big"),
+    ("i4", 8192, 1024, 8192, "sigmoid", "sp_gemm16"), ("i4", 8192, 1056, 8192, "sigmoid", "sp_gemm16_big"),
+    ("f16", 4567, 1536, 8192, "tanh", "sp_gemm16"), ("f16", 4567, 1544, 8192, "sigmoid", "sp_gemm16_big"),
+    ("i8", 4567, 2048, 4736, "tanh", "sp_gemm16"), ("i8", 4567, 2064, 4736, "tanh", "sp_gemm16_big"),
+    ("i8", 4567, 512, 4736, "relu", "sp_gemm16"), ("i8", 4567, 528, 4736, "relu", "sp_gemm16_big"),
+])
+def test_which_kernel_takes_short_sums(S, fmt, n, K, N, act, name):
+    """Both sides of each line of gemm16_shared_limit (nothing is launched)."""
+    bits = {"f16": 16, "bf16": 16, "i8": 8, "i4": 4, "i2": 2}[fmt]
+    prec = {"f16": S.PRECISION_FP16, "bf16": S.PRECISION_BFLOAT16, "i8": S.PRECISION_INT8, "i4": S.PRECISION_INT4, "i2": S.PRECISION_INT2}[fmt]
+    d = S.DeviceNet([K, N], [{"sigmoid": S.ACT_SIGMOID, "tanh": S.ACT_TANH, "relu": S.ACT_RELU}[act]], prec)
+    for which, count in ((0, K * N), (1, N)):
+        d.upload(0, which, np.zeros(count * bits // 8, np.uint8), 1.0 if bits < 16 else 0.0)
+    got = S.lib().sphip_layer_kernel_name(d.h, 1, n, 0).decode()
+    d.destroy()
+    assert got == name
+
+
 @pytest.mark.parametrize("fmt,n,K,N,act", [
     ("f16", 4095, 576, 4088, "tanh"), ("i8", 4090, 576, 4086, "sigmoid"),      # whole units, and rows that are not
     ("i2", 4090, 640, 4086, "tanh"), ("bf16", 3900, 528, 4083, "sigmoid"),
@@ -625,6 +661,31 @@ def test_large_tiles_with_sigmoid_and_tanh(S, O, fmt, n, K, N, act):
         got = S.forward_batch(net, X)
         S.free_network(net)
         assert rel_max_abs(got, ref.forward_batch_f64(X)) <= (8e-3 if fmt == "bf16" else 2e-3)
+
+
+def test_large_tiles_apply_the_library_s_tanh(S):
+    """tanh of sp_gemm16_big, written without tanhf's branch, bit by bit that of the single-stage kernel: both sides of 0.625,
+    zeros of either sign, subnormal and huge sums, infinities and NaN.  (One term per sum, so that no order of sums matters.)"""
+    N, n = 4096, 4096
+    edge = np.array([0.0, -0.0, 0.625, -0.625, 0.62451171875, 0.62548828125, 6e-8, -6e-8, 1e-4, 9.0, 9.1, -20.0, 65504.0,
+                     np.inf, -np.inf, np.nan], np.float16)
+    w = np.concatenate([edge, np.linspace(-10, 10, N - edge.size).astype(np.float16)])
+    X = np.zeros((n, 576), F32)
+    X[:, 0] = np.linspace(0.5, 1.5, n).astype(np.float16)
+    out = []
+    for K, name in ((576, "sp_gemm16_big"), (512, "sp_gemm16")):
+        W = np.zeros((N, K), np.float16)
+        W[:, 0] = w
+        d = S.DeviceNet([K, N], [S.ACT_TANH], S.PRECISION_FP16)
+        d.upload(0, 0, W.ravel().view(np.uint8))
+        d.upload(0, 1, np.zeros(N, np.float16).view(np.uint8))
+        assert S.lib().sphip_layer_kernel_name(d.h, 1, n, 0).decode() == name
+        out.append(d.forward(np.ascontiguousarray(X[:, :K])))
+        d.destroy()
+    a, b = (o.view(np.uint32) for o in out)
+    assert np.array_equal(a[:, :13], b[:, :13]) and np.array_equal(a[:, 16:], b[:, 16:])
+    assert np.array_equal(out[0][:, 13:], out[1][:, 13:], equal_nan=True) and np.all(np.isnan(out[0][:, 15]))
+    assert np.all(out[0][:, 13] == 1.0) and np.all(out[0][:, 14] == -1.0)
 
 
 def test_large_tiles_saturate_and_keep_infinities_block_by_block(S):
