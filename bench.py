@@ -183,7 +183,9 @@ def load_traffic():
             entries = json.load(f)["entries"]
     except (OSError, ValueError, KeyError):
         return {}
-    return {(e["kernel"], tuple(e["shape"])): e["bytes"] for e in entries}
+    from bench_traffic import kernel_source
+    now = {k: kernel_source(k) for k in {e["kernel"] for e in entries}}       # (a kernel replaced under its name has none)
+    return {(e["kernel"], tuple(e["shape"])): e["bytes"] for e in entries if e.get("source") == now[e["kernel"]]}
 
 
 PROFILED_TRAFFIC = load_traffic()

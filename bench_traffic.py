@@ -11,18 +11,38 @@ FETCH_SIZE / WRITE_SIZE are read per dispatch.  The dispatches of the dominant l
 whose reading is within 20 % of that kernel's largest (the other layers of the net are smaller).  Each counter is scaled
 by what it reads for the plain copy of the net's largest array that --calibrate-copy makes in the same run (a copy
 kernel reads and writes exactly that many bytes).  bytes = fetch + write of one launch (times --launches for a batch that
-runs in blocks of rows), what bench.py reports as roofline.traffic.  No GPU is needed to run this script.
+runs in blocks of rows), what bench.py reports as roofline.traffic, as long as the kernel's definition is the measured
+one.  No GPU is needed to run this script.
 """
 from __future__ import annotations
 
 import argparse
 import csv
 import glob
+import hashlib
 import json
 import os
+import re
 import sys
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
+
+
+def kernel_source(kernel: str) -> str:
+    """Digest of the kernel's definition, comments and white space left out; None where no source defines it.  An entry
+    measured on another definition is none of this kernel."""
+    body = []
+    for f in sorted(glob.glob(os.path.join(ROOT, "spingalett_amd", "csrc", "hip_*"))):
+        if not f.endswith((".inl", ".hip")):
+            continue
+        with open(f) as fh:
+            text = fh.read()
+        for m in re.finditer(r"__global__[^{;]*?\b%s\(" % re.escape(kernel), text):
+            body.append(text[m.start():text.index("\n}\n", m.start())])
+    if not body:
+        return None
+    plain = re.sub(r"\s+", "", re.sub(r"//[^\n]*", "", "\n".join(body)))
+    return hashlib.sha256(plain.encode()).hexdigest()[:16]
 
 
 def readings(directory: str, counter: str):
@@ -89,7 +109,7 @@ def main():
     f_factor = copy_bytes / 1024.0 / copy_reading(fetch_rows)      # KiB of real traffic per counter unit
     w_factor = copy_bytes / 1024.0 / copy_reading(write_rows)
     entry = {
-        "kernel": args.kernel, "shape": [args.batch, N, K], "workload": args.workload, "batch": args.batch,
+        "kernel": args.kernel, "source": kernel_source(args.kernel), "shape": [args.batch, N, K], "workload": args.workload, "batch": args.batch,
         "fetch_per_dispatch": round(fetch, 1), "write_per_dispatch": round(write, 1), "dispatches_averaged": nf,
         "fetch_factor_kib": round(f_factor, 4), "write_factor_kib": round(w_factor, 4),
         "calibration_copy_bytes": copy_bytes,
