@@ -1096,8 +1096,8 @@ struct ThinPlan {
 // against 41 / 54 us and 16384 x 16384 INT8 108 / 175 against 119 / 145 us (tiles from 129); 16384 x 16384 INT4 82 / 141
 // against 104 / 143 us, 4096 x 16384 INT4 34 / 54 against 52 / 71 us, 8192 x 8192 INT2 29 / 44 against 40 / 52 us (streaming
 // up to 256).  The fewer bytes a code has, the longer re-reading the weights per block of 64 samples pays.
-// Layers of a few megabytes stay with the streaming kernel up to 256 samples (the 784-512-1000-10 INT8 net: 36 us
-// against 57 us at 256 samples).
+// Layers of a few megabytes stay with the streaming kernel up to 256 samples, where the tiles would be a handful.  Sums of up to
+// 1024 leave it at 65: the tiles take them without a K split (8192 x 784 INT8 at 128 samples 20 -> 13 us).
 uint32_t thin_max_samples(int fmt, uint32_t N, uint32_t K)
 {
     if (K <= 1024u) return 64u;

@@ -594,7 +594,7 @@ __device__ __forceinline__ void frag_reads(u32x4 *dst, uint32_t addr)
 //
 // The accumulators are accumulation registers by number (mfma_acc, acc_read): left to the compiler, 256 of them next to the
 // fragments are spilled.  Nothing else here lives in those registers (the first statement claims all of them, and the
-// vector registers suffice for the rest).
+// vector registers suffice for the rest; the Makefile refuses a build with a spill in this kernel, which could go there).
 //
 // One wave per SIMD has nobody to hide behind, so the loop is straight-line code with everything asked for ahead:
 //   * A K tile is RM quads of sixteen products (four row tiles x four column tiles).  Consecutive quads share one of their
@@ -1283,8 +1283,8 @@ __global__ __launch_bounds__(256, 1) void sp_gemm16_big(const GemmArgs g)
 }
 
 // The parts of four neighbouring sums, `stride` float4 apart: the first `splits` added in order into sum, the others into low.
-// Four are on their way at a time: one after the other, each is a round trip to memory (four parts of 50 x 8192 sums 4.9 ->
-// RED us, sixteen of 50 x 1000 7.4 -> RED2).
+// Four are on their way at a time: one after the other, each is a round trip to memory (sixteen parts of 50 x 1000 sums 6.9 ->
+// 6.4 us; four of 50 x 8192, which fill the chip, 4.8 / 4.9).
 __device__ __forceinline__ void add_parts(const float4 *at, uint64_t stride, uint32_t splits, uint32_t parts, float4 &sum, float4 &low)
 {
     sum = low = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
