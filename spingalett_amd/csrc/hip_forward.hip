@@ -981,28 +981,27 @@ void launch_gemv(int prec, const Workspace &wk, const LayerArgs &L, const float 
 
 // Rows of a tile of the big GEMM.  128 x 256 tiles instead of partly filled or too few 256 x 256 ones: up to 128
 // samples always (a single row of tiles), and for 16-bit weights, which reach LDS by DMA, whenever 256-row tiles
-// would be fewer than 192 (8192 x 8192 BF16 at 256 / 512 / 1024 samples 47.9 / 79.5 / 137 against 53.5 / 82.3 / 150 us,
-// 4096 x 4096 at 1024 samples 50.5 against 54.4, 8192 x 2048 FP16 at 768 samples 37.7 against 64.2 us: twice the
-// tiles, half the K splits or none).  Integer weights pass through registers and are unpacked once per tile: half the
-// rows per unpacked tile cost more than the tiles bring (8192 x 8192 INT2 at 512 samples 93.9 against 81.5 us, INT8
-// at 1024 samples 171 against 162).  With enough 256 x 256 tiles the smaller tile is no faster (8192-wide layers
-// from 1536 samples).
+// would be fewer than 192 (8192 x 8192 BF16 at 256 / 512 / 1024 samples 48.5 / 85.0 / 132 against 58.0 / 85.9 / 144 us, 4096 x
+// 4096 at 1024 samples 53.7 against 59.3: twice the tiles, half the K splits or none; but sums of 8192 into 2048 outputs at 768
+// samples 58.7 against 53.5).  Integer weights are unpacked once per tile: half the rows per unpacked tile cost more than the
+// tiles bring (8192 x 8192 INT2 at 512 samples 91.4 against 86.1 us, INT8 at 1024 samples 155 against 149).  With enough
+// 256 x 256 tiles the smaller tile is no faster (8192-wide layers from 1536 samples).
 uint32_t gemm16_tile_rows(int fmt, uint32_t M, uint32_t N)
 {
     if (M <= 128u) return 128u;
     if (fmt_bits(fmt) != 16) return 256u;
-    // ... and 128-row tiles are at most one per compute unit (more of them run in two rounds, the second mostly
-    // empty: 8192 x 8192 at 1100 samples 242 against 225 us)
+    // ... and 128-row tiles are at most one per compute unit (more of them run in two rounds; where the line lay for the kernel
+    // of eight waves, 8192 x 8192 at 1100 samples 242 against 225 us, and for this one not measured but there, 202 against 221)
     const uint32_t cols = (N + 255u) / 256u;
     return ((M + 255u) / 256u) * cols < 192u && ((M + 127u) / 128u) * cols <= 256u ? 128u : 256u;
 }
 
 // K splits of the tile GEMM when its tiles would leave compute units idle: from K = 4096 on (16-bit weights, which reach
-// LDS by DMA: 3072), at least eight K tiles each.  Below, the single-stage kernel's small tiles fill the chip in one launch and no partial sums travel (forward
-// of one layer, conversion of the input included, K split here against single stage: 4096 x 512 x 1024 FP16 24.8
-// against 13.3 us, 1024 x 4096 x 1024 32.6 against 26.1 us, 1024 x 2048 x 2048 31.1 against 26.0 us, INT8 34.4 against
-// 27.3 us; at K = 3072 FP16 128 x 4096 x 3072 21.7 against 26.9 us, 1024 x 2048 x 3072 even, INT8 40.5 against 37.6 us; from
-// K = 4096 the long walk pays: 512 x 2048 x 4096 30.4 against 37.1 us, 256 x 8192 x 8192 53 against 82 us)
+// LDS by DMA: 3072), at least eight K tiles each.  Below, the single-stage kernel's small tiles fill the chip in one launch and
+// no partial sums travel (forward of one layer, conversion of the input included, K split here against single stage: 1024 x 2048
+// x 2048 FP16 31.0 against 25.5 us, at K = 3072 128 x 4096 21.7 against 26.5 and 1024 x 2048 even, 512 x 2048 x 4096 30.5 against
+// 36.2, 256 x 8192 x 8192 49 against 84; INT8 1024 x 2048 x 3072 42.5 against 36.9, x 4096 47.8 against 45.9, INT4 600 x 4096 x
+// 3584 59 against 50)
 uint32_t gemm16_splits(int fmt, uint32_t M, uint32_t N, uint32_t K, uint32_t *kper)
 {
     const uint32_t bm = gemm16_tile_rows(fmt, M, N);
