@@ -1577,11 +1577,12 @@ uint32_t gemm32_parts_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper)
 // Tiles of 64 rows where those of 128 would be one on some compute units and two on others (256 to 383: twice as many are
 // still resident at once; 10000 x 512 x 784 82 -> 71 us, 4096 x 1000 x 1000 78 -> 68, but 512 tiles of 2000 x 4096 x 4096 359
 // -> 390), and for short sums, which are mostly load, split and store (8192 x 16384 x 64 230 -> 200 us)
-void launch_gemm32_parts(const PartsGemm32Args &g, uint32_t splits)
+void launch_gemm32_parts(const PartsGemm32Args &g, uint32_t splits, bool rows64)
 {
     const uint32_t cols = (g.N + 127u) / 128u;
     const uint64_t tiles = (g.M + 127ull) / 128u * cols;
-    if (splits == 1u && ((tiles >= 256u && tiles < 384u) || g.K <= 128u)) sp_gemm32_bf16_parts<1><<<(g.M + 63u) / 64u * cols, 256, 0, g_stream>>>(g);
+    if (rows64 || (splits == 1u && ((tiles >= 256u && tiles < 384u) || g.K <= 128u)))
+        sp_gemm32_bf16_parts<1><<<dim3((g.M + 63u) / 64u * cols, splits), 256, 0, g_stream>>>(g);
     else sp_gemm32_bf16_parts<2><<<dim3((g.M + 127u) / 128u * cols, splits), 256, 0, g_stream>>>(g);
 }
 
@@ -1596,6 +1597,19 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
     if (!training && gemm32_parts_pay(batch, L.N, L.K)) {
         PartsGemm32Args b{};
         uint32_t parts = gemm32_parts_splits(M, L.N, L.K, &b.kper);
+        // A block of rows of a larger batch, which would be cut into many partial sums: tiles of 64 rows, in as few parts as
+        // give every compute unit one (10000 samples of 784-512-1000-10 evaluated in blocks of 2560 rows 976 -> 910 us in
+        // 128-row tiles of six and four parts / these; 870 in the FP32 kernels, whose sums are further off).
+        const uint64_t tiles64 = (M + 63ull) / 64u * ((L.N + 127u) / 128u);
+        const bool rows64 = M < batch && parts > 1;
+        if (rows64) {
+            const uint32_t ktiles = (L.K + 31u) / 32u, fewer = (uint32_t)((255u + tiles64) / tiles64);
+            if (fewer < parts) {
+                const uint32_t per = (ktiles + fewer - 1u) / fewer;
+                b.kper = per * 32u;
+                parts = (ktiles + per - 1u) / per;
+            }
+        }
         if (parts > 1 && (uint64_t)parts * M * L.N > ws_floats) { parts = 1; b.kper = (L.K + 31u) / 32u * 32u; }
         tl_route.name = "sp_gemm32_bf16_parts";
         if (tl_route.dry) return false;
@@ -1603,7 +1617,7 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
         b.M = M; b.N = L.N; b.K = L.K;
         b.vec = vec;
         b.bias = L.bias; b.bscale = L.bscale; b.bias_fmt = L.bias_fmt; b.act = L.act;
-        launch_gemm32_parts(b, parts);
+        launch_gemm32_parts(b, parts, rows64);
         if (parts > 1) {
             g.ws = ws;
             sp_gemm32_reduce<<<(uint32_t)(((uint64_t)M * L.N + 255) / 256), 256, 0, g_stream>>>(g, parts);
