@@ -1078,14 +1078,15 @@ struct ThinCtx {
 struct ThinPlan {
     bool use;
     bool mode_b;
-    bool kw;               // thin operand of <= 8 rows (<= 16 outputs): K split among the waves of a workgroup (sp_skinny16_kw)
-    int ncp;               // thin rows held in LDS in that case
+    bool kw;               // thin operand of <= 8 rows: K split among the waves of a workgroup (sp_skinny16_kw)
     int nw;                // waves per workgroup in that case (4 or 8)
+    bool head;             // few outputs: sp_skinny16_kw_head
+    int nt;                // sixteens of outputs in that case
     uint32_t R, NC;        // streamed rows, thin rows
     int rt, ct;
     int nwv;               // waves per workgroup of sp_skinny16_regs
     bool regs;             // sp_skinny16_regs instead of sp_skinny16
-    int st;                // sixteens of samples per workgroup of sp_skinny16
+    int st;                // sixteens of samples per workgroup of sp_skinny16 and sp_skinny16_kw_head
     uint32_t splits, kper, row_blocks, cblocks;
 };
 
@@ -1135,7 +1136,32 @@ uint32_t thin_splits(int fmt, int st, uint32_t wgs, uint32_t chunks, uint64_t ou
 ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K, uint64_t most_sums = ~0ull)
 {
     ThinPlan p{};
-    if (N <= 64 && K % 8u == 0 && M >= 1) {
+    // Few outputs: sp_skinny16_kw_head, one launch.  Against sp_skinny16_regs and its reduction (more than 16 outputs; us, FP16):
+    // 1024 x 20 at 16 / 1000 / 16384 samples 12.8 / 15.5 / 42.4 -> 7.6 / 8.7 / 27.6, 1536 x 48 14.5 / 18.4 / 56.6 -> 12.5 / 14.4 /
+    // 43.6.  Its eight waves are all the K split there is, and a workgroup reads all weights for its samples: few samples of
+    // longer sums into 33 to 64 outputs are left to the split (2048 x 50 at 16 samples 12.7 against 13.1, at 256 18.4 against
+    // 16.5; 3072 x 40 at 64 16.4 against 17.3, at 1000 21.7 against 20.4).  Up to 16 outputs a split pays beyond 4096 only (4096 x 10 at
+    // 64 samples 11.1 without, 14.0 in two parts; 8192 x 10 17.9 and, in four, 14.5).  Two sixteens of samples a workgroup where
+    // there are enough to fill the chip with them (1024 x 33 at 8192 samples 23.4 -> 20.9, at 4096 16.5 -> 17.2), not with one of
+    // outputs (1000 x 10 at 8192 samples 15.3 -> 16.7 in workgroups of 64).
+    const int nt = N <= 16u ? 1 : N <= 32u ? 2 : 4;
+    if (N <= 64 && K % 8u == 0 && M >= 1 &&
+        (nt == 1 || K * nt <= 6144u || (K <= 2048u && M >= 128u) || (K <= 3072u && M >= 1000u))) {
+        p.use = p.mode_b = p.head = true; p.R = M; p.NC = N;
+        p.nt = nt;
+        p.st = p.nt > 1 && M >= 8192u ? 2 : 1;
+        p.cblocks = 1;
+        p.row_blocks = (M + 16u * p.st - 1u) / (16u * p.st);
+        const uint32_t steps = (K + 31u) / 32u;
+        uint32_t splits = K > 4096u ? K / 2048u : 1u;
+        if (splits > 256u / p.row_blocks) splits = 256u / p.row_blocks;
+        if (splits > 16u) splits = 16u;
+        if (splits < 1u) splits = 1u;
+        const uint32_t per = (steps + splits - 1u) / splits;
+        p.kper = per * 32u;
+        p.splits = (steps + per - 1u) / per;
+        return p;
+    } else if (N <= 64 && K % 8u == 0 && M >= 1) {
         p.use = true; p.mode_b = true; p.R = M; p.NC = N;
     } else if (M >= 16u && (uint64_t)N * K <= (128u << 10)) {
         // a layer of a few hundred rows and columns gives this kernel two or three workgroups, each fetching the whole
@@ -1160,21 +1186,17 @@ ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K, uint64_t most_su
     // up to 32 MB of streamed bytes, slower beyond (16384 x 16384 INT4 at 8 samples: 40 us against 34 us).
     const uint64_t streamed_bytes = (uint64_t)p.R * K * (uint64_t)fmt_bits(sfmt) / 8u;
     const bool kw_pays = sfmt == I8 || streamed_bytes <= ((sfmt == I4 || sfmt == I2) ? (64ull << 20) : (32ull << 20));
-    // A classifier head (at most 16 outputs, activations streamed) takes the same kernel with 16 thin rows; up to 32
-    // chunks of K it runs without a K split across workgroups: one launch, and a softmax can be done in its epilogue.
-    const bool head = p.mode_b && p.NC <= 16u;
-    if ((p.NC <= 8u && kw_pays) || head) {
+    if (p.NC <= 8u && kw_pays) {
         // one workgroup per 32 streamed rows, its four waves share K; K is split across workgroups as well only
         // when the rows alone do not fill the chip
         p.kw = true;
-        p.ncp = p.NC <= 8u ? 8 : 16;
         p.rt = p.ct = 1;
         p.cblocks = 1;
         p.row_blocks = (p.R + 31u) / 32u;
         const uint32_t chunks = (K + bkc - 1) / bkc;
         // 6144 to 12287 streamed rows: eight waves per workgroup instead of a K split across two workgroups
-        p.nw = (p.ncp == 8 && p.row_blocks >= 192u && p.row_blocks < 384u && chunks >= 16u) ? 8 : 4;
-        uint32_t splits = (p.row_blocks >= 192u || (head && chunks <= 32u)) ? 1u : (512u + p.row_blocks - 1) / p.row_blocks;
+        p.nw = (p.row_blocks >= 192u && p.row_blocks < 384u && chunks >= 16u) ? 8 : 4;
+        uint32_t splits = p.row_blocks >= 192u ? 1u : (512u + p.row_blocks - 1) / p.row_blocks;
         if (splits > 16u) splits = 16u;
         if (splits > chunks / 4u) splits = chunks / 4u;
         if (splits < 1u) splits = 1u;
@@ -1249,36 +1271,45 @@ void launch_thin_dma(const SkinnyArgs &a, const ThinPlan &p)
     kern<<<dim3(gx, p.splits * a.halves, 1), 512, lds, g_stream>>>(a);
 }
 
-template <int SFMT, bool F16T, int NCP, int NW>
+template <int SFMT, bool F16T, int NW>
 void launch_thin_kw(const SkinnyArgs &a, const ThinPlan &p)
 {
     if (tl_route.dry) return;
-    constexpr size_t lds = (size_t)NW * 2 * NCP * SkinnyFmt<SFMT>::PITCH + (size_t)NW * (NCP / 2) * 64 * sizeof(float);
-    auto kern = sp_skinny16_kw<SFMT, F16T, NCP, NW>;
+    constexpr size_t lds = (size_t)NW * 2 * 8 * SkinnyFmt<SFMT>::PITCH + (size_t)NW * 4 * 64 * sizeof(float);
+    auto kern = sp_skinny16_kw<SFMT, F16T, NW>;
     static bool once = ((void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), true);
     (void)once;
     kern<<<dim3(p.row_blocks, p.splits * a.halves, 1), 64 * NW, lds, g_stream>>>(a);
 }
 
+template <bool F16T, int HALVES>
+void launch_thin_head(const SkinnyArgs &a, const ThinPlan &p)
+{
+    if (tl_route.dry) return;
+    const dim3 grid(p.row_blocks, p.splits);
+    if (p.nt == 1) sp_skinny16_kw_head<F16T, 1, 1, HALVES><<<grid, 512, 0, g_stream>>>(a);
+    else if (p.nt == 2 && p.st == 1) sp_skinny16_kw_head<F16T, 2, 1, HALVES><<<grid, 512, 0, g_stream>>>(a);
+    else if (p.nt == 2) sp_skinny16_kw_head<F16T, 2, 2, HALVES><<<grid, 512, 0, g_stream>>>(a);
+    else if (p.st == 1) sp_skinny16_kw_head<F16T, 4, 1, HALVES><<<grid, 512, 0, g_stream>>>(a);
+    else sp_skinny16_kw_head<F16T, 4, 2, HALVES><<<grid, 512, 0, g_stream>>>(a);
+}
+
 template <int SFMT, bool F16T>
 void launch_thin(SkinnyArgs a, const ThinPlan &p)
 {
-    if (p.splits == 1 && a.halves == 1) a.ws = nullptr;
+    if (p.splits == 1 && (a.halves == 1 || p.head)) a.ws = nullptr;
     a.ksplits = p.splits;
-    if (p.kw) {
-        bool wide = false;                      // 16 thin rows: classifier heads only, which stream 16-bit activations
-        if constexpr (SFMT == F16 || SFMT == BF16) {
-            if (p.ncp == 16) {
-                launch_thin_kw<SFMT, F16T, 16, 4>(a, p);
-                wide = true;
-            }
-        }
-        if (wide) {
-        } else if (p.nw == 8) {
-            launch_thin_kw<SFMT, F16T, 8, 8>(a, p);
+    a.parts = p.head ? p.splits : p.splits * a.halves;
+    if (p.head) {
+        if constexpr (F16T) {
+            if (a.halves == 2) launch_thin_head<true, 2>(a, p);
+            else launch_thin_head<true, 1>(a, p);
         } else {
-            launch_thin_kw<SFMT, F16T, 8, 4>(a, p);
+            launch_thin_head<false, 1>(a, p);
         }
+    } else if (p.kw) {
+        if (p.nw == 8) launch_thin_kw<SFMT, F16T, 8>(a, p);
+        else launch_thin_kw<SFMT, F16T, 4>(a, p);
     } else if (!p.regs) {
         if (p.st == 1) launch_thin_dma<SFMT, F16T, 1>(a, p);
         else if (p.st == 2) launch_thin_dma<SFMT, F16T, 2>(a, p);
@@ -1343,13 +1374,13 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     }
     const ThinPlan tp = plan_thin(FMT, M, L.N, L.K, ctx.ws_floats / halves);
     if (tp.use && !single && (!tp.mode_b || ctx.w16) &&
-        ((tp.splits == 1 && halves == 1) || (uint64_t)tp.splits * halves * tp.NC * tp.R <= ctx.ws_floats)) {
+        ((tp.splits == 1 && (halves == 1 || tp.head)) || (uint64_t)tp.splits * halves * tp.NC * tp.R <= ctx.ws_floats)) {
         SkinnyArgs a{};
         a.halves = halves; a.half_elems = (uint64_t)M * L.K;
         a.L = L; a.C = C; a.ws = ctx.ws; a.R = tp.R; a.NC = tp.NC; a.row_blocks = tp.row_blocks; a.cblocks = tp.cblocks; a.kper = tp.kper; a.out_f32 = out_f32; a.mode_b = tp.mode_b ? 1 : 0;
-        tl_route.name = tp.kw ? "sp_skinny16_kw" : tp.regs ? "sp_skinny16_regs" : "sp_skinny16";
+        tl_route.name = tp.kw || tp.head ? "sp_skinny16_kw" : tp.regs ? "sp_skinny16_regs" : "sp_skinny16";
         if (tp.mode_b) {
-            if (ctx.soft_out && tp.kw && tp.splits == 1 && halves == 1) {
+            if (ctx.soft_out && tp.head && tp.splits == 1 && ctx.soft_kind != 3) {
                 a.soft_out = ctx.soft_out;
                 a.soft_kind = ctx.soft_kind;
                 *ctx.soft_done = true;
@@ -1722,7 +1753,7 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             const ThinPlan tp = plan_thin(F16, n, N, K3);
             if (tp.use) {
                 if (tp.splits > 1) ws = (uint64_t)tp.splits * tp.NC * tp.R;
-                if (!tp.kw && !tp.regs) spare = ws;
+                if (!tp.kw && !tp.regs && !tp.head) spare = ws;
             } else {
                 const uint32_t sp = gemm16_splits(F16, n, N, K3, &kper);
                 if (sp > 1) ws = (uint64_t)sp * n * N;
@@ -1737,7 +1768,7 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             const ThinPlan tp = plan_thin(net->prec, n, N, K);
             if (tp.use) {
                 if (tp.splits > 1 || halves > 1) ws = (uint64_t)tp.splits * halves * tp.NC * tp.R;
-                if (!tp.kw && !tp.regs) spare = ws - (halves > 1 ? (uint64_t)halves * tp.NC * tp.R : 0u);
+                if (!tp.kw && !tp.regs && !tp.head) spare = ws - (halves > 1 ? (uint64_t)halves * tp.NC * tp.R : 0u);
             } else {
                 const uint32_t sp = gemm16_splits(net->prec, n, N, K, &kper);
                 if (sp > 1 || halves > 1) ws = (uint64_t)sp * halves * n * N;

@@ -27,12 +27,13 @@ struct SkinnyArgs {
     uint32_t kper;           // codes per K split (whole chunks)
     int out_f32;
     int mode_b;              // 0: streamed rows are outputs, thin rows samples; 1: the reverse
-    void *soft_out;          // sp_skinny16_kw, mode_b, no K split: softmax over a sample's outputs goes here instead of C
+    void *soft_out;          // sp_skinny16_kw_head without a K split: softmax over a sample's outputs goes here instead of C
     int soft_kind;           // its element type: 0 FP32, 1 BF16, 2 FP16
     // Split activations (GemmArgs has the layout): grid y = halves x ksplits, y / ksplits picks the activation matrix
     // (the thin operand, or the streamed one in mode b), y % ksplits the K range.
     uint32_t ksplits;        // K splits (>= 1)
     uint32_t halves;         // 1, or 2 with split activations
+    uint32_t parts;          // partial sums of an output in ws: ksplits x halves, or ksplits where a workgroup adds the halves
     uint64_t half_elems;     // elements between the two activation matrices (samples x K)
 };
 
@@ -775,16 +776,17 @@ __global__ __launch_bounds__(512) void sp_skinny16(const SkinnyArgs a)
     });
 }
 
-// Variant for a thin operand of at most NCP (8 or 16; the host uses 8) rows: the NW waves of a workgroup share one tile of 32
+// Variant for a thin operand of at most eight rows: the NW waves of a workgroup share one tile of 32
 // streamed rows and split K among themselves (wave w takes chunks w, w + NW, ...), so that a layer with many streamed
 // rows needs no K split across workgroups, no partial sums in memory and no second launch.  Each wave stages its own
 // thin chunks in its own LDS region (no workgroup barrier in the loop); the NW accumulator tiles meet in LDS at the
 // end and are added in wave order.  Loads and their bookkeeping are those of sp_skinny16_regs.
-template <int FMT, bool F16T, int NCP, int NW>
+template <int FMT, bool F16T, int NW>
 __global__ __launch_bounds__(64 * NW) void sp_skinny16_kw(const SkinnyArgs a)
 {
     using F = SkinnyFmt<FMT>;
     constexpr int EPL = F::EPL, LPC = F::LPC, BKC = F::BKC, STEPS = F::STEPS, PITCH = F::PITCH;
+    constexpr int NCP = 8;                                 // thin rows held in LDS
     constexpr int UNITS = NCP * (BKC / 16);                // 16-code units of one thin chunk
     constexpr int UPL = (UNITS + 63) / 64;                 // units per lane
     constexpr int STAGE = NCP * PITCH;
@@ -797,8 +799,8 @@ __global__ __launch_bounds__(64 * NW) void sp_skinny16_kw(const SkinnyArgs a)
     const uint32_t K = a.L.K;
     const uint32_t r_out = blockIdx.x * 32u + n31;
     const uint32_t half = blockIdx.y / a.ksplits;
-    const uint8_t *const stream = a.mode_b ? a.stream + (size_t)half * a.half_elems * 2u : a.stream;
-    const uint16_t *const thin = a.mode_b ? a.thin : a.thin + (size_t)half * a.half_elems;
+    const uint8_t *const stream = a.stream;
+    const uint16_t *const thin = a.thin + (size_t)half * a.half_elems;
     const uint32_t kbeg = (blockIdx.y % a.ksplits) * a.kper;
     const uint32_t kend = kbeg + a.kper < K ? kbeg + a.kper : K;
     const uint32_t nchunks = (kend - kbeg + BKC - 1) / BKC;
@@ -961,43 +963,6 @@ __global__ __launch_bounds__(64 * NW) void sp_skinny16_kw(const SkinnyArgs a)
     for (int q = 0; q < NQ; ++q) red[(wave * NQ + q) * 64 + lane] = acc[q];
     __syncthreads();
     if (wave != 0 || r_out >= a.R) return;
-    if (a.soft_out) {
-        // the thin rows are all the outputs of sample r_out, half of them in lane n31 and half in lane n31 + 32:
-        // softmax as Activation.c:5-21 (largest logit subtracted, exponentials, one division by their sum)
-        float v[NQ];
-        float m = -3.402823466e+38f;
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const uint32_t c = 8u * (q >> 2) + 4u * h + (q & 3);
-            float sum = 0.0f;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) sum += red[(w * NQ + q) * 64 + lane];
-            const float bias = elem_value_rt(a.L.bias_fmt, a.L.bias, c < a.NC ? c : 0u) * a.L.bscale;
-            v[q] = c < a.NC ? fmaf(sum, a.L.wscale, bias) : -3.402823466e+38f;
-            m = fmaxf(m, v[q]);
-        }
-        m = fmaxf(m, __shfl_xor(m, 32));
-        float s = 0.0f;
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const uint32_t c = 8u * (q >> 2) + 4u * h + (q & 3);
-            v[q] = c < a.NC ? expf(v[q] - m) : 0.0f;
-            s += v[q];
-        }
-        s += __shfl_xor(s, 32);
-        const float inv = s > 0.0f ? 1.0f / s : 1.0f;
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const uint32_t c = 8u * (q >> 2) + 4u * h + (q & 3);
-            if (c >= a.NC) continue;
-            const size_t o = (size_t)r_out * a.L.N + c;
-            const float y = v[q] * inv;
-            if (a.soft_kind == 0) reinterpret_cast<float *>(a.soft_out)[o] = y;
-            else if (a.soft_kind == 1) reinterpret_cast<uint16_t *>(a.soft_out)[o] = f32_to_bf16_rne(y);
-            else reinterpret_cast<uint16_t *>(a.soft_out)[o] = f32_to_f16_sat(y);
-        }
-        return;
-    }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const uint32_t c = 8u * (q >> 2) + 4u * h + (q & 3);
@@ -1010,9 +975,6 @@ __global__ __launch_bounds__(64 * NW) void sp_skinny16_kw(const SkinnyArgs a)
     }
 }
 
-// adds the partial sums of sp_skinny16 (K splits in split order; with split activations the sums of the second matrix,
-// scaled by 2^-11, after those of the first) and applies bias and activation; a thread takes four neighbouring
-// streamed rows (VEC: R is a multiple of four and the rows are outputs, so they are neighbours in C as well) or one
 template <bool F16T>
 __device__ __forceinline__ void skinny_store(const SkinnyArgs &a, size_t o, float v)
 {
@@ -1026,11 +988,185 @@ __device__ __forceinline__ void skinny_store(const SkinnyArgs &a, size_t o, floa
     } else reinterpret_cast<uint16_t *>(a.C)[o] = f32_to_t16<F16T>(v);
 }
 
+// Layers of at most 64 outputs (classifier heads, narrow layers): a workgroup owns 16 ST samples and all NT sixteens of outputs,
+// its eight waves split K.  Nothing is staged: lane (l15, q4) loads 16 bytes of row l15 of a tile at k = 32 s + 8 q4 straight
+// into registers, U steps of both operands at once and the next U while these are multiplied, and the waves' sums meet in
+// LDS.  What bounds such a layer below a few thousand samples is the latency of its chain of loads, not their bytes: up to
+// K = 1024 there is one round of them.  (The kernels before staged the samples of each chunk of K through LDS, a round trip
+// to memory per chunk, and cut K over the grid with a second launch for more than 16 outputs.)  From a few thousand samples on the
+// weights' reads from L2 count, so workgroups take more samples (ST).  A layer, conversion of its input included: 1000 x 10 at 16 /
+// 256 / 8192 samples 8.3 / 8.8 / 17.0 -> 6.4 / 6.5 / 14.9 us, 4096 x 10 at 256 16.5 -> 11.9; more outputs at plan_thin.
+// HALVES == 2: split activations as in sp_gemm16_small.
+template <bool F16T, int NT, int ST, int HALVES>
+__global__ __launch_bounds__(512) void sp_skinny16_kw_head(const SkinnyArgs a)
+{
+    static_assert(HALVES == 1 || F16T, "split activations are FP16");
+    constexpr int NW = 8, U = NT + ST * HALVES <= 5 ? 4 : 2;
+    __shared__ f32x4 part[NW][NT * ST * 64];
+    __shared__ float bias_of[NT * 16];
+    const uint32_t t = threadIdx.x, lane = t & 63u, l15 = lane & 15u, q4 = lane >> 4;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t >> 6));
+    const uint32_t K = a.L.K, m0 = blockIdx.x * (16u * ST);
+    const uint32_t kbeg = blockIdx.y * a.kper, kend = kbeg + a.kper < K ? kbeg + a.kper : K;
+    const uint32_t steps = (kend - kbeg + 31u) / 32u, per = (steps + NW - 1) / NW;
+    const uint32_t s0 = wave * per, s1 = s0 + per < steps ? s0 + per : steps;
+
+    if (t < NT * 16u && !a.ws) bias_of[t] = t < a.NC ? elem_value_rt(a.L.bias_fmt, a.L.bias, t) * a.L.bscale : 0.0f;
+    const uint16_t *wp[NT], *xp[ST];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const uint32_t n = 16u * i + l15;
+        wp[i] = a.thin + (size_t)(n < a.NC ? n : a.NC - 1u) * K;
+    }
+#pragma unroll
+    for (int j = 0; j < ST; ++j) {
+        const uint32_t m = m0 + 16u * j + l15;
+        xp[j] = reinterpret_cast<const uint16_t *>(a.stream) + (size_t)(m < a.R ? m : a.R - 1u) * K;
+    }
+    struct Frag { u32x4 w[NT], x[ST * HALVES]; };
+    // (K is a multiple of eight: a piece is inside its row, or beyond K and taken for zeros)
+    auto ld = [&](uint32_t s) __attribute__((always_inline)) -> Frag {
+        Frag f;
+        if (s >= s1) return f;                              // (a wave's last round may be short)
+        const uint32_t k = kbeg + 32u * s + 8u * q4, at = k < kend ? k : 0u;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) f.w[i] = *reinterpret_cast<const u32x4 *>(wp[i] + at);
+#pragma unroll
+        for (int j = 0; j < ST; ++j) {
+            f.x[j] = *reinterpret_cast<const u32x4 *>(xp[j] + at);
+            if constexpr (HALVES == 2) f.x[ST + j] = *reinterpret_cast<const u32x4 *>(xp[j] + a.half_elems + at);
+        }
+        return f;
+    };
+    f32x4 acc[NT][ST * HALVES];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < ST * HALVES; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto fma = [&](Frag &f, uint32_t s) __attribute__((always_inline)) {
+        if (s >= s1) return;
+        const uint32_t keep = kbeg + 32u * s + 8u * q4 < kend ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) f.w[i] &= keep;
+#pragma unroll
+        for (int j = 0; j < ST * HALVES; ++j) {
+            f.x[j] &= keep;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                if constexpr (F16T) {
+                    f16x8 av, bv;
+                    __builtin_memcpy(&av, &f.w[i], 16);
+                    __builtin_memcpy(&bv, &f.x[j], 16);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, acc[i][j], 0, 0, 0);
+                } else {
+                    bf16x8 av, bv;
+                    __builtin_memcpy(&av, &f.w[i], 16);
+                    __builtin_memcpy(&bv, &f.x[j], 16);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc[i][j], 0, 0, 0);
+                }
+            }
+        }
+    };
+    if (s0 < s1) {
+        Frag cur[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) cur[u] = ld(s0 + u);
+        uint32_t s = s0;
+        for (; s + U < s1; s += U) {
+            Frag next[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) next[u] = ld(s + U + u);
+#pragma unroll
+            for (int u = 0; u < U; ++u) fma(cur[u], s + u);
+#pragma unroll
+            for (int u = 0; u < U; ++u) cur[u] = next[u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) fma(cur[u], s + u);
+    }
+#pragma unroll
+    for (int j = 0; j < ST; ++j)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            f32x4 v = acc[i][j];
+            if constexpr (HALVES == 2)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = fmaf(acc[i][ST + j][r], kLoScale, v[r]);
+            part[wave][(j * NT + i) * 64 + lane] = v;
+        }
+    __syncthreads();
+
+    // lane (l15, q4) of a tile: outputs 16 i + 4 q4 .. + 3 of sample 16 j + l15; the waves' sums in wave order
+    for (uint32_t slot = t; slot < NT * ST * 64u; slot += 64u * NW) {
+        f32x4 z = part[0][slot];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) z += part[w][slot];
+        if (a.soft_out) {
+            part[0][slot] = z;
+            continue;
+        }
+        const uint32_t tile = slot >> 6, m = m0 + 16u * (tile / NT) + l15, n0 = 16u * (tile % NT) + 4u * q4;
+        if (m >= a.R) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t n = n0 + r;
+            if (n >= a.NC) continue;
+            if (a.ws) a.ws[((size_t)blockIdx.y * a.NC + n) * a.R + m] = z[r];
+            else skinny_store<F16T>(a, (size_t)m * a.L.N + n, apply_act(layer_sum(a.L, z[r], bias_of[n], n), a.L.act));
+        }
+    }
+    if (a.soft_out) {
+        // softmax as Activation.c:5-21 (largest logit subtracted, exponentials, one division by their sum), a wave per tile
+        __syncthreads();
+        if (wave >= (uint32_t)ST) return;
+        const uint32_t m = m0 + 16u * wave + l15;
+        float v[NT][4], top = -3.402823466e+38f, s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const f32x4 z = part[0][(wave * NT + i) * 64u + lane];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t n = 16u * i + 4u * q4 + r;
+                v[i][r] = n < a.NC ? fmaf(z[r], a.L.wscale, bias_of[n]) : -3.402823466e+38f;
+                top = fmaxf(top, v[i][r]);
+            }
+        }
+        top = fmaxf(top, __shfl_xor(top, 16));
+        top = fmaxf(top, __shfl_xor(top, 32));
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v[i][r] = 16u * i + 4u * q4 + r < a.NC ? expf(v[i][r] - top) : 0.0f;
+                s += v[i][r];
+            }
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        const float inv = s > 0.0f ? 1.0f / s : 1.0f;
+        if (m >= a.R) return;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t n = 16u * i + 4u * q4 + r;
+                if (n >= a.NC) continue;
+                const size_t o = (size_t)m * a.L.N + n;
+                const float y = v[i][r] * inv;
+                if (a.soft_kind == 0) reinterpret_cast<float *>(a.soft_out)[o] = y;
+                else if (a.soft_kind == 1) reinterpret_cast<uint16_t *>(a.soft_out)[o] = f32_to_bf16_rne(y);
+                else reinterpret_cast<uint16_t *>(a.soft_out)[o] = f32_to_f16_sat(y);
+            }
+    }
+}
+
+// adds the partial sums of sp_skinny16 (K splits in split order; with split activations the sums of the second matrix,
+// scaled by 2^-11, after those of the first) and applies bias and activation; a thread takes four neighbouring
+// streamed rows (VEC: R is a multiple of four and the rows are outputs, so they are neighbours in C as well) or one
 template <bool F16T, bool VEC>
 __global__ __launch_bounds__(256) void sp_skinny_reduce(const SkinnyArgs a, uint32_t splits)
 {
     const uint64_t total = (uint64_t)a.NC * a.R;
-    const uint32_t parts = splits * a.halves;
+    const uint32_t parts = a.parts;
     if constexpr (VEC) {
         const uint64_t idx = ((uint64_t)blockIdx.x * 256u + threadIdx.x) * 4u;
         if (idx >= total) return;

@@ -606,6 +606,29 @@ def test_streamed_weights_at_the_edges_of_their_tiles(S, O, fmt, n, K, N):
     assert rel_max_abs(got, ref.forward_batch_f64(X)) <= 2e-3
 
 
+@pytest.mark.parametrize("fmt,mode", [("f16", "plain"), ("bf16", "plain"), ("bf16", "bf16"), ("i8", "split"), ("i4", "plain"), ("i2", "split")])
+@pytest.mark.parametrize("n,K,N,act", [
+    (5, 8, 1, "none"), (16, 40, 16, "softmax"), (17, 1000, 17, "softmax"), (33, 2048, 32, "tanh"), (300, 1536, 33, "leaky_relu"),
+    (129, 2048, 64, "softmax"), (1001, 3072, 50, "sigmoid"), (40, 8200, 10, "softmax"), (70, 16384, 16, "none"),   # K in parts
+    (8192, 264, 31, "softmax"), (8200, 72, 64, "relu"),                                          # two sixteens of samples
+])
+def test_few_outputs_at_the_edges_of_their_tiles(S, O, fmt, mode, n, K, N, act):
+    """sp_skinny16_kw_head against the float64 forward.  (FP16 inputs: 2^-12 of each, at random over K terms; BF16 ones 2^-9; split
+    ones 2^-22 beside the sums' 2^-24 per term.)"""
+    src = make_oracle_net(O, [K, N], [act], seed=n + K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    if mode != "plain":
+        which = S.NET_ACTIVATIONS_SPLIT if mode == "split" else S.NET_ACTIVATIONS_BF16
+        assert S.lib().spingalett_set_net_activations(net, which) == 0
+    X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    part = S.forward_batch(net, X[:n // 2 + 5])                    # other tiles' edges, through the same buffers
+    S.free_network(net)
+    want, tol = ref.forward_batch_f64(X), {"plain": 2e-3, "bf16": 1.6e-2, "split": 2e-5}[mode]
+    assert rel_max_abs(got, want) <= tol
+    assert rel_max_abs(part, want[:n // 2 + 5]) <= tol
+
+
 @pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
 @pytest.mark.parametrize("n,K,N", [(100, 128, 49152), (100, 192, 49160), (128, 320, 49410), (65, 1024, 49153)])
 def test_tiles_of_128_rows_in_every_format(S, O, fmt, n, K, N):
