@@ -283,15 +283,11 @@ static bool train_download(sp_net *sn)
 {
     NeuralNetwork *net = &sn->pub;
     sn->opt_loaded = true;            /* the host gradient / moment arrays hold content from here on: layer() carries them */
-    for (uint32_t l = 0; l + 1 < net->layers; ++l) {
-        const uint64_t wo = net->weight_offsets[l], bo = net->bias_offsets[l];
-        if (sphip_train_get(sn->dev, SPHIP_TRAIN_W, l, net->weights + wo) || sphip_train_get(sn->dev, SPHIP_TRAIN_B, l, net->biases + bo) ||
-            sphip_train_get(sn->dev, SPHIP_TRAIN_MW, l, net->opt_m_weights + wo) || sphip_train_get(sn->dev, SPHIP_TRAIN_VW, l, net->opt_v_weights + wo) ||
-            sphip_train_get(sn->dev, SPHIP_TRAIN_MB, l, net->opt_m_biases + bo) || sphip_train_get(sn->dev, SPHIP_TRAIN_VB, l, net->opt_v_biases + bo) ||
-            sphip_train_get(sn->dev, SPHIP_TRAIN_GW, l, net->grad_weights + wo) || sphip_train_get(sn->dev, SPHIP_TRAIN_GB, l, net->grad_biases + bo)) {
-            report(SPINGALETT_ERR_INVALID, "HIP back-end: train (download)");
-            return false;
-        }
+    const sp_train_host all = {net->weights, net->biases, net->opt_m_weights, net->opt_m_biases, net->opt_v_weights, net->opt_v_biases,
+                               net->grad_weights, net->grad_biases};
+    if (sp_train_arrays && sp_train_arrays(sn->dev, &all, true)) {
+        report(SPINGALETT_ERR_INVALID, "HIP back-end: train (download)");
+        return false;
     }
     return true;
 }
@@ -394,21 +390,18 @@ void train_struct_arguments(TrainArgs args)
     const uint32_t eff_batch = small ? args.batch_size : per_sample ? 1u : sample_count;
     /* a net that fits one compute unit trains inside one launch, which takes and returns the arrays itself */
     const bool tiny = sp_train_tiny_fits && sp_train_tiny_fits(net->layers, net->topology, sample_count, eff_batch, small);
-    if (sn->dev && !tiny && !upload_arrays(sn, sn->dev)) {
-        sp_hip_release(sn);
-        return;
-    }
+    const bool had_device = sn->dev != NULL;
     if (!ensure_device(sn)) return;
     if (sphip_train_begin(sn->dev)) {
         report(SPINGALETT_ERR_ALLOC, "HIP back-end: train");
         return;
     }
-    for (uint32_t l = 0; l + 1 < net->layers && !tiny; ++l) {
-        const uint64_t wo = net->weight_offsets[l], bo = net->bias_offsets[l];
-        if (sphip_train_set(sn->dev, SPHIP_TRAIN_MW, l, net->opt_m_weights + wo) || sphip_train_set(sn->dev, SPHIP_TRAIN_VW, l, net->opt_v_weights + wo) ||
-            sphip_train_set(sn->dev, SPHIP_TRAIN_MB, l, net->opt_m_biases + bo) || sphip_train_set(sn->dev, SPHIP_TRAIN_VB, l, net->opt_v_biases + bo)) {
+    if (!tiny && sp_train_arrays) {
+        const sp_train_host state = {had_device ? net->weights : NULL, had_device ? net->biases : NULL, net->opt_m_weights,
+                                     net->opt_m_biases, net->opt_v_weights, net->opt_v_biases, NULL, NULL};
+        if (sp_train_arrays(sn->dev, &state, false)) {
             report(SPINGALETT_ERR_INVALID, "HIP back-end: train (upload)");
-            sphip_train_end(sn->dev);
+            sp_hip_release(sn);           /* (it may hold half of the weights) */
             return;
         }
     }

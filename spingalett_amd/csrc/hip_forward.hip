@@ -23,6 +23,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -2337,100 +2339,27 @@ static int grow_pinned(float **p, uint64_t *cap, uint64_t need)
     return 0;
 }
 
-// Large uploads from ordinary (pageable) host memory.  Left to the runtime, a 64 MB array moved at about 4 GB/s
-// here; copied by a few threads into a ring of pinned chunks, each handed to the copy engine as soon as it is full,
-// the host-side copy and the transfer overlap.  Like hipMemcpyAsync from pageable memory, the call returns when
-// all of src has been read; the transfers themselves are ordered on g_stream.
-//
-// With a `landed`, the transfers run on a stream of their own, and landed(upto) is called after each chunk: what it
-// enqueues on g_stream may read the first upto bytes of dst and runs beside the transfers that follow.  The ways without a
-// ring call it once.
-namespace {
-constexpr size_t kStageChunk = 8u << 20;
-constexpr int kStageSlots = 3, kStageThreads = 4;
-struct UploadRing {
-    void *buf[kStageSlots] = {};
-    hipEvent_t ev[kStageSlots] = {}, start = nullptr;
-    hipStream_t side = nullptr;
-    bool ready = false;
-    std::mutex mu;
-} g_upload;
-}  // namespace
-
-// host memory that the copy engine reads as it is
-static bool host_registered(const void *src)
-{
-    hipPointerAttribute_t attr{};
-    if (hipPointerGetAttributes(&attr, src) == hipSuccess && attr.type != hipMemoryTypeUnregistered) return true;
-    (void)hipGetLastError();                                   // an unknown pointer leaves an error behind
-    return false;
-}
-
-static int upload_from_host(void *dst, const void *src, size_t bytes, const std::function<int(size_t)> &landed = {})
-{
-    if (bytes < 2 * kStageChunk || host_registered(src)) {
-        HCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
-        return landed ? landed(bytes) : 0;
-    }
-    std::lock_guard<std::mutex> lock(g_upload.mu);
-    if (!g_upload.ready) {
-        for (int i = 0; i < kStageSlots; ++i) {
-            HCHECK(hipHostMalloc(&g_upload.buf[i], kStageChunk, hipHostMallocDefault));
-            HCHECK(hipEventCreateWithFlags(&g_upload.ev[i], hipEventDisableTiming));
-        }
-        HCHECK(hipEventCreateWithFlags(&g_upload.start, hipEventDisableTiming));
-        HCHECK(hipStreamCreateWithFlags(&g_upload.side, hipStreamNonBlocking));
-        g_upload.ready = true;
-    }
-    const hipStream_t stream = landed ? g_upload.side : g_stream;
-    if (landed) {
-        HCHECK(hipEventRecord(g_upload.start, g_stream));     // what is still reading dst
-        HCHECK(hipStreamWaitEvent(stream, g_upload.start, 0));
-    }
-    size_t off = 0;
-    for (int i = 0; off < bytes; ++i, off += kStageChunk) {
-        const int slot = i % kStageSlots;
-        const size_t len = bytes - off < kStageChunk ? bytes - off : kStageChunk;
-        HCHECK(hipEventSynchronize(g_upload.ev[slot]));         // its last transfer, of this call or the one before, has left the chunk
-        const char *s = static_cast<const char *>(src) + off;
-        char *d = static_cast<char *>(g_upload.buf[slot]);
-        const size_t part = (len / kStageThreads + 4096) & ~(size_t)4095;
-        std::thread helpers[kStageThreads - 1];
-        int started = 0;
-        for (int t = 1; t < kStageThreads; ++t) {
-            const size_t b = (size_t)t * part;
-            if (b >= len) break;
-            const size_t l = len - b < part ? len - b : part;
-            helpers[started++] = std::thread([=] { memcpy(d + b, s + b, l); });
-        }
-        memcpy(d, s, len < part ? len : part);
-        for (int t = 0; t < started; ++t) helpers[t].join();
-        HCHECK(hipMemcpyAsync(static_cast<char *>(dst) + off, d, len, hipMemcpyHostToDevice, stream));
-        HCHECK(hipEventRecord(g_upload.ev[slot], stream));
-        if (landed) {
-            HCHECK(hipStreamWaitEvent(g_stream, g_upload.ev[slot], 0));
-            if (landed(off + len)) { (void)hipStreamSynchronize(stream); return 1; }
-        }
-    }
-    return 0;
-}
+}  // extern "C"
+#include "hip_transfer.inl"
+extern "C" {
 
 // Rows per block when a batch comes from the host and its layers run over the rows that have landed while the others are
 // under way, 0 if they wait for all of them.  Only where the layers are the shorter part by far, so that running them in
 // smaller blocks costs nothing: per value of a sample the bus takes 0.085 ns, a multiply-add of FP32 layers at 100 TFLOP/s
-// 0.00002 ns; the line lies at half of that.  A block is what one chunk holds, in whole tiles of 256 rows, and 2048 at
+// 0.00002 ns; the line lies at half of that.  A block is what 8 MB hold, in whole tiles of 256 rows, and 2048 at
 // least (10000 samples of 784-512-1000-10 FP32 from the host 955 -> 865 us, 20000 1780 -> 1575; 20000 of 784-128-10 1570
 // -> 1455); a rest of fewer than kLastRows joins the block before it, so that no few rows take a path for few rows.
 static const uint32_t kLastRows = 512;
+static const size_t kLandedBytes = 8u << 20;
 static uint32_t landing_rows(const sphip_net *net, const float *x, uint32_t n, uint32_t flags)
 {
     const uint32_t in_w = net->topo[0];
-    if ((flags & SPHIP_WHOLE_BATCH) || (uint64_t)n * in_w * sizeof(float) < 2u * kStageChunk || host_registered(x)) return 0;
+    if ((flags & SPHIP_WHOLE_BATCH) || (uint64_t)n * in_w * sizeof(float) < 2u * kLandedBytes || host_registered(x)) return 0;
     if (pick_regime(net, n, flags) == R_GEMV || batch_block_rows(net, n, flags) < n) return 0;
     uint64_t macs = 0;
     for (uint32_t l = 1; l < net->layers; ++l) macs += (uint64_t)net->topo[l - 1] * net->topo[l];
     if (macs > 2000ull * in_w) return 0;
-    uint32_t rows = (uint32_t)(kStageChunk / sizeof(float) / in_w / 256u * 256u);
+    uint32_t rows = (uint32_t)(kLandedBytes / sizeof(float) / in_w / 256u * 256u);
     if (rows < 2048u) rows = 2048u;
     return rows + kLastRows <= n ? rows : 0;
 }
@@ -2496,8 +2425,7 @@ int sphip_forward(sphip_net *net, const float *x, uint32_t n, float *y, uint32_t
             if (wait_for_small_results(net)) return 1;
             memcpy(y, net->pin_out, out_cnt * sizeof(float));
         } else {
-            HCHECK(hipMemcpyAsync(y, d_y, out_cnt * sizeof(float), hipMemcpyDeviceToHost, g_stream));
-            HCHECK(hipStreamSynchronize(g_stream));
+            if (download_to_host(y, d_y, out_cnt * sizeof(float))) return 1;
         }
     }
     return 0;

@@ -997,9 +997,34 @@ int sphip_train_get(sphip_net *net, int which, uint32_t l, float *host)
     uint64_t cnt = 0;
     const float *src = train_array(net, which, l, &cnt);
     if (!src) return fail_msg("sphip_train_get: unknown array");
-    HCHECK(hipMemcpyAsync(host, src, cnt * sizeof(float), hipMemcpyDeviceToHost, g_stream));
-    HCHECK(hipStreamSynchronize(g_stream));
+    if (cnt > kSmallOut) return download_to_host(host, src, cnt * sizeof(float));
+    if (grow_pinned(&net->pin_out, &net->pin_out_cap, cnt)) return 1;
+    sp_copy32<<<(uint32_t)((cnt + 255) / 256), 256, 0, g_stream>>>(src, net->pin_out, cnt);
+    if (wait_for_small_results(net)) return 1;
+    memcpy(host, net->pin_out, cnt * sizeof(float));
     return 0;
+}
+
+int sp_train_arrays(sphip_net *net, const sp_train_host *h, bool to_host)
+{
+    if (!net || !net->train) return fail_msg("sp_train_arrays: sphip_train_begin was not called for this net");
+    sphip_train_state *ts = net->train;
+    std::vector<Segment> seg;
+    auto add = [&](float *host, void *dev, uint64_t cnt) {
+        if (host) seg.push_back({reinterpret_cast<char *>(host), static_cast<char *>(dev), cnt * sizeof(float)});
+    };
+    for (uint32_t l = 0; l + 1 < net->layers; ++l) {
+        add(h->weights ? h->weights + ts->woff[l] : nullptr, net->W[l].base, net->W[l].count);
+        add(h->biases ? h->biases + ts->boff[l] : nullptr, net->B[l].base, net->B[l].count);
+        if (!to_host && h->weights) net->W[l].cat3_valid = false;          // the FP16 parts describe the old weights
+    }
+    add(h->m_weights, ts->mW, ts->total_w);
+    add(h->v_weights, ts->vW, ts->total_w);
+    add(h->g_weights, ts->gW, ts->total_w);
+    add(h->m_biases, ts->mB, ts->total_b);
+    add(h->v_biases, ts->vB, ts->total_b);
+    add(h->g_biases, ts->gB, ts->total_b);
+    return move_arrays(seg.data(), (uint32_t)seg.size(), to_host);
 }
 
 int sphip_train_step(sphip_net *net, const float *x, const float *targets, uint32_t n, const sphip_train_args *args,

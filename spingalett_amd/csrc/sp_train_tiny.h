@@ -1,5 +1,6 @@
 /*
- * sp_train_tiny.h — the training of small nets inside one launch (hip_train_tiny.inl), as the C side calls it.
+ * sp_train_tiny.h — the training of small nets inside one launch (hip_train_tiny.inl) and the host arrays of any training on
+ * their way to the device and back (hip_transfer.inl), as the C side calls them.
  * Internal: not part of the library's interface.
  */
 #ifndef SP_TRAIN_TINY_H
@@ -29,7 +30,12 @@ typedef struct {
     double *total_loss;              /* sum of the losses of the last epoch's places covered here, or NULL */
 } sp_tiny_run;
 
-/* A build of the C side alone (the host sanitizer's) has neither: weak there, checked before use. */
+/* Arrays of a net, flat like NeuralNetwork's, or NULL for those that stay where they are */
+typedef struct {
+    float *weights, *biases, *m_weights, *m_biases, *v_weights, *v_biases, *g_weights, *g_biases;
+} sp_train_host;
+
+/* A build of the C side alone (the host sanitizer's) has none of these: weak there, checked before use. */
 #if defined(__cplusplus)
 #define SP_TINY_API __attribute__((visibility("hidden")))
 #else
@@ -37,6 +43,7 @@ typedef struct {
 #endif
 SP_TINY_API bool sp_train_tiny_fits(uint32_t layers, const uint32_t *topology, uint32_t samples, uint32_t batch, bool ordered);
 SP_TINY_API int  sp_train_tiny_run(sphip_net *net, const sp_tiny_run *run);
+SP_TINY_API int  sp_train_arrays(sphip_net *net, const sp_train_host *arrays, bool to_host);
 
 #ifdef __cplusplus
 }
