@@ -6,7 +6,8 @@
 // the sizes; the arithmetic is nothing.  Here one workgroup keeps weights, moments, activations and (where they fit)
 // the samples in LDS and walks through the steps; the phases of a step are separated by workgroup barriers, and with 64
 // threads (nets whose phases have no more items than that) the barriers cost nothing.  What bounds it is the latency
-// of a phase: an LDS read, a short dependent sum, a store.  2-8-1 with four samples: 39 -> 2.0 us per step.
+// of a phase: an LDS read, a short dependent sum, a store, and the branches around them.  2-8-1 with four samples: 39 -> 2.0 us
+// per step, 1.5 in sp_train_tiny_one.
 
 namespace {
 
@@ -23,6 +24,8 @@ struct TinyArgs {
     uint32_t lds_b, lds_z, lds_desc;   // ... biases, logits, what each parameter's gradient reads
     uint32_t lds_x, lds_t, lds_o;               // ... all samples and targets, the sample order of an epoch
     uint32_t lds_tb;                            // ... the batch's targets, where they are staged
+    uint32_t ld[kTinyLayers + 1];               // sp_train_tiny_one: floats from row to row of a layer's values and weights
+    uint32_t lds_end;                           // ... floats of LDS
     uint32_t total_w, total_b;
     const float *in;                            // weights | biases | mW | mB | vW | vB, flat
     float *out;                                 // the same, then gW | gB (host memory)
@@ -120,6 +123,37 @@ __device__ __forceinline__ float tiny_colsum(const float *d, uint32_t ld, uint32
     return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
+// one output's share of a sample's loss (compute_sample_loss, SIMD.c:522-552)
+__device__ __forceinline__ double tiny_loss(const TinyArgs &g, float a, float t)
+{
+    if (g.loss_func == 0) {
+        const float d = a - t;
+        return (double)(d * d);
+    }
+    if (g.sigmoid_out) {
+        float c = a < 1e-9f ? 1e-9f : a;
+        c = c > 1.0f - 1e-9f ? 1.0f - 1e-9f : c;
+        return -(double)(t * logf(c) + (1.0f - t) * logf(1.0f - c));
+    }
+    return -(double)(t * logf(a < 1e-9f ? 1e-9f : a));
+}
+
+// a softmax's output r of n logits, its target, and its delta
+__device__ __forceinline__ float tiny_soft_delta(const float *z, const float *tr, uint32_t n, uint32_t r, int mode, float &a, float &t)
+{
+    float m = z[0];
+    for (uint32_t k = 1; k < n; ++k) m = fmaxf(m, z[k]);
+    float sum = 0.0f;
+    for (uint32_t k = 0; k < n; ++k) sum += expf(z[k] - m);
+    const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
+    a = expf(z[r] - m) * inv;
+    t = tr[r];
+    if (mode != 0) return a - t;
+    float c = 0.0f;
+    for (uint32_t k = 0; k < n; ++k) { const float ak = expf(z[k] - m) * inv; c += (ak - tr[k]) * ak; }
+    return a * ((a - t) - c);
+}
+
 // T threads, NL weight layers (compile-time, so that the layers' sizes and offsets live in scalar registers: read from
 // the argument block by a layer index they cost a scalar load each, more than the phase itself)
 template <int T, int NL>
@@ -203,18 +237,7 @@ __global__ __launch_bounds__(T) void sp_train_tiny(const TinyArgs g)
             b2pow *= opt.b2;
             opt.mf = 1.0f / (1.0f - b1pow);
             opt.vf = 1.0f / (1.0f - b2pow);
-            auto add_loss = [&](float a, float t) {
-                if (g.loss_func == 0) {
-                    const float d = a - t;
-                    loss += (double)(d * d);
-                } else if (g.sigmoid_out) {
-                    float c = a < 1e-9f ? 1e-9f : a;
-                    c = c > 1.0f - 1e-9f ? 1.0f - 1e-9f : c;
-                    loss -= (double)(t * logf(c) + (1.0f - t) * logf(1.0f - c));
-                } else {
-                    loss -= (double)(t * logf(a < 1e-9f ? 1e-9f : a));
-                }
-            };
+            auto add_loss = [&](float a, float t) { loss += tiny_loss(g, a, t); };
 
             // forward; without a softmax the last layer's threads go straight on to their deltas
 #pragma unroll
@@ -240,19 +263,8 @@ __global__ __launch_bounds__(T) void sp_train_tiny(const TinyArgs g)
                 __syncthreads();
                 for (uint32_t p = tid; p < n * n_out; p += T) {
                     const TinyPos o(p, n_out);
-                    const float *z = L + g.lds_z + o.q * ldo, *tr = L + to + o.q * ldo;
-                    float m = z[0];
-                    for (uint32_t k = 1; k < n_out; ++k) m = fmaxf(m, z[k]);
-                    float sum = 0.0f;
-                    for (uint32_t k = 0; k < n_out; ++k) sum += expf(z[k] - m);
-                    const float inv = sum > 0.0f ? 1.0f / sum : 1.0f, a = expf(z[o.r] - m) * inv, t = tr[o.r];
-                    float d = a - t;
-                    if (g.mode == 0) {
-                        float c = 0.0f;
-                        for (uint32_t k = 0; k < n_out; ++k) { const float ak = expf(z[k] - m) * inv; c += (ak - tr[k]) * ak; }
-                        d = a * (d - c);
-                    }
-                    L[g.lds_d[NL - 1] + o.q * ldo + o.r] = d;
+                    float a, t;
+                    L[g.lds_d[NL - 1] + o.q * ldo + o.r] = tiny_soft_delta(L + g.lds_z + o.q * ldo, L + to + o.q * ldo, n_out, o.r, g.mode, a, t);
                     if (want_loss) add_loss(a, t);
                 }
             }
@@ -348,16 +360,305 @@ __global__ __launch_bounds__(T) void sp_train_tiny(const TinyArgs g)
     }
 }
 
+// The same training where every phase has at most one item a thread and every thread at most one parameter.  A step of such a
+// net is a few hundred instructions, and what it cost in the kernel above was its branches: the rests of sums term by
+// term, each waiting for LDS in turn, loops of one round, places worked out anew in each phase.  Here rows are padded with
+// zeros to whole groups of four, which change no sum, every place is a pointer worked out once, a thread's parameter and
+// its moments stay in registers, and the corrections of the moments are formed for 64 steps at a time, one a lane.
+// A step of 2-8-1 with 4 / 70 samples 2.2 / 6.0 -> 1.5 / 3.2 us, of 7-5-3 with 16 and a softmax 4.3 -> 2.3, of 13-29-17-3
+// with 16 9.3 -> 4.0, of 16-16-4 with one 2.7 -> 1.7 (a two-hundredth of a call's 50 us among them).
+constexpr uint32_t kTinyOne = 1024u;            // items and parameters at most
+
+// as tiny_row_dot, rows padded with zeros to a multiple of four
+__device__ __forceinline__ float tiny_padded_dot(const float *w, const float *a, uint32_t K)
+{
+    float s0 = 0.0f, s1 = 0.0f;
+    uint32_t k = 0;
+    for (; k + 8u <= K; k += 8u) {
+        float wv[8], av[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { wv[u] = w[k + u]; av[u] = a[k + u]; }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { s0 = fmaf(wv[u], av[u], s0); s1 = fmaf(wv[4 + u], av[4 + u], s1); }
+    }
+    if (const uint32_t left = K - k) {
+        float wv[8], av[8];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { wv[u] = w[k + u]; av[u] = a[k + u]; }
+        if (left == 4u) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s0 = fmaf(wv[u], av[u], s0);
+        } else {
+            s0 = fmaf(wv[2], av[2], fmaf(wv[0], av[0], s0));
+            s1 = fmaf(wv[3], av[3], fmaf(wv[1], av[1], s1));
+            if (left > 4u) {
+#pragma unroll
+                for (int u = 4; u < 8; ++u) { wv[u] = w[k + u]; av[u] = a[k + u]; }
+                s0 = fmaf(wv[6], av[6], fmaf(wv[4], av[4], s0));
+                s1 = fmaf(wv[7], av[7], fmaf(wv[5], av[5], s1));
+            }
+        }
+    }
+    return s0 + s1;
+}
+
+// Gradient of a weight (tiny_chain over the batch) or of a bias (tiny_colsum) side by side: lanes of one wave need either
+__device__ __forceinline__ float tiny_gradient(const float *d, uint32_t ds, const float *a, uint32_t as, uint32_t n, bool bias)
+{
+    float s = 0.0f, c[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t i = 0;
+    for (; i + 4u <= n; i += 4u) {
+        float dv[4], av[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { dv[u] = *d; av[u] = *a; d += ds; a += as; }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { s = fmaf(dv[u], av[u], s); c[u] += dv[u]; }
+    }
+    if (const uint32_t left = n - i) {
+        float dv[3], av[3];
+#pragma unroll
+        for (uint32_t u = 0; u < 3u; ++u) { const uint32_t at = u < left ? u : 0u; dv[u] = d[at * ds]; av[u] = a[at * as]; }
+#pragma unroll
+        for (uint32_t u = 0; u < 3u; ++u) { s = u < left ? fmaf(dv[u], av[u], s) : s; c[u] = u < left ? c[u] + dv[u] : c[u]; }
+    }
+    return bias ? (c[0] + c[1]) + (c[2] + c[3]) : s;
+}
+
+// apply_act and act_derivative with the smooth activations, which small nets have, asked for first: each question is a branch
+__device__ __forceinline__ float tiny_act(float x, int act)
+{
+    if (__builtin_expect(act == A_TANH, 1)) return tanh_straight(x);
+    if (__builtin_expect(act == A_SIGMOID, 1)) return 1.0f / (1.0f + expf(-x));
+    return apply_act(x, act);
+}
+
+__device__ __forceinline__ float tiny_derivative(float a, int act)
+{
+    if (__builtin_expect(act == A_TANH, 1)) return 1.0f - a * a;
+    if (__builtin_expect(act == A_SIGMOID, 1)) return a * (1.0f - a);
+    return act_derivative(a, act);
+}
+
+template <int T, int NL>
+__global__ __launch_bounds__(T) void sp_train_tiny_one(const TinyArgs g)
+{
+    extern __shared__ __attribute__((aligned(16))) float L[];
+    __shared__ double red[16];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, total = g.total_w + g.total_b;
+    const uint32_t n_in = g.width[0], n_out = g.width[NL], ldx = g.ld[0], ldo = g.ld[NL];
+    const bool x_lds = g.lds_x != 0u, staged = g.order || !x_lds;
+    const bool soft = g.act[NL - 1] == A_SOFTMAX, clip = g.max_norm > 0.0f;
+    uint32_t *Lu = reinterpret_cast<uint32_t *>(L);
+
+    for (uint32_t p = tid; p < g.lds_end; p += T) L[p] = 0.0f;
+    __syncthreads();
+    if (x_lds) {
+        for (uint32_t p = tid; p < g.samples * n_in; p += T) {
+            const TinyPos o(p, n_in);
+            L[g.lds_x + o.q * ldx + o.r] = g.x[p];
+        }
+        for (uint32_t p = tid; p < g.samples * n_out; p += T) {
+            const TinyPos o(p, n_out);
+            L[g.lds_t + o.q * ldo + o.r] = g.t[p];
+        }
+    }
+    // this thread's parameter: where it lies, what its gradient multiplies, its own values
+    float *par = L;
+    const float *par_d = L, *par_a = L;
+    uint32_t par_ld_d = 0, par_ld_a = 0;
+    bool bias = false, input = false;
+    float w = 0.0f, m = 0.0f, v = 0.0f, grad = 0.0f;
+    if (tid < total) {
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+            const uint32_t K = g.width[l], N = g.width[l + 1], p = tid - g.wofs[l], j = tid - g.total_w - g.bofs[l];
+            if (tid < g.total_w && tid >= g.wofs[l] && p < K * N) {
+                const TinyPos o(p, K);
+                par = L + g.lds_w[l] + o.q * g.ld[l] + o.r;
+                par_d = L + g.lds_d[l] + o.q;
+                par_a = l ? L + g.lds_a[l] + o.r : L + o.r;
+                par_ld_d = g.ld[l + 1];
+                par_ld_a = g.ld[l];
+                input = l == 0;
+            } else if (tid >= g.total_w + g.bofs[l] && j < N) {
+                par = L + g.lds_b + g.bofs[l] + j;
+                par_d = par_a = L + g.lds_d[l] + j;
+                par_ld_d = par_ld_a = g.ld[l + 1];
+                bias = true;
+            }
+        }
+        w = g.in[tid];
+        m = g.in[total + tid];
+        v = g.in[2u * total + tid];
+        *par = w;
+    }
+    // its items of the phases: forward (row of weights, row of inputs, bias, output), hidden deltas (row of deltas, column of
+    // weights, the value, output)
+    struct Fwd { const float *w, *a, *b; float *out; uint32_t q; } fwd[NL];
+    struct Back { const float *d, *w, *a; float *out; } back[NL];
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+        const uint32_t N = g.width[l + 1];
+        TinyPos o(tid, N);
+        if (tid >= N * g.batch) o.q = o.r = 0u;
+        fwd[l].w = L + g.lds_w[l] + o.r * g.ld[l];
+        fwd[l].a = L + (l ? g.lds_a[l] : 0u) + o.q * g.ld[l];
+        fwd[l].b = L + g.lds_b + g.bofs[l] + o.r;
+        fwd[l].out = L + (l + 1 < NL ? g.lds_a[l + 1 < NL ? l + 1 : 0] : g.lds_d[l]) + o.q * g.ld[l + 1] + o.r;
+        fwd[l].q = o.q * g.ld[l + 1] + o.r;
+        if (l == 0) continue;
+        TinyPos i(tid, g.width[l]);
+        if (tid >= g.width[l] * g.batch) i.q = i.r = 0u;
+        back[l].d = L + g.lds_d[l] + i.q * g.ld[l + 1];
+        back[l].w = L + g.lds_w[l] + i.r;
+        back[l].a = L + g.lds_a[l] + i.q * g.ld[l] + i.r;
+        back[l].out = L + g.lds_d[l - 1] + i.q * g.ld[l] + i.r;
+    }
+
+    float b1pow = g.b1pow, b2pow = g.b2pow, mf = 0.0f, vf = 0.0f;
+    double loss = 0.0;
+    OptArgs opt = g.opt;
+    opt.decay = bias ? 0.0f : g.opt.decay;
+    const float batch_scale = 1.0f / (float)g.batch;
+    uint32_t step = 0;
+    for (uint32_t epoch = 0; epoch < g.epochs; ++epoch) {
+        const bool want_loss = g.loss && epoch + 1u == g.epochs;
+        if (g.order) {
+            __syncthreads();
+            for (uint32_t p = tid; p < g.samples; p += T) Lu[g.lds_o + p] = g.order[(size_t)epoch * g.samples + p];
+        }
+        for (uint32_t first = 0; first < g.samples; first += g.batch, ++step) {
+            const uint32_t n = g.samples - first < g.batch ? g.samples - first : g.batch;
+            uint32_t xo = g.lds_x + first * ldx, to = g.lds_t + first * ldo;
+            if (staged) {
+                xo = g.lds_a[0];
+                to = g.lds_tb;
+                __syncthreads();
+                for (uint32_t p = tid; p < n * n_in; p += T) {
+                    const TinyPos o(p, n_in);
+                    const uint32_t r = g.order ? Lu[g.lds_o + first + o.q] : first + o.q;
+                    L[xo + o.q * ldx + o.r] = x_lds ? L[g.lds_x + r * ldx + o.r] : g.x[(size_t)r * n_in + o.r];
+                }
+                for (uint32_t p = tid; p < n * n_out; p += T) {
+                    const TinyPos o(p, n_out);
+                    const uint32_t r = g.order ? Lu[g.lds_o + first + o.q] : first + o.q;
+                    L[to + o.q * ldo + o.r] = x_lds ? L[g.lds_t + r * ldo + o.r] : g.t[(size_t)r * n_out + o.r];
+                }
+            }
+            if (step % 64u == 0u) {
+                // beta^t of the next 64 steps, one a lane, each the product of as many factors as the host's
+                float p1 = 0.0f, p2 = 0.0f;
+                for (uint32_t i = 0; i < 64u; ++i) {
+                    b1pow *= opt.b1;
+                    b2pow *= opt.b2;
+                    p1 = i == lane ? b1pow : p1;
+                    p2 = i == lane ? b2pow : p2;
+                }
+                mf = 1.0f / (1.0f - p1);
+                vf = 1.0f / (1.0f - p2);
+            }
+            opt.mf = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mf), (int)(step % 64u)));
+            opt.vf = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, vf), (int)(step % 64u)));
+            auto add_loss = [&](float a, float t) { loss += tiny_loss(g, a, t); };
+
+            // forward; without a softmax the last layer's threads go straight on to their deltas
+#pragma unroll
+            for (int l = 0; l < NL; ++l) {
+                __syncthreads();
+                if (tid < n * g.width[l + 1]) {
+                    const float z = tiny_padded_dot(fwd[l].w, l ? fwd[l].a : fwd[l].a + xo, g.width[l]) + *fwd[l].b;
+                    if (l + 1 < NL) {
+                        *fwd[l].out = tiny_act(z, g.act[l]);
+                    } else if (soft) {
+                        L[g.lds_z + fwd[l].q] = z;
+                    } else {
+                        const float a = tiny_act(z, g.act[l]), t = L[to + fwd[l].q], diff = a - t;
+                        *fwd[l].out = g.mode == 1 ? diff : diff * tiny_derivative(a, g.act[l]);
+                        if (want_loss) add_loss(a, t);
+                    }
+                }
+            }
+            if (soft) {
+                __syncthreads();
+                if (tid < n * n_out) {
+                    const TinyPos o(tid, n_out);
+                    float a, t;
+                    *fwd[NL - 1].out = tiny_soft_delta(L + g.lds_z + o.q * ldo, L + to + o.q * ldo, n_out, o.r, g.mode, a, t);
+                    if (want_loss) add_loss(a, t);
+                }
+            }
+
+            // hidden deltas
+#pragma unroll
+            for (int l = NL - 1; l > 0; --l) {
+                __syncthreads();
+                if (tid < n * g.width[l]) {
+                    const float *wc = back[l].w;
+                    float s = 0.0f;
+                    for (uint32_t k = 0; k < g.width[l + 1]; k += 4u) {
+                        float dv[4], wv[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) { dv[u] = back[l].d[k + u]; wv[u] = *wc; wc += g.ld[l]; }
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) s = fmaf(dv[u], wv[u], s);
+                    }
+                    *back[l].out = s * tiny_derivative(*back[l].a, g.act[l - 1]);
+                }
+            }
+
+            // gradients and updates
+            __syncthreads();
+            double sq = 0.0;
+            if (tid < total) {
+                grad = tiny_gradient(par_d, par_ld_d, input ? par_a + xo : par_a, par_ld_a, n, bias) * (n == g.batch ? batch_scale : 1.0f / (float)n);
+                if (clip) sq = (double)grad * (double)grad;
+            }
+            if (clip) {
+                const float norm = sqrtf((float)tiny_block_sum<T>(sq, red));
+                grad *= norm > g.max_norm ? g.max_norm / norm : 1.0f;
+            }
+            if (tid < total) {
+                opt_update(opt, w, grad, m, v);
+                *par = w;
+            }
+        }
+    }
+
+    // results: to the net's device arrays, and flat into host memory
+    if (tid < total) {
+        const bool is_w = tid < g.total_w;
+        const uint32_t q = is_w ? tid : tid - g.total_w;
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+            const uint32_t at = q - (is_w ? g.wofs[l] : g.bofs[l]);
+            if (at < (is_w ? g.width[l] : 1u) * g.width[l + 1]) (is_w ? g.dW : g.dB)[l][at] = w;
+        }
+        (is_w ? g.dmW : g.dmB)[q] = m;
+        (is_w ? g.dvW : g.dvB)[q] = v;
+        (is_w ? g.dgW : g.dgB)[q] = grad;
+        g.out[tid] = w;
+        g.out[total + tid] = m;
+        g.out[2u * total + tid] = v;
+        g.out[3u * total + tid] = grad;
+    }
+    if (g.loss) {
+        const double sum = tiny_block_sum<T>(loss, red);
+        if (tid == 0) *g.loss = sum;
+    }
+}
+
 // LDS layout of a net and batch; false where the net belongs to the launch-by-launch step
 struct TinyPlan {
     TinyArgs a;
     uint32_t lds_floats;
-    bool x_lds;
+    bool x_lds, one;
     uint32_t threads, nl;
 };
 
-bool tiny_plan(uint32_t layers, const uint32_t *topo, uint32_t samples, uint32_t batch, bool ordered, TinyPlan *out)
+// one: for sp_train_tiny_one, rows and columns of weights padded to whole groups of four
+bool tiny_layout(uint32_t layers, const uint32_t *topo, uint32_t samples, uint32_t batch, bool ordered, bool one, TinyPlan *out)
 {
+    auto row = [&](uint32_t w) { return one ? ((w + 3u) & ~3u) + 1u : tiny_ld(w); };
     if (layers < 2 || layers - 1u > kTinyLayers || batch == 0 || batch > samples) return false;
     TinyPlan p{};
     TinyArgs &a = p.a;
@@ -366,6 +667,7 @@ bool tiny_plan(uint32_t layers, const uint32_t *topo, uint32_t samples, uint32_t
     for (uint32_t l = 0; l < layers; ++l) {
         if (topo[l] > 512u) return false;
         a.width[l] = topo[l];
+        a.ld[l] = row(topo[l]);
         if (topo[l] > widest) widest = topo[l];
         if (!l) continue;
         a.wofs[l - 1u] = (uint32_t)w;
@@ -381,19 +683,21 @@ bool tiny_plan(uint32_t layers, const uint32_t *topo, uint32_t samples, uint32_t
     a.total_b = (uint32_t)b;
     uint64_t at = 2;                                      // (offset 0 means "not there")
     auto take = [&](uint64_t floats) { const uint64_t o = at; at += floats; return (uint32_t)o; };
-    a.lds_desc = take(2u * (w + b));
-    const uint64_t x = (uint64_t)samples * tiny_ld(topo[0]), t = (uint64_t)samples * tiny_ld(topo[p.nl]);
-    const uint64_t xb = (uint64_t)batch * tiny_ld(topo[0]), tb = (uint64_t)batch * tiny_ld(topo[p.nl]);
+    if (!one) a.lds_desc = take(2u * (w + b));
+    const uint64_t x = (uint64_t)samples * row(topo[0]), t = (uint64_t)samples * row(topo[p.nl]);
+    const uint64_t xb = (uint64_t)batch * row(topo[0]), tb = (uint64_t)batch * row(topo[p.nl]);
     for (uint32_t l = 0; l < p.nl; ++l) {
-        a.lds_w[l] = take((uint64_t)tiny_ld(topo[l]) * topo[l + 1]);
-        a.lds_d[l] = take((uint64_t)batch * tiny_ld(topo[l + 1]));
-        if (l) a.lds_a[l] = take((uint64_t)batch * tiny_ld(topo[l]));
+        a.lds_w[l] = take((uint64_t)row(topo[l]) * (one ? (topo[l + 1] + 3u) & ~3u : topo[l + 1]));
+        a.lds_d[l] = take((uint64_t)batch * row(topo[l + 1]));
+        if (l) a.lds_a[l] = take((uint64_t)batch * row(topo[l]));
     }
     a.lds_z = take(tb);
     a.lds_b = take(b);
-    a.lds_m = take(w + b);
-    a.lds_v = take(w + b);
-    a.lds_g = take(w + b);
+    if (!one) {
+        a.lds_m = take(w + b);
+        a.lds_v = take(w + b);
+        a.lds_g = take(w + b);
+    }
     if (ordered) a.lds_o = take(samples);
     // all samples in LDS where they fit (with room for a gathered batch if there is an order), else batch by batch
     p.x_lds = (at + x + t + (ordered ? xb + tb : 0)) * sizeof(float) <= kTinyLds;
@@ -407,19 +711,39 @@ bool tiny_plan(uint32_t layers, const uint32_t *topo, uint32_t samples, uint32_t
     // one wave where the phases hold a round or two of it, sixteen where they hold many
     uint64_t items = widest * batch;
     if (w + b > items) items = w + b;
-    p.threads = items <= 128u ? 64u : items <= 1024u ? 256u : 1024u;
+    if (one && items > kTinyOne) return false;
+    p.one = one;
+    p.threads = items <= (one ? 64u : 128u) ? 64u : items <= (one ? 256u : 1024u) ? 256u : 1024u;
+    a.lds_end = (uint32_t)at;
     p.lds_floats = (uint32_t)at;
     *out = p;
     return true;
 }
 
-template <int T, int NL>
-int launch_tiny_inst(const TinyArgs &a, size_t lds)
+bool tiny_plan(uint32_t layers, const uint32_t *topo, uint32_t samples, uint32_t batch, bool ordered, TinyPlan *out)
 {
+    if (!tiny_layout(layers, topo, samples, batch, ordered, false, out)) return false;
+    // (the samples in LDS or not as without the padding: trainings are cut into launches by that)
+    TinyPlan one;
+    if (tiny_layout(layers, topo, samples, batch, ordered, true, &one) && one.x_lds == out->x_lds) *out = one;
+    return true;
+}
+
+template <int T, int NL>
+int launch_tiny_inst(const TinyPlan &p, size_t lds)
+{
+    if (p.one) {
+        auto kern = sp_train_tiny_one<T, NL>;
+        static bool once = ((void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTinyLds), true);
+        (void)once;
+        kern<<<1, T, lds, g_stream>>>(p.a);
+        HCHECK(hipGetLastError());
+        return 0;
+    }
     auto kern = sp_train_tiny<T, NL>;
     static bool once = ((void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTinyLds), true);
     (void)once;
-    kern<<<1, T, lds, g_stream>>>(a);
+    kern<<<1, T, lds, g_stream>>>(p.a);
     HCHECK(hipGetLastError());
     return 0;
 }
@@ -429,10 +753,10 @@ int launch_tiny(const TinyPlan &p)
 {
     const size_t lds = (size_t)p.lds_floats * sizeof(float);
     switch (p.nl) {
-    case 1:  return launch_tiny_inst<T, 1>(p.a, lds);
-    case 2:  return launch_tiny_inst<T, 2>(p.a, lds);
-    case 3:  return launch_tiny_inst<T, 3>(p.a, lds);
-    default: return launch_tiny_inst<T, 4>(p.a, lds);
+    case 1:  return launch_tiny_inst<T, 1>(p, lds);
+    case 2:  return launch_tiny_inst<T, 2>(p, lds);
+    case 3:  return launch_tiny_inst<T, 3>(p, lds);
+    default: return launch_tiny_inst<T, 4>(p, lds);
     }
 }
 

@@ -564,6 +564,24 @@ def test_small_nets_match_the_oracle(topo, acts, loss, n, batch, epochs, opt, kw
     S.free_network(net)
 
 
+@pytest.mark.parametrize("topo,acts,loss,n,batch,epochs,opt,kw", [
+    # the largest number of items and parameters of one, four and sixteen waves and one more; sums of 1 to 12 terms and their rests
+    ([3, 5, 4], ["tanh", "sigmoid"], 0, 12, 0, 9, S.OPTIMIZER_ADAM, {}),                          # 60 items of a phase
+    ([1, 13, 4], ["sigmoid", "softmax"], 1, 5, 0, 9, S.OPTIMIZER_ADAMW, {"weight_decay": 1e-3}),    # 65
+    ([4, 8, 2], ["relu", "none"], 0, 32, 0, 6, S.OPTIMIZER_MOMENTUM, {"weight_decay": 1e-3}),       # 256
+    ([7, 6, 11, 1], ["tanh", "leaky_relu", "sigmoid"], 1, 23, 0, 6, S.OPTIMIZER_RMSPROP, {}),       # 253, three layers
+    ([12, 9, 10], ["sigmoid", "softmax"], 0, 29, 0, 5, S.OPTIMIZER_ADAM, {"max_grad_norm": 1e-3}),  # 348, clipped, squared error
+    ([5, 8, 8, 8, 2], ["tanh", "foo52", "sigmoid", "none"], 0, 128, 0, 4, S.OPTIMIZER_SGD, {}),     # 1024, four layers
+    ([5, 8, 8, 8, 2], ["tanh", "foo52", "sigmoid", "none"], 0, 129, 0, 4, S.OPTIMIZER_SGD, {}),     # 1032: more than an item a thread
+    ([10, 60, 5], ["tanh", "sigmoid"], 1, 3, 0, 6, S.OPTIMIZER_ADAM, {}),                           # 965 parameters
+    ([7, 5, 3], ["tanh", "softmax"], 1, 131, 1, 1, S.OPTIMIZER_ADAM, {}),                           # 131 steps: moments' corrections anew
+    ([9, 6, 2], ["sigmoid", "none"], 0, 14, 14, 5, S.OPTIMIZER_ADAM, {}),                           # shuffled
+])
+def test_small_nets_with_one_item_a_thread_match_the_oracle(topo, acts, loss, n, batch, epochs, opt, kw):
+    """sp_train_tiny_one, as above."""
+    test_small_nets_match_the_oracle(topo, acts, loss, n, batch, epochs, opt, kw)
+
+
 def test_an_epoch_of_many_steps_runs_in_several_launches():
     """60,000 updates of a small net, one per sample, are three launches; without momentum four trainings over a quarter
     of the samples each are the same updates, bit for bit.  A shuffled order of equal samples is no order at all."""
