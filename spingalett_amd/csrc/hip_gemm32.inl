@@ -298,7 +298,8 @@ __device__ __forceinline__ void load_piece(float (&v)[4], const float *row, uint
 // steps of eight, and their sums meet in LDS.  No operand staging: lane (r, h) loads four consecutive k of row r of both
 // operands (k = 8 s + 4 h .. + 3 of step s) straight into registers and feeds them to four MFMA steps (a sum over k in
 // any order).  For outputs of up to 512 tiles and K up to 1024, where sp_gemm32_f32 needs a K split over the grid and a
-// second launch to fill the chip (256 x 512 x 784: 8 us against 12 us for the two).  A softmax layer of at most 32
+// second launch to fill the chip (256 x 512 x 784: 8 us against 12 us for the two).  Biases are asked for with the first loads:
+// behind the barrier their latency was a tenth of the kernel (four 256 x 256 layers at 256 samples 16.4 -> 15.6 us).  A softmax layer of at most 32
 // outputs is normalised here (Activation.c:5-21), soft_out != nullptr.  Rows are 16-byte aligned (K % 4 == 0).
 __global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float *__restrict__ soft_out)
 {
@@ -313,6 +314,8 @@ __global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float
     const uint32_t am = m0 + q < M ? m0 + q : M - 1, wn = n0 + q < N ? n0 + q : N - 1;
     const float *ap = g.A + (size_t)am * K + 4 * h;
     const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)wn * K + 4 * h;
+    // (of this thread's two outputs, which are in one column)
+    float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, n0 + (t & 31) < N ? n0 + (t & 31) : N - 1) * g.L.bscale;
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
@@ -336,6 +339,7 @@ __global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float
     for (; s < s1; ++s) fma4(ld(ap, s), ld(wp, s));
 #pragma unroll
     for (int r = 0; r < 16; ++r) part[wave][(8 * (r >> 2) + 4 * h + (r & 3)) * 33 + q] = acc[r];
+    here(bias);
     __syncthreads();
     // the waves' sums in wave order, bias, activation; 512 threads, two outputs each
 #pragma unroll
@@ -344,8 +348,7 @@ __global__ __launch_bounds__(512) void sp_gemm32_small(const Gemm32Args g, float
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += part[w][row * 33 + col];
-        const uint32_t n = n0 + col < N ? n0 + col : N - 1;
-        v = apply_act(v + elem_value_rt(g.L.bias_fmt, g.L.bias, n) * g.L.bscale, g.L.act);
+        v = apply_act(v + bias, g.L.act);
         if (soft_out) part[0][row * 33 + col] = v;               // (every thread has read part[0][its own two slots] only)
         else if (m0 + row < M && n0 + col < N) g.C[(size_t)(m0 + row) * N + n0 + col] = v;
     }
@@ -380,6 +383,12 @@ __global__ __launch_bounds__(512) void sp_gemm32_small16(const Gemm32Args g, con
     const uint32_t m0 = (blockIdx.x / tiles_n) * T, n0 = (blockIdx.x % tiles_n) * T;
     const float *ap = g.A + (size_t)(m0 + q < M ? m0 + q : M - 1) * K;
     const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)(n0 + q < N ? n0 + q : N - 1) * K;
+    // 16 neighbouring threads of the first four waves hold a row in the end: this thread's output, its bias and target
+    const int row = t / T, col = t % T;
+    const bool in = t < T * T && m0 + row < M && n0 + col < N;
+    const size_t o = (size_t)(m0 + row) * N + n0 + col;
+    float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, n0 + col < N ? n0 + col : N - 1) * g.L.bscale;
+    float target = in && tail.targets ? tail.targets[o] : 0.0f;
     for (uint32_t sg = wave; sg < seg.count; sg += NW) {
         const uint32_t k0 = sg * seg.len, k1 = k0 + seg.len < K ? k0 + seg.len : K;
         f32x4 acc;
@@ -406,11 +415,10 @@ __global__ __launch_bounds__(512) void sp_gemm32_small16(const Gemm32Args g, con
 #pragma unroll
         for (int r = 0; r < 4; ++r) part[sg][(4 * h + r) * (T + 1) + q] = acc[r];
     }
+    here(bias);
+    here(target);
     __syncthreads();
-    // the segments' sums in order, bias, activation: 16 neighbouring threads of the first four waves hold a row
-    const int row = t / T, col = t % T;
-    const bool in = t < T * T && m0 + row < M && n0 + col < N;
-    const size_t o = (size_t)(m0 + row) * N + n0 + col;
+    // the segments' sums in order, bias, activation
     float v = 0.0f;
     if (t < T * T) {
 #pragma unroll
@@ -423,8 +431,7 @@ __global__ __launch_bounds__(512) void sp_gemm32_small16(const Gemm32Args g, con
             for (int w = 0; w < 8; ++w)
                 if ((uint32_t)(w0 + w) < seg.count) v += x[w];
         }
-        const uint32_t n = n0 + col < N ? n0 + col : N - 1;
-        v = apply_act(v + elem_value_rt(g.L.bias_fmt, g.L.bias, n) * g.L.bscale, g.L.act);
+        v = apply_act(v + bias, g.L.act);
         if (soft_out) part[0][row * (T + 1) + col] = v;               // (every thread has read its own slots only)
     }
     if (soft_out) {                                                   // (uniform; N <= 16: the tile holds whole rows)
@@ -448,7 +455,7 @@ __global__ __launch_bounds__(512) void sp_gemm32_small16(const Gemm32Args g, con
         g.C[o] = v;
     }
     if (!tail.targets || t >= T * T) return;                          // (uniform in a wave)
-    const float d = in ? v - tail.targets[o] : 0.0f;
+    const float d = in ? v - target : 0.0f;
     float out = tail.mode == 1 ? d : d * act_derivative(v, tail.act);
     if (tail.mode == 0) {                                             // squared error through a softmax
         float c = in ? d * v : 0.0f;

@@ -182,6 +182,10 @@ __device__ __forceinline__ uint16_t f32_to_t16(float x)
     else return f32_to_bf16_rne(x);
 }
 
+// A value loaded at the start of a kernel for its end is here from now on: said in front of the last barrier, it keeps the
+// compiler from asking for it behind that, where nothing hides the latency
+__device__ __forceinline__ void here(float &v) { asm volatile("" : "+v"(v)); }
+
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>)
