@@ -998,7 +998,7 @@ int sphip_train_get(sphip_net *net, int which, uint32_t l, float *host)
     const float *src = train_array(net, which, l, &cnt);
     if (!src) return fail_msg("sphip_train_get: unknown array");
     if (cnt > kSmallOut) return download_to_host(host, src, cnt * sizeof(float));
-    if (grow_pinned(&net->pin_out, &net->pin_out_cap, cnt)) return 1;
+    if (grow_pinned(&net->pin_out, &net->pin_out_cap, kSmallOut)) return 1;
     sp_copy32<<<(uint32_t)((cnt + 255) / 256), 256, 0, g_stream>>>(src, net->pin_out, cnt);
     if (wait_for_small_results(net)) return 1;
     memcpy(host, net->pin_out, cnt * sizeof(float));

@@ -13,8 +13,8 @@ namespace {
 constexpr size_t kStageChunk = 8u << 20, kFirstChunk = 512u << 10, kStagePart = 256u << 10;
 // Single arrays below these sizes are left to the runtime, which has the bus read the caller's pages up to 8 MB (2 / 5.5 / 8 /
 // 15 / 31 MiB up 81 / 174 / 253 / 553 / 795 us, the last two copied into 8 MB chunks by four threads, against 105 / 202 / 278 /
-// 408 / 739 here; 2 MB down 107 against 96).
-constexpr size_t kStagedUp = 10u << 20, kStagedDown = 1u << 20;
+// 408 / 739 here; 2 MB down 107 against 96, for which the ring is not worth its pinned memory).
+constexpr size_t kStagedUp = 10u << 20, kStagedDown = 4u << 20, kHelperLeast = 1u << 20;
 constexpr uint32_t kStageSlots = 4, kStageHelpers = 3;
 
 struct StageRing {
@@ -63,7 +63,7 @@ public:
     int run(hipStream_t stream, const std::function<int(size_t)> &landed)
     {
         std::thread helpers[kStageHelpers];
-        uint32_t started = 0, wanted = total_ / kStagedDown < kStageHelpers ? (uint32_t)(total_ / kStagedDown) : kStageHelpers;
+        uint32_t started = 0, wanted = total_ / kHelperLeast < kStageHelpers ? (uint32_t)(total_ / kHelperLeast) : kStageHelpers;
         const int rc = pump(stream, landed, [&] {
             // (down: when the first chunk is here, which may be long after the call, behind everything the stream still does)
             try {
