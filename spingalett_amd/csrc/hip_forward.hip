@@ -265,6 +265,133 @@ __global__ __launch_bounds__(256) void sp_softmax_rows(const float *__restrict__
     });
 }
 
+// Softmax of rows of any sums: of the partial sums [part][rows][N] of a layer whose K was split over the grid (those of split
+// activations' second matrix, from `splits` on, times 2^-11; biases added here), in one launch with their addition, or of
+// logits.  NWV waves to a row, 4 PER values a thread, all in registers.  Written by the reduction and read again by a launch of its
+// own, the logits of a split layer cost 4 us, and a wave alone with a row of more than 1024 walks it value by value (whole
+// nets, before -> with it, us: 4096 x 1000 INT4 at 16 / 64 samples 15.6 / 18.2 -> 12.1 / 14.5, FP32 at 64 20.2 -> 16.8, 8192 x 4000
+// FP16 at 16 / 600 60.7 / 116 -> 26.4 / 79.8).  A wave to a row up to 256 outputs, with which four waves have nothing to do (1500 x
+// 100 FP32 at 2000 samples 26.4 before, 28.5 with four, 23.5 with one).  Finished logits take it beyond 1024 outputs: 512 x 3000 FP16 at
+// 1 / 64 / 8192 samples 27.8 / 40.5 / 124 -> 8.7 / 12.2 / 97.
+struct SoftSums {
+    const float *ws;
+    uint32_t splits, parts, rows, N;
+    LayerArgs L;
+    void *out;
+    int kind;                // as sp_softmax_rows
+    int logits;              // ws holds one set of finished logits
+};
+constexpr uint32_t kSoftSumsMost = 16384u;
+
+template <int PER, bool VEC, int NWV>
+__global__ __launch_bounds__(256) void sp_sum_softmax(const SoftSums a)
+{
+    __shared__ float red[2][4];
+    const uint32_t t = NWV == 1 ? threadIdx.x & 63u : threadIdx.x, N = a.N;
+    const uint32_t row = NWV == 1 ? blockIdx.x * 4u + (threadIdx.x >> 6) : blockIdx.x;
+    if (row >= a.rows) return;                             // (whole waves; NWV == 4: none)
+    const uint64_t total = (uint64_t)a.rows * N, first = (uint64_t)row * N;
+    float v[PER][4], top = -3.402823466e+38f, sum = 0.0f;
+    // value e of group g: outputs 4 (t + T g) + e, or t + T (4 g + e) where rows are not whole float4s
+    constexpr uint32_t T = 64u * NWV;
+    auto at = [&](int g, int e) { return VEC ? 4u * (t + T * g) + e : t + T * (4u * g + e); };
+#pragma unroll
+    for (int g = 0; g < PER; ++g) {
+        float low[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (VEC) {
+            const uint32_t n = at(g, 0);
+            float4 s, l;
+            add_parts(reinterpret_cast<const float4 *>(a.ws + first + (n < N ? n : 0u)), total / 4u, a.splits, a.parts, s, l);
+            v[g][0] = s.x; v[g][1] = s.y; v[g][2] = s.z; v[g][3] = s.w;
+            low[0] = l.x; low[1] = l.y; low[2] = l.z; low[3] = l.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[g][e] = 0.0f;
+            for (uint32_t p = 0; p < a.parts; ++p) {
+                float x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = a.ws[p * total + first + (at(g, e) < N ? at(g, e) : 0u)];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) (p < a.splits ? v[g][e] : low[e]) += x[e];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t n = at(g, e);
+            if (!a.logits) {
+                const float bias = elem_value_rt(a.L.bias_fmt, a.L.bias, n < N ? n : 0u) * a.L.bscale;
+                v[g][e] = fmaf(fmaf(low[e], kLoScale, v[g][e]), a.L.wscale, bias);
+            }
+            v[g][e] = n < N ? v[g][e] : -3.402823466e+38f;
+            top = fmaxf(top, v[g][e]);
+        }
+    }
+    top = wave_max(top);
+    if constexpr (NWV == 4) {
+        if ((t & 63u) == 0) red[0][t >> 6] = top;
+        __syncthreads();
+        top = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    }
+#pragma unroll
+    for (int g = 0; g < PER; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[g][e] = at(g, e) < N ? expf(v[g][e] - top) : 0.0f;
+            sum += v[g][e];
+        }
+    sum = wave_sum(sum);
+    if constexpr (NWV == 4) {
+        if ((t & 63u) == 0) red[1][t >> 6] = sum;
+        __syncthreads();
+        sum = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    }
+    const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
+#pragma unroll
+    for (int g = 0; g < PER; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t n = at(g, e);
+            if (n >= N) continue;
+            const uint64_t o = first + n;
+            const float y = v[g][e] * inv;
+            if (a.kind == 0) {
+                reinterpret_cast<float *>(a.out)[o] = y;
+            } else if (a.kind == 1) {
+                reinterpret_cast<uint16_t *>(a.out)[o] = f32_to_bf16_rne(y);
+            } else if (a.kind == 2) {
+                reinterpret_cast<uint16_t *>(a.out)[o] = f32_to_f16_sat(y);
+            } else {
+                uint16_t hi, lo;
+                split_f16(y, hi, lo);
+                reinterpret_cast<uint16_t *>(a.out)[o] = hi;
+                reinterpret_cast<uint16_t *>(a.out)[total + o] = lo;
+            }
+        }
+}
+
+void launch_sum_softmax(const SoftSums &a)
+{
+    const bool vec = a.N % 4u == 0 && (reinterpret_cast<uintptr_t>(a.ws) & 15u) == 0;
+    auto go = [&](auto per_c, auto nwv_c) {
+        constexpr int PER = decltype(per_c)::value, NWV = decltype(nwv_c)::value;
+        const uint32_t grid = NWV == 1 ? (a.rows + 3u) / 4u : a.rows;
+        if (vec) sp_sum_softmax<PER, true, NWV><<<grid, 256, 0, g_stream>>>(a);
+        else sp_sum_softmax<PER, false, NWV><<<grid, 256, 0, g_stream>>>(a);
+    };
+    using std::integral_constant;
+    if (a.N <= 256u) go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    else if (a.N <= 1024u) go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    else if (a.N <= 4096u) go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    else go(integral_constant<int, 16>{}, integral_constant<int, 4>{});
+}
+
+// rows of finished logits; up to 1024 of them a wave holds in registers (sp_softmax_rows)
+void launch_softmax(const float *logits, void *out, int kind, uint32_t rows, uint32_t N)
+{
+    if (N > 1024u && N <= kSoftSumsMost) launch_sum_softmax({logits, 1, 1, rows, N, LayerArgs{}, out, kind, 1});
+    else sp_softmax_rows<<<(rows + 3) / 4, 256, 0, g_stream>>>(logits, out, kind, rows, N);
+}
+
 // FP32 -> 16-bit activations for the first GEMM layer
 template <bool F16T>
 __global__ __launch_bounds__(256) void sp_cvt16(const float *__restrict__ in, uint16_t *__restrict__ out, uint64_t n)
@@ -1326,7 +1453,9 @@ void launch_thin(SkinnyArgs a, const ThinPlan &p)
             if (p.ct == 2) launch_thin_inst<SFMT, F16T, 1, 2>(a, p); else launch_thin_inst<SFMT, F16T, 1, 1>(a, p);
         }
     }
-    if (a.ws && !tl_route.dry) {
+    if (a.ws && a.soft_out && !tl_route.dry) {
+        launch_sum_softmax({a.ws, p.splits, a.parts, a.NC, a.R, a.L, a.soft_out, a.soft_kind, 0});
+    } else if (a.ws && !tl_route.dry) {
         const uint64_t total = (uint64_t)a.NC * a.R;
         // four rows per thread where they are neighbours in the workspace and in C, and both are 16-byte aligned
         const bool vec = !a.mode_b && a.R % 4u == 0 && (reinterpret_cast<uintptr_t>(a.ws) & 15u) == 0 &&
@@ -1391,6 +1520,11 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
             a.thin = ctx.w16;
             launch_thin<F16T ? F16 : BF16, F16T>(a, tp);
         } else {
+            if (ctx.soft_out && (tp.splits > 1 || halves == 2) && L.N <= kSoftSumsMost) {
+                a.soft_out = ctx.soft_out;
+                a.soft_kind = ctx.soft_kind;
+                *ctx.soft_done = true;
+            }
             a.stream = L.w;
             a.thin = A;
             launch_thin<FMT, F16T>(a, tp);
@@ -1398,6 +1532,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         return;
     }
     GemmArgs g{L, A, C, M, out_f32, nullptr, 0, 1, halves};
+    const bool soft_sums = ctx.soft_out && L.N <= kSoftSumsMost;          // if there are partial sums
     const bool aligned = rows_aligned(FMT, L.K) && (L.K % 8u == 0);
     const bool fits32 = (uint64_t)M * L.K * 2u < (1ull << 32) && (uint64_t)L.N * L.K * 2u < (1ull << 32);   // 32-bit DMA offsets
     // the 256 x 256 tiles need about a tile per compute unit; smaller problems fill the chip better with 128 x 128
@@ -1429,7 +1564,10 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
             (void)once;
             kern<<<grid, 256, lds, g_stream>>>(g);
         }
-        if (g.ws) {
+        if (g.ws && soft_sums) {
+            launch_sum_softmax({g.ws, g.ksplits, g.ksplits * halves, M, L.N, L, ctx.soft_out, ctx.soft_kind, 0});
+            *ctx.soft_done = true;
+        } else if (g.ws) {
             const uint64_t total = (uint64_t)M * L.N;
             const bool vec = L.N % 4u == 0 && (reinterpret_cast<uintptr_t>(g.ws) & 15u) == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
             if (vec) sp_gemm16_reduce<F16T, true><<<(uint32_t)((total / 4u + 255) / 256), 256, 0, g_stream>>>(g, g.ksplits);
@@ -1491,7 +1629,10 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     if (shape == 22) go(I2c{}, I2c{});
     else if (shape == 12) go(I1{}, I2c{});
     else go(I1{}, I1{});
-    if (g.ws) {
+    if (g.ws && soft_sums) {
+        launch_sum_softmax({g.ws, g.ksplits, g.ksplits * halves, M, L.N, L, ctx.soft_out, ctx.soft_kind, 0});
+        *ctx.soft_done = true;
+    } else if (g.ws) {
         const uint64_t total = (uint64_t)M * L.N;
         const bool vec = L.N % 4u == 0 && (reinterpret_cast<uintptr_t>(g.ws) & 15u) == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
         if (vec) sp_gemm16_reduce<F16T, true><<<(uint32_t)((total / 4u + 255) / 256), 256, 0, g_stream>>>(g, g.ksplits);
@@ -1651,6 +1792,10 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
         b.vec = vec;
         b.bias = L.bias; b.bscale = L.bscale; b.bias_fmt = L.bias_fmt; b.act = L.act;
         launch_gemm32_parts(b, parts, rows64);
+        if (parts > 1 && soft_out && L.N <= kSoftSumsMost) {
+            launch_sum_softmax({ws, parts, parts, M, L.N, L, soft_out, 0, 0});
+            return true;
+        }
         if (parts > 1) {
             g.ws = ws;
             sp_gemm32_reduce<<<(uint32_t)(((uint64_t)M * L.N + 255) / 256), 256, 0, g_stream>>>(g, parts);
@@ -1691,6 +1836,10 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
     }
     if (splits > 1 && soft_out && L.N <= 64u) {
         sp_gemm32_reduce_softmax<<<(M + 15u) / 16u, 256, 0, g_stream>>>(g, splits, soft_out);
+        return true;
+    }
+    if (splits > 1 && soft_out && !training && L.N <= kSoftSumsMost) {     // (training keeps the order of its sums)
+        launch_sum_softmax({ws, splits, splits, M, L.N, L, soft_out, 0, 0});
         return true;
     }
     if (splits > 1) sp_gemm32_reduce<<<(uint32_t)(((uint64_t)M * L.N + 255) / 256), 256, 0, g_stream>>>(g, splits);
@@ -2054,7 +2203,7 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
             *logits = wk.soft_tmp;
         } else if (softmax && !only_layer && !soft_done) {
             const int kind = (reg == R_GEMM16 && !is_last) ? (split ? 3 : f16t ? 2 : 1) : 0;
-            sp_softmax_rows<<<(n + 3) / 4, 256, 0, g_stream>>>(wk.soft_tmp, dst, kind, n, net->topo[l]);
+            launch_softmax(wk.soft_tmp, dst, kind, n, net->topo[l]);
         }
         in = dst;
     }
@@ -2542,8 +2691,10 @@ int sphip_forward_layers(sphip_net *net, const float *x, float *host_neurons)
     memcpy(net->pin_in, x, (size_t)net->topo[0] * sizeof(float));
     sp_copy32<<<(net->topo[0] + 255) / 256, 256, 0, g_stream>>>(net->pin_in, net->layers_buf, net->topo[0]);
     const bool one_launch = net->layers <= 16u && net->total_neurons <= kGatherMost;
+    // (a softmax of more than 1024 outputs wants more than the gathering launch's last wave)
     const float *logits = nullptr;
-    if (enqueue_forward(net, net->workspace(), net->layers_buf, 1, net->layers_buf + net->slot_off[last], 0, 0, true, one_launch ? &logits : nullptr)) return 1;
+    if (enqueue_forward(net, net->workspace(), net->layers_buf, 1, net->layers_buf + net->slot_off[last], 0, 0, true,
+                        one_launch && net->topo[last] <= 1024u ? &logits : nullptr)) return 1;
     // all slots, densely packed, straight into pinned memory
     uint32_t dense = 0;
     for (uint32_t l0 = 0; l0 < net->layers; l0 += 16) {

@@ -629,6 +629,32 @@ def test_few_outputs_at_the_edges_of_their_tiles(S, O, fmt, mode, n, K, N, act):
     assert rel_max_abs(part, want[:n // 2 + 5]) <= tol
 
 
+@pytest.mark.parametrize("fmt,mode", [("f32", "plain"), ("f32", "split"), ("bf16", "bf16"), ("f16", "plain"), ("i8", "split"), ("i2", "plain")])
+@pytest.mark.parametrize("n,topo,acts", [
+    (19, [4096, 65], ["softmax"]), (37, [6000, 256], ["softmax"]), (50, [4100, 257], ["softmax"]), (9, [8192, 1000], ["softmax"]),
+    (300, [8192, 1024], ["softmax"]), (21, [3000, 1025], ["softmax"]), (70, [128, 1027], ["softmax"]), (17, [4096, 4095], ["softmax"]),
+    (33, [64, 4097], ["softmax"]), (6, [2048, 16384], ["softmax"]), (5, [64, 16385], ["softmax"]), (1, [96, 2500], ["softmax"]),
+    (40, [4096, 1500, 20], ["softmax", "tanh"]), (11, [256, 300, 9], ["softmax", "none"]),       # hidden ones, in each 16-bit form
+])
+def test_softmax_of_split_sums_and_of_wide_rows(S, O, fmt, mode, n, topo, acts):
+    """sp_sum_softmax at the edges of what a thread, a wave and a workgroup hold, against the float64 forward.  (As for few outputs; a
+    softmax turns the error of a logit into a relative one, and FP32 logits have 2^-24 per term.)"""
+    src = make_oracle_net(O, topo, acts, seed=n + topo[1], bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    if mode != "plain":
+        which = S.NET_ACTIVATIONS_SPLIT if mode == "split" else S.NET_ACTIVATIONS_BF16
+        assert S.lib().spingalett_set_net_activations(net, which) == 0
+    X = np.random.default_rng(n).standard_normal((n, topo[0])).astype(F32)
+    got, want = S.forward_batch(net, X), ref.forward_batch_f64(X)
+    one = S.forward(net, X[0]).copy()
+    S.free_network(net)
+    tol = {"plain": 2e-5 if fmt == "f32" else 4e-3, "bf16": 3e-2, "split": 4e-5}[mode]
+    assert rel_max_abs(got, want) <= tol
+    assert rel_max_abs(one, want[0]) <= 2e-5
+    if len(topo) == 2:
+        assert np.abs(got.astype(np.float64).sum(axis=1) - 1).max() <= 1e-5
+
+
 @pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
 @pytest.mark.parametrize("n,K,N", [(100, 128, 49152), (100, 192, 49160), (128, 320, 49410), (65, 1024, 49153)])
 def test_tiles_of_128_rows_in_every_format(S, O, fmt, n, K, N):
