@@ -466,6 +466,97 @@ __global__ __launch_bounds__(512) void sp_gemm32_small16(const Gemm32Args g, con
     if (in) tail.delta[o] = out;
 }
 
+// The same for up to 16 outputs of many samples: a wave owns 16 samples and walks through all of K, the segments' sums added in
+// their order, so that the products, the softmax and a training step's output deltas are one launch and the samples' rows are
+// read once.  Bound by its reads of 64 bytes of a row at a time (1.5 TB/s of 16384 x 1000, where whole lines by DMA reach 1.9);
+// the next round's loads are under way during a round's products.  Times at gemm32_head_takes.
+__global__ __launch_bounds__(256) void sp_gemm32_head(const Gemm32Args g, const KSegments seg, float *__restrict__ soft_out, const DeltaTail tail)
+{
+    constexpr int U = 8;                                              // blocks of 16 k per round
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const uint32_t M = g.M, N = g.L.N, K = g.L.K, lane = threadIdx.x & 63u, q = lane & 15u, h = lane >> 4;
+    const uint32_t m0 = (blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * 16u;
+    if (m0 >= M) return;                                              // (a whole wave)
+    const float *ap = g.A + (size_t)(m0 + q < M ? m0 + q : M - 1u) * K;
+    const float *wp = reinterpret_cast<const float *>(g.L.w) + (size_t)(q < N ? q : N - 1u) * K;
+    float bias = elem_value_rt(g.L.bias_fmt, g.L.bias, q < N ? q : N - 1u) * g.L.bscale;
+    float target[4];
+#pragma unroll
+    for (uint32_t r = 0; r < 4u; ++r) {
+        const uint32_t m = m0 + 4u * h + r;
+        target[r] = tail.targets && q < N ? tail.targets[(size_t)(m < M ? m : M - 1u) * N + q] : 0.0f;
+    }
+    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    struct Round { float a[U][4], b[U][4]; } cur, next;
+    auto fetch = [&](Round &f, uint32_t k, uint32_t k1) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t kb = k + 16u * u;
+            if (kb >= k1) break;                                      // (uniform)
+            load_piece(f.a[u], ap, kb, h, k1, K);
+            load_piece(f.b[u], wp, kb, h, k1, K);
+        }
+    };
+    uint32_t k = 0, k1 = seg.len < K ? seg.len : K;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    fetch(cur, 0, k1);
+    for (;;) {
+        uint32_t nk = k + 16u * U, nk1 = k1;                          // the next round: on in this segment, or the next one's first
+        if (nk >= k1) {
+            nk = k1;
+            nk1 = k1 + seg.len < K ? k1 + seg.len : K;
+        }
+        if (nk < K) fetch(next, nk, nk1);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k + 16u * u >= k1) break;
+            chain_order<false>(cur.a[u]);
+            chain_order<false>(cur.b[u]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.a[u][i], cur.b[u][i], acc, 0, 0, 0);
+        }
+        if (nk == k1) {                                               // (the end of a segment)
+            sum += acc;
+            acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        if (nk >= K) break;
+        cur = next;
+        k = nk;
+        k1 = nk1;
+    }
+    // register r of lane (q, h): output q of sample 4 h + r
+#pragma unroll
+    for (uint32_t r = 0; r < 4u; ++r) {
+        const uint32_t m = m0 + 4u * h + r;
+        const bool in = m < M && q < N;
+        const size_t o = (size_t)m * N + q;
+        float v = apply_act(sum[r] + bias, g.L.act);
+        if (soft_out) {                                               // (uniform; the order of sp_softmax_rows)
+            float mx = q < N ? v : -3.402823466e+38f;
+#pragma unroll
+            for (int off = 8; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+            const float ex = q < N ? expf(v - mx) : 0.0f;
+            float all = ex;
+#pragma unroll
+            for (int off = 8; off; off >>= 1) all += __shfl_xor(all, off);
+            v = ex * (all > 0.0f ? 1.0f / all : 1.0f);
+            if (in) soft_out[o] = v;
+        } else if (in) {
+            g.C[o] = v;
+        }
+        if (!tail.targets) continue;
+        const float d = in ? v - target[r] : 0.0f;
+        float out = tail.mode == 1 ? d : d * act_derivative(v, tail.act);
+        if (tail.mode == 0) {
+            float c = in ? d * v : 0.0f;
+#pragma unroll
+            for (int off = 8; off; off >>= 1) c += __shfl_xor(c, off);
+            out = v * (d - c);
+        }
+        if (in) tail.delta[o] = out;
+    }
+}
+
 // adds the K splits of sp_gemm32_f32 (in split order) and applies bias and activation
 __global__ __launch_bounds__(256) void sp_gemm32_reduce(const Gemm32Args g, uint32_t splits)
 {

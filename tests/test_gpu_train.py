@@ -128,6 +128,31 @@ OPT_CASES = [
 ]
 
 
+@pytest.mark.parametrize("topo,acts,loss,n", [
+    ([40, 500, 10], ["relu", "softmax"], 1, 2049), ([33, 131, 16], ["tanh", "softmax"], 0, 2500),       # few outputs of many samples:
+    ([16, 512, 1], ["tanh", "sigmoid"], 0, 4097), ([20, 1024, 3], ["relu", "none"], 0, 16400),          # K in segments and whole,
+    ([9, 65, 15], ["sigmoid", "softmax"], 1, 20011), ([24, 1000, 12], ["leaky_relu", "softmax"], 1, 16385),   # ragged rows and ends
+])
+def test_heads_of_many_samples_match_the_oracle(topo, acts, loss, n):
+    """sp_gemm32_head and sp_train_head_grad: outputs, loss and gradients of a batch against the oracle."""
+    net, onet = public_net(topo, acts, loss, seed=n)
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, topo[0])).astype(np.float32)
+    T = targets_for(rng, n, topo[-1], loss == 1)
+    seen = []
+    S.train(net, X, T, 1, S.STRATEGY_FULL_BATCH, S.OPTIMIZER_SGD, learning_rate=1e-6, callback=lambda p, epoch, err: seen.append(err) or False)
+    assert S.last_error()[0] == S.SPINGALETT_OK, S.last_error()
+    gW, gB, out = onet.batch_gradients(X, T)
+    nc = net.contents
+    arr = lambda name, cnt: np.ctypeslib.as_array(getattr(nc, name), shape=(int(cnt),))
+    assert rel_max_abs(arr("grad_weights", nc.total_weights), gW) <= TOL
+    assert rel_max_abs(arr("grad_biases", nc.total_biases), gB) <= TOL
+    assert seen[0] == pytest.approx(O.batch_loss(out, T, loss, O.ACT[acts[-1]]) / n, rel=1e-4)
+    onet.apply_gradients(O.TrainState(onet), gW, gB, S.OPTIMIZER_SGD, lr=1e-6)
+    assert rel_max_abs(S.forward_batch(net, X), onet.forward_batch(X)) <= TOL          # (behind the update)
+    S.free_network(net)
+
+
 def test_gradients_of_a_large_layer_match_float64():
     """Weights beyond the L2s (1000 x 1052, 4.2 MB) and 512 tiles of 128 x 128: the forward product of this step is
     sp_gemm32_f32_big's, in one order of sums however many multiply-adds it has (the inference forward's kernel on BF16
