@@ -565,7 +565,7 @@ __global__ __launch_bounds__(256) void sp_pad_rows(const uint8_t *__restrict__ i
     out[id] = v;
 }
 
-// The caller's rows of K floats as rows of Kp (a multiple of 4), zeros behind; KIND 1 BF16, 2 FP16, 3 split FP16
+// The caller's rows of K floats as rows of Kp (a multiple of 4), zeros behind; KIND 0 FP32, 1 BF16, 2 FP16, 3 split FP16
 // (sp_cvt16_split's two matrices).  A thread makes four elements of a row.
 template <int KIND>
 __global__ __launch_bounds__(256) void sp_pad_input(const float *__restrict__ x, void *__restrict__ out, uint32_t n, uint32_t K, uint32_t Kp)
@@ -577,6 +577,10 @@ __global__ __launch_bounds__(256) void sp_pad_input(const float *__restrict__ x,
 #pragma unroll
     for (uint32_t e = 0; e < 4u; ++e) v[e] = k + e < K ? x[(size_t)r * K + k + e] : 0.0f;
     const size_t o = (size_t)r * Kp + k;
+    if constexpr (KIND == 0) {
+        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(out) + o) = make_float4(v[0], v[1], v[2], v[3]);
+        return;
+    }
     uint16_t h[4], l[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -877,13 +881,16 @@ Regime pick_regime(const sphip_net *net, uint32_t n, uint32_t flags)
 // caller's, and not a hidden softmax, whose sum runs over its real neurons.
 // Integer rows of eight codes' multiples (1000 INT8 codes) have kernels of their own, which are as good on small layers
 // and take the input as it is; hidden widths of that kind are padded in front of half a million weights and more, where
-// the streaming and DMA kernels, which want 16-byte rows, are the better ones.  FP32 rows stay as they are.
+// the streaming and DMA kernels, which want 16-byte rows, are the better ones, and so are inputs wider than what the small kernel
+// takes (one layer, as they are -> padded, us: 4104 x 3000 INT8 at 16 / 300 samples 35 / 44.5 -> 13.1 / 37.5, 9040 x 2576 INT2 at 16 61
+// -> 13.9; rows that are no whole words ran code by code: 11864 x 5968 INT2 at 16 / 1590 166 / 3029 -> 18 / 286).  FP32 rows stay as
+// they are.
 uint32_t padded_width(int fmt, uint32_t w, uint32_t next, bool hidden)
 {
     if (fmt == F32) return w;
     const uint32_t unit = fmt_bits(fmt) == 16 ? 8u : 128u / (uint32_t)fmt_bits(fmt);
     if (w % unit == 0) return w;
-    if (w % 8u == 0 && !(hidden && (uint64_t)w * next > (512u << 10))) return w;
+    if (w % 8u == 0 && !((hidden || w > 2048u) && (uint64_t)w * next > (512u << 10))) return w;
     const uint32_t to = w >= 256u ? 64u : unit;
     return (w + to - 1u) / to * to;
 }
@@ -907,6 +914,21 @@ LayerArgs make_layer_args(const sphip_net *net, uint32_t l /*1-based layer*/, bo
 }
 
 bool rows_aligned(int fmt, uint32_t K) { return ((uint64_t)K * (uint64_t)fmt_bits(fmt)) % 128u == 0; }
+
+// Whether the vector kernels read a first layer's weights as they were uploaded, next to the caller's rows.  Not where those
+// rows are no whole words, which leaves only the kernel that reads code by code, a wave to a row (1.5 us per 1000 codes, FP16 4.5),
+// and are long enough to pay for the launch that pads the input (one sample, as they are -> padded, us: 1531 x 777 FP16 8.9 -> 6.8,
+// BF16 5.2 -> 6.5, 4099 x 600 FP16 19.7 -> 8.0, BF16 9.5 -> 8.0, INT2 9.0 -> 8.4, 10078 x 112 INT8 19.3 -> 9.9, 7298 x 8070 FP16 80 ->
+// 21, INT4 43 -> 11; at four samples 4099 x 600 BF16 10.9 -> 11.4, 4097 x 9000 46.9 -> 23.5).  Integer layers of more than two samples only where
+// they reach the integer matrix cores (launch_gemv_i8): 5003 x 100 INT2 at four samples 12.2 against 17.3, 7298 x 8070 41 -> 20.
+bool raw_rows(int fmt, uint32_t K, uint32_t N, uint32_t n)
+{
+    if (fmt == F32 || rows_aligned(fmt, K) || K < (fmt == F16 ? 1280u : n > 2u && N < 2048u ? 5000u : 4096u)) return true;
+    const uint64_t row_bits = (uint64_t)K * (uint64_t)fmt_bits(fmt);
+    if (fmt_bits(fmt) < 16)
+        return row_bits % 32u == 0 || (n > 2u && N > 64u && (uint64_t)N * K * n <= (fmt == I2 ? (2ull << 20) : (4ull << 20)));
+    return row_bits % 32u == 0 && N <= 64u && row_bits / 32u >= 256u;
+}
 
 template <int FMT>
 void launch_gemv_fmt(const LayerArgs &L, const float *x, float *y, uint32_t n, bool padded = false)
@@ -2136,7 +2158,12 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
     const uint32_t in_w = net->topo[0], in_pw = net->ptopo[0];
     const bool x_fused = reg == R_GEMM16 && in_pw == in_w && gemm16_small_layer(n, net->ptopo[1], in_w, tl_route.halves) &&
                          (reinterpret_cast<uintptr_t>(d_x) & 15u) == 0;
-    if (x_fused) {
+    const bool raw = raw_rows(net->prec, in_w, net->ptopo[1], n);
+    if (reg == R_GEMV && in_pw != in_w && !raw && only_layer <= 1u) {
+        const uint64_t quads = (uint64_t)n * (in_pw / 4u);
+        sp_pad_input<0><<<(uint32_t)((quads + 255u) / 256u), 256, 0, g_stream>>>(d_x, wk.buf[1], n, in_w, in_pw);
+        in = wk.buf[1];
+    } else if (x_fused) {
         // (the first layer's kernel rounds, or splits, the FP32 input itself)
     } else if (in_pw != in_w && reg == R_GEMM16 && !only_layer) {
         // rows of a padded input, converted on the way
@@ -2162,7 +2189,7 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
 
     for (uint32_t l = 1; l <= last; ++l) {
         const DevArray &wa = net->w(l - 1);
-        LayerArgs L = make_layer_args(net, l, l == 1 && reg == R_GEMV);
+        LayerArgs L = make_layer_args(net, l, l == 1 && reg == R_GEMV && raw);
         if (wide) {
             L.w = reinterpret_cast<const uint8_t *>(wa.wide16);
             L.wscale = ldexpf(L.wscale, -wa.wide_shift);
@@ -2184,7 +2211,7 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
         bool soft_done = false;                 // the layer's own kernel wrote the softmax
         if (run) {
             if (reg == R_GEMV) launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n,
-                                          only_layer != 0 && net->aq_valid_layer == l && net->aq_valid_n == n, net->ptopo[l - 1] != net->topo[l - 1]);
+                                          only_layer != 0 && net->aq_valid_layer == l && net->aq_valid_n == n, net->ptopo[l - 1] != net->topo[l - 1] && (l > 1 || raw));
             if (reg == R_GEMV) { net->aq_valid_layer = l; net->aq_valid_n = n; }
             else if ((reg == R_GEMM32 || (reg == R_CAT3 && !cat3)) && f32_thin_vector(L, n))
                 launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n, false);
@@ -2935,11 +2962,12 @@ const char *sphip_layer_kernel_name(sphip_net *net, uint32_t layer, uint32_t n, 
     // pointers as aligned, which is how sphip_forward calls it
     tl_route.dry = true;
     tl_route.name = "";
-    const LayerArgs L = make_layer_args(net, layer, layer == 1 && pick_regime(net, n, flags) == R_GEMV);
+    const LayerArgs L = make_layer_args(net, layer, layer == 1 && pick_regime(net, n, flags) == R_GEMV && raw_rows(net->prec, net->topo[0], net->ptopo[1], n));
     const float *aligned_ptr = reinterpret_cast<const float *>(uintptr_t{256});     // never dereferenced
     switch (pick_regime(net, n, flags)) {
     case R_GEMV:
-        launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false, net->ptopo[layer - 1] != net->topo[layer - 1]);
+        launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false,
+                    net->ptopo[layer - 1] != net->topo[layer - 1] && (layer > 1 || raw_rows(net->prec, net->topo[0], net->ptopo[1], n)));
         break;
     case R_GEMM32:
         if (f32_thin_vector(L, n)) launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false);

@@ -656,6 +656,43 @@ def test_softmax_of_split_sums_and_of_wide_rows(S, O, fmt, mode, n, topo, acts):
 
 
 @pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
+@pytest.mark.parametrize("K,N", [(1279, 70), (1283, 70), (4095, 65), (4097, 65), (4999, 129), (5002, 300), (5003, 64), (9002, 1100), (7297, 901)])
+def test_few_samples_of_rows_that_are_no_whole_words(S, O, fmt, K, N):
+    """The vector kernels on such rows as they are and padded (raw_rows), one to four samples, against the float64 forward; forward()
+    hands out the padded layer's outputs and its input unchanged.  (FP32 sums of K terms: 2^-24 each, at random.)"""
+    src = make_oracle_net(O, [K, N, 7], ["tanh", "none"], seed=K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    X = np.random.default_rng(K).standard_normal((4, K)).astype(F32)
+    want = ref.forward_batch_f64(X)
+    for n in (1, 2, 3, 4):
+        assert rel_max_abs(S.forward_batch(net, X[:n]), want[:n]) <= 1e-5
+    assert rel_max_abs(S.forward(net, X[1]), want[1]) <= 1e-5
+    c = net.contents
+    neurons = np.ctypeslib.as_array(c.neurons, shape=(int(c.total_neurons),))
+    assert np.array_equal(neurons[:K], X[1])
+    hidden = np.tanh(X[1].astype(np.float64) @ ref.W(0).astype(np.float64).T + ref.b(0))
+    assert rel_max_abs(neurons[K:K + N], hidden) <= 1e-5
+    S.free_network(net)
+
+
+@pytest.mark.parametrize("fmt,mode", [("i8", "plain"), ("i4", "plain"), ("i2", "plain"), ("i2", "split")])
+@pytest.mark.parametrize("K,N", [(2056, 300), (2072, 260), (4008, 131), (6024, 1030)])
+def test_wide_inputs_of_integer_nets_run_padded(S, O, fmt, mode, K, N):
+    """Inputs of more than 2048 values whose rows of codes are no whole 16-byte units (padded_width), from a sample to several tiles,
+    against the float64 forward.  (FP16 inputs 2^-12, split ones 2^-22.)"""
+    src = make_oracle_net(O, [K, N, 12], ["relu", "softmax"], seed=K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    if mode == "split":
+        assert S.lib().spingalett_set_net_activations(net, S.NET_ACTIVATIONS_SPLIT) == 0
+    X = np.random.default_rng(K).standard_normal((700, K)).astype(F32)
+    want = ref.forward_batch_f64(X)
+    for n in (1, 4, 5, 17, 64, 300, 700):
+        tol = 2e-5 if n <= 4 else 4e-5 if mode == "split" else 5e-3
+        assert rel_max_abs(S.forward_batch(net, X[:n]), want[:n]) <= tol, n
+    S.free_network(net)
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
 @pytest.mark.parametrize("n,K,N", [(100, 128, 49152), (100, 192, 49160), (128, 320, 49410), (65, 1024, 49153)])
 def test_tiles_of_128_rows_in_every_format(S, O, fmt, n, K, N):
     """sp_gemm16_big with 128-row tiles, whole and partial K tiles, against the float64 forward.  (As above.)"""
