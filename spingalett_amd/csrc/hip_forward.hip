@@ -1829,7 +1829,6 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
         if (tl_route.dry) return false;
         b.A = A; b.B = reinterpret_cast<const float *>(L.w); b.C = C; b.ws = parts > 1 ? ws : nullptr;
         b.M = M; b.N = L.N; b.K = L.K;
-        b.vec = vec;
         b.bias = L.bias; b.bscale = L.bscale; b.bias_fmt = L.bias_fmt; b.act = L.act;
         launch_gemm32_parts(b, parts, rows64);
         if (parts > 1 && soft_out && L.N <= kSoftSumsMost) {

@@ -11,7 +11,6 @@ struct PartsGemm32Args {
     int bias_fmt, act;
     uint32_t M, N, K;
     uint32_t kper;         // k range of one split (multiple of 32)
-    int vec;               // rows are 16-byte aligned
 };
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -52,7 +51,9 @@ __device__ __forceinline__ void bf16_parts2(float x, float y, uint32_t &h, uint3
 // share a compute unit, and one's splitting runs beside another's products.  Bound by the matrix cores and the splitting's
 // vector instructions together: 4096 x 4096 x 4096 1070 -> 732 us (188 TFLOP/s of FP32 products, 1.13 PFLOP/s of BF16),
 // 20000 x 1000 x 512 221 -> 124, 2000 x 4096 x 4096 600 -> 353, 512 x 4096 x 4096 (split over K) 178 -> 107.  (Of that the
-// scaling of the operands costs between -3 and 4 %: 723, 123, 364 and 110 us without it.)
+// scaling of the operands costs between -3 and 4 %: 723, 123, 364 and 110 us without it.)  Rows that are not whole 16-byte
+// units are loaded 16 bytes at a time all the same (10000 x 1000 x 1001 278 -> 142 us, 10000 x 1872 x 4650
+// 1980 -> 1005; element by element before).
 // Infinities and operands from 2^104 on have no such parts, sums from 2^80 on no room for their scale: an element whose sum
 // comes out infinite or NaN is formed again as a chain of FP32 products.
 template <int TM>
@@ -100,8 +101,9 @@ __global__ __launch_bounds__(256) void sp_gemm32_bf16_parts(const PartsGemm32Arg
     float fa[TM][8], fb[2][8];
     auto fetch = [&](float (&f)[8], const float *p, uint32_t k0) {
         const uint32_t k = k0 + unit * 8u;
-        if (g.vec && k0 + BK <= kend) {
-            const float4 v0 = *reinterpret_cast<const float4 *>(p + k), v1 = *reinterpret_cast<const float4 *>(p + k + 4u);
+        if (k0 + BK <= kend) {
+            // (rows begin anywhere: the wide loads want no more than the alignment of a float)
+            const float4_any v0 = *reinterpret_cast<const float4_any *>(p + k), v1 = *reinterpret_cast<const float4_any *>(p + k + 4u);
             f[0] = v0.x; f[1] = v0.y; f[2] = v0.z; f[3] = v0.w;
             f[4] = v1.x; f[5] = v1.y; f[6] = v1.z; f[7] = v1.w;
         } else {

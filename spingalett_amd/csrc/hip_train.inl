@@ -22,14 +22,15 @@ struct TrGemmArgs {
     uint32_t kper;         // k range of one split (multiple of 32)
     int act;               // TR_EPI_DELTA: activation kind of aux
     float scale;           // TR_EPI_SCALE
-    int vecA, vecB;        // operand may be read as float4 (leading dimension and base 16-byte aligned)
 };
 
 // C[m][n] = sum_k A(m, k) B(n, k) where an operand's rows are not whole 16-byte units (else sp_gemm32_f32 of hip_tile32.inl, with
 // the same order of sums), through registers.  Tile 64 x 64 x 32, four waves in a 2 x 2 grid.  Each operand is either
 // k-contiguous (element (r, k) at r * ld + k; LDS tile [row][33]) or row-contiguous (element (r, k) at k * ld + r; LDS tile
 // [k][96]): the hidden deltas read the weights row-contiguous, the gradients read both operands so.  Both LDS layouts
-// are conflict-free for the matrix-core operand reads (lane -> row, half-wave -> k).
+// are conflict-free for the matrix-core operand reads (lane -> row, half-wave -> k).  Whole pieces are loaded 16 bytes at a time
+// from wherever they begin (an epoch of 8000 samples of 785-513-1001-20 803 -> 560 us, a step of 512 180 -> 157 with the same in
+// sp_train_grad_update; element by element before).
 template <bool AMC, bool BMC, int EPI>
 __global__ __launch_bounds__(256) void sp_train_gemm32(const TrGemmArgs g)
 {
@@ -63,8 +64,11 @@ __global__ __launch_bounds__(256) void sp_train_gemm32(const TrGemmArgs g)
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
     // four consecutive elements starting at p, of which the first `valid` exist
-    auto load4 = [](const float *p, bool vec, int valid) -> float4 {
-        if (vec && valid >= 4) return *reinterpret_cast<const float4 *>(p);
+    auto load4 = [](const float *p, int valid) -> float4 {
+        if (valid >= 4) {
+            const float4_any x = *reinterpret_cast<const float4_any *>(p);
+            return make_float4(x.x, x.y, x.z, x.w);
+        }
         float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -72,22 +76,22 @@ __global__ __launch_bounds__(256) void sp_train_gemm32(const TrGemmArgs g)
         return make_float4(v[0], v[1], v[2], v[3]);
     };
     // piece p of a tile: k-contiguous -> row p / 8, k (p % 8) * 4; row-contiguous -> k p / (BM / 4), row (p % (BM / 4)) * 4
-    auto fetch_one = [&](const float *base, uint32_t ld, bool mc, bool vec, uint32_t r0, uint32_t R, uint32_t k0, int p) -> float4 {
+    auto fetch_one = [&](const float *base, uint32_t ld, bool mc, uint32_t r0, uint32_t R, uint32_t k0, int p) -> float4 {
         if (mc) {
             const uint32_t k = k0 + (uint32_t)(p / (BM / 4)), r = r0 + (uint32_t)(p % (BM / 4)) * 4u;
             const int valid = (k < kend && r < R) ? (int)(R - r < 4u ? R - r : 4u) : 0;
-            return load4(base + (size_t)(k < K ? k : K - 1) * ld + (r < R ? r : 0u), vec, valid);
+            return load4(base + (size_t)(k < K ? k : K - 1) * ld + (r < R ? r : 0u), valid);
         }
         const uint32_t r = r0 + (uint32_t)(p >> 3), k = k0 + (uint32_t)(p & 7) * 4u;
         const int valid = (r < R && k < kend) ? (int)(kend - k < 4u ? kend - k : 4u) : 0;
-        return load4(base + (size_t)(r < R ? r : R - 1) * ld + (k < kend ? k : 0u), vec, valid);
+        return load4(base + (size_t)(r < R ? r : R - 1) * ld + (k < kend ? k : 0u), valid);
     };
     float4 ra[PIECES], rb[PIECES];
     auto fetch = [&](uint32_t k0) {
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
-            ra[i] = fetch_one(g.A, g.lda, AMC, g.vecA != 0, m0, M, k0, t + 256 * i);
-            rb[i] = fetch_one(g.B, g.ldb, BMC, g.vecB != 0, n0, N, k0, t + 256 * i);
+            ra[i] = fetch_one(g.A, g.lda, AMC, m0, M, k0, t + 256 * i);
+            rb[i] = fetch_one(g.B, g.ldb, BMC, n0, N, k0, t + 256 * i);
         }
     };
     auto stash_one = [&](float *tile, bool mc, const float4 &v, int p) {
@@ -431,7 +435,6 @@ struct GradLayer {
     float *W, *gW, *mW, *vW, *B, *gB, *mB, *vB;
     uint32_t out, in, tiles_n, first;          // column tiles; first workgroup of the layer
     uint32_t kper;         // samples per segment of the sums (the tiled kernel's K splits, added in split order: the same bits)
-    int vec_d, vec_a;      // rows may be read as float4
 };
 
 constexpr uint32_t kGradLayers = 16, kGroupedSamples = 512;
@@ -484,10 +487,13 @@ __global__ __launch_bounds__(256) void sp_train_grad_update(const GradArgs g)
         }
 
     // piece p of a tile of width W: sample p / (W / 4), element (p % (W / 4)) * 4; one piece of A, two of B per thread
-    auto load4 = [](const float *base, uint32_t ld, uint32_t R, uint32_t r, uint32_t k, bool kin, bool vec) -> float4 {
+    auto load4 = [](const float *base, uint32_t ld, uint32_t R, uint32_t r, uint32_t k, bool kin) -> float4 {
         if (!kin || r >= R) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         const float *p = base + (size_t)k * ld + r;
-        if (vec && r + 4u <= R) return *reinterpret_cast<const float4 *>(p);
+        if (r + 4u <= R) {
+            const float4_any x = *reinterpret_cast<const float4_any *>(p);
+            return make_float4(x.x, x.y, x.z, x.w);
+        }
         float e[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (uint32_t i = 0; i < 4u; ++i)
@@ -496,11 +502,11 @@ __global__ __launch_bounds__(256) void sp_train_grad_update(const GradArgs g)
     };
     float4 ra, rb[2];
     auto fetch = [&](uint32_t k0) {
-        ra = load4(L.d, M, M, m0 + (t & 7) * 4u, k0 + (t >> 3), k0 + (t >> 3) < n, L.vec_d != 0);
+        ra = load4(L.d, M, M, m0 + (t & 7) * 4u, k0 + (t >> 3), k0 + (t >> 3) < n);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const uint32_t p = t + 256u * i, k = k0 + (p >> 4);
-            rb[i] = load4(L.a, N, N, n0 + (p & 15u) * 4u, k, k < n, L.vec_a != 0);
+            rb[i] = load4(L.a, N, N, n0 + (p & 15u) * 4u, k, k < n);
         }
     };
     // column sums of the deltas, in the order of sp_train_colsum_part: chunks of 256 samples, in a chunk thread (q, c) adds
@@ -755,12 +761,6 @@ int train_reserve(sphip_net *net, uint32_t n)
     return 0;
 }
 
-void set_vec(TrGemmArgs &g)
-{
-    g.vecA = g.lda % 4u == 0 && (reinterpret_cast<uintptr_t>(g.A) & 15u) == 0;
-    g.vecB = g.ldb % 4u == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15u) == 0;
-}
-
 Tile32Args tile32_args(const TrGemmArgs &g)
 {
     return {g.A, g.B, g.C, g.ws, g.aux, nullptr, F32, 1.0f, g.M, g.N, g.K, g.lda, g.ldb, g.kper, g.act, g.scale};
@@ -783,7 +783,6 @@ void launch_train_delta(TrGemmArgs g, float *ws, uint64_t ws_floats)
     }
     if (splits > 1 && (uint64_t)splits * g.M * g.N > ws_floats) { splits = 1; g.kper = (g.K + 31u) / 32u * 32u; }
     g.ws = splits > 1 ? ws : nullptr;
-    set_vec(g);
     if (gemm32_tile_takes(g.A, g.B, g.lda, g.ldb))
         launch_gemm32_tile<T32_DELTA, false, true>(tile32_args(g), splits);
     else
@@ -851,8 +850,6 @@ void train_gradients(sphip_net *net, const float *d_x, uint32_t n, const sphip_t
                 (void)gemm32_splits(q.out, q.in, n, &q.kper);
                 q.tiles_n = (q.in + 63u) / 64u;
                 q.first = blocks;
-                q.vec_d = q.out % 4u == 0 && aligned(q.d);
-                q.vec_a = q.in % 4u == 0 && aligned(q.a);
                 blocks += (q.out + 31u) / 32u * q.tiles_n;
             }
             sp_train_grad_update<<<blocks, 256, 0, g_stream>>>(g);
@@ -894,7 +891,6 @@ void train_gradients(sphip_net *net, const float *d_x, uint32_t n, const sphip_t
         g.M = net->topo[l + 1]; g.N = net->topo[l]; g.K = n;
         g.ws = ts->ws;
         const uint32_t splits = gemm32_splits(g.M, g.N, g.K, &g.kper);
-        set_vec(g);
         if (g.M <= 16u)
             sp_train_head_grad<<<dim3((g.N + 63u) / 64u, splits), 256, 0, g_stream>>>(g);
         else if (gemm32_tile_takes(g.A, g.B, g.lda, g.ldb))

@@ -128,6 +128,27 @@ OPT_CASES = [
 ]
 
 
+@pytest.mark.parametrize("topo,n", [
+    ([33, 35, 65, 31], 70), ([97, 66, 129, 18], 513), ([63, 127, 34, 21], 512), ([131, 70, 99, 37], 1025),       # tiles of 32 k and their
+    ([1001, 514, 203], 2050), ([785, 257, 67], 700),                                                            # rests, ragged rows
+])
+def test_ragged_fp32_layers_match_the_oracle(topo, n):
+    """Rows of FP32 values that begin anywhere: forwards, and gradients through sp_train_gemm32 and sp_train_grad_update."""
+    net, onet = public_net(topo, ["tanh"] * (len(topo) - 2) + ["softmax"], 1, seed=n)
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, topo[0])).astype(np.float32)
+    T = targets_for(rng, n, topo[-1], True)
+    assert rel_max_abs(S.forward_batch(net, X), onet.forward_batch(X)) <= TOL
+    S.train(net, X, T, 1, S.STRATEGY_FULL_BATCH, S.OPTIMIZER_SGD, learning_rate=1e-6)
+    assert S.last_error()[0] == S.SPINGALETT_OK, S.last_error()
+    gW, gB, _ = onet.batch_gradients(X, T)
+    nc = net.contents
+    arr = lambda name, cnt: np.ctypeslib.as_array(getattr(nc, name), shape=(int(cnt),))
+    assert rel_max_abs(arr("grad_weights", nc.total_weights), gW) <= TOL
+    assert rel_max_abs(arr("grad_biases", nc.total_biases), gB) <= TOL
+    S.free_network(net)
+
+
 @pytest.mark.parametrize("topo,acts,loss,n", [
     ([40, 500, 10], ["relu", "softmax"], 1, 2049), ([33, 131, 16], ["tanh", "softmax"], 0, 2500),       # few outputs of many samples:
     ([16, 512, 1], ["tanh", "sigmoid"], 0, 4097), ([20, 1024, 3], ["relu", "none"], 0, 16400),          # K in segments and whole,
