@@ -30,6 +30,9 @@ typedef struct {
     double *total_loss;              /* sum of the losses of the last epoch's places covered here, or NULL */
 } sp_tiny_run;
 
+/* sphip_train_step flag: the batch is the whole training set, which goes to the device once */
+#define SP_TRAIN_WHOLE_SET (1u << 30)
+
 /* Arrays of a net, flat like NeuralNetwork's, or NULL for those that stay where they are */
 typedef struct {
     float *weights, *biases, *m_weights, *m_biases, *v_weights, *v_biases, *g_weights, *g_biases;
