@@ -1215,6 +1215,31 @@ uint32_t gemm16_ragged_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper
 }
 
 // What the thin-operand kernel needs beyond the layer itself
+// K splits of the single-stage kernel for the other rows.  A tile walks its sums one K tile behind the other with a single one in
+// flight, 0.7 us each of 128, so a layer of few tiles and long sums waits on that chain, the chip nearly empty.  Up to a tile
+// per compute unit, two workgroups on each, at least four K tiles a part.  Forward of one layer, unsplit / split, us:
+//            samples x outputs   INT8 at K 1024    2048        3072        8192        FP16 at K 3072   8192
+//              260 x 100            8.6 /  8.6                 25.9 / 13.3 58.4 / 17.7   24.2 / 13.4   53.2 / 17.7
+//             1000 x 250           13.6 / 13.6   22.0 / 22.1   31.5 / 20.4 67.4 / 27.8   30.7 / 20.0   63.1 / 28.5
+//             2000 x 130           17.1 / 17.0   22.7 / 18.2   30.8 / 21.4 69.6 / 36.9   29.3 / 21.3   64.3 / 37.1
+//             6500 x  73           18.6 / 18.7   30.2 / 27.7   41.9 / 37.1  106 / 86     41.0 / 37.3    102 / 86
+// From 257 tiles on it loses below K = 3000 and gains little above: 2000 x 640 at K = 1024 16.4 / 22.8, 2048 26.1 / 26.5, 3584
+// 38.6 / 36.7; 1300 x 1250 at 1024 17.8 / 26.5, 3584 39.9 / 42.9.  1024 workgroups are no faster (1000 x 250 at 8192 30.4), 256
+// lose at large batches (2000 x 130 at 8192 41.3), and parts of two K tiles cost short sums (1000 x 640 at 1024 17.7 / 19.7).
+uint32_t gemm16_single_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper)
+{
+    const uint32_t tiles = ((M + 63u) / 64u) * ((N + 63u) / 64u), ktiles = (K + 127u) / 128u;
+    *kper = 0;
+    if (tiles > 256u) return 1;
+    uint32_t splits = (512u + tiles - 1) / tiles;
+    if (splits > 16u) splits = 16u;
+    if (splits > K / 512u) splits = K / 512u;
+    if (splits <= 1u) return 1;
+    const uint32_t per = (ktiles + splits - 1) / splits;
+    *kper = per * 128u;
+    return (ktiles + per - 1) / per;
+}
+
 struct ThinCtx {
     const uint16_t *w16;   // [N][K] 16-bit weights (raw 16-bit formats, or FP16 codes) when N <= 64, else nullptr
     float *ws;             // split-K workspace
@@ -1601,9 +1626,10 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     g.ksplits = 1;
     if (halves == 2) g.ws = ctx.ws;                  // one partial sum per activation matrix, added by the reduction
     const bool words = !aligned && L.K % 8u == 0 && ((uint64_t)L.K * fmt_bits(FMT)) % 32u == 0 && (FMT == I8 || FMT == I4 || FMT == I2);
-    if ((!aligned && !words) || single) {
+    {
+        const bool plain = (!aligned && !words) || single;
         uint32_t kper = 0;
-        const uint32_t sp = gemm16_ragged_splits(M, L.N, L.K, &kper);
+        const uint32_t sp = plain ? gemm16_ragged_splits(M, L.N, L.K, &kper) : gemm16_single_splits(M, L.N, L.K, &kper);
         if (sp > 1 && (uint64_t)sp * halves * M * L.N <= ctx.ws_floats) {
             g.kper = kper;
             g.ksplits = sp;
@@ -1621,7 +1647,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     const int shape = !(aligned || words) ? 11 : tiles(128, 128) >= 512u ? 22 : tiles(64, 128) >= 512u ? 12 : 11;
     // K of 1024 and more: K tiles of 128 instead of 64, half as many rounds of load, barrier, store, barrier (600 x 1280 x
     // 1536 FP16 18.2 -> 14.1 us, 4096 x 512 x 4096 48.6 -> 37.9 us; below 1024 no gain: 4096 x 512 x 784 INT8 12.5 / 13.0 us)
-    const bool deep = (aligned || words) && g.kper == 0 && L.K >= 1024u;
+    const bool deep = (aligned || words) && (single ? g.kper == 0 : g.kper % 128u == 0) && L.K >= 1024u;
     auto go = [&](auto tm_c, auto tn_c) {
         constexpr int TM = decltype(tm_c)::value, TN = decltype(tn_c)::value;
         const dim3 grid(tiles(64 * TM, 64 * TN), g.ksplits * halves);
@@ -1898,7 +1924,7 @@ struct WorkspaceNeed {
     uint64_t plane_bytes;      // digit planes: 4 bytes per element (+ padding of the last chunk) ...
     uint64_t plane_recs;       // ... and one scale (+ four digit sums) per 64 elements
     uint64_t split_floats;
-    uint64_t split_least;      // what of it no layer can do without (sp_skinny16 cuts K into as many parts as there is room for)
+    uint64_t split_least;      // what of it no layer can do without (sp_skinny16 and sp_gemm16 split K as far as there is room)
     uint64_t parts_floats;     // the partial sums that sp_gemm32_bf16_parts would like room for (it runs without them too)
     uint64_t cat_elems;        // split mode of an FP32 net: FP16 elements of the widest three-part layer input
 };
@@ -1953,6 +1979,11 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             } else {
                 const uint32_t sp = gemm16_splits(F16, n, N, K3, &kper);
                 if (sp > 1) ws = (uint64_t)sp * n * N;
+                const uint64_t single = gemm16_single_splits(n, N, K3, &kper);
+                if (single > 1 && single * n * N > ws) {
+                    spare = single * n * N - ws;
+                    ws += spare;
+                }
             }
         } else if (net->prec == F32) {
             if (reg == R_GEMV) continue;
@@ -1973,6 +2004,12 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
                 if (!aligned && !words) {
                     const uint32_t rs = gemm16_ragged_splits(n, N, K, &kper);
                     if (rs > 1) ws = (uint64_t)rs * halves * n * N;
+                } else {
+                    const uint64_t single = (uint64_t)gemm16_single_splits(n, N, K, &kper) * halves;
+                    if (single > halves && single * n * N > ws) {
+                        spare = single * n * N - ws;
+                        ws += spare;
+                    }
                 }
             }
         }
@@ -2683,7 +2720,7 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
         if (rows > 4u) rows = (rows + 3u) & ~3u;             // the next block's rows start as aligned as the first one's
         need = workspace_need(net, net->ptopo, rows, flags);
     }
-    // Partial sums of sp_skinny16 take what the rest leaves.
+    // Partial sums of sp_skinny16 and sp_gemm16 take what the rest leaves.
     const size_t total = all(net->ptopo, need);
     if (total > kScratchRoom) {
         const uint64_t over = (total - kScratchRoom + 255u) / 256u * (256u / sizeof(float));

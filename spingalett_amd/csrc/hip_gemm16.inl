@@ -119,7 +119,7 @@ __device__ __forceinline__ void unpack_word16(uint32_t w, uint32_t *o)
 }
 
 // Tile: BM x BN x BK (BK = 64, or 128 for a K of 1024 and more), 256 threads = 2 x 2 waves, each wave TM x TN tiles of
-// 32x32.  A K split (g.kper, whole tiles of 64) goes with BK = 64 only.
+// 32x32.  A K split (g.kper) is of whole tiles.
 // LDS rows are padded by 8 elements so that 128-bit fragment reads of 32
 // consecutive rows spread over the banks.
 // W4 (integer codes, ALIGNED activations): the weight rows are whole 32-bit words but not whole 16-byte units

@@ -692,6 +692,23 @@ def test_wide_inputs_of_integer_nets_run_padded(S, O, fmt, mode, K, N):
     S.free_network(net)
 
 
+@pytest.mark.parametrize("fmt,mode", [("f16", "plain"), ("bf16", "plain"), ("i8", "plain"), ("i4", "plain"), ("i2", "plain"), ("f16", "split"), ("i4", "split"), ("f32", "split")])
+@pytest.mark.parametrize("n,K,N", [(257, 1024, 65), (300, 1016, 200), (259, 1152, 130), (1100, 3000, 73), (500, 8192, 255), (1000, 1088, 1024),
+                                   (1030, 2064, 1020)])
+@pytest.mark.parametrize("act", ["tanh", "softmax"])
+def test_long_sums_of_few_tiles_are_split(S, O, fmt, mode, n, K, N, act):
+    """K splits of sp_gemm16 (gemm16_single_splits): even and uneven ones, partial K tiles, rows of whole words and of 16-byte units, a
+    layer of just as many tiles as run unsplit, against the float64 forward.  (FP16 inputs 2^-12, BF16 2^-9, split ones 2^-22.)"""
+    src = make_oracle_net(O, [K, N], [act], seed=n + K + N, bias_std=0.1)
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    if mode == "split":
+        assert S.lib().spingalett_set_net_activations(net, S.NET_ACTIVATIONS_SPLIT) == 0
+    X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
+    got = S.forward_batch(net, X)
+    S.free_network(net)
+    assert rel_max_abs(got, ref.forward_batch_f64(X)) <= (4e-5 if mode == "split" else 2e-2 if fmt == "bf16" else 5e-3)
+
+
 @pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
 @pytest.mark.parametrize("n,K,N", [(100, 128, 49152), (100, 192, 49160), (128, 320, 49410), (65, 1024, 49153)])
 def test_tiles_of_128_rows_in_every_format(S, O, fmt, n, K, N):
