@@ -918,16 +918,21 @@ bool rows_aligned(int fmt, uint32_t K) { return ((uint64_t)K * (uint64_t)fmt_bit
 // Whether the vector kernels read a first layer's weights as they were uploaded, next to the caller's rows.  Not where those
 // rows are no whole words, which leaves only the kernel that reads code by code, a wave to a row (1.5 us per 1000 codes, FP16 4.5),
 // and are long enough to pay for the launch that pads the input (one sample, as they are -> padded, us: 1531 x 777 FP16 8.9 -> 6.8,
-// BF16 5.2 -> 6.5, 4099 x 600 FP16 19.7 -> 8.0, BF16 9.5 -> 8.0, INT2 9.0 -> 8.4, 10078 x 112 INT8 19.3 -> 9.9, 7298 x 8070 FP16 80 ->
-// 21, INT4 43 -> 11; at four samples 4099 x 600 BF16 10.9 -> 11.4, 4097 x 9000 46.9 -> 23.5).  Integer layers of more than two samples only where
-// they reach the integer matrix cores (launch_gemv_i8): 5003 x 100 INT2 at four samples 12.2 against 17.3, 7298 x 8070 41 -> 20.
+// BF16 5.2 -> 6.5, 4099 x 600 FP16 19.7 -> 8.0, BF16 9.5 -> 8.0, INT8 9.1 -> 9.0, INT4 9.2 -> 7.2, INT2 8.8 -> 7.2, 9002 x 100 INT8 17.2
+// -> 13.6, 7297 x 8070 FP16 80 -> 21, INT4 42 -> 16; 3001 x 600 INT8 7.2 -> 7.9; at four samples 4099 x 600 BF16 10.9 -> 11.4, 4097 x
+// 9000 46.9 -> 23.5).  Padded rows stay in FP32 arithmetic, a word of codes a lane, whose decoding costs at three and four samples what the
+// wider loads bring in INT2 (12287 x 2048 25.3 -> 28.2; thin layers, a workgroup to a row, 24.4 -> 10.8) and in shorter rows of
+// INT8 (5003 x 1100 12.0 -> 13.0, 7297 x 1100 16.3 -> 16.6, 9002 x 1100 19.3 -> 19.2, 4099 x 8070 24.6 -> 22.6).
 bool raw_rows(int fmt, uint32_t K, uint32_t N, uint32_t n)
 {
-    if (fmt == F32 || rows_aligned(fmt, K) || K < (fmt == F16 ? 1280u : n > 2u && N < 2048u ? 5000u : 4096u)) return true;
+    if (fmt == F32 || rows_aligned(fmt, K)) return true;
     const uint64_t row_bits = (uint64_t)K * (uint64_t)fmt_bits(fmt);
-    if (fmt_bits(fmt) < 16)
-        return row_bits % 32u == 0 || (n > 2u && N > 64u && (uint64_t)N * K * n <= (fmt == I2 ? (2ull << 20) : (4ull << 20)));
-    return row_bits % 32u == 0 && N <= 64u && row_bits / 32u >= 256u;
+    if (fmt_bits(fmt) == 16) {
+        if (K < (fmt == F16 ? 1280u : n > 2u && N < 2048u ? 5000u : 4096u)) return true;
+        return row_bits % 32u == 0 && N <= 64u && row_bits / 32u >= 256u;
+    }
+    if (K < 4096u || row_bits % 32u == 0) return true;
+    return n > 2u && N > 64u && (fmt == I2 || (fmt == I8 && N < 4096u && K < 7168u));
 }
 
 template <int FMT>
@@ -2247,7 +2252,7 @@ int enqueue_forward(sphip_net *net, const Workspace &wk, const float *d_x, uint3
         bool soft_done = false;                 // the layer's own kernel wrote the softmax
         if (run) {
             if (reg == R_GEMV) launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n,
-                                          only_layer != 0 && net->aq_valid_layer == l && net->aq_valid_n == n, net->ptopo[l - 1] != net->topo[l - 1] && (l > 1 || raw));
+                                          only_layer != 0 && net->aq_valid_layer == l && net->aq_valid_n == n, net->ptopo[l - 1] != net->topo[l - 1]);
             if (reg == R_GEMV) { net->aq_valid_layer = l; net->aq_valid_n = n; }
             else if ((reg == R_GEMM32 || (reg == R_CAT3 && !cat3)) && f32_thin_vector(L, n))
                 launch_gemv(net->prec, wk, L, (const float *)in, (float *)main_out, n, false);
@@ -3002,8 +3007,7 @@ const char *sphip_layer_kernel_name(sphip_net *net, uint32_t layer, uint32_t n, 
     const float *aligned_ptr = reinterpret_cast<const float *>(uintptr_t{256});     // never dereferenced
     switch (pick_regime(net, n, flags)) {
     case R_GEMV:
-        launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false,
-                    net->ptopo[layer - 1] != net->topo[layer - 1] && (layer > 1 || raw_rows(net->prec, net->topo[0], net->ptopo[1], n)));
+        launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false, net->ptopo[layer - 1] != net->topo[layer - 1]);
         break;
     case R_GEMM32:
         if (f32_thin_vector(L, n)) launch_gemv(net->prec, net->workspace(), L, aligned_ptr, nullptr, n, false);

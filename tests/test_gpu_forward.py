@@ -675,6 +675,23 @@ def test_few_samples_of_rows_that_are_no_whole_words(S, O, fmt, K, N):
     S.free_network(net)
 
 
+@pytest.mark.parametrize("fmt,K,N", [("i8", 5003, 1000), ("i8", 7297, 901), ("i4", 5002, 1300), ("i4", 9001, 4100), ("i2", 9002, 1100), ("i2", 4104, 2600)])
+def test_few_large_inputs_cost_the_others_no_bits_in_ragged_rows(S, O, fmt, K, N):
+    """One to four samples, inputs of a million in front of weights of zero among ones of one: the activations of rows that are whole
+    units by padding only stay FP32 values of their own.  (FP32 sums: 2^-24 per term; 22 bits of a chunk's largest would be 0.5.)"""
+    src = make_oracle_net(O, [K, N], ["none"], seed=K + N, bias_std=0.1)
+    large = [0, 1, K // 3, 2048, K - 1]
+    src.W(0)[:, large] = 0.0
+    _, ref, net = quantized_pair(O, S, src, fmt)
+    X = np.random.default_rng(K).standard_normal((4, K)).astype(F32)
+    X[:, large] = np.array([1e6, -3e5, 2e5, -1e6, 7e5], F32)
+    want = ref.forward_batch_f64(X)
+    for n in (1, 2, 3, 4):
+        assert rel_max_abs(S.forward_batch(net, X[:n]), want[:n]) <= 1e-5, n
+    assert rel_max_abs(S.forward(net, X[1]), want[1]) <= 1e-5
+    S.free_network(net)
+
+
 @pytest.mark.parametrize("fmt,mode", [("i8", "plain"), ("i4", "plain"), ("i2", "plain"), ("i2", "split")])
 @pytest.mark.parametrize("K,N", [(2056, 300), (2072, 260), (4008, 131), (6024, 1030)])
 def test_wide_inputs_of_integer_nets_run_padded(S, O, fmt, mode, K, N):
