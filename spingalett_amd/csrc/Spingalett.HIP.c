@@ -285,7 +285,7 @@ static bool train_download(sp_net *sn)
     sn->opt_loaded = true;            /* the host gradient / moment arrays hold content from here on: layer() carries them */
     const sp_train_host all = {net->weights, net->biases, net->opt_m_weights, net->opt_m_biases, net->opt_v_weights, net->opt_v_biases,
                                net->grad_weights, net->grad_biases};
-    if (sp_train_arrays && sp_train_arrays(sn->dev, &all, true)) {
+    if (!sp_train_arrays || sp_train_arrays(sn->dev, &all, true)) {
         report(SPINGALETT_ERR_INVALID, "HIP back-end: train (download)");
         return false;
     }
@@ -396,10 +396,10 @@ void train_struct_arguments(TrainArgs args)
         report(SPINGALETT_ERR_ALLOC, "HIP back-end: train");
         return;
     }
-    if (!tiny && sp_train_arrays) {
+    if (!tiny) {
         const sp_train_host state = {had_device ? net->weights : NULL, had_device ? net->biases : NULL, net->opt_m_weights,
                                      net->opt_m_biases, net->opt_v_weights, net->opt_v_biases, NULL, NULL};
-        if (sp_train_arrays(sn->dev, &state, false)) {
+        if (!sp_train_arrays || sp_train_arrays(sn->dev, &state, false)) {
             report(SPINGALETT_ERR_INVALID, "HIP back-end: train (upload)");
             sp_hip_release(sn);           /* (it may hold half of the weights) */
             return;

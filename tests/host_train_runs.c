@@ -4,7 +4,9 @@
  * kernel translation unit: the device calls succeed, sp_train_tiny_run checks what it is given and counts.  A launch is
  * taken to last 5000 cycles and a quarter of a cycle per weight and sample for every step; none may pass 120 M cycles (50
  * ms) by more than a step.  The places of an epoch come in order, whole batches at a time, each exactly once, so do the
- * samples of a shuffled epoch, and the loss of an epoch is the sum over its parts.  tests/test_host_sanitizers.py builds and runs it. */
+ * samples of a shuffled epoch, and the loss of an epoch is the sum over its parts.
+ * Larger nets hand their arrays to sp_train_arrays, which here reads or writes every one at its full length.  Built with
+ * NO_ARRAYS it is missing, and train() has to say so.  tests/test_host_sanitizers.py builds and runs both. */
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -30,9 +32,10 @@ void sphip_train_end(sphip_net *n) { (void)n; }
 int sphip_train_set(sphip_net *n, int w, uint32_t l, const float *h) { (void)n; (void)w; (void)l; (void)h; return 0; }
 int sphip_train_get(sphip_net *n, int w, uint32_t l, float *h) { (void)n; (void)w; (void)l; (void)h; return 0; }
 int sphip_train_step(sphip_net *n, const float *x, const float *t, uint32_t k, const sphip_train_args *a, uint32_t f, float *tl)
-{ (void)n; (void)x; (void)t; (void)k; (void)a; (void)f; (void)tl; return 1; }
+{ (void)n; (void)x; (void)t; (void)k; (void)a; (void)f; if (tl) *tl = 0.0f; return 0; }
 
-static uint64_t g_weights;
+static uint64_t g_weights, g_biases;
+static bool g_large;                          /* the net does not fit one launch */
 static uint32_t g_next, g_runs;
 static uint64_t g_places, g_steps;
 static int g_bad;
@@ -40,7 +43,7 @@ static uint8_t *g_seen;                       /* per sample: how often it came *
 static double g_reported;
 
 bool sp_train_tiny_fits(uint32_t layers, const uint32_t *topology, uint32_t samples, uint32_t batch, bool ordered)
-{ (void)layers; (void)topology; (void)samples; (void)batch; (void)ordered; return true; }
+{ (void)layers; (void)topology; (void)samples; (void)batch; (void)ordered; return !g_large; }
 
 #define CHECK(c) do { if (!(c)) { fprintf(stderr, "run %u: %s\n", g_runs, #c); ++g_bad; } } while (0)
 int sp_train_tiny_run(sphip_net *net, const sp_tiny_run *r)
@@ -65,6 +68,32 @@ int sp_train_tiny_run(sphip_net *net, const sp_tiny_run *r)
     if (r->total_loss) *r->total_loss = 0.5 * r->count;
     return 0;
 }
+
+#ifndef NO_ARRAYS
+static uint32_t g_ups, g_downs;
+static float g_sum;                           /* of what went up */
+int sp_train_arrays(sphip_net *net, const sp_train_host *h, bool to_host)
+{
+    (void)net;
+    float *const arrays[8] = {h->weights, h->m_weights, h->v_weights, h->g_weights, h->biases, h->m_biases, h->v_biases, h->g_biases};
+    for (int a = 0; a < 8; ++a) {
+        if (!arrays[a]) continue;
+        for (uint64_t i = 0; i < (a < 4 ? g_weights : g_biases); ++i) {
+            if (to_host) arrays[a][i] = (float)(a + 1);
+            else g_sum += arrays[a][i];
+        }
+    }
+    if (to_host) {
+        for (int a = 0; a < 8; ++a) CHECK(arrays[a]);
+        ++g_downs;
+    } else {
+        CHECK(h->m_weights && h->m_biases && h->v_weights && h->v_biases);
+        CHECK((h->weights != NULL) == (g_ups > 0) && (h->biases != NULL) == (g_ups > 0));      /* (a new device net got them when it was made) */
+        ++g_ups;
+    }
+    return 0;
+}
+#endif
 
 static bool look(NeuralNetwork *net, size_t epoch, float error)
 {
@@ -100,10 +129,47 @@ static int one(uint32_t samples, uint32_t hidden, TrainingStrategy strategy, uin
     return g_bad;
 }
 
+/* a net whose steps are launches of their own, trained twice */
+static void large(void)
+{
+    enum { IN = 33, HIDDEN = 129, OUT = 7, SAMPLES = 50 };
+    NeuralNetwork *net = new_spingalett(.loss_func = LOSS_MSE);
+    layer(.net = net, .neurons_amount = IN);
+    layer(.net = net, .neurons_amount = HIDDEN, .act_func = ACT_TANH, .weight_initialization = WEIGHT_INITIALIZATION_XAVIER);
+    layer(.net = net, .neurons_amount = OUT, .act_func = ACT_NONE, .weight_initialization = WEIGHT_INITIALIZATION_XAVIER);
+    float *x = (float *)calloc(SAMPLES * IN, sizeof *x), *t = (float *)calloc(SAMPLES * OUT, sizeof *t);
+    g_large = true;
+    g_weights = net->total_weights;
+    g_biases = net->total_biases;
+    for (uint32_t run = 0; run < 2u; ++run) {
+        const float first = net->weights[0], last = net->biases[g_biases - 1u];
+        spingalett_clear_error();
+        train(.net = net, .inputs = x, .targets = t, .sample_count = SAMPLES, .epochs = 3, .training_strategy = STRATEGY_FULL_BATCH);
+#ifdef NO_ARRAYS
+        CHECK(spingalett_last_error_code() != SPINGALETT_OK);
+        CHECK(net->weights[0] == first && net->biases[g_biases - 1u] == last && net->time_step == 0);
+#else
+        (void)first;
+        (void)last;
+        CHECK(spingalett_last_error_code() == SPINGALETT_OK);
+        CHECK(g_ups == run + 1u && g_downs == run + 1u);
+        float *const arrays[8] = {net->weights, net->opt_m_weights, net->opt_v_weights, net->grad_weights,
+                                  net->biases, net->opt_m_biases, net->opt_v_biases, net->grad_biases};
+        for (int a = 0; a < 8; ++a) CHECK(arrays[a][0] == (float)(a + 1) && arrays[a][(a < 4 ? g_weights : g_biases) - 1u] == (float)(a + 1));
+#endif
+    }
+    printf("arrays of a larger net: %s\n", g_bad ? "not as they should be" : "as they should be");
+    g_large = false;
+    free(x);
+    free(t);
+    free_network(net);
+}
+
 int main(void)
 {
     spingalett_set_verbose(false);
     spingalett_set_log_level(LOG_NONE);
+    large();
     one(1000000, 8, STRATEGY_SAMPLE, 0, 2);                  /* an epoch of a million steps */
     one(24011, 8, STRATEGY_SAMPLE, 0, 3);                    /* a few steps more than a launch takes */
     one(100, 8, STRATEGY_SAMPLE, 0, 1000);                   /* many epochs to a launch */

@@ -34,3 +34,17 @@ def test_trainings_of_small_nets_are_cut_into_short_launches():
                          text=True, env=env, timeout=300)
     assert run.returncode == 0, run.stdout[-4000:]
     assert "1000000 samples" in run.stdout
+
+
+def test_trainings_hand_over_whole_arrays_or_say_that_they_cannot():
+    """`make train_runs`: the arrays of a larger net at their full lengths, there and back, under the sanitizers; a build without
+    sp_train_arrays reports an error instead of training on what the device happens to hold."""
+    res = subprocess.run(["make", "-C", CSRC, "train_runs"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0, res.stdout
+    env = dict(os.environ)
+    env.pop("LD_PRELOAD", None)
+    for name in ("host_train_runs", "host_train_runs_no_arrays"):
+        run = subprocess.run([os.path.join(CSRC, "build", name)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=env,
+                             timeout=300)
+        assert run.returncode == 0, run.stdout[-4000:]
+        assert "arrays of a larger net: as they should be" in run.stdout
