@@ -1219,7 +1219,6 @@ uint32_t gemm16_ragged_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper
     return (ktiles + per - 1) / per;
 }
 
-// What the thin-operand kernel needs beyond the layer itself
 // K splits of the single-stage kernel for the other rows.  A tile walks its sums one K tile behind the other with a single one in
 // flight, 0.7 us each of 128, so a layer of few tiles and long sums waits on that chain, the chip nearly empty.  Up to a tile
 // per compute unit, two workgroups on each, at least four K tiles a part.  Forward of one layer, unsplit / split, us:
@@ -1228,6 +1227,16 @@ uint32_t gemm16_ragged_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper
 //             1000 x 250           13.6 / 13.6   22.0 / 22.1   31.5 / 20.4 67.4 / 27.8   30.7 / 20.0   63.1 / 28.5
 //             2000 x 130           17.1 / 17.0   22.7 / 18.2   30.8 / 21.4 69.6 / 36.9   29.3 / 21.3   64.3 / 37.1
 //             6500 x  73           18.6 / 18.7   30.2 / 27.7   41.9 / 37.1  106 / 86     41.0 / 37.3    102 / 86
+// The partial sums and their launch cost 3 us and 4.4 a million, so the more outputs, the longer the sums for which that pays (INT8,
+// us):
+//            samples x outputs      K 1280        1536          1792          2048          2304          2560          3072
+//             5000 x  75         20.0 / 19.0   22.3 / 19.9   24.6 / 21.6   27.6 / 23.4   29.7 / 25.0
+//             1600 x 256                       17.5 / 17.2   20.0 / 18.1   21.8 / 19.3   24.1 / 19.7
+//             2000 x 250         16.0 / 16.5   18.2 / 18.1   20.1 / 18.5   22.2 / 18.9   24.2 / 19.3
+//             1024 x 512         14.4 / 15.6   16.3 / 17.2   18.2 / 18.0   20.0 / 19.4   21.9 / 20.5
+//             1000 x 640         14.5 / 16.8   16.2 / 17.9   18.2 / 19.2   19.9 / 21.4   22.0 / 21.3   24.3 / 21.9   28.4 / 23.7
+//             1000 x 1000        14.9 / 19.2   16.9 / 20.5   18.7 / 21.6   20.5 / 22.1   23.2 / 22.6   25.3 / 23.6   29.0 / 25.8
+//             INT4               14.6 / 18.7   16.7 / 20.2   18.4 / 21.4   19.9 / 22.7   22.2 / 24.4   24.1 / 25.5   (at 2688 25.1 / 25.6)
 // From 257 tiles on it loses below K = 3000 and gains little above: 2000 x 640 at K = 1024 16.4 / 22.8, 2048 26.1 / 26.5, 3584
 // 38.6 / 36.7; 1300 x 1250 at 1024 17.8 / 26.5, 3584 39.9 / 42.9.  1024 workgroups are no faster (1000 x 250 at 8192 30.4), 256
 // lose at large batches (2000 x 130 at 8192 41.3), and parts of two K tiles cost short sums (1000 x 640 at 1024 17.7 / 19.7).
@@ -1236,6 +1245,8 @@ uint32_t gemm16_single_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper
     const uint32_t tiles = ((M + 63u) / 64u) * ((N + 63u) / 64u), ktiles = (K + 127u) / 128u;
     *kper = 0;
     if (tiles > 256u) return 1;
+    const uint32_t outputs = M * N;                                          // (a million at most)
+    if (K < (outputs <= 430000u ? 1024u : outputs <= 530000u ? 1792u : outputs <= 700000u ? 2560u : 2816u)) return 1;
     uint32_t splits = (512u + tiles - 1) / tiles;
     if (splits > 16u) splits = 16u;
     if (splits > K / 512u) splits = K / 512u;
@@ -1245,6 +1256,7 @@ uint32_t gemm16_single_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper
     return (ktiles + per - 1) / per;
 }
 
+// What the thin-operand kernel needs beyond the layer itself
 struct ThinCtx {
     const uint16_t *w16;   // [N][K] 16-bit weights (raw 16-bit formats, or FP16 codes) when N <= 64, else nullptr
     float *ws;             // split-K workspace

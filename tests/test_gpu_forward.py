@@ -1745,6 +1745,22 @@ def test_streamed_rows_a_little_below_8192_take_no_longer(S, fmt):
     assert us[8100] <= 1.2 * us[8192]
 
 
+@pytest.mark.parametrize("fmt", ["f16", "i8"])
+def test_sums_too_short_for_a_split_take_no_longer(S, fmt):
+    """gemm16_single_splits: a million outputs of 1024 terms in 256 tiles, against a tenth more in 288 tiles, which are never split
+    (in two parts 1.3 times as long; now 0.95)."""
+    N, K, us = 1000, 1024, {}
+    net, W, b = _decoded_layer(S, fmt, N, K, seed=N)
+    for n in (1000, 1100):
+        assert S.lib().sphip_layer_kernel_name(net.h, 1, n, 0).decode() == "sp_gemm16"
+        X = np.random.default_rng(n).standard_normal((n, K)).astype(F32)
+        pre = X.astype(np.float64) @ W.T + b
+        assert rel_max_abs(net.forward(X), np.where(pre > 0, pre, 0.01 * pre)) <= 1e-3
+        us[n] = min(S.time_layer([net], 1, n, 100) for _ in range(5))
+    net.destroy()
+    assert us[1000] <= 1.12 * us[1100]
+
+
 def test_streamed_rows_of_8_kib_take_no_longer_than_others(S):
     """sp_skinny16 on rows that are a power of two of bytes long: read in step, they lay in a few of the memory's channels
     (16384 x 16384 INT4 1.35 times as long as 16384 x 15872; now even).  Weights larger than the memory-side cache."""
