@@ -1789,15 +1789,24 @@ void launch_gemm32_small(const Gemm32Args &g, uint32_t tile, const KSegments &se
 
 // FP32 layers of up to 16 outputs and many samples: sp_gemm32_head up to K = 512 (16384 samples, softmax included: 128 x 10 16.8 ->
 // 7.1 us, 256 x 16 19.3 -> 10.9, 512 x 16 24.2 -> 18.1; 777 x 10 26.9 against 34.9, 1000 x 10 35.8 against 42.8: its loads take 64
-// bytes of 16 rows, the tiles' DMA whole lines), and where it also forms a training step's output deltas up to K = 1024 in one
-// segment (an epoch of 20000 samples of 784-512-1000-10 932 -> 909 us; 8000 x 3 x 1500, in segments, 252 against 283).
+// bytes of 16 rows, the tiles' DMA whole lines).  Where it also forms a training step's output deltas, the launch and the passes it
+// saves pay up to K = 1024 in one segment, from the second round of tiles on (a step of 32-K-N, tiles / head, us):
+//                 K x N   640 x 1      640 x 10     784 x 1      784 x 10     1000 x 1     1000 x 10    1000 x 16
+//   16384 samples       135 / 136    145 / 139    152 / 157    161 / 164    168 / 177    178 / 182    183 / 190
+//   20000               163 / 163    175 / 165    177 / 178    191 / 182    203 / 206    216 / 210    225 / 222
+//   50000                                         392 / 393                 467 / 475
+// (a single output has no softmax to save).  Rows that are not whole 16-byte units: its loads lie across lines, while the tiles'
+// go through LDS once (a layer alone, tiles / head, us: 10 outputs of 6000 samples K = 129 7.9 / 7.7, 301 10.1 / 11.2, 511 12.5 /
+// 16.5; 10000 301 12.8 / 11.4, 402 13.4 / 13.2, 511 15.1 / 20.5; 20000 301 16.4 / 13.6, 482 21.9 / 24.5; 32768 402 24.4 / 22.5, 511
+// 27.5 / 27.5; 66000 402 78 / 42).
 bool gemm32_head_takes(uint32_t M, uint32_t N, uint32_t K, bool deltas, KSegments *seg)
 {
     if (N > 16u || M < 2048u || K > 1024u) return false;
     uint32_t kper = 0;
     const uint32_t splits = gemm32_fwd_splits(M, N, K, &kper);
     *seg = KSegments{kper, splits, 0};
-    return K <= 512u || (deltas && splits == 1u);
+    if (K <= 512u) return K % 4u == 0 || K <= 128u || M >= 32768u || (K <= 320u && M >= 10000u);
+    return deltas && splits == 1u && (K <= 640u || (N > 1u && M > 16384u));
 }
 
 void launch_gemm32_head(const Gemm32Args &g, const KSegments &seg, float *soft_out, const DeltaTail &tail)

@@ -1761,6 +1761,42 @@ def test_sums_too_short_for_a_split_take_no_longer(S, fmt):
     assert us[1000] <= 1.12 * us[1100]
 
 
+def _fp32_layer(S, N, K, seed):
+    rng = np.random.default_rng(seed)
+    W, b = (rng.standard_normal((N, K)) * 0.05).astype(F32), (rng.standard_normal(N) * 0.1).astype(F32)
+    net = S.DeviceNet([K, N], [S.ACT_LEAKY_RELU], S.PRECISION_FLOAT32)
+    net.upload(0, 0, W)
+    net.upload(0, 1, b)
+    return net, W.astype(np.float64), b.astype(np.float64)
+
+
+@pytest.mark.parametrize("n,K,N,kernel", [
+    (17000, 128, 10, "head"), (6000, 129, 10, "tiles"), (17000, 512, 16, "head"), (10001, 319, 3, "head"), (9999, 319, 3, "tiles"),
+    (10001, 321, 3, "tiles"), (8192, 511, 10, "tiles"), (32769, 511, 2, "head"), (8192, 516, 10, "tiles"),
+])
+def test_few_fp32_outputs_on_both_sides_of_their_kernels(S, n, K, N, kernel):
+    """gemm32_head_takes: rows of whole 16-byte units up to K = 512, others where the kernel of tiles is the slower one, against
+    float64.  (FP32 sums: 2^-24 per term.)"""
+    net, W, b = _fp32_layer(S, N, K, seed=n + K)
+    name = S.lib().sphip_layer_kernel_name(net.h, 1, n, 0).decode()
+    assert (name == "sp_gemm32_head") == (kernel == "head"), name
+    X = np.random.default_rng(n).standard_normal((n, K)).astype(F32)
+    pre = X.astype(np.float64) @ W.T + b
+    got = net.forward(X)
+    net.destroy()
+    assert rel_max_abs(got, np.where(pre > 0, pre, 0.01 * pre)) <= 1e-5
+
+
+def test_ragged_rows_into_few_fp32_outputs_take_no_longer(S):
+    """8192 samples of 511 values into 10 outputs against 513, which the kernel of tiles takes (sp_gemm32_head 1.4 times as long)."""
+    us = {}
+    for K in (511, 513):
+        net, _, _ = _fp32_layer(S, 10, K, seed=K)
+        us[K] = min(S.time_layer([net], 1, 8192, 100) for _ in range(5))
+        net.destroy()
+    assert us[511] <= 1.15 * us[513]
+
+
 def test_streamed_rows_of_8_kib_take_no_longer_than_others(S):
     """sp_skinny16 on rows that are a power of two of bytes long: read in step, they lay in a few of the memory's channels
     (16384 x 16384 INT4 1.35 times as long as 16384 x 15872; now even).  Weights larger than the memory-side cache."""
