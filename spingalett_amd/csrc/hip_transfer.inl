@@ -4,9 +4,9 @@
 // Array by array each transfer begins when the one before has ended: the arrays of a training of 784-512-1000-10, 26 MB there
 // and back in 42 calls of the runtime's, took 1.9 ms; 0.77 here with the launches of one epoch.  A few threads copy between the
 // caller's memory and a ring of pinned chunks while other chunks are on the bus (54 GB/s): the bus is the bound as long as the
-// host's copies keep up, which four threads do (55 GB/s; one thread 31, eight no more than four).  The helpers start once per call and
-// take parts of chunks in order.  The first chunks are small, so that the bus does not wait for a whole one to be filled, nor
-// the host for a whole one to arrive.
+// host's copies keep up, which four threads do (55 GB/s; one thread 31, eight no more than four).  The helpers start once per call,
+// take parts of chunks in order and sleep while there is none.  The first chunks are small, so that the bus does not wait for a whole
+// one to be filled, nor the host for a whole one to arrive.
 
 namespace {
 
@@ -15,7 +15,7 @@ constexpr size_t kStageChunk = 8u << 20, kFirstChunk = 512u << 10, kStagePart = 
 // 15 / 31 MiB up 81 / 174 / 253 / 553 / 795 us, the last two copied into 8 MB chunks by four threads, against 105 / 202 / 278 /
 // 408 / 739 here; 2 MB down 107 against 96, for which the ring is not worth its pinned memory).
 constexpr size_t kStagedUp = 10u << 20, kStagedDown = 4u << 20, kHelperLeast = 1u << 20;
-constexpr uint32_t kStageSlots = 4, kStageHelpers = 3;
+constexpr uint32_t kStageSlots = 4, kStageHelpers = 3, kIdleLooks = 64;
 
 struct StageRing {
     void *buf[kStageSlots] = {};
@@ -67,12 +67,16 @@ public:
         const int rc = pump(stream, landed, [&] {
             // (down: when the first chunk is here, which may be long after the call, behind everything the stream still does)
             try {
-                for (; started < wanted; ++started) helpers[started] = std::thread([this] { while (!stop_.load(std::memory_order_relaxed)) if (!copy_one()) std::this_thread::yield(); });
+                for (; started < wanted; ++started) helpers[started] = std::thread([this] { help(); });
             } catch (...) {
                 wanted = started;                       // no more threads to be had: fewer helpers
             }
         });
-        stop_.store(true);
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            stop_.store(true);
+        }
+        more_.notify_all();
         for (uint32_t t = 0; t < started; ++t) helpers[t].join();
         return rc;
     }
@@ -123,6 +127,23 @@ private:
         return true;
     }
 
+    // A helper looks for the next part a little and then sleeps until there is one: the chunk before it may be behind everything
+    // that the stream still does, for as long as that takes.
+    void help()
+    {
+        for (uint32_t idle = 0; !stop_.load(std::memory_order_relaxed);) {
+            if (copy_one()) {
+                idle = 0;
+            } else if (++idle < kIdleLooks) {
+                std::this_thread::yield();
+            } else {
+                std::unique_lock<std::mutex> lock(mu_);
+                more_.wait(lock, [this] { return stop_.load() || next_.load() < open_.load(); });
+                idle = 0;
+            }
+        }
+    }
+
     int submit(uint32_t c, hipStream_t stream)
     {
         char *const pin = static_cast<char *>(g_ring.buf[c % kStageSlots]);
@@ -169,8 +190,12 @@ private:
         uint32_t open = 0, sent = 0, freed = 0;        // chunks that may be copied, are on the bus or past it, (down) have been copied
         auto open_next = [&] {
             if (!to_host_) done_[open % kStageSlots].store(0u, std::memory_order_relaxed);
-            open_.store(chunk_end(open++), std::memory_order_release);
+            {
+                std::lock_guard<std::mutex> lock(mu_);
+                open_.store(chunk_end(open++), std::memory_order_release);
+            }
             if (open == 1u) start_helpers();
+            else more_.notify_all();
         };
         auto copied = [&](uint32_t c) { return done_[c % kStageSlots].load(std::memory_order_acquire) == (chunk_end(c) - chunk_at(c) + kStagePart - 1u) / kStagePart; };
         while (to_host_ ? freed < chunks_ : sent < chunks_) {
@@ -206,7 +231,10 @@ private:
                     }
                 }
             }
-            if (!copy_one() && !moved) std::this_thread::yield();
+            if (copy_one() || moved) continue;
+            // nothing to copy, to send or to hand out: a chunk on the bus is waited for where there is no other, else the helpers' copies
+            if (to_host_ ? freed == open : sent == open) HCHECK(hipEventSynchronize(g_ring.ev[open % kStageSlots]));
+            else std::this_thread::yield();
         }
         return 0;
     }
@@ -218,6 +246,8 @@ private:
     std::atomic<size_t> next_{0}, open_{0};        // bytes of the transfer that have been taken, that may be taken
     std::atomic<uint32_t> done_[kStageSlots] = {};
     std::atomic<bool> stop_{false};
+    std::mutex mu_;                                // open_ and stop_ change with it held, so that no helper sleeps through it
+    std::condition_variable more_;
 };
 
 // the ring's buffers, with its lock held

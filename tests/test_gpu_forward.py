@@ -17,6 +17,7 @@ agree 100 %.
 import ctypes as C
 import os
 import tempfile
+import time
 
 import numpy as np
 import pytest
@@ -1726,6 +1727,30 @@ def test_large_uploads_arrive_whole(S, nbytes):
         a = rng.integers(0, 256, nbytes, dtype=np.uint8)
         assert S.lib().sphip_memcpy_h2d(dst.ptr.value + shift, a.ctypes.data, nbytes) == 0
         assert np.array_equal(dst.to_numpy(np.uint8, nbytes + 4)[shift:shift + nbytes], a)
+
+
+def test_nobody_spins_behind_a_busy_stream(S):
+    """A large upload behind 0.1 s and more of kernels: the threads that copy sleep until a chunk is free (the caller and three helpers
+    looked for one all the time, four processors for as long as the kernels ran), and what arrives is whole."""
+    net = S.DeviceNet([4096] * 4, [S.ACT_RELU] * 3, S.PRECISION_FP16)
+    for l in range(3):
+        net.upload(l, 0, np.zeros(4096 * 4096, np.uint16))
+        net.upload(l, 1, np.zeros(4096, np.uint16))
+    n = 16384
+    d_x, d_y = S.DeviceBuffer.from_numpy(np.zeros((n, 4096), F32)), S.DeviceBuffer(n * 4096 * 4)
+    a = np.random.default_rng(3).random(16 << 20, dtype=F32)
+    dst = S.DeviceBuffer.from_numpy(a[::-1].copy())
+    net.forward_device(d_x, n, d_y)
+    S.synchronize()
+    for _ in range(120):
+        net.forward_device(d_x, n, d_y)
+    wall, cpu = time.perf_counter(), time.process_time()
+    assert S.lib().sphip_memcpy_h2d(dst.ptr, a.ctypes.data, a.nbytes) == 0
+    wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+    assert wall >= 0.05                                             # (it did wait)
+    assert cpu <= 2.0 * wall, (cpu, wall)
+    assert np.array_equal(dst.to_numpy(F32, a.size), a)
+    net.destroy()
 
 
 @pytest.mark.parametrize("fmt", ["i4", "i2"])
