@@ -15,7 +15,8 @@ constexpr size_t kStageChunk = 8u << 20, kFirstChunk = 512u << 10, kStagePart = 
 // 15 / 31 MiB up 81 / 174 / 253 / 553 / 795 us, the last two copied into 8 MB chunks by four threads, against 105 / 202 / 278 /
 // 408 / 739 here; 2 MB down 107 against 96, for which the ring is not worth its pinned memory).
 constexpr size_t kStagedUp = 10u << 20, kStagedDown = 4u << 20, kHelperLeast = 1u << 20;
-constexpr uint32_t kStageSlots = 4, kStageHelpers = 3, kIdleLooks = 64;
+constexpr uint32_t kStageSlots = 4, kStageHelpers = 3, kIdleLooks = 1000;
+constexpr uint32_t kInFlight = 8;              // chunks in the slots at once: seven at most (slot_of)
 
 struct StageRing {
     void *buf[kStageSlots] = {};
@@ -94,6 +95,12 @@ private:
     }
     size_t chunk_end(uint32_t c) const { return std::min(chunk_at(c + 1u), total_); }
 
+    // The slot a chunk lies in, and whether it is the first one there.  Up: the four that make 8 MB share one, so that the slots hold
+    // 32 MB of a transfer that has to wait for the stream, and the call need not.
+    uint32_t slot_of(uint32_t c) const { return (to_host_ ? c : c < 4u ? 0u : c - 3u) % kStageSlots; }
+    bool begins_slot(uint32_t c) const { return to_host_ || c == 0u || c >= 4u; }
+    char *chunk_pin(uint32_t c) const { return static_cast<char *>(g_ring.buf[slot_of(c)]) + (begins_slot(c) ? 0u : chunk_at(c)); }
+
     // f(segment, offset in it, offset from `from`, bytes) for what lies in [from, to) of the transfer
     template <class F>
     void each(size_t from, size_t to, F &&f) const
@@ -118,16 +125,16 @@ private:
         uint32_t c = 0;
         while (chunk_at(c + 1u) <= from) ++c;
         const size_t to = std::min(from + kStagePart, total_);
-        char *const pin = static_cast<char *>(g_ring.buf[c % kStageSlots]) + (from - chunk_at(c));
+        char *const pin = chunk_pin(c) + (from - chunk_at(c));
         each(from, to, [&](const Segment &s, size_t at, size_t in, size_t n) {
             if (to_host_) memcpy(s.host + at, pin + in, n);
             else memcpy(pin + in, s.host + at, n);
         });
-        done_[c % kStageSlots].fetch_add(1u, std::memory_order_release);
+        done_[c % kInFlight].fetch_add(1u, std::memory_order_release);
         return true;
     }
 
-    // A helper looks for the next part a little and then sleeps until there is one: the chunk before it may be behind everything
+    // A helper looks for the next part for some 0.2 ms, longer than a chunk takes, and then sleeps: the next chunk may be behind everything
     // that the stream still does, for as long as that takes.
     void help()
     {
@@ -146,7 +153,7 @@ private:
 
     int submit(uint32_t c, hipStream_t stream)
     {
-        char *const pin = static_cast<char *>(g_ring.buf[c % kStageSlots]);
+        char *const pin = chunk_pin(c);
         if (count_ == 1u) {
             const size_t at = chunk_at(c), n = std::min(chunk_end(c), seg_[0].bytes) - at;
             HCHECK(to_host_ ? hipMemcpyAsync(pin, seg_[0].dev + at, n, hipMemcpyDeviceToHost, stream)
@@ -169,7 +176,7 @@ private:
             flush();
             HCHECK(hipGetLastError());
         }
-        HCHECK(hipEventRecord(g_ring.ev[c % kStageSlots], stream));
+        HCHECK(hipEventRecord(g_ring.ev[slot_of(c)], stream));
         return 0;
     }
 
@@ -187,9 +194,9 @@ private:
     template <class Start>
     int pump(hipStream_t stream, const std::function<int(size_t)> &landed, Start &&start_helpers)
     {
-        uint32_t open = 0, sent = 0, freed = 0;        // chunks that may be copied, are on the bus or past it, (down) have been copied
+        uint32_t idle = 0, open = 0, sent = 0, freed = 0;        // chunks that may be copied, are on the bus or past it, (down) have been copied
         auto open_next = [&] {
-            if (!to_host_) done_[open % kStageSlots].store(0u, std::memory_order_relaxed);
+            if (!to_host_) done_[open % kInFlight].store(0u, std::memory_order_relaxed);
             {
                 std::lock_guard<std::mutex> lock(mu_);
                 open_.store(chunk_end(open++), std::memory_order_release);
@@ -197,18 +204,18 @@ private:
             if (open == 1u) start_helpers();
             else more_.notify_all();
         };
-        auto copied = [&](uint32_t c) { return done_[c % kStageSlots].load(std::memory_order_acquire) == (chunk_end(c) - chunk_at(c) + kStagePart - 1u) / kStagePart; };
+        auto copied = [&](uint32_t c) { return done_[c % kInFlight].load(std::memory_order_acquire) == (chunk_end(c) - chunk_at(c) + kStagePart - 1u) / kStagePart; };
         while (to_host_ ? freed < chunks_ : sent < chunks_) {
             bool moved = false;
             if (to_host_) {
                 for (; sent < chunks_ && sent < freed + kStageSlots; ++sent, moved = true) {
-                    done_[sent % kStageSlots].store(0u, std::memory_order_relaxed);
+                    done_[sent % kInFlight].store(0u, std::memory_order_relaxed);
                     if (submit(sent, stream)) return 1;
                 }
                 // (everything the stream does before the first chunk: waited for, not polled)
                 if (open == 0u) HCHECK(hipEventSynchronize(g_ring.ev[0]));
                 for (; open < sent; moved = true) {
-                    const int busy = slot_busy(open % kStageSlots);
+                    const int busy = slot_busy(slot_of(open));
                     if (busy < 0) return 1;
                     if (busy) break;
                     open_next();
@@ -216,8 +223,8 @@ private:
                 for (; freed < open && copied(freed); moved = true) ++freed;
             } else {
                 // (a slot's last transfer may be one of the call before)
-                for (; open < chunks_ && open < sent + kStageSlots; moved = true) {
-                    const int busy = slot_busy(open % kStageSlots);
+                for (; open < chunks_ && (open < 3u + kStageSlots || open < sent + kStageSlots); moved = true) {
+                    const int busy = begins_slot(open) ? slot_busy(slot_of(open)) : 0;
                     if (busy < 0) return 1;
                     if (busy) break;
                     open_next();
@@ -226,14 +233,18 @@ private:
                     if (submit(sent, stream)) return 1;
                     ++sent;
                     if (landed) {
-                        HCHECK(hipStreamWaitEvent(g_stream, g_ring.ev[(sent - 1u) % kStageSlots], 0));
+                        HCHECK(hipStreamWaitEvent(g_stream, g_ring.ev[slot_of(sent - 1u)], 0));
                         if (landed(std::min(chunk_end(sent - 1u), seg_[0].bytes))) return 1;
                     }
                 }
             }
-            if (copy_one() || moved) continue;
-            // nothing to copy, to send or to hand out: a chunk on the bus is waited for where there is no other, else the helpers' copies
-            if (to_host_ ? freed == open : sent == open) HCHECK(hipEventSynchronize(g_ring.ev[open % kStageSlots]));
+            if (copy_one() || moved) {
+                idle = 0;
+                continue;
+            }
+            // Nothing to copy, to send or to hand out.  Where it is a chunk on the bus that is missing, and for long, the runtime waits for
+            // it; else the helpers' copies are under way.
+            if (++idle >= kIdleLooks && (to_host_ ? freed == open : sent == open)) HCHECK(hipEventSynchronize(g_ring.ev[slot_of(open)]));
             else std::this_thread::yield();
         }
         return 0;
@@ -244,7 +255,7 @@ private:
     bool to_host_;
     size_t total_ = 0;
     std::atomic<size_t> next_{0}, open_{0};        // bytes of the transfer that have been taken, that may be taken
-    std::atomic<uint32_t> done_[kStageSlots] = {};
+    std::atomic<uint32_t> done_[kInFlight] = {};   // parts of a chunk that have been copied
     std::atomic<bool> stop_{false};
     std::mutex mu_;                                // open_ and stop_ change with it held, so that no helper sleeps through it
     std::condition_variable more_;

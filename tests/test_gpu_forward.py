@@ -1729,28 +1729,80 @@ def test_large_uploads_arrive_whole(S, nbytes):
         assert np.array_equal(dst.to_numpy(np.uint8, nbytes + 4)[shift:shift + nbytes], a)
 
 
+class _Busy:
+    """enqueue(): about 0.15 s of kernels."""
+
+    def __init__(self, S):
+        self.n = 16384
+        self.net = S.DeviceNet([4096] * 4, [S.ACT_RELU] * 3, S.PRECISION_FP16)
+        for l in range(3):
+            self.net.upload(l, 0, np.zeros(4096 * 4096, np.uint16))
+            self.net.upload(l, 1, np.zeros(4096, np.uint16))
+        self.x, self.y = S.DeviceBuffer.from_numpy(np.zeros((self.n, 4096), F32)), S.DeviceBuffer(self.n * 4096 * 4)
+        self.net.forward_device(self.x, self.n, self.y)
+        S.synchronize()
+
+    def enqueue(self):
+        for _ in range(120):
+            self.net.forward_device(self.x, self.n, self.y)
+
+
 def test_nobody_spins_behind_a_busy_stream(S):
-    """A large upload behind 0.1 s and more of kernels: the threads that copy sleep until a chunk is free (the caller and three helpers
-    looked for one all the time, four processors for as long as the kernels ran), and what arrives is whole."""
-    net = S.DeviceNet([4096] * 4, [S.ACT_RELU] * 3, S.PRECISION_FP16)
-    for l in range(3):
-        net.upload(l, 0, np.zeros(4096 * 4096, np.uint16))
-        net.upload(l, 1, np.zeros(4096, np.uint16))
-    n = 16384
-    d_x, d_y = S.DeviceBuffer.from_numpy(np.zeros((n, 4096), F32)), S.DeviceBuffer(n * 4096 * 4)
+    """A large upload behind kernels: the threads that copy sleep until a chunk is free (the caller and three helpers looked for one
+    all the time, four processors for as long as the kernels ran), and what arrives is whole."""
+    busy = _Busy(S)
     a = np.random.default_rng(3).random(16 << 20, dtype=F32)
     dst = S.DeviceBuffer.from_numpy(a[::-1].copy())
-    net.forward_device(d_x, n, d_y)
-    S.synchronize()
-    for _ in range(120):
-        net.forward_device(d_x, n, d_y)
+    busy.enqueue()
     wall, cpu = time.perf_counter(), time.process_time()
     assert S.lib().sphip_memcpy_h2d(dst.ptr, a.ctypes.data, a.nbytes) == 0
     wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
     assert wall >= 0.05                                             # (it did wait)
     assert cpu <= 2.0 * wall, (cpu, wall)
     assert np.array_equal(dst.to_numpy(F32, a.size), a)
-    net.destroy()
+    busy.net.destroy()
+
+
+class _LargeBatch:
+    """A net, a batch of 22.5 MB and what a step on it makes of the first layer's gradients."""
+
+    def __init__(self, S):
+        self.topo, n, rng = [256, 16, 10], 23000, np.random.default_rng(5)
+        self.net = S.DeviceNet(self.topo, [S.ACT_TANH, S.ACT_SOFTMAX], S.PRECISION_FLOAT32)
+        for l in range(2):
+            self.net.upload(l, 0, (rng.standard_normal(self.topo[l] * self.topo[l + 1]) * 0.1).astype(F32))
+            self.net.upload(l, 1, np.zeros(self.topo[l + 1], F32))
+        self.net.train_begin()
+        self.x, self.t = rng.standard_normal((n, 256)).astype(F32), np.zeros((n, 10), F32)
+        self.t[np.arange(n), rng.integers(0, 10, n)] = 1.0
+        self.args = S.SphipTrainArgs(S.OPTIMIZER_SGD, S.LOSS_CROSS_ENTROPY, 0.0, 0.0, 0.9, 0.9, 0.999, 1e-8, 0.0, 0.9, 0.999)
+        self.step()
+        self.want = self.gradients(S)
+
+    def step(self, x=None):
+        self.net.train_step(self.x if x is None else x, self.t, self.args)
+
+    def gradients(self, S):
+        return self.net.train_get(S.SPHIP_TRAIN_GW, 0).copy()
+
+
+def test_large_batch_is_staged_behind_a_busy_stream(S):
+    """A step's batch of 22.5 MB: the slots hold all of it, the call returns long before the kernels in front of it are done, and has
+    read the caller's array by then."""
+    busy, batch = _Busy(S), _LargeBatch(S)
+    for _ in range(2):
+        x = batch.x.copy()
+        S.synchronize()
+        busy.enqueue()
+        start = time.perf_counter()
+        batch.step(x)
+        back = time.perf_counter() - start
+        x[:] = 0.0
+        S.synchronize()
+        done = time.perf_counter() - start
+        assert done >= 0.05 and back <= 0.5 * done, (back, done)
+        assert np.array_equal(batch.gradients(S), batch.want)
+    busy.net.destroy()
 
 
 @pytest.mark.parametrize("fmt", ["i4", "i2"])
