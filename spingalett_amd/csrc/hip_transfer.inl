@@ -18,13 +18,17 @@ constexpr size_t kStagedUp = 10u << 20, kStagedDown = 4u << 20, kHelperLeast = 1
 constexpr uint32_t kStageSlots = 4, kStageHelpers = 3, kIdleLooks = 1000;
 constexpr uint32_t kInFlight = 8;              // chunks in the slots at once: seven at most (slot_of)
 
+// One ring for each direction: a download holds its own until all before it on the stream is done, which must not keep another
+// thread's upload from filling chunks.
 struct StageRing {
+    const size_t chunk;                            // the longest
     void *buf[kStageSlots] = {};
     hipEvent_t ev[kStageSlots] = {}, start = nullptr;
-    hipStream_t side = nullptr;
+    hipStream_t side = nullptr;                    // (with start: up only)
     bool ready = false;
     std::mutex mu;
-} g_ring;
+    explicit StageRing(size_t bytes) : chunk(bytes) {}
+} g_up{kStageChunk}, g_down{4u * kFirstChunk};
 
 // a contiguous part of a transfer; a transfer is its segments in a row, each beginning at a multiple of 64 bytes of it
 struct Segment {
@@ -53,14 +57,15 @@ __global__ __launch_bounds__(256) void sp_move_pieces(const PieceArgs a)
 
 class StagedTransfer {
 public:
-    StagedTransfer(const Segment *segments, uint32_t count, bool to_host) : seg_(segments), count_(count), to_host_(to_host)
+    StagedTransfer(const Segment *segments, uint32_t count, bool to_host)
+        : seg_(segments), count_(count), to_host_(to_host), ring_(to_host ? g_down : g_up)
     {
         for (uint32_t i = 0; i < count; ++i) total_ += padded(segments[i].bytes);
         chunks_ = 0;
         while (chunk_at(chunks_) < total_) ++chunks_;
     }
 
-    // The caller holds the ring's lock.  landed: see upload_from_host.
+    // The caller holds its ring's lock.  landed: see upload_from_host.
     int run(hipStream_t stream, const std::function<int(size_t)> &landed)
     {
         std::thread helpers[kStageHelpers];
@@ -99,7 +104,7 @@ private:
     // 32 MB of a transfer that has to wait for the stream, and the call need not.
     uint32_t slot_of(uint32_t c) const { return (to_host_ ? c : c < 4u ? 0u : c - 3u) % kStageSlots; }
     bool begins_slot(uint32_t c) const { return to_host_ || c == 0u || c >= 4u; }
-    char *chunk_pin(uint32_t c) const { return static_cast<char *>(g_ring.buf[slot_of(c)]) + (begins_slot(c) ? 0u : chunk_at(c)); }
+    char *chunk_pin(uint32_t c) const { return static_cast<char *>(ring_.buf[slot_of(c)]) + (begins_slot(c) ? 0u : chunk_at(c)); }
 
     // f(segment, offset in it, offset from `from`, bytes) for what lies in [from, to) of the transfer
     template <class F>
@@ -176,14 +181,14 @@ private:
             flush();
             HCHECK(hipGetLastError());
         }
-        HCHECK(hipEventRecord(g_ring.ev[slot_of(c)], stream));
+        HCHECK(hipEventRecord(ring_.ev[slot_of(c)], stream));
         return 0;
     }
 
     // 0: the slot's last transfer has ended, 1: not yet, -1: an error
-    static int slot_busy(uint32_t slot)
+    int slot_busy(uint32_t slot) const
     {
-        const hipError_t e = hipEventQuery(g_ring.ev[slot]);
+        const hipError_t e = hipEventQuery(ring_.ev[slot]);
         if (e == hipSuccess) return 0;
         (void)hipGetLastError();
         if (e == hipErrorNotReady) return 1;
@@ -213,7 +218,7 @@ private:
                     if (submit(sent, stream)) return 1;
                 }
                 // (everything the stream does before the first chunk: waited for, not polled)
-                if (open == 0u) HCHECK(hipEventSynchronize(g_ring.ev[0]));
+                if (open == 0u) HCHECK(hipEventSynchronize(ring_.ev[0]));
                 for (; open < sent; moved = true) {
                     const int busy = slot_busy(slot_of(open));
                     if (busy < 0) return 1;
@@ -233,7 +238,7 @@ private:
                     if (submit(sent, stream)) return 1;
                     ++sent;
                     if (landed) {
-                        HCHECK(hipStreamWaitEvent(g_stream, g_ring.ev[slot_of(sent - 1u)], 0));
+                        HCHECK(hipStreamWaitEvent(g_stream, ring_.ev[slot_of(sent - 1u)], 0));
                         if (landed(std::min(chunk_end(sent - 1u), seg_[0].bytes))) return 1;
                     }
                 }
@@ -244,7 +249,7 @@ private:
             }
             // Nothing to copy, to send or to hand out.  Where it is a chunk on the bus that is missing, and for long, the runtime waits for
             // it; else the helpers' copies are under way.
-            if (++idle >= kIdleLooks && (to_host_ ? freed == open : sent == open)) HCHECK(hipEventSynchronize(g_ring.ev[slot_of(open)]));
+            if (++idle >= kIdleLooks && (to_host_ ? freed == open : sent == open)) HCHECK(hipEventSynchronize(ring_.ev[slot_of(open)]));
             else std::this_thread::yield();
         }
         return 0;
@@ -253,6 +258,7 @@ private:
     const Segment *seg_;
     uint32_t count_, chunks_ = 0;
     bool to_host_;
+    StageRing &ring_;
     size_t total_ = 0;
     std::atomic<size_t> next_{0}, open_{0};        // bytes of the transfer that have been taken, that may be taken
     std::atomic<uint32_t> done_[kInFlight] = {};   // parts of a chunk that have been copied
@@ -261,17 +267,19 @@ private:
     std::condition_variable more_;
 };
 
-// the ring's buffers, with its lock held
-int ring_ready()
+// a ring's buffers, with its lock held
+int ring_ready(StageRing &r)
 {
-    if (g_ring.ready) return 0;
+    if (r.ready) return 0;
     for (uint32_t i = 0; i < kStageSlots; ++i) {
-        if (!g_ring.buf[i]) HCHECK(hipHostMalloc(&g_ring.buf[i], kStageChunk, hipHostMallocDefault));
-        if (!g_ring.ev[i]) HCHECK(hipEventCreateWithFlags(&g_ring.ev[i], hipEventDisableTiming));
+        if (!r.buf[i]) HCHECK(hipHostMalloc(&r.buf[i], r.chunk, hipHostMallocDefault));
+        if (!r.ev[i]) HCHECK(hipEventCreateWithFlags(&r.ev[i], hipEventDisableTiming));
     }
-    if (!g_ring.start) HCHECK(hipEventCreateWithFlags(&g_ring.start, hipEventDisableTiming));
-    if (!g_ring.side) HCHECK(hipStreamCreateWithFlags(&g_ring.side, hipStreamNonBlocking));
-    g_ring.ready = true;
+    if (&r == &g_up) {
+        if (!r.start) HCHECK(hipEventCreateWithFlags(&r.start, hipEventDisableTiming));
+        if (!r.side) HCHECK(hipStreamCreateWithFlags(&r.side, hipStreamNonBlocking));
+    }
+    r.ready = true;
     return 0;
 }
 
@@ -296,12 +304,12 @@ int upload_from_host(void *dst, const void *src, size_t bytes, const std::functi
         HCHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, g_stream));
         return landed ? landed(bytes) : 0;
     }
-    std::lock_guard<std::mutex> lock(g_ring.mu);
-    if (ring_ready()) return 1;
-    const hipStream_t stream = landed ? g_ring.side : g_stream;
+    std::lock_guard<std::mutex> lock(g_up.mu);
+    if (ring_ready(g_up)) return 1;
+    const hipStream_t stream = landed ? g_up.side : g_stream;
     if (landed) {
-        HCHECK(hipEventRecord(g_ring.start, g_stream));     // what is still reading dst
-        HCHECK(hipStreamWaitEvent(stream, g_ring.start, 0));
+        HCHECK(hipEventRecord(g_up.start, g_stream));       // what is still reading dst
+        HCHECK(hipStreamWaitEvent(stream, g_up.start, 0));
     }
     const Segment one{const_cast<char *>(static_cast<const char *>(src)), static_cast<char *>(dst), bytes};
     const int rc = StagedTransfer(&one, 1u, false).run(stream, landed);
@@ -317,8 +325,8 @@ int download_to_host(void *dst, const void *src, size_t bytes)
         HCHECK(hipStreamSynchronize(g_stream));
         return 0;
     }
-    std::lock_guard<std::mutex> lock(g_ring.mu);
-    if (ring_ready()) return 1;
+    std::lock_guard<std::mutex> lock(g_down.mu);
+    if (ring_ready(g_down)) return 1;
     const Segment one{static_cast<char *>(dst), const_cast<char *>(static_cast<const char *>(src)), bytes};
     const int rc = StagedTransfer(&one, 1u, true).run(g_stream, {});
     if (rc) (void)hipStreamSynchronize(g_stream);
@@ -328,8 +336,9 @@ int download_to_host(void *dst, const void *src, size_t bytes)
 // several arrays of whole floats at once, up (ordered on g_stream, the host arrays read when the call returns) or down
 int move_arrays(const Segment *segments, uint32_t count, bool to_host)
 {
-    std::lock_guard<std::mutex> lock(g_ring.mu);
-    if (ring_ready()) return 1;
+    StageRing &ring = to_host ? g_down : g_up;
+    std::lock_guard<std::mutex> lock(ring.mu);
+    if (ring_ready(ring)) return 1;
     const int rc = StagedTransfer(segments, count, to_host).run(g_stream, {});
     if (rc) (void)hipStreamSynchronize(g_stream);
     return rc;

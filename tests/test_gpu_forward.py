@@ -17,6 +17,7 @@ agree 100 %.
 import ctypes as C
 import os
 import tempfile
+import threading
 import time
 
 import numpy as np
@@ -1802,6 +1803,33 @@ def test_large_batch_is_staged_behind_a_busy_stream(S):
         done = time.perf_counter() - start
         assert done >= 0.05 and back <= 0.5 * done, (back, done)
         assert np.array_equal(batch.gradients(S), batch.want)
+    busy.net.destroy()
+
+
+def test_upload_does_not_wait_for_another_threads_download(S):
+    """Thread A waits for 8 MB of outputs behind a busy stream; a large batch of this thread's is staged meanwhile (the two shared a
+    lock)."""
+    busy, batch = _Busy(S), _LargeBatch(S)
+    net, W, b = _fp32_layer(S, 2000, 64, seed=9)
+    X = np.random.default_rng(9).standard_normal((1000, 64)).astype(F32)
+    net.forward(X)                                                  # (its buffers and the slots are there)
+    S.synchronize()
+    busy.enqueue()
+    got = []
+    other = threading.Thread(target=lambda: got.append(net.forward(X)))
+    other.start()
+    time.sleep(0.02)                                                # (it waits by then)
+    start = time.perf_counter()
+    batch.step()
+    back = time.perf_counter() - start
+    other.join()
+    done = time.perf_counter() - start
+    S.synchronize()
+    assert done >= 0.05 and back <= 0.5 * done, (back, done)
+    pre = X.astype(np.float64) @ W.T + b
+    assert rel_max_abs(got[0], np.where(pre > 0, pre, 0.01 * pre)) <= 1e-5
+    assert np.array_equal(batch.gradients(S), batch.want)
+    net.destroy()
     busy.net.destroy()
 
 
