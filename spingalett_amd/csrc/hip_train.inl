@@ -1050,9 +1050,11 @@ int sp_train_arrays(sphip_net *net, const sp_train_host *h, bool to_host)
 {
     if (!net || !net->train) return fail_msg("sp_train_arrays: sphip_train_begin was not called for this net");
     sphip_train_state *ts = net->train;
-    std::vector<Segment> seg;
+    const std::unique_ptr<Segment[]> seg(new (std::nothrow) Segment[2u * net->layers + 6u]);
+    if (!seg) return fail_msg("sp_train_arrays: out of host memory");
+    uint32_t count = 0;
     auto add = [&](float *host, void *dev, uint64_t cnt) {
-        if (host) seg.push_back({reinterpret_cast<char *>(host), static_cast<char *>(dev), cnt * sizeof(float)});
+        if (host) seg[count++] = {reinterpret_cast<char *>(host), static_cast<char *>(dev), cnt * sizeof(float)};
     };
     for (uint32_t l = 0; l + 1 < net->layers; ++l) {
         add(h->weights ? h->weights + ts->woff[l] : nullptr, net->W[l].base, net->W[l].count);
@@ -1065,7 +1067,7 @@ int sp_train_arrays(sphip_net *net, const sp_train_host *h, bool to_host)
     add(h->m_biases, ts->mB, ts->total_b);
     add(h->v_biases, ts->vB, ts->total_b);
     add(h->g_biases, ts->gB, ts->total_b);
-    return move_arrays(seg.data(), (uint32_t)seg.size(), to_host);
+    return move_arrays(seg.get(), count, to_host);
 }
 
 int sphip_train_step(sphip_net *net, const float *x, const float *targets, uint32_t n, const sphip_train_args *args,
