@@ -1327,30 +1327,41 @@ uint32_t thin_splits(int fmt, int st, uint32_t wgs, uint32_t chunks, uint64_t ou
     return best;
 }
 
-// mode_b streams 16-bit activations (fmt = the activation type), mode a the weights.  most_sums: thin_splits().
-ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K, uint64_t most_sums = ~0ull)
+// mode_b streams 16-bit activations (fmt = the activation type), mode a the weights.  most_sums: thin_splits().  halves: activation
+// matrices.
+ThinPlan plan_thin(int fmt, uint32_t M, uint32_t N, uint32_t K, uint64_t most_sums = ~0ull, uint32_t halves = 1)
 {
     ThinPlan p{};
     // Few outputs: sp_skinny16_kw_head, one launch.  Against sp_skinny16_regs and its reduction (more than 16 outputs; us, FP16):
     // 1024 x 20 at 16 / 1000 / 16384 samples 12.8 / 15.5 / 42.4 -> 7.6 / 8.7 / 27.6, 1536 x 48 14.5 / 18.4 / 56.6 -> 12.5 / 14.4 /
-    // 43.6.  Its eight waves are all the K split there is, and a workgroup reads all weights for its samples: few samples of
-    // longer sums into 33 to 64 outputs are left to the split (2048 x 50 at 16 samples 12.7 against 13.1, at 256 18.4 against
-    // 16.5; 3072 x 40 at 64 16.4 against 17.3, at 1000 21.7 against 20.4).  Up to 16 outputs a split pays beyond 4096 only (4096 x 10 at
-    // 64 samples 11.1 without, 14.0 in two parts; 8192 x 10 17.9 and, in four, 14.5).  Two sixteens of samples a workgroup where
-    // there are enough to fill the chip with them (1024 x 33 at 8192 samples 23.4 -> 20.9, at 4096 16.5 -> 17.2), not with one of
-    // outputs (1000 x 10 at 8192 samples 15.3 -> 16.7 in workgroups of 64).
+    // 43.6.  Its eight waves are all the K split there is for more than 16 outputs, and a workgroup reads all weights for its samples:
+    // few samples of longer sums into many outputs are left to the split (2048 x 50 at 16 samples 12.7 against 13.1, at 256 18.4
+    // against 16.5; 3072 x 32 at 16 samples 12.0 against 13.0, x 20 11.9 against 11.6, with split activations 15.8 against 16.1;
+    // 3072 x 40 at 64 16.4 against 17.3, at 1000 21.7 against 20.4).  Up to 16 outputs K is cut over the grid as well where the samples
+    // are few, in parts of 1024 from 3072 on (x 16 at K = 4096, 16 / 64 / 1000 samples 11.8 / 12.1 / 15.7 whole, 9.2 / 9.9 / 14.5 in
+    // four; with split activations 15.8 / 16.1 / 20.7 and 10.0 / 11.2 / 16.8, x 1 12.6 / 13.0 / 17.4 and 9.3 / 10.3 / 15.6), up to eight
+    // of them (x 16 at 16384 and 64 samples 14.4, in four 16.3); up to eight outputs of unsplit activations, or of as few samples, in parts of
+    // 2048 beyond 4096, below which the second launch costs what they bring (x 8 at 4096 and 64 samples 10.8 whole, 11.3 in four).  From 129
+    // workgroups on no longer (x 16 at 4096 and 4096 samples 25.9 whole, 28.9 in two), but for rows of split activations that L2 does
+    // not hold (x 10 at 16384 and 4096 samples 178 and 163).  Two sixteens of samples a workgroup where there are enough to fill the
+    // chip with them (1024 x 33 at 8192 samples 23.4 -> 20.9, at 4096 16.5 -> 17.2), not with one of outputs (1000 x 10 at 8192
+    // samples 15.3 -> 16.7 in workgroups of 64).
     const int nt = N <= 16u ? 1 : N <= 32u ? 2 : 4;
     if (N <= 64 && K % 8u == 0 && M >= 1 &&
-        (nt == 1 || K * nt <= 6144u || (K <= 2048u && M >= 128u) || (K <= 3072u && M >= 1000u))) {
+        (nt == 1 || (K * nt <= 6144u && (halves == 2u || N * K <= (84u << 10))) || (K <= 2048u && M >= 128u) || (K <= 3072u && M >= 1000u))) {
         p.use = p.mode_b = p.head = true; p.R = M; p.NC = N;
         p.nt = nt;
         p.st = p.nt > 1 && M >= 8192u ? 2 : 1;
         p.cblocks = 1;
         p.row_blocks = (M + 16u * p.st - 1u) / (16u * p.st);
         const uint32_t steps = (K + 31u) / 32u;
+        const bool fine = nt == 1 && (N > 8u || (halves == 2u && M > 8u));
         uint32_t splits = K > 4096u ? K / 2048u : 1u;
-        if (splits > 256u / p.row_blocks) splits = 256u / p.row_blocks;
+        if (fine && K >= 3072u && splits < 8u) splits = K / 1024u < 8u ? K / 1024u : 8u;
+        const uint32_t room = (halves == 2u && K >= 16384u ? 512u : 256u) / p.row_blocks;
+        if (splits > room) splits = room;
         if (splits > 16u) splits = 16u;
+        if (splits > most_sums / ((uint64_t)M * N)) splits = (uint32_t)(most_sums / ((uint64_t)M * N));
         if (splits < 1u) splits = 1u;
         const uint32_t per = (steps + splits - 1u) / splits;
         p.kper = per * 32u;
@@ -1569,7 +1580,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         else sp_gemm16_small<FMT, F16T, false><<<grid, 512, 0, g_stream>>>(g);
         return;
     }
-    const ThinPlan tp = plan_thin(FMT, M, L.N, L.K, ctx.ws_floats / halves);
+    const ThinPlan tp = plan_thin(FMT, M, L.N, L.K, ctx.ws_floats / halves, halves);
     if (tp.use && !single && (!tp.mode_b || ctx.w16) &&
         ((tp.splits == 1 && (halves == 1 || tp.head)) || (uint64_t)tp.splits * halves * tp.NC * tp.R <= ctx.ws_floats)) {
         SkinnyArgs a{};
@@ -1952,7 +1963,7 @@ struct WorkspaceNeed {
     uint64_t plane_bytes;      // digit planes: 4 bytes per element (+ padding of the last chunk) ...
     uint64_t plane_recs;       // ... and one scale (+ four digit sums) per 64 elements
     uint64_t split_floats;
-    uint64_t split_least;      // what of it no layer can do without (sp_skinny16 and sp_gemm16 split K as far as there is room)
+    uint64_t split_least;      // what of it no layer can do without (sp_skinny16, sp_skinny16_kw_head and sp_gemm16 split K as far as there is room)
     uint64_t parts_floats;     // the partial sums that sp_gemm32_bf16_parts would like room for (it runs without them too)
     uint64_t cat_elems;        // split mode of an FP32 net: FP16 elements of the widest three-part layer input
 };
@@ -2003,7 +2014,7 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             const ThinPlan tp = plan_thin(F16, n, N, K3);
             if (tp.use) {
                 if (tp.splits > 1) ws = (uint64_t)tp.splits * tp.NC * tp.R;
-                if (!tp.kw && !tp.regs && !tp.head) spare = ws;
+                if (!tp.kw && !tp.regs) spare = ws;
             } else {
                 const uint32_t sp = gemm16_splits(F16, n, N, K3, &kper);
                 if (sp > 1) ws = (uint64_t)sp * n * N;
@@ -2020,10 +2031,10 @@ WorkspaceNeed workspace_need(const sphip_net *net, const std::vector<uint32_t> &
             const uint64_t parts = gemm32_parts_pay(batch, N, K) ? gemm32_parts_splits(n, N, K, &kper) : 1u;
             if (parts > 1 && parts * n * N > w.parts_floats) w.parts_floats = parts * n * N;
         } else {
-            const ThinPlan tp = plan_thin(net->prec, n, N, K);
+            const ThinPlan tp = plan_thin(net->prec, n, N, K, ~0ull, halves);
             if (tp.use) {
                 if (tp.splits > 1 || halves > 1) ws = (uint64_t)tp.splits * halves * tp.NC * tp.R;
-                if (!tp.kw && !tp.regs && !tp.head) spare = ws - (halves > 1 ? (uint64_t)halves * tp.NC * tp.R : 0u);
+                if (!tp.kw && !tp.regs) spare = ws - (halves > 1 ? (uint64_t)halves * tp.NC * tp.R : 0u);
             } else {
                 const uint32_t sp = gemm16_splits(net->prec, n, N, K, &kper);
                 if (sp > 1 || halves > 1) ws = (uint64_t)sp * halves * n * N;
@@ -2748,7 +2759,7 @@ int sphip_forward_noalloc(sphip_net *net, const float *d_x, uint32_t n, float *d
         if (rows > 4u) rows = (rows + 3u) & ~3u;             // the next block's rows start as aligned as the first one's
         need = workspace_need(net, net->ptopo, rows, flags);
     }
-    // Partial sums of sp_skinny16 and sp_gemm16 take what the rest leaves.
+    // Partial sums of sp_skinny16, sp_skinny16_kw_head and sp_gemm16 take what the rest leaves.
     const size_t total = all(net->ptopo, need);
     if (total > kScratchRoom) {
         const uint64_t over = (total - kScratchRoom + 255u) / 256u * (256u / sizeof(float));
