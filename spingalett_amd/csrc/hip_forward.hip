@@ -1586,7 +1586,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         SkinnyArgs a{};
         a.halves = halves; a.half_elems = (uint64_t)M * L.K;
         a.L = L; a.C = C; a.ws = ctx.ws; a.R = tp.R; a.NC = tp.NC; a.row_blocks = tp.row_blocks; a.cblocks = tp.cblocks; a.kper = tp.kper; a.out_f32 = out_f32; a.mode_b = tp.mode_b ? 1 : 0;
-        tl_route.name = tp.kw || tp.head ? "sp_skinny16_kw" : tp.regs ? "sp_skinny16_regs" : "sp_skinny16";
+        tl_route.name = tp.head ? "sp_skinny16_kw_head" : tp.kw ? "sp_skinny16_kw" : tp.regs ? "sp_skinny16_regs" : "sp_skinny16";
         if (tp.mode_b) {
             if (ctx.soft_out && tp.head && tp.splits == 1 && ctx.soft_kind != 3) {
                 a.soft_out = ctx.soft_out;

@@ -622,6 +622,8 @@ def test_few_outputs_at_the_edges_of_their_tiles(S, O, fmt, mode, n, K, N, act):
     if mode != "plain":
         which = S.NET_ACTIVATIONS_SPLIT if mode == "split" else S.NET_ACTIVATIONS_BF16
         assert S.lib().spingalett_set_net_activations(net, which) == 0
+    flags = {"plain": 0, "split": S.SPHIP_SPLIT_ACTIVATIONS, "bf16": S.SPHIP_BF16_ACTIVATIONS}[mode]
+    assert S.lib().sphip_layer_kernel_name(S.lib().spingalett_hip_handle(net), 1, n, flags).decode() == "sp_skinny16_kw_head"
     X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
     got = S.forward_batch(net, X)
     part = S.forward_batch(net, X[:n // 2 + 5])                    # other tiles' edges, through the same buffers
@@ -1237,7 +1239,7 @@ def _same_nonfinite(got, want):
     ("i2", 8192, 8192, 4, 0, "sp_gemv_i8mfma"), ("i8", 1030, 1040, 17, 16, "sp_gemv_i8mfma"),
     ("i4", 512, 1024, 2, 0, "sp_gemv"), ("bf16", 600, 512, 4, 0, "sp_gemv"), ("i2", 301, 250, 3, 0, "sp_gemv_generic"),
     ("i4", 16384, 2048, 8, 0, "sp_skinny16_kw"), ("i8", 2100, 2064, 48, 0, "sp_skinny16"),
-    ("f16", 1500, 4096, 60, 0, "sp_skinny16"), ("bf16", 10, 1000, 300, 0, "sp_skinny16_kw"),
+    ("f16", 1500, 4096, 60, 0, "sp_skinny16"), ("bf16", 10, 1000, 300, 0, "sp_skinny16_kw_head"),
     ("f16", 1500, 1000, 77, 0, "sp_gemm16_small"), ("i2", 600, 1000, 200, 0, "sp_gemm16_small"),
     ("bf16", 2048, 4096, 600, 0, "sp_gemm16_big"), ("i2", 2048, 4096, 1000, 0, "sp_gemm16_big"),
     ("bf16", 2048, 2048, 600, 0, "sp_gemm16"),
