@@ -713,17 +713,28 @@ def test_wide_inputs_of_integer_nets_run_padded(S, O, fmt, mode, K, N):
     S.free_network(net)
 
 
-@pytest.mark.parametrize("fmt,mode", [("f16", "plain"), ("bf16", "plain"), ("i8", "plain"), ("i4", "plain"), ("i2", "plain"), ("f16", "split"), ("i4", "split"), ("f32", "split")])
-@pytest.mark.parametrize("n,K,N", [(257, 1024, 65), (300, 1016, 200), (259, 1152, 130), (1100, 3000, 73), (500, 8192, 255), (1000, 1088, 1024),
-                                   (1030, 2064, 1020)])
-@pytest.mark.parametrize("act", ["tanh", "softmax"])
+_PLAIN_AND_SPLIT = [("f16", "plain"), ("bf16", "plain"), ("i8", "plain"), ("i4", "plain"), ("i2", "plain"), ("f16", "split"), ("i4", "split")]
+
+
+@pytest.mark.parametrize("n,K,N,act,fmt,mode", [(*layer, *how) for layer, hows in [
+    ((257, 2064, 65, "tanh"), _PLAIN_AND_SPLIT),               # four parts, the last of two K tiles; rows of words in INT4 and INT2
+    ((5000, 1168, 75, "softmax"), _PLAIN_AND_SPLIT),           # two parts, the last K tile partial
+    ((300, 3024, 200, "softmax"), _PLAIN_AND_SPLIT),           # padded INT4 and INT2 rows
+    ((1100, 3024, 73, "tanh"), _PLAIN_AND_SPLIT),
+    ((1100, 3000, 73, "softmax"), [("f16", "plain"), ("i8", "plain"), ("i4", "split")]),           # rows of words in INT8
+    ((500, 8192, 255, "tanh"), _PLAIN_AND_SPLIT),
+    ((1000, 8200, 250, "softmax"), _PLAIN_AND_SPLIT),
+    ((1000, 8200, 250, "tanh"), [("f32", "split")]), ((3000, 2056, 250, "softmax"), [("f32", "split")]),   # sums three times as long
+] for how in hows])
 def test_long_sums_of_few_tiles_are_split(S, O, fmt, mode, n, K, N, act):
-    """K splits of sp_gemm16 (gemm16_single_splits): even and uneven ones, partial K tiles, rows of whole words and of 16-byte units, a
-    layer of just as many tiles as run unsplit, against the float64 forward.  (FP16 inputs 2^-12, BF16 2^-9, split ones 2^-22.)"""
+    """K splits of sp_gemm16 (gemm16_single_splits): even and uneven ones, partial K tiles, rows of whole words and of 16-byte units,
+    against the float64 forward.  (FP16 inputs 2^-12, BF16 2^-9, split ones 2^-22.)"""
     src = make_oracle_net(O, [K, N], [act], seed=n + K + N, bias_std=0.1)
     _, ref, net = quantized_pair(O, S, src, fmt)
     if mode == "split":
         assert S.lib().spingalett_set_net_activations(net, S.NET_ACTIVATIONS_SPLIT) == 0
+    flags = S.SPHIP_SPLIT_ACTIVATIONS if mode == "split" else 0
+    assert S.lib().sphip_layer_kernel_name(S.lib().spingalett_hip_handle(net), 1, n, flags).decode() == "sp_gemm16"
     X = np.random.default_rng(K).standard_normal((n, K)).astype(F32)
     got = S.forward_batch(net, X)
     S.free_network(net)
