@@ -48,6 +48,13 @@ CASES = [
     ("bf16", [512, 1024, 1000], ["leaky_relu", "softmax"], (2048, 70), 128),
     ("i8", [777, 1030, 515, 33], ["relu", "tanh", "none"], (64, 5), 0),            # ragged rows: K split of the single-stage kernel
     ("i2", [256, 256, 256, 64, 10], ["relu", "relu", "tanh", "softmax"], (3, 1), 0),   # word-per-lane vector kernel
+    ("i8", [3072, 250, 10], ["relu", "softmax"], (1000, 300), 0),                  # K splits of the single-stage kernel
+    ("i4", [1024, 4096, 1000], ["tanh", "softmax"], (64, 17), 0),                  # softmax with the addition of the parts
+    ("bf16", [8192, 300, 9], ["softmax", "none"], (40, 9), 128),                   # ... of a hidden layer, into both matrices
+    ("f16", [4096, 16, 16384, 12], ["tanh", "relu", "softmax"], (300, 20), 0),     # few outputs, K in parts
+    ("f16", [4099, 600, 7], ["tanh", "none"], (4, 1), 0),                          # padded input of the vector kernels
+    ("i8", [9002, 1100, 7], ["tanh", "none"], (4, 2), 0),
+    ("i2", [4104, 2600, 7], ["tanh", "none"], (2, 1), 0),
 ]
 
 
@@ -151,6 +158,8 @@ def test_noalloc_forward_cuts_k_into_as_many_parts_as_fit(S, topo, n, flags):
     ("i2", [3, 1, 33, 2], 250001, 0),                     # widths below one unit, a batch that blocks do not divide
     ("i8", [777, 1030, 515, 33], 4000, 128),              # split activations: partial sums of both matrices
     ("i8", [16, 400001, 40, 10], 8, 0),                   # the FP16 copy of the codes does not fit: the tile kernel
+    ("i8", [8192, 250], 900, 0),                          # 59.0 MB of activations: eight parts of sp_gemm16's sums are 7.2 MB too many
+    ("f16", [16384, 16], 511, 0),                         # 67.0 MB: five of sp_skinny16_kw_head's eight parts fit
 ])
 def test_noalloc_forward_takes_what_fits_without_the_padding(S, fmt, topo, n, flags):
     """What is accepted goes by the net's own widths; 2e-2 against sphip_forward like every 16-bit route against another
