@@ -1743,6 +1743,20 @@ def test_large_uploads_arrive_whole(S, nbytes):
         assert np.array_equal(dst.to_numpy(np.uint8, nbytes + 4)[shift:shift + nbytes], a)
 
 
+@pytest.mark.parametrize("nbytes", [(4 << 20) - 4, 4 << 20, (4 << 20) + 4, (11 << 19) + 4, (15 << 19) - 4, (35 << 20) + 4])
+def test_large_downloads_arrive_whole(S, nbytes):
+    """Downloads at, below and past the line of the ring of chunks and its borders: a net that hands out what it was given."""
+    net = S.new_spingalett(S.LOSS_MSE)
+    S.layer(net, 1)
+    S.layer(net, 1, S.ACT_NONE, S.WEIGHT_INITIALIZATION_NONE)
+    S.weights_view(net, 0)[:] = 1.0
+    S.biases_view(net, 0)[:] = 0.0
+    for seed in (nbytes, 1):
+        X = np.random.default_rng(seed).standard_normal((nbytes // 4, 1)).astype(F32)
+        assert np.array_equal(S.forward_batch(net, X), X)
+    S.free_network(net)
+
+
 class _Busy:
     """enqueue(): about 0.15 s of kernels."""
 

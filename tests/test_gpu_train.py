@@ -692,3 +692,29 @@ def test_steps_from_host_batches_match_oracle(topo, acts, loss, n):
         assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_MW, l), st.mW[wo: wo + wc]) <= 2 * TOL, l
         assert rel_max_abs(d.train_get(S.SPHIP_TRAIN_VB, l), st.vB[bo: bo + bc]) <= 2 * TOL, l
     d.destroy()
+
+
+@pytest.mark.parametrize("topo,n", [
+    ([33] * 21, 64),                      # 46 pieces in a chunk, more than a launch moves at once
+    ([701, 997, 3], 70),                  # arrays of odd lengths across the chunks' borders
+    ([512, 256, 16], 600), ([1021, 2053, 7], 40),
+])
+def test_arrays_of_a_training_arrive_whole(topo, n):
+    """Weights, biases and moments there and back: a step of gradient descent at a rate of 1e-30 leaves every bit of them.  The second
+    call finds a device net and takes the edited weights along."""
+    net, _ = public_net(topo, ["tanh"] * (len(topo) - 2) + ["softmax"], 1, seed=n)
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, topo[0])).astype(np.float32)
+    T = targets_for(rng, n, topo[-1], True)
+    nc = net.contents
+    arrays = {name: np.ctypeslib.as_array(getattr(nc, name), shape=(int(nc.total_weights if name.endswith("weights") else nc.total_biases),))
+              for name in ("weights", "biases", "opt_m_weights", "opt_m_biases", "opt_v_weights", "opt_v_biases")}
+    for _ in range(2):
+        for a in arrays.values():
+            a[:] = rng.standard_normal(a.size).astype(np.float32) * np.float32(0.05)
+        want = {name: a.copy() for name, a in arrays.items()}
+        S.train(net, X, T, 1, S.STRATEGY_FULL_BATCH, S.OPTIMIZER_SGD, learning_rate=1e-30)
+        assert S.last_error()[0] == S.SPINGALETT_OK, S.last_error()
+        for name, a in arrays.items():
+            assert np.array_equal(a, want[name]), name
+    S.free_network(net)
