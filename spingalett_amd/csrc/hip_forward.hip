@@ -1258,6 +1258,18 @@ uint32_t gemm16_single_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t *kper
     return (ktiles + per - 1) / per;
 }
 
+// Whether the single-stage kernel is the better one where the 256 x 256 tiles of integer codes would be split over K: up to K = 4608,
+// and longer ones of more than two of its tiles a compute unit whose workgroups would leave most of a second round idle.  Inputs of
+// such widths took it before they ran padded (unpadded / padded on large tiles / padded here, 4104 x 1030 INT4 at 700 / 1500 / 4000
+// samples 40 / 44 / 31, 44 / 53 / 45, 88 / 112 / 91 us; 6024 x 1030 at 4000 125 / 140 / 129; tiles / here, 4104 x 2050 at 1000 70 / 55,
+// x 3000 at 2500 116 / 120; 8200 x 1500 at 2500 130 / 135; 6024 x 770 at 4000, in one round, 96 / 110).
+bool gemm16_split_wasted(uint32_t M, uint32_t N, uint32_t K, uint32_t workgroups)
+{
+    if (K <= 4608u) return true;
+    const uint64_t tiles = (uint64_t)((M + 63u) / 64u) * ((N + 63u) / 64u);
+    return K <= 8192u && tiles > 512u && 2u * ((workgroups + 255u) / 256u * 256u) >= 3u * workgroups;
+}
+
 // What the thin-operand kernel needs beyond the layer itself
 struct ThinCtx {
     const uint16_t *w16;   // [N][K] 16-bit weights (raw 16-bit formats, or FP16 codes) when N <= 64, else nullptr
@@ -1620,7 +1632,8 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
     const bool halves_ok = halves == 1 || (uint64_t)halves * M * L.N <= ctx.ws_floats;     // (checked by the caller's reserve)
     // (too few tiles and no K split, gemm16_splits: the single-stage kernel below)
     const bool shared_cu = halves == 1 && bm == 256u && L.K <= gemm16_shared_limit(FMT, L.act, big_tiles, (uint64_t)M * L.N);
-    if (aligned && !shared_cu && L.K >= 128u && M > 64 && L.N >= 256 && fits32 && (big_tiles >= 192u || split_ok) && halves_ok) {
+    const bool wasted = ctx.padded_in && fmt_bits(FMT) < 16 && splits > 1u && gemm16_split_wasted(M, L.N, L.K, big_tiles * splits);
+    if (aligned && !shared_cu && !wasted && L.K >= 128u && M > 64 && L.N >= 256 && fits32 && (big_tiles >= 192u || split_ok) && halves_ok) {
         if (big_tiles >= 192u) g.kper = 0;
         else g.ksplits = splits;
         if (g.kper || halves == 2) g.ws = ctx.ws;

@@ -1904,6 +1904,20 @@ def test_shorter_sums_of_few_outputs_take_no_longer(S):
     assert us[4096] <= 1.05 * us[6144]
 
 
+def test_padded_integer_inputs_take_no_longer_than_unpadded_ones(S):
+    """700 to 4000 samples of 4104 INT4 codes into 1030 outputs, which run padded, against 4088 codes of the kernel of one stage (on
+    large tiles split over K 1.2 to 1.3 times as long; now even)."""
+    us = {}
+    for K in (4088, 4104):
+        net, _, _ = _decoded_layer(S, "i4", 1030, K, seed=K)
+        for n in (700, 1500, 4000):
+            assert S.lib().sphip_layer_kernel_name(net.h, 1, n, 0).decode() == "sp_gemm16"
+            us[K, n] = min(S.time_layer([net], 1, n, 50) for _ in range(5))
+        net.destroy()
+    for n in (700, 1500, 4000):
+        assert us[4104, n] <= 1.12 * us[4088, n], n
+
+
 def _fp32_layer(S, N, K, seed):
     rng = np.random.default_rng(seed)
     W, b = (rng.standard_normal((N, K)) * 0.05).astype(F32), (rng.standard_normal(N) * 0.1).astype(F32)
