@@ -272,9 +272,12 @@ __global__ __launch_bounds__(256) void sp_softmax_rows(const float *__restrict__
 // logits.  NWV waves to a row, 4 PER values a thread, all in registers.  Written by the reduction and read again by a launch of its
 // own, the logits of a split layer cost 4 us, and a wave alone with a row of more than 1024 walks it value by value (whole
 // nets, before -> with it, us: 4096 x 1000 INT4 at 16 / 64 samples 15.6 / 18.2 -> 12.1 / 14.5, FP32 at 64 20.2 -> 16.8, 8192 x 4000
-// FP16 at 16 / 600 60.7 / 116 -> 26.4 / 79.8).  A wave to a row up to 256 outputs, with which four waves have nothing to do (1500 x
-// 100 FP32 at 2000 samples 26.4 before, 28.5 with four, 23.5 with one).  Finished logits take it beyond 1024 outputs: 512 x 3000 FP16 at
-// 1 / 64 / 8192 samples 27.8 / 40.5 / 124 -> 8.7 / 12.2 / 97.
+// FP16 at 600 116 -> 79.8).  A wave to a row up to 256 outputs, with which four waves have nothing to do (1500 x 100 FP32 at 2000 samples
+// 26.4 before, 28.5 with four, 23.5 with one), and of many rows up to 768 (64 x 400 INT2 with split activations at 8192 samples 31.5,
+// with four 36.2; x 513 36.7 and 40.1, at 2000 19.1 and 18.3; x 1000 at 4000 35.0 and 31.2).  A thread's place for 64 values where 20
+// are needed costs registers and a sixth of the time (64 x 4097 FP16 at 8192 samples 130 before, 253 with 64 of them all gone
+// through, 117 without those beyond the row, 106 with 32).  Finished logits take it beyond 1024 outputs: 512 x 3000 FP16 at 1 / 64 /
+// 8192 samples 27.8 / 40.5 / 124 -> 8.7 / 12.2 / 97.
 struct SoftSums {
     const float *ws;
     uint32_t splits, parts, rows, N;
@@ -285,6 +288,12 @@ struct SoftSums {
 };
 constexpr uint32_t kSoftSumsMost = 16384u;
 
+// Whether a layer's partial sums meet in this launch: beyond 1024 outputs, a few rows' workgroups would add the parts of a row one
+// after the other (added by a reduction of their own, which spreads them over the chip, and here, us: 8192 x 4097 FP16 at 16 / 64 / 256
+// samples 27.7 / 33.4 / 63.1 and 33.3 / 39.0 / 66.7, 8192 x 2000 INT2 with split activations at 16 23.4 and 27.1, 2048 x 6000 at 16 /
+// 3000 23.3 / 256 and 30.8 / 234).
+bool soft_sums_pay(uint32_t rows, uint32_t N) { return N <= 1024u || (N <= kSoftSumsMost && rows >= 512u); }
+
 template <int PER, bool VEC, int NWV>
 __global__ __launch_bounds__(256) void sp_sum_softmax(const SoftSums a)
 {
@@ -294,11 +303,14 @@ __global__ __launch_bounds__(256) void sp_sum_softmax(const SoftSums a)
     if (row >= a.rows) return;                             // (whole waves; NWV == 4: none)
     const uint64_t total = (uint64_t)a.rows * N, first = (uint64_t)row * N;
     float v[PER][4], top = -3.402823466e+38f, sum = 0.0f;
-    // value e of group g: outputs 4 (t + T g) + e, or t + T (4 g + e) where rows are not whole float4s
+    // value e of group g: outputs 4 (t + T g) + e, or t + T (4 g + e) where rows are not whole float4s; groups beyond the row are
+    // left out (uniform)
     constexpr uint32_t T = 64u * NWV;
     auto at = [&](int g, int e) { return VEC ? 4u * (t + T * g) + e : t + T * (4u * g + e); };
+    auto live = [&](int g) { return 4u * T * g < N; };
 #pragma unroll
     for (int g = 0; g < PER; ++g) {
+        if (!live(g)) continue;
         float low[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if constexpr (VEC) {
             const uint32_t n = at(g, 0);
@@ -309,12 +321,21 @@ __global__ __launch_bounds__(256) void sp_sum_softmax(const SoftSums a)
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[g][e] = 0.0f;
-            for (uint32_t p = 0; p < a.parts; ++p) {
-                float x[4];
+            const float *src[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = a.ws[p * total + first + (at(g, e) < N ? at(g, e) : 0u)];
+            for (int e = 0; e < 4; ++e) src[e] = a.ws + first + (at(g, e) < N ? at(g, e) : 0u);
+            for (uint32_t p0 = 0; p0 < a.parts; p0 += 4u) {              // (four parts on their way, as add_parts)
+                float x[4][4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) (p < a.splits ? v[g][e] : low[e]) += x[e];
+                for (uint32_t i = 0; i < 4u; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[i][e] = src[e][(p0 + i < a.parts ? p0 + i : p0) * total];
+#pragma unroll
+                for (uint32_t i = 0; i < 4u; ++i) {
+                    if (p0 + i >= a.parts) continue;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) (p0 + i < a.splits ? v[g][e] : low[e]) += x[i][e];
+                }
             }
         }
 #pragma unroll
@@ -335,12 +356,14 @@ __global__ __launch_bounds__(256) void sp_sum_softmax(const SoftSums a)
         top = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     }
 #pragma unroll
-    for (int g = 0; g < PER; ++g)
+    for (int g = 0; g < PER; ++g) {
+        if (!live(g)) continue;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             v[g][e] = at(g, e) < N ? expf(v[g][e] - top) : 0.0f;
             sum += v[g][e];
         }
+    }
     sum = wave_sum(sum);
     if constexpr (NWV == 4) {
         if ((t & 63u) == 0) red[1][t >> 6] = sum;
@@ -349,7 +372,8 @@ __global__ __launch_bounds__(256) void sp_sum_softmax(const SoftSums a)
     }
     const float inv = sum > 0.0f ? 1.0f / sum : 1.0f;
 #pragma unroll
-    for (int g = 0; g < PER; ++g)
+    for (int g = 0; g < PER; ++g) {
+        if (!live(g)) continue;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const uint32_t n = at(g, e);
@@ -369,6 +393,7 @@ __global__ __launch_bounds__(256) void sp_sum_softmax(const SoftSums a)
                 reinterpret_cast<uint16_t *>(a.out)[total + o] = lo;
             }
         }
+    }
 }
 
 void launch_sum_softmax(const SoftSums &a)
@@ -382,8 +407,11 @@ void launch_sum_softmax(const SoftSums &a)
     };
     using std::integral_constant;
     if (a.N <= 256u) go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+    else if (a.N <= 512u && a.rows >= 2048u) go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    else if (a.N <= 768u && a.rows >= 4096u) go(integral_constant<int, 3>{}, integral_constant<int, 1>{});
     else if (a.N <= 1024u) go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
     else if (a.N <= 4096u) go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    else if (a.N <= 8192u) go(integral_constant<int, 8>{}, integral_constant<int, 4>{});
     else go(integral_constant<int, 16>{}, integral_constant<int, 4>{});
 }
 
@@ -1609,7 +1637,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
             a.thin = ctx.w16;
             launch_thin<F16T ? F16 : BF16, F16T>(a, tp);
         } else {
-            if (ctx.soft_out && (tp.splits > 1 || halves == 2) && L.N <= kSoftSumsMost) {
+            if (ctx.soft_out && (tp.splits > 1 || halves == 2) && soft_sums_pay(M, L.N)) {
                 a.soft_out = ctx.soft_out;
                 a.soft_kind = ctx.soft_kind;
                 *ctx.soft_done = true;
@@ -1621,7 +1649,7 @@ void launch_gemm16_fmt(const LayerArgs &L, const uint16_t *A, void *C, uint32_t 
         return;
     }
     GemmArgs g{L, A, C, M, out_f32, nullptr, 0, 1, halves};
-    const bool soft_sums = ctx.soft_out && L.N <= kSoftSumsMost;          // if there are partial sums
+    const bool soft_sums = ctx.soft_out && soft_sums_pay(M, L.N);          // if there are partial sums
     const bool aligned = rows_aligned(FMT, L.K) && (L.K % 8u == 0);
     const bool fits32 = (uint64_t)M * L.K * 2u < (1ull << 32) && (uint64_t)L.N * L.K * 2u < (1ull << 32);   // 32-bit DMA offsets
     // the 256 x 256 tiles need about a tile per compute unit; smaller problems fill the chip better with 128 x 128
@@ -1909,7 +1937,7 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
         b.M = M; b.N = L.N; b.K = L.K;
         b.bias = L.bias; b.bscale = L.bscale; b.bias_fmt = L.bias_fmt; b.act = L.act;
         launch_gemm32_parts(b, parts, rows64);
-        if (parts > 1 && soft_out && L.N <= kSoftSumsMost) {
+        if (parts > 1 && soft_out && soft_sums_pay(M, L.N)) {
             launch_sum_softmax({ws, parts, parts, M, L.N, L, soft_out, 0, 0});
             return true;
         }
@@ -1961,7 +1989,7 @@ bool launch_gemm32(const LayerArgs &L, const float *A, float *C, uint32_t M, flo
         sp_gemm32_reduce_softmax<<<(M + 15u) / 16u, 256, 0, g_stream>>>(g, splits, soft_out);
         return true;
     }
-    if (splits > 1 && soft_out && !training && L.N <= kSoftSumsMost) {     // (training keeps the order of its sums)
+    if (splits > 1 && soft_out && !training && soft_sums_pay(M, L.N)) {     // (training keeps the order of its sums)
         launch_sum_softmax({ws, splits, splits, M, L.N, L, soft_out, 0, 0});
         return true;
     }

@@ -659,6 +659,38 @@ def test_softmax_of_split_sums_and_of_wide_rows(S, O, fmt, mode, n, topo, acts):
         assert np.abs(got.astype(np.float64).sum(axis=1) - 1).max() <= 1e-5
 
 
+@pytest.mark.parametrize("fmt,mode,n,topo,acts", [
+    ("f16", "split", 2048, [64, 512], ["softmax"]), ("i2", "split", 2049, [72, 258], ["softmax"]),           # a wave to a row of
+    ("i4", "split", 4096, [64, 513], ["softmax"]), ("bf16", "split", 4099, [64, 768], ["softmax"]),          # up to 768, and
+    ("i8", "split", 4097, [64, 769], ["softmax"]), ("f32", "plain", 2100, [300, 401], ["softmax"]),          # just not
+    ("i2", "split", 512, [1024, 1025], ["softmax"]), ("f16", "split", 511, [1024, 2051], ["softmax"]),       # with the parts, and not
+    ("i8", "split", 600, [256, 8192], ["softmax"]), ("f16", "plain", 513, [64, 8191], ["softmax"]), ("bf16", "plain", 70, [64, 8193], ["softmax"]),
+    ("i4", "split", 520, [256, 5001, 9], ["softmax", "none"]),
+])
+def test_softmax_rows_at_the_lines_between_their_kernels(S, O, fmt, mode, n, topo, acts):
+    """sp_sum_softmax's instances at both sides of the lines between them, as above."""
+    test_softmax_of_split_sums_and_of_wide_rows(S, O, fmt, mode, n, topo, acts)
+
+
+def test_rows_of_logits_take_no_longer_past_a_border(S):
+    """8192 rows of 4097 logits against 4096 (every thread went through 64 places for 17 values: 2.4 times as long; now 1.2)."""
+    n, us = 8192, {}
+    for N in (4096, 4097):
+        net = S.DeviceNet([64, N], [S.ACT_SOFTMAX], S.PRECISION_FP16)
+        net.upload(0, 0, np.zeros(64 * N, np.uint16))
+        net.upload(0, 1, np.zeros(N, np.uint16))
+        d_x, d_y = S.DeviceBuffer.from_numpy(np.zeros((n, 64), F32)), S.DeviceBuffer(n * N * 4)
+        us[N] = np.inf
+        for _ in range(6):
+            start = time.perf_counter()
+            for _ in range(20):
+                net.forward_device(d_x, n, d_y)
+            S.synchronize()
+            us[N] = min(us[N], time.perf_counter() - start)
+        net.destroy()
+    assert us[4097] <= 1.6 * us[4096]
+
+
 @pytest.mark.parametrize("fmt", ["f16", "bf16", "i8", "i4", "i2"])
 @pytest.mark.parametrize("K,N", [(1279, 70), (1283, 70), (4095, 65), (4097, 65), (4999, 129), (5002, 300), (5003, 64), (9002, 1100), (7297, 901)])
 def test_few_samples_of_rows_that_are_no_whole_words(S, O, fmt, K, N):
