@@ -16,19 +16,21 @@ constexpr size_t kStageChunk = 8u << 20, kFirstChunk = 512u << 10, kStagePart = 
 // 408 / 739 here; 2 MB down 107 against 96, for which the ring is not worth its pinned memory).
 constexpr size_t kStagedUp = 10u << 20, kStagedDown = 4u << 20, kHelperLeast = 1u << 20;
 constexpr uint32_t kStageSlots = 4, kStageHelpers = 3, kIdleLooks = 1000;
-constexpr uint32_t kInFlight = 8;              // chunks in the slots at once: seven at most (slot_of)
+constexpr uint32_t kInFlight = 8;              // chunks in the slots at once: six at most (slot_of)
 
 // One ring for each direction: a download holds its own until all before it on the stream is done, which must not keep another
-// thread's upload from filling chunks.
+// thread's upload from filling chunks.  Three slots up: with a fourth, the slots and an array that is sent again and again no longer
+// fit the host's cache together (32 MB 870 us, 805 with three; new arrays 751 and 750).
 struct StageRing {
     const size_t chunk;                            // the longest
+    const uint32_t slots;                          // kStageSlots at most
     void *buf[kStageSlots] = {};
     hipEvent_t ev[kStageSlots] = {}, start = nullptr;
     hipStream_t side = nullptr;                    // (with start: up only)
     bool ready = false;
     std::mutex mu;
-    explicit StageRing(size_t bytes) : chunk(bytes) {}
-} g_up{kStageChunk}, g_down{4u * kFirstChunk};
+    StageRing(size_t bytes, uint32_t count) : chunk(bytes), slots(count) {}
+} g_up{kStageChunk, 3u}, g_down{4u * kFirstChunk, 4u};
 
 // a contiguous part of a transfer; a transfer is its segments in a row, each beginning at a multiple of 64 bytes of it
 struct Segment {
@@ -101,8 +103,8 @@ private:
     size_t chunk_end(uint32_t c) const { return std::min(chunk_at(c + 1u), total_); }
 
     // The slot a chunk lies in, and whether it is the first one there.  Up: the four that make 8 MB share one, so that the slots hold
-    // 32 MB of a transfer that has to wait for the stream, and the call need not.
-    uint32_t slot_of(uint32_t c) const { return (to_host_ ? c : c < 4u ? 0u : c - 3u) % kStageSlots; }
+    // 24 MB of a transfer that has to wait for the stream, and the call need not.
+    uint32_t slot_of(uint32_t c) const { return (to_host_ ? c : c < 4u ? 0u : c - 3u) % ring_.slots; }
     bool begins_slot(uint32_t c) const { return to_host_ || c == 0u || c >= 4u; }
     char *chunk_pin(uint32_t c) const { return static_cast<char *>(ring_.buf[slot_of(c)]) + (begins_slot(c) ? 0u : chunk_at(c)); }
 
@@ -213,7 +215,7 @@ private:
         while (to_host_ ? freed < chunks_ : sent < chunks_) {
             bool moved = false;
             if (to_host_) {
-                for (; sent < chunks_ && sent < freed + kStageSlots; ++sent, moved = true) {
+                for (; sent < chunks_ && sent < freed + ring_.slots; ++sent, moved = true) {
                     done_[sent % kInFlight].store(0u, std::memory_order_relaxed);
                     if (submit(sent, stream)) return 1;
                 }
@@ -228,7 +230,7 @@ private:
                 for (; freed < open && copied(freed); moved = true) ++freed;
             } else {
                 // (a slot's last transfer may be one of the call before)
-                for (; open < chunks_ && (open < 3u + kStageSlots || open < sent + kStageSlots); moved = true) {
+                for (; open < chunks_ && (open < 3u + ring_.slots || open < sent + ring_.slots); moved = true) {
                     const int busy = begins_slot(open) ? slot_busy(slot_of(open)) : 0;
                     if (busy < 0) return 1;
                     if (busy) break;
@@ -271,7 +273,7 @@ private:
 int ring_ready(StageRing &r)
 {
     if (r.ready) return 0;
-    for (uint32_t i = 0; i < kStageSlots; ++i) {
+    for (uint32_t i = 0; i < r.slots; ++i) {
         if (!r.buf[i]) HCHECK(hipHostMalloc(&r.buf[i], r.chunk, hipHostMallocDefault));
         if (!r.ev[i]) HCHECK(hipEventCreateWithFlags(&r.ev[i], hipEventDisableTiming));
     }
