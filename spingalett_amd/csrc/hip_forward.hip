@@ -1305,7 +1305,7 @@ struct ThinCtx {
     uint64_t ws_floats;
     bool x_f32;            // A is still the caller's FP32 input (the layer is one gemm16_small_layer() accepts)
     void *soft_out;        // softmax layer: where the normalised outputs go if the layer's kernel can do it itself ...
-    int soft_kind;         // ... as 0 FP32, 1 BF16, 2 FP16
+    int soft_kind;         // ... as 0 FP32, 1 BF16, 2 FP16, 3 FP16 in two halves (not by sp_skinny16_kw_head, which has no place for the second)
     bool *soft_done;       // ... and whether it did
     bool padded_in;        // the first layer, with the caller's rows padded (padded_width)
 };

@@ -27,8 +27,10 @@ struct SkinnyArgs {
     uint32_t kper;           // codes per K split (whole chunks)
     int out_f32;
     int mode_b;              // 0: streamed rows are outputs, thin rows samples; 1: the reverse
-    void *soft_out;          // sp_skinny16_kw_head without a K split: softmax over a sample's outputs goes here instead of C
-    int soft_kind;           // its element type: 0 FP32, 1 BF16, 2 FP16
+    // Softmax over a sample's outputs goes here instead of C: by sp_skinny16_kw_head itself where K is not split, by sp_sum_softmax
+    // with the addition of the parts behind streamed weights (launch_thin)
+    void *soft_out;
+    int soft_kind;           // its element type: 0 FP32, 1 BF16, 2 FP16, 3 FP16 in two halves (sp_sum_softmax only)
     // Split activations (GemmArgs has the layout): grid y = halves x ksplits, y / ksplits picks the activation matrix
     // (the thin operand, or the streamed one in mode b), y % ksplits the K range.
     uint32_t ksplits;        // K splits (>= 1)

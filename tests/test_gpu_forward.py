@@ -1396,8 +1396,9 @@ def test_seeded_random_layer_shapes(S, fmt, N, K, n):
 
 
 def test_large_host_input_goes_up_in_chunks(S):
-    """Host inputs of 16 MB and more are uploaded through a ring of pinned 8 MB chunks filled by several threads;
-    sizes that are no multiple of a chunk, twice in a row (the ring is reused), against FP64 on every row."""
+    """Host inputs of 10 MB and more are uploaded through a ring of pinned chunks, of 0.5 to 4.5 MB up to the eighth megabyte and of 8
+    from there, filled by several threads, and from 16 MB on the layers of the rows that have landed run beside the rest; sizes
+    that are no multiple of a chunk, twice in a row (the ring is reused), against FP64 on every row."""
     net, W, b = _decoded_layer(S, "bf16", 16, 1030, seed=77)
     for n in (5000, 4200):                                  # 20.6 MB and 17.3 MB
         X = np.random.default_rng(n).standard_normal((n, 1030)).astype(F32)
